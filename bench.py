@@ -143,8 +143,8 @@ def bench_chem(api, problems, torch, n, seed, steps, h=1e3):
     p_ms, p_st = run(True, max(2, steps // 2))
     assert b_st["newton_iters"] == p_st["newton_iters"] and b_st["hist"] == p_st["hist"]
     rhs_fl, jac_fl, rhs_trans = CHEM_RHS_FLOPS, CHEM_JAC_FLOPS, CHEM_RHS_TRANSCENDENTALS
-    # RHS evaluations: one per Newton iteration plus one before each Jacobian setup
-    nrhs = b_st["newton_iters"] + b_st["setups"]
+    # RHS evaluations: one per Newton iteration (a step's Jacobian setup uses its first)
+    nrhs = b_st["newton_iters"]
     lu_fl = 2 * 10 ** 3 // 3 + 10 ** 2            # factor, per setup (approx.)
     solve_fl = 2 * 10 ** 2                        # triangular solves, per iteration
     flops = nrhs * rhs_fl + b_st["setups"] * (jac_fl + lu_fl) + b_st["newton_iters"] * solve_fl

@@ -391,20 +391,21 @@ int mvd_chem_dirk_tune(mvd_context *ctx, double h, const mvd_dirk_opts *o, const
 /* Set the batched kernel's launch shape by hand (what mvd_chem_dirk_tune chooses): block
  * threads per block (64, 128 or 256; blocks whose LDS would not fit a CU are split at
  * launch) and waves resident waves of the persistent grid (0: one per SIMD of the device).
- * Each wave takes 64-cell chunks, the first by its index and the rest from the work queue,
- * so waves smaller than the number of chunks exercises the queue. The results do not
+ * Each wave takes chunks of up to 64 cells (as few turns per wave as that allows, of even
+ * size), the first by its index and the rest from the work queue, so waves smaller than the
+ * number of 64-cell chunks exercises the queue. The results do not
  * depend on the shape. get_shape returns the shape the next launch uses (waves resolved). */
 int mvd_chem_dirk_set_shape(mvd_context *ctx, int block, int waves);
 /* The block split of a batched launch (no GPU needed; diagnostics and tests): the threads
  * per block a launch asked for `block` threads runs with for an nstage-stage table, when the
  * kernel's static LDS is static_lds bytes and the device allows lds_limit bytes per block
- * (the launch asks the runtime for both). The dynamic LDS is 8 * (4*1024 + waves * (24 +
- * 10*nstage) * 64) bytes: the gamma tables, then per wave its cells' constants, the stage
- * derivatives of the earlier stages and the step start; for tables of more than four stages
- * (and explicit-first-stage tables, which this call does not see) the stage derivatives go
- * to a device buffer of 80 * (nstage - 1) bytes per thread of the persistent grid instead,
- * 8 * (4*1024 + waves * 34 * 64) bytes of LDS. Halves the block until it fits; 0 when not
- * even one wave fits. */
+ * (the launch asks the runtime for both). The dynamic LDS is 8 * (4*1024 + waves * words *
+ * 64) bytes: the gamma tables, then per wave its cells' constants, the step start and the
+ * work slots (stage derivatives, stage right-hand side, a correction); words = 54 up to
+ * three stages and 64 with four; for tables of more than four stages (and
+ * explicit-first-stage tables, which this call does not see) 54, the stage derivatives
+ * going to a device buffer of 80 * (nstage - 1) bytes per thread of the persistent grid
+ * instead. Halves the block until it fits; 0 when not even one wave fits. */
 int mvd_chem_dirk_fit_block(int block, int nstage, long static_lds, long lds_limit);
 int mvd_chem_dirk_get_shape(mvd_context *ctx, int *block, int *waves);
 

@@ -1,15 +1,14 @@
 // One diagonally implicit RK step of the per-cell primordial chemistry (the fast implicit
 // stage of the reacting-flow demo), two ways:
 //
-//   batched  - one persistent launch. Each wave pulls 64-cell chunks from an atomic work
-//              queue (work stealing across waves and CUs: cells need 3 to 9+ Newton
+//   batched  - one persistent launch. Each wave pulls chunks of up to 64 cells from an atomic
+//              work queue (work stealing across waves and CUs: cells need 3 to 9+ Newton
 //              iterations) and each lane runs all stages and Newton iterations of its cell:
 //              RHS with the temperature solve, analytic Jacobian, M = I - h a_ii s J, 10x10
 //              LU with partial pivoting, triangular solves, WRMS convergence test, re-setup
-//              after max_iters. The iterate, the stage right-hand side and the LU factors
-//              stay in the register file for the whole step (one wave per SIMD: 512 VGPR +
-//              AGPR); only the stage derivatives, read once per stage, go to a per-chunk
-//              scratch block. Statistics are accumulated per block in LDS.
+//              after max_iters. The iterate and the LU factors stay in the register file for
+//              the whole step (one wave per SIMD: 512 VGPR + AGPR); what is read once per
+//              pass or stage is in LDS. Statistics are accumulated per block in LDS.
 //   plain    - the reference's structure (primordial_ode_main.cpp with SUNDIALS + MAGMA):
 //              one-thread-per-cell kernels for the RHS, the Jacobian into column-major 10x10
 //              blocks, the batched LU factorisation, and the Newton update with the
@@ -17,8 +16,9 @@
 //              round trip per Newton iteration to test convergence.
 //
 // Both follow the same per-cell algorithm (stage predictor, modified Newton with the
-// Jacobian from y_n, re-setup after max_iters) and the same operation order, so they agree
-// with each other bitwise and with the CPU oracle iteration for iteration.
+// Jacobian from y_n, whose RHS evaluation is also the first iteration's, re-setup after
+// max_iters) and share their arithmetic, so they agree with each other bitwise and with the
+// CPU oracle iteration for iteration.
 #include <mutex>
 #include "mvd_chem.hpp"
 #include "mvd_dirk.hpp"
@@ -49,7 +49,7 @@ template <bool PAIRS = false>
 __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
                                 double &Ts, double &dTs, const double (&y)[NSP], double srhs,
                                 double (&f)[NSP], bool solve_t = true) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double ya[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = y[s] * c.s(s);
@@ -79,55 +79,17 @@ __device__ inline void cell_rhs(const ChemConst &cc, const CellIn &c, double &Ts
   cell_rhs<PAIRS>(cc, gamma_tabs(cc), c, Ts, dTs, y, srhs, f);
 }
 
-// A cell's 10x10 matrix in memory: element (r, c) at b[r*rs + c*cs]. The batched solver
-// uses its element-major chunk block (rs = 640, cs = 64); the plain solver the reference's
-// column-major blocks (rs = 1, cs = 10).
-struct Mat {
-  double *b;
-  long rs, cs;
-  __device__ double &operator()(int r, int c) const { return b[r * rs + c * cs]; }
-};
-
-// M = I - hg * srhs * J(y), J = calculate_jacobian_cvklu from the current temperature.
-// The species rows (reaction tables) are formed and stored before the gas-energy row
-// (cooling tables) is evaluated; the fence keeps the two groups of table loads apart so that
-// both never occupy registers at once.
-__device__ inline void cell_matrix(const ChemConst &cc, const CellIn &c, double Ts, double dTs,
-                                   const double (&y)[NSP], double hg, double srhs,
-                                   const Mat &m) {
-#pragma clang fp contract(off)
-  double ya[NSP];
-#pragma unroll
-  for (int s = 0; s < NSP; s++) ya[s] = y[s] * c.s(s);
-  double k[NRATE], dk[NRATE], J[NSP][NSP];
-#pragma unroll
-  for (int r = 0; r < NRATE; r++) k[r] = dk[r] = 0.0;
-#pragma unroll
-  for (int r = 0; r < NSP; r++)
-#pragma unroll
-    for (int q = 0; q < NSP; q++) J[r][q] = 0.0;
-  chem_rates_range<0, C_BREM>(cc, Ts, k, dk);
-  chem_jac_species(ya, k, dk, dTs, J);
-#pragma unroll
-  for (int r = 0; r < NSP - 1; r++)
-#pragma unroll
-    for (int q = 0; q < NSP; q++)
-      m(r, q) = (r == q ? 1.0 : 0.0) - hg * (srhs * (J[r][q] * (c.is(r) * c.s(q))));
-  __asm__ volatile("" ::: "memory");
-  chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
-  chem_jac_energy(ya, k, dk, Ts, cc.z, dTs, c.ax, J);
-#pragma unroll
-  for (int q = 0; q < NSP; q++)
-    m(NSP - 1, q) = (NSP - 1 == q ? 1.0 : 0.0) -
-                    hg * (srhs * (J[NSP - 1][q] * (c.is(NSP - 1) * c.s(q))));
-}
-
 // Packed pivots of a factorisation without row exchanges (pivot k at step k).
 constexpr unsigned long long PIV_IDENTITY = 0x9876543210ULL;
 
 // LU with partial pivoting (first maximum wins, LAPACK getrf row interchanges) with the
 // whole matrix in registers (right-looking, predicated row exchanges so that the runtime
-// pivot never indexes a register array). Returns the pivots packed 4 bits each.
+// pivot never indexes a register array; a column in which no lane of the wave pivots skips
+// them, 1800 selects in all). Returns the pivots packed 4 bits each.
+// INVD (the Newton solvers' form): FMA updates, fast_rcp pivots, and the diagonal of U left
+// as its reciprocals for lu_solve_regs. Without it: LAPACK's separate products and IEEE
+// reciprocals, which meet an exact zero pivot (a singular block) as its getrf would.
+template <bool INVD>
 __device__ inline unsigned long long lu_factor_regs(double (&a)[NSP][NSP]) {
 #pragma clang fp contract(off)
   unsigned long long pv = 0;
@@ -141,30 +103,34 @@ __device__ inline unsigned long long lu_factor_regs(double (&a)[NSP][NSP]) {
       if (v > best) { best = v; p = r; }
     }
     pv |= (unsigned long long)p << (4 * k);
+    if (p != k) {
 #pragma unroll
-    for (int r = k + 1; r < NSP; r++) {
-      const bool sw = (r == p);
+      for (int r = k + 1; r < NSP; r++) {
+        const bool sw = (r == p);
 #pragma unroll
-      for (int q = 0; q < NSP; q++) {
-        const double x = a[k][q], y = a[r][q];
-        a[k][q] = sw ? y : x;
-        a[r][q] = sw ? x : y;
+        for (int q = 0; q < NSP; q++) {
+          const double x = a[k][q], y = a[r][q];
+          a[k][q] = sw ? y : x;
+          a[r][q] = sw ? x : y;
+        }
       }
     }
-    const double ik = 1.0 / a[k][k];
+    const double ik = INVD ? fast_rcp(a[k][k]) : 1.0 / a[k][k];
 #pragma unroll
     for (int r = k + 1; r < NSP; r++) {
       const double l = a[r][k] * ik;
       a[r][k] = l;
 #pragma unroll
-      for (int q = k + 1; q < NSP; q++) a[r][q] -= l * a[k][q];
+      for (int q = k + 1; q < NSP; q++)
+        a[r][q] = INVD ? fma(-l, a[k][q], a[r][q]) : a[r][q] - l * a[k][q];
     }
+    if (INVD) a[k][k] = ik;
   }
   return pv;
 }
 
-__device__ inline void lu_solve(const Mat &a, unsigned long long pv, double (&b)[NSP]) {
-#pragma clang fp contract(off)
+// b's rows exchanged as the factorisation exchanged the matrix's
+__device__ inline void lu_exchange(unsigned long long pv, double (&b)[NSP]) {
 #pragma unroll
   for (int k = 0; k < NSP; k++) {
     const int p = (int)((pv >> (4 * k)) & 15);
@@ -176,28 +142,18 @@ __device__ inline void lu_solve(const Mat &a, unsigned long long pv, double (&b)
       b[r] = sw ? bk : br;
     }
   }
-#pragma unroll
-  for (int r = 1; r < NSP; r++)
-#pragma unroll
-    for (int q = 0; q < r; q++) b[r] -= a(r, q) * b[q];
-#pragma unroll
-  for (int r = NSP - 1; r >= 0; r--) {
-#pragma unroll
-    for (int q = r + 1; q < NSP; q++) b[r] -= a(r, q) * b[q];
-    b[r] /= a(r, r);
-  }
 }
 
 __device__ inline double wrms_norm(const double (&d)[NSP], const double (&z)[NSP],
                                    double rtol, double atol) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double s = 0.0;
 #pragma unroll
   for (int k = 0; k < NSP; k++) {
-    const double w = d[k] / (rtol * fabs(z[k]) + atol);
+    const double w = d[k] * fast_rcp(rtol * fabs(z[k]) + atol);
     s += w * w;
   }
-  return sqrt(s / NSP);
+  return sqrt(s * (1.0 / NSP));
 }
 
 // ARKODE's Newton convergence test (arkStep_NlsConvTest, ARKODE 5.2 / SUNDIALS 6.2.0, the
@@ -214,12 +170,12 @@ __device__ inline double conv_rate(double crate, double del, double delp) {
 }
 
 __device__ inline bool conv_ok(double crate, double del, double tol) {
-#pragma clang fp contract(off)
-  return (crate < 1.0 ? crate : 1.0) * del / tol <= 1.0;
+#pragma clang fp contract(on)
+  return (crate < 1.0 ? crate : 1.0) * del <= tol;
 }
 
 __device__ inline bool conv_diverging(double del, double delp) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   return del > 2.3 * delp;
 }
 
@@ -306,58 +262,59 @@ static inline unsigned stats_blocks(long nrow) {
 // batched path
 // ------------------------------------------------------------------------------------
 
-// M = I - hg * srhs * J into registers (same expressions and order as cell_matrix). The
-// rates come from the rate-major tables here: with the factors held in registers, the pair
-// table's wider loads cost this kernel spills, and it measured faster this way.
+// The structural nonzeros of the analytic Jacobian (chem_jac_species, chem_jac_energy).
+__device__ constexpr bool CHEM_JNZ[NSP][NSP] = {
+    {1, 1, 1, 1, 1, 0, 0, 0, 1, 1}, {1, 1, 1, 1, 1, 0, 0, 0, 1, 1}, {1, 1, 1, 1, 1, 0, 0, 0, 1, 1},
+    {1, 1, 1, 1, 1, 0, 0, 0, 1, 1}, {0, 1, 1, 1, 1, 0, 0, 0, 1, 1}, {0, 0, 0, 0, 0, 1, 1, 0, 1, 1},
+    {0, 0, 0, 0, 0, 1, 1, 1, 1, 1}, {0, 0, 0, 0, 0, 0, 1, 1, 1, 1}, {0, 1, 1, 1, 1, 1, 1, 1, 1, 1},
+    {1, 0, 1, 1, 0, 1, 1, 1, 1, 1}};
+
+// M = I - hg * srhs * J into registers, J = calculate_jacobian_cvklu from the current
+// temperature: the species rows (reaction tables), then the gas-energy row (cooling tables),
+// so that both groups of rates never occupy registers at once. The rates come from the
+// rate-major tables here: with the factors held in registers, the pair table's wider loads
+// cost the batched kernel spills, and it measured faster this way.
 __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, double Ts,
                                         double dTs, const double (&y)[NSP], double hg,
                                         double srhs, double (&M)[NSP][NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double ya[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = y[s] * c.s(s);
   double k[NRATE], dk[NRATE];
 #pragma unroll
   for (int r = 0; r < NRATE; r++) k[r] = dk[r] = 0.0;
-#pragma unroll
-  for (int r = 0; r < NSP; r++)
-#pragma unroll
-    for (int q = 0; q < NSP; q++) M[r][q] = 0.0;
+  const double hs = hg * srhs;
   chem_rates_range<0, C_BREM>(cc, Ts, k, dk);
   chem_jac_species(ya, k, dk, dTs, M);
 #pragma unroll
-  for (int r = 0; r < NSP - 1; r++)
+  for (int r = 0; r < NSP - 1; r++) {
+    const double row = hs * c.is(r);
 #pragma unroll
-    for (int q = 0; q < NSP; q++)
-      M[r][q] = (r == q ? 1.0 : 0.0) - hg * (srhs * (M[r][q] * (c.is(r) * c.s(q))));
-  chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
-  chem_jac_energy(ya, k, dk, Ts, cc.z, dTs, c.ax, M);
-#pragma unroll
-  for (int q = 0; q < NSP; q++)
-    M[NSP - 1][q] = (NSP - 1 == q ? 1.0 : 0.0) -
-                    hg * (srhs * (M[NSP - 1][q] * (c.is(NSP - 1) * c.s(q))));
-}
-
-// Solve with the factors of lu_factor_regs. The row exchanges are applied only when some
-// lane of the wave pivoted: for I - h*gamma*J of the stiff network the diagonal is the
-// column maximum in nearly every cell and step, and applying the packed pivots costs 180
-// selects per solve.
-__device__ inline void lu_solve_regs(const double (&a)[NSP][NSP], unsigned long long pv,
-                                     double (&b)[NSP]) {
-#pragma clang fp contract(off)
-  if (__builtin_amdgcn_ballot_w64(pv != PIV_IDENTITY) != 0) {   // wave-uniform
-#pragma unroll
-    for (int k = 0; k < NSP; k++) {
-      const int p = (int)((pv >> (4 * k)) & 15);
-#pragma unroll
-      for (int r = k + 1; r < NSP; r++) {
-        const bool sw = (r == p);
-        const double bk = b[k], br = b[r];
-        b[k] = sw ? br : bk;
-        b[r] = sw ? bk : br;
-      }
+    for (int q = 0; q < NSP; q++) {
+      const double eye = r == q ? 1.0 : 0.0;
+      M[r][q] = CHEM_JNZ[r][q] ? eye - row * (M[r][q] * c.s(q)) : eye;
     }
   }
+  chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
+  chem_jac_energy(ya, k, dk, Ts, cc.z, dTs, c.ax, M);
+  const double row = hs * c.is(NSP - 1);
+#pragma unroll
+  for (int q = 0; q < NSP; q++) {
+    const double eye = NSP - 1 == q ? 1.0 : 0.0;
+    M[NSP - 1][q] = CHEM_JNZ[NSP - 1][q] ? eye - row * (M[NSP - 1][q] * c.s(q)) : eye;
+  }
+}
+
+// Solve with the factors of lu_factor_regs<true> (reciprocal diagonal). The row exchanges
+// are applied only when some lane of the wave pivoted: for I - h*gamma*J of the stiff
+// network the diagonal is the column maximum in nearly every cell and step, and applying
+// the packed pivots costs 180 selects per solve.
+__device__ inline void lu_solve_regs(const double (&a)[NSP][NSP], unsigned long long pv,
+                                     double (&b)[NSP]) {
+#pragma clang fp contract(on)
+  if (__builtin_amdgcn_ballot_w64(pv != PIV_IDENTITY) != 0)      // wave-uniform
+    lu_exchange(pv, b);
 #pragma unroll
   for (int r = 1; r < NSP; r++)
 #pragma unroll
@@ -366,23 +323,28 @@ __device__ inline void lu_solve_regs(const double (&a)[NSP][NSP], unsigned long 
   for (int r = NSP - 1; r >= 0; r--) {
 #pragma unroll
     for (int q = r + 1; q < NSP; q++) b[r] -= a[r][q] * b[q];
-    b[r] /= a[r][r];
+    b[r] *= a[r][r];
   }
 }
 
 // Per-cell values a wave keeps in LDS, element-major ([word][64 lanes]): scale, inv_scale,
-// mdensity, inv_mdensity, the two optical-depth factors, the stage derivatives F_j of the
-// first nstage - 1 stages (F_j[s] of lane l at (j*10+s)*64 + l; for the wide tables, with
-// an explicit first stage or more than FST_LDS_MAX stages, they live in a global buffer
-// instead, [(j*10+s)][thread of the grid], so that four waves still share a block) and the
-// (sub)step start y_n.
+// mdensity, inv_mdensity, the two optical-depth factors, the (sub)step start y_n, then the
+// work slots of NSP words each.
+// Narrow tables (SDIRK of up to FST_LDS_MAX stages): slot j keeps the stage derivative F_j.
+// The current stage's right-hand side r sits in the slot that the stage's own F will take
+// (the last stage, whose F is not needed: in slot 0, whose F_0 is consumed when that r is
+// formed), and the first correction of a step across its matrix set-up in slot 1, free until
+// the second stage; tables of one or two stages have two slots for these.
+// Wide tables (an explicit first stage or more than FST_LDS_MAX stages): slot 0 is r, slot 1
+// the correction, and the stage derivatives live in a global buffer, [(j*10+s)][thread of the
+// grid], so that four waves still share a block.
 constexpr int CELL_WORDS = 2 * NSP + 4;
 constexpr int FST_LDS_MAX = 4;
 __host__ __device__ inline bool dirk_wide(int nstage, bool esdirk) {
   return esdirk || nstage > FST_LDS_MAX;
 }
 __host__ __device__ inline int dirk_wave_words(int nstage, bool wide) {
-  return CELL_WORDS + (wide ? 0 : (nstage - 1) * NSP) + NSP;
+  return CELL_WORDS + NSP + (wide || nstage <= 3 ? 2 : nstage - 1) * NSP;
 }
 // dynamic LDS of the batched kernel for `wpb` waves per block
 inline size_t dirk_lds_bytes(int wpb, int nstage, bool wide) {
@@ -421,44 +383,49 @@ template <bool FORCED, bool SUBSTEP, bool WIDE>
 __global__ void __launch_bounds__(256)
 chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double *y,
                   const double *force, const int *order, const double2 *tdt, int *queue,
-                  int *rows, int nsteps, double *fglob) {
-#pragma clang fp contract(off)
+                  int *rows, int nsteps, double *fglob, int chunk) {
+#pragma clang fp contract(on)
   // block statistics in LDS (the per-cell updates are LDS atomics; one row per block).
   // Dynamic LDS: the gamma tables of the temperature solve (32 KB; the ten-step Newton loop
   // gathers from them at every step of every RHS evaluation), then per wave the values of
-  // its 64 cells (WAVE_WORDS): the constants read at every RHS evaluation, loaded from HBM
+  // its cells (dirk_wave_words): the constants read at every RHS evaluation, loaded from HBM
   // once per cell, and the stage derivatives and step start read at stage changes.
   __shared__ int bs[NSTAT];
   extern __shared__ double lds[];
   if (threadIdx.x < NSTAT) bs[threadIdx.x] = 0;
+  // the wide tables' matrix, for a stage index held per lane
+  __shared__ double tabA[WIDE ? MAXSTAGE * MAXSTAGE : 1];
+  if (WIDE && threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < MAXSTAGE * MAXSTAGE; k++) tabA[k] = o.A[k];
+  }
   for (int e = threadIdx.x; e < 4 * TLEN; e += blockDim.x) lds[e] = cc.tab[G_GH2_1 * TLEN + e];
   __syncthreads();
   const GammaTabs gt = gamma_tabs(lds);
   const int lane = threadIdx.x & 63;
   double *const cst = lds + 4 * TLEN + (threadIdx.x >> 6) * (dirk_wave_words(o.nstage, WIDE) * 64);
-  // F_j[s] at (j*10 + s) * fstr: in LDS (fstr 64), or for the wide tables in the global
-  // buffer (one column per thread of the grid)
+  double *const yst = cst + CELL_WORDS * 64 + lane;        // y_n[s] at s*64
+  double *const slots = yst + NSP * 64;                    // work slot k, element s: (10 k + s)*64
+  // F_j[s] at (j*10 + s) * fstr: in the work slots (fstr 64), or for the wide tables in the
+  // global buffer (one column per thread of the grid)
   const long fstr = WIDE ? (long)gridDim.x * blockDim.x : 64;
-  constexpr int QS = WIDE ? MAXSTAGE : FST_LDS_MAX;        // most stages of this instantiation
-  double *const Fst = WIDE ? fglob + (long)blockIdx.x * blockDim.x + threadIdx.x
-                           : cst + CELL_WORDS * 64 + lane;
-  double *const yst = cst + (CELL_WORDS + (WIDE ? 0 : (o.nstage - 1) * NSP)) * 64 + lane;  // y_n[s] at s*64
+  double *const Fst = WIDE ? fglob + (long)blockIdx.x * blockDim.x + threadIdx.x : slots;
   // The first chunk of each wave is its global wave index; later ones come from the queue
   // (which starts after them), each fetched while the previous chunk is being solved: lane
   // 0 issues the atomic after the chunk's prologue loads and the wave reads its result at
   // the end.
   const int nwaves = (int)(gridDim.x * (blockDim.x >> 6));
-  int next = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
+  int next = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * chunk;
   for (;;) {
     const int base = next;
     if ((long)base >= n) break;
     int q = 0;
-    if (SUBSTEP && lane == 0) q = atomicAdd(queue, 64) + nwaves * 64;
-    if ((long)base + lane < n) {   // lanes past the end idle to the end of the chunk
+    if (SUBSTEP && lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
+    if (lane < chunk && (long)base + lane < n) {   // the other lanes idle to the chunk's end
     // the lane's cell: queue positions run over the cells in temperature order
     const int cell = order ? order[base + lane] : base + lane;
-    // per-lane state for the whole step: iterate, stage right-hand side, LU factors
-    double Ts, dTs, Ts0, dTs0, z[NSP], r[NSP], lu[NSP][NSP];
+    // per-lane state for the whole step: iterate and LU factors
+    double Ts, dTs, Ts0, dTs0, z[NSP], lu[NSP][NSP];
     {
       const long i = cell;
       Ts0 = p.Ts[i];                                       // warm start at the substep start
@@ -472,7 +439,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
         dTs = dTs0;
       }
 #pragma unroll
-      for (int s = 0; s < NSP; s++) { z[s] = y[NSP * i + s]; r[s] = z[s] + h * 0.0; }
+      for (int s = 0; s < NSP; s++) z[s] = y[NSP * i + s];
 #pragma unroll
       for (int s = 0; s < NSP; s++) {
         yst[s * 64] = z[s];
@@ -484,25 +451,43 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
       cst[(2 * NSP + 2) * 64 + lane] = p.cie[i];
       cst[(2 * NSP + 3) * 64 + lane] = p.h2o[i];
     }
-    // One loop, one RHS evaluation per pass; the sequence of evaluations (and so of the
-    // temperature warm starts) is that of the stage/Newton/re-setup loops:
-    //   RHS(y_n), setup; per stage: RHS(z), Newton update, ... ; after max_iters without
-    //   convergence: RHS(z), setup, and the stage's Newton loop restarts.
+    // One loop, one RHS evaluation per pass. A pass is one Newton iteration of the cell's
+    // stage; where a setup is due (at y_n, or after max_iters without convergence) the pass
+    // forms and factors the matrix at the iterate between that evaluation and the update,
+    // so the evaluation serves both.
+    // The cells of a wave keep step with each other: one whose stage has converged waits
+    // until the others' have too, and the stage changes (and the next step's setups, which
+    // fall due together) are taken by all lanes at once. A wave runs to its slowest cell
+    // anyway; without the waiting, the lanes' stage changes and setups spread over nearly
+    // every pass and each of them was paid for by the whole wave. r and the first correction
+    // live in LDS: in registers across the matrix set-up they cost 170 spilled VGPRs. With
+    // the contracted arithmetic (mvd_chem.hpp) and the even chunks, against lanes that ran
+    // on alone and evaluated the RHS again after a setup: 4096 cells, 167 forced
+    // seven-stage steps 72.4 -> 39.0 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
+    // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included).
     // the next chunk's queue position, requested once the cell's loads are in flight (lane
     // 0 is active whenever the chunk is; the substepping variants request it at the chunk's
     // start, which costs them fewer registers)
-    if (!SUBSTEP && lane == 0) q = atomicAdd(queue, 64) + nwaves * 64;
+    if (!SUBSTEP && lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
     // (the substepping variants, which hold more state, solve it again: skipping there
     // costs registers that are worth more than the solve)
     bool setup = true, solved = !SUBSTEP && tdt != nullptr;
+    bool busy = true;                                      // iterating (else waiting)
+    bool fend = false;                                     // the step ended by failing
+    bool start = true;                                     // z is the (sub)step start y_n
+    int rslot = 0;                                         // offset of r's slot
     int st = 0, it = 0, setups = 0, nit = 0, nsetup = 0, nst = 0, nfail = 0;
     double crate = 1.0, delp = 0.0;                        // Newton rate estimate, last norm
     int lsetup = 0;                                        // step of the last Jacobian setup
-    bool fset = false;                                     // this step failed
     double hs = h;                                         // current (sub)step
     double hg = h * o.gamma;                               // one implicit diagonal value
     int halv = 0, done = 0;                                // substep level, units done
     unsigned long long pv = 0;
+    // With forcing, r holds the stage's right-hand side plus hg * force, the constant part
+    // of z - hg f(z) - r; the forcing is then read at stage changes only.
+#pragma unroll
+    for (int s = 0; s < NSP; s++)
+      slots[s * 64] = FORCED ? z[s] + hg * force[NSP * (long)cell + s] : z[s];
     for (;;) {
       // The lane offset and cell index are made opaque on every pass so that the per-lane
       // addresses of the cell's inputs are formed where they are used instead of being held
@@ -511,133 +496,193 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
       int ci = cell;
       __asm__ volatile("" : "+v"(lo), "+v"(ci));
       const long i = ci;
-      const double *cl = cst + lo;
-      const CellIn c{cl, cl + NSP * 64, 64,
-                     CellAux{cl[(2 * NSP) * 64], cl[(2 * NSP + 1) * 64], cl[(2 * NSP + 2) * 64],
-                             cl[(2 * NSP + 3) * 64]}};
-      double f[NSP];
-      cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !solved);
-      solved = false;
-      if (WIDE && o.esdirk && st == 0) {
-        // explicit first stage (ESDIRK): its value is y_n and F_0 = f(y_n), this pass's
-        // RHS; the first implicit stage's r = y_n + hs a_10 F_0. The pass goes on as that
-        // stage's setup or first Newton iteration, with this f at its predictor y_n.
-#pragma unroll
-        for (int s = 0; s < NSP; s++) {
-          const double F0 = FORCED ? f[s] + force[NSP * i + s] : f[s];
-          Fst[s * fstr] = F0;
-          double a = 0.0;
-          a += dirk_coef(o, 1, 0) * F0;
-          r[s] = yst[s * 64] + hs * a;
-        }
-        st = 1;
-      }
-      if (setup) {
-        cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, lu);
-        pv = lu_factor_regs(lu);
-        nsetup++;
-        setup = false;
-        it = 0;
-        crate = 1.0;
-        lsetup = nst;
-        continue;
-      }
-      double d[NSP];
-      if (FORCED) {
-#pragma unroll
-        for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * (f[s] + force[NSP * i + s]) - r[s]);
-      } else {
-#pragma unroll
-        for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * f[s] - r[s]);
-      }
-      lu_solve_regs(lu, pv, d);
-#pragma unroll
-      for (int s = 0; s < NSP; s++) z[s] += d[s];
-      nit++;
-      it++;
-      bool step_end = false;
-      const double del = wrms_norm(d, z, o.rtol, o.atol);
-      if (it > 1) crate = conv_rate(crate, del, delp);
-      const bool diverging = it > 1 && conv_diverging(del, delp);
-      delp = del;
-      if (conv_ok(crate, del, o.ntol)) {
-        if (++st == o.nstage) {
-          if (SUBSTEP) done += 1 << (o.max_halvings - halv);
-          step_end = !SUBSTEP || done >= (1 << o.max_halvings);
-          if (!step_end) {
-            // substep accepted: it becomes the start of the next one
-#pragma unroll
-            for (int s = 0; s < NSP; s++) { yst[s * 64] = z[s]; r[s] = z[s] + hs * 0.0; }
-            Ts0 = Ts;
-            dTs0 = dTs;
-            st = 0;
-            it = 0;
-            setups = 0;
-            setup = true;
-            continue;
-          }
-        } else {
-          // F_{st-1} = (z - r)/hg (ARKODE's implicit-stage derivative); the next stage's r
-#pragma unroll
-          for (int s = 0; s < NSP; s++) Fst[((st - 1) * NSP + s) * fstr] = (z[s] - r[s]) / hg;
+      if (busy) {
+        const double *cl = cst + lo;
+        const CellIn c{cl, cl + NSP * 64, 64,
+                       CellAux{cl[(2 * NSP) * 64], cl[(2 * NSP + 1) * 64],
+                               cl[(2 * NSP + 2) * 64], cl[(2 * NSP + 3) * 64]}};
+        double f[NSP];
+        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !solved);
+        solved = false;
+        if (WIDE && o.esdirk && st == 0) {
+          // explicit first stage (ESDIRK): its value is y_n and F_0 = f(y_n), this pass's
+          // RHS; the first implicit stage's r = y_n + hs a_10 F_0. The pass goes on as that
+          // stage's first Newton iteration, with this f at its predictor y_n.
 #pragma unroll
           for (int s = 0; s < NSP; s++) {
+            const double fo = FORCED ? force[NSP * i + s] : 0.0;
+            const double F0 = FORCED ? f[s] + fo : f[s];
+            Fst[s * fstr] = F0;
             double a = 0.0;
-#pragma unroll
-            for (int j = 0; j < QS - 1; j++)
-              if (j < st) a += dirk_coef<QS>(o, st, j) * Fst[(j * NSP + s) * fstr];
-            r[s] = yst[s * 64] + hs * a;                   // the (sub)step start
+            a += dirk_coef(o, 1, 0) * F0;
+            double rs = yst[s * 64] + hs * a;
+            if (FORCED) rs += hg * fo;
+            slots[s * 64] = rs;
           }
-          it = 0;
-          setups = 0;
+          st = 1;
         }
-      } else if (it == o.max_iters || diverging) {
-        if (++setups > o.max_setups) {
-          if (SUBSTEP) {
-            // back to the substep start
+        double *const rs = slots + rslot + (lo - lane);
+        double d[NSP];
 #pragma unroll
-            for (int s = 0; s < NSP; s++) z[s] = yst[s * 64];
-            Ts = Ts0;
-            dTs = dTs0;
-            if (halv < o.max_halvings) {
-              halv++;
-              hs = ldexp(h, -halv);
-              hg = hs * o.gamma;
+        for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * f[s] - rs[s * 64]);
+        if (setup) {
+          // at a step's start the correction waits in its slot (and z is y_n), so that
+          // neither occupies registers while the matrix is formed and factored; a setup at
+          // a later iterate (rare) evaluates the RHS again in the next pass instead
+          double *const ds = slots + NSP * 64 + (lo - lane);
+          if (start) {
 #pragma unroll
-              for (int s = 0; s < NSP; s++) r[s] = z[s] + hs * 0.0;
-              st = 0;
-              it = 0;
-              setups = 0;
-              setup = true;
-              continue;
+            for (int s = 0; s < NSP; s++) ds[s * 64] = d[s];
+          }
+          cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, lu);
+          pv = lu_factor_regs<true>(lu);
+          nsetup++;
+          setup = false;
+          it = 0;
+          crate = 1.0;
+          lsetup = nst;
+          if (!start) continue;
+          __asm__ volatile("" ::: "memory");
+#pragma unroll
+          for (int s = 0; s < NSP; s++) {
+            d[s] = ds[s * 64];
+            z[s] = yst[s * 64 + (lo - lane)];
+          }
+        }
+        start = false;
+        lu_solve_regs(lu, pv, d);
+#pragma unroll
+        for (int s = 0; s < NSP; s++) z[s] += d[s];
+        nit++;
+        it++;
+        const double del = wrms_norm(d, z, o.rtol, o.atol);
+        if (it > 1) crate = conv_rate(crate, del, delp);
+        const bool diverging = it > 1 && conv_diverging(del, delp);
+        delp = del;
+        if (conv_ok(crate, del, o.ntol)) {
+          busy = false;
+        } else if (it == o.max_iters || diverging) {
+          if (++setups > o.max_setups) {
+            bool retry = false;
+            if (SUBSTEP) {
+              // back to the substep start
+#pragma unroll
+              for (int s = 0; s < NSP; s++) z[s] = yst[s * 64];
+              Ts = Ts0;
+              dTs = dTs0;
+              if (halv < o.max_halvings) {
+                retry = true;
+                halv++;
+                hs = ldexp(h, -halv);
+                hg = hs * o.gamma;
+#pragma unroll
+                for (int s = 0; s < NSP; s++)
+                  slots[s * 64] = FORCED ? z[s] + hg * force[NSP * i + s] : z[s];
+                rslot = 0;
+                st = 0;
+                it = 0;
+                setups = 0;
+                setup = true;
+                start = true;
+              }
+            }
+            if (!retry) {                                  // the step failed
+              nfail++;
+              fend = true;
+              busy = false;
+            }
+          } else {
+            setup = true;
+          }
+        }
+      }
+      if (__ballot(busy) != 0) continue;                   // some cell of the wave iterates
+      busy = true;
+      if (!fend && ++st < o.nstage) {
+        // F_{st-1} = (z - r)/hg (ARKODE's implicit-stage derivative; with forcing r holds
+        // hg * force too); the next stage's r
+        const double ihg = 1.0 / hg;
+        double *const rold = slots + rslot;
+        // (narrow: r_{st-1} and F_{st-1} share slot st - 1; the last stage's r takes slot 0)
+        if (!WIDE) rslot = st + 1 < o.nstage ? st * NSP * 64 : 0;
+        double *const rnew = slots + rslot;
+#pragma unroll
+        for (int s = 0; s < NSP; s++) {
+          const double F = (z[s] - rold[s * 64]) * ihg;
+          Fst[((st - 1) * NSP + s) * fstr] = FORCED ? F + force[NSP * i + s] : F;
+        }
+        double a[NSP];
+#pragma unroll
+        for (int s = 0; s < NSP; s++) a[s] = 0.0;
+        if (WIDE) {
+          // two earlier stages' loads in flight at a time: all of them at once cost this
+          // variant 70 spilled VGPRs
+#pragma unroll 1
+          for (int j = 0; j < st; j += 2) {
+            const double c0 = tabA[st * MAXSTAGE + j], c1 = tabA[st * MAXSTAGE + j + 1];
+            const bool two = j + 1 < st;
+            const double *const F0 = Fst + (long)j * NSP * fstr;
+            const double *const F1 = two ? F0 + NSP * fstr : F0;
+            double u[NSP], v[NSP];
+#pragma unroll
+            for (int s = 0; s < NSP; s++) u[s] = F0[s * fstr];
+#pragma unroll
+            for (int s = 0; s < NSP; s++) v[s] = F1[s * fstr];
+#pragma unroll
+            for (int s = 0; s < NSP; s++) {
+              a[s] += c0 * u[s];
+              if (two) a[s] += c1 * v[s];
             }
           }
-          nfail++;                                         // the step failed
-          fset = true;
-          step_end = true;
         } else {
-          setup = true;
+#pragma unroll
+          for (int s = 0; s < NSP; s++)
+#pragma unroll
+            for (int j = 0; j < FST_LDS_MAX - 1; j++)
+              if (j < st) a[s] += dirk_coef<FST_LDS_MAX>(o, st, j) * Fst[(j * NSP + s) * 64];
         }
+#pragma unroll
+        for (int s = 0; s < NSP; s++) {
+          double rs = yst[s * 64] + hs * a[s];             // the (sub)step start
+          if (FORCED) rs += hg * force[NSP * i + s];
+          rnew[s * 64] = rs;
+        }
+        it = 0;
+        setups = 0;
+        continue;
+      }
+      // end of the (sub)step
+      bool step_end = true;
+      if (SUBSTEP && !fend) {
+        done += 1 << (o.max_halvings - halv);
+        step_end = done >= (1 << o.max_halvings);
       }
       if (step_end) {
         if (++nst >= nsteps) break;
-        // the next step from the state the cell kept (as the next launch would start it)
-#pragma unroll
-        for (int s = 0; s < NSP; s++) { yst[s * 64] = z[s]; r[s] = z[s] + h * 0.0; }
-        Ts0 = Ts;
-        dTs0 = dTs;
-        st = 0;
-        it = 0;
-        setups = 0;
+        // the next step from the state the cell kept (as the next launch would start it).
         // ARKODE's lsetup frequency: a setup at y_n after a failed or split step and once
         // msbp steps have passed since the last one; else Newton starts with the held factors
-        setup = fset || halv > 0 || nst - lsetup >= o.msbp;
-        fset = false;
+        setup = fend || halv > 0 || nst - lsetup >= o.msbp;
+        fend = false;
         hs = h;
         hg = h * o.gamma;
         halv = 0;
         done = 0;
+      } else {
+        setup = true;                                      // substep accepted: the next one
       }
+#pragma unroll
+      for (int s = 0; s < NSP; s++) {
+        yst[s * 64] = z[s];
+        slots[s * 64] = FORCED ? z[s] + hg * force[NSP * i + s] : z[s];
+      }
+      rslot = 0;
+      start = true;
+      Ts0 = Ts;
+      dTs0 = dTs;
+      st = 0;
+      it = 0;
+      setups = 0;
     }
     {
       const long i = cell;
@@ -718,10 +763,15 @@ plain_jac(long n, ChemConst cc, ChemPtrsD p, double hg, double srhs, const doubl
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || !todo[i]) return;
   const CellIn c = load_cell(p, i);
-  double zz[NSP];
+  double zz[NSP], M[NSP][NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) zz[s] = z[NSP * i + s];
-  cell_matrix(cc, c, p.Ts[i], p.dTs[i], zz, hg, srhs, Mat{LU + (long)NSP * NSP * i, 1, NSP});
+  cell_matrix_regs(cc, c, p.Ts[i], p.dTs[i], zz, hg, srhs, M);
+  double *blk = LU + (long)NSP * NSP * i;
+#pragma unroll
+  for (int q = 0; q < NSP; q++)
+#pragma unroll
+    for (int r = 0; r < NSP; r++) blk[NSP * q + r] = M[r][q];
 }
 
 // batched getrf: each thread factors its cell's block in registers
@@ -735,7 +785,7 @@ plain_getrf(long n, double *LU, unsigned long long *piv, const int *todo) {
   for (int q = 0; q < NSP; q++)
 #pragma unroll
     for (int r = 0; r < NSP; r++) a[r][q] = blk[NSP * q + r];
-  piv[i] = lu_factor_regs(a);
+  piv[i] = lu_factor_regs<true>(a);
 #pragma unroll
   for (int q = 0; q < NSP; q++)
 #pragma unroll
@@ -746,7 +796,7 @@ plain_getrf(long n, double *LU, unsigned long long *piv, const int *todo) {
 __global__ void __launch_bounds__(256)
 plain_stage_init(long n, int st, double h, DirkDev o, const double *yn, const double *F,
                  double *r, int *active, const int *failed) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
 #pragma unroll
@@ -767,7 +817,7 @@ __global__ void __launch_bounds__(256)
 plain_newton(long n, double hg, DirkDev o, double *LU, const unsigned long long *piv,
              const double *f, const double *r, double *z, int *active, int *cell_iters,
              double *crate, double *delp, int m, int *count) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || active[i] != 1) return;
   double d[NSP], zz[NSP];
@@ -776,7 +826,13 @@ plain_newton(long n, double hg, DirkDev o, double *LU, const unsigned long long 
     zz[s] = z[NSP * i + s];
     d[s] = -(zz[s] - hg * f[NSP * i + s] - r[NSP * i + s]);
   }
-  lu_solve(Mat{LU + (long)NSP * NSP * i, 1, NSP}, piv[i], d);
+  double a[NSP][NSP];
+  const double *blk = LU + (long)NSP * NSP * i;
+#pragma unroll
+  for (int q = 0; q < NSP; q++)
+#pragma unroll
+    for (int r = 0; r < NSP; r++) a[r][q] = blk[NSP * q + r];
+  lu_solve_regs(a, piv[i], d);
 #pragma unroll
   for (int s = 0; s < NSP; s++) {
     zz[s] += d[s];
@@ -809,12 +865,12 @@ plain_resume(long n, int *active, double *crate) {
 // stage end: F_st = (z - r)/hg
 __global__ void __launch_bounds__(256)
 plain_stage_finish(long n, int st, double hg, const double *z, const double *r, double *F) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
 #pragma unroll
   for (int s = 0; s < NSP; s++)
-    F[(long)st * n * NSP + NSP * i + s] = (z[NSP * i + s] - r[NSP * i + s]) / hg;
+    F[(long)st * n * NSP + NSP * i + s] = (z[NSP * i + s] - r[NSP * i + s]) * (1.0 / hg);
 }
 
 // per-wave statistics rows of the plain path
@@ -927,7 +983,7 @@ constexpr int TORD_CBLOCK = 256;
 __global__ void __launch_bounds__(TORD_CBLOCK)
 tord_count(long n, ChemConst cc, ChemPtrsD p, const double *y, const double *force, double h,
            double srhs, unsigned short *key, int *cnt, double2 *tdt) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   __shared__ int hc[TORD_NBK];
   __shared__ double gl[4 * TLEN];        // the gamma tables of the temperature solve
   for (int e = threadIdx.x; e < TORD_NBK; e += blockDim.x) hc[e] = 0;
@@ -953,7 +1009,7 @@ tord_count(long n, ChemConst cc, ChemPtrsD p, const double *y, const double *for
       v = fabs(v);
       m = v > m ? v : m;
     }
-    const int kt = chem_bin(cc, log(T > cc.tmin ? (T < cc.tmax ? T : cc.tmax) : cc.tmin)) >> 3;
+    const int kt = chem_bin(cc, chem_log(T > cc.tmin ? (T < cc.tmax ? T : cc.tmax) : cc.tmin)) >> 3;
     const int k = kt * TORD_RC + tord_rate_class(h * m);
     key[i] = (unsigned short)k;
     atomicAdd(&hc[k], 1);
@@ -1016,8 +1072,8 @@ tord_scatter(long n, const unsigned short *key, int *cnt, int *order) {
 // running offsets | keys | temperatures at y_n).
 struct BatchedPlan {
   void (*kern)(long, ChemConst, ChemPtrsD, DirkDev, double, double *, const double *,
-               const int *, const double2 *, int *, int *, int, double *);
-  int block, wpb;
+               const int *, const double2 *, int *, int *, int, double *, int);
+  int block, wpb, chunk;
   long grid, nrow;
   bool sorted;
   size_t b_rows, b_ord, b_cnt, b_key, b_tdt, b_fst;
@@ -1052,9 +1108,15 @@ static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, boo
   p.block = dirk_fit_block(block, o.nstage, fa.sharedSizeBytes, (size_t)lim, o.esdirk != 0);
   if (p.block == 0) return -1;
   p.wpb = p.block / 64;
-  const size_t chunks = (size_t)(n + 63) / 64;
-  long waves = grid_waves > 0 ? grid_waves : 1;
-  if (waves > (long)chunks) waves = (long)chunks;
+  // Cells per wave and turn: up to 64, spread evenly over the waves of the grid and the turns
+  // each of them takes. A batch of fewer than 64 cells per wave of the device then runs on
+  // all waves with fewer cells each, so that fewer cells wait for a wave's slowest one and a
+  // wave pays for fewer cells' setups and retries.
+  const long want = grid_waves > 0 ? grid_waves : 1;
+  const long turns = (n + 64 * want - 1) / (64 * want);
+  p.chunk = (int)((n + turns * want - 1) / (turns * want));
+  const long chunks = (n + p.chunk - 1) / p.chunk;
+  const long waves = want < chunks ? want : chunks;
   p.grid = (waves + p.wpb - 1) / p.wpb;
   p.nrow = p.grid;                                         // one statistics row per block
   p.sorted = n >= TORD_MIN;
@@ -1102,7 +1164,8 @@ static int batched_enqueue(const BatchedPlan &p, ChemState &s, const DirkDev &o,
       p.b_fst ? (double *)(work + p.b_rows + p.b_ord + p.b_cnt + p.b_key + p.b_tdt) : nullptr;
   hipLaunchKernelGGL(p.kern, dim3((unsigned)p.grid), dim3(p.block), lds, st, n, s.cc,
                      ptrs_d(s), o, h, y, force, (const int *)order,
-                     sub ? nullptr : (const double2 *)tdt, counters, rows, nsteps, fglob);
+                     sub ? nullptr : (const double2 *)tdt, counters, rows, nsteps, fglob,
+                     p.chunk);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1210,6 +1273,7 @@ int dirk_plain_run(ChemState &s, const DirkDev &o, double h, double *y, hipStrea
   hipLaunchKernelGGL(count_setups, dim3(nb(n)), dim3(256), 0, st, n, active, csetups);
   hipLaunchKernelGGL(plain_resume, dim3(nb(n)), dim3(256), 0, st, n, active, crate);
   int *hcnt = s.host_counters;
+  bool fresh = true;              // f holds the RHS at the iterate y_n (the setup's evaluation)
   for (int stg = o.esdirk ? 1 : 0; stg < o.nstage; stg++) {
     const double hg = h * o.A[stg * MAXSTAGE + stg];
     hipLaunchKernelGGL(plain_stage_init, dim3(nb(n)), dim3(256), 0, st, n, stg, h, o, yn, acc, r,
@@ -1219,8 +1283,10 @@ int dirk_plain_run(ChemState &s, const DirkDev &o, double h, double *y, hipStrea
       bool all_done = false;
       hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, st, 2L, nact, 0);
       for (int it = 0; it < o.max_iters; it++) {
-        hipLaunchKernelGGL(plain_rhs, dim3(nb(n)), dim3(256), 0, st, n, s.cc, p, o.rhs_scale, z,
-                           f, active, PLAIN_ITERATING);
+        if (!fresh)
+          hipLaunchKernelGGL(plain_rhs, dim3(nb(n)), dim3(256), 0, st, n, s.cc, p, o.rhs_scale,
+                             z, f, active, PLAIN_ITERATING);
+        fresh = false;
         hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, st, 1L, nact, 0);
         hipLaunchKernelGGL(plain_newton, dim3(nb(n)), dim3(256), 0, st, n, hg, o, LU, piv, f, r,
                            z, active, iters, crate, delp, it, nact);
@@ -1280,7 +1346,7 @@ ls_setup_kernel(long n, double gamma, const double *J, double *LU, unsigned long
 #pragma unroll
     for (int r = 0; r < NSP; r++)
       a[r][q] = formed ? jb[NSP * q + r] : (r == q ? 1.0 : 0.0) - gamma * jb[NSP * q + r];
-  piv[i] = lu_factor_regs(a);
+  piv[i] = lu_factor_regs<false>(a);
   bool sing = false;
   double *blk = LU + (long)NSP * NSP * i;
 #pragma unroll
@@ -1295,12 +1361,24 @@ ls_setup_kernel(long n, double gamma, const double *J, double *LU, unsigned long
 __global__ void __launch_bounds__(256)
 ls_solve_kernel(long n, const double *LU, const unsigned long long *piv, const double *b,
                 double *x) {
+#pragma clang fp contract(off)
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double v[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) v[s] = b[NSP * i + s];
-  lu_solve(Mat{const_cast<double *>(LU) + (long)NSP * NSP * i, 1, NSP}, piv[i], v);
+  const double *a = LU + (long)NSP * NSP * i;            // element (r, q) at 10 q + r
+  lu_exchange(piv[i], v);
+#pragma unroll
+  for (int r = 1; r < NSP; r++)
+#pragma unroll
+    for (int q = 0; q < r; q++) v[r] -= a[NSP * q + r] * v[q];
+#pragma unroll
+  for (int r = NSP - 1; r >= 0; r--) {
+#pragma unroll
+    for (int q = r + 1; q < NSP; q++) v[r] -= a[NSP * q + r] * v[q];
+    v[r] /= a[NSP * r + r];
+  }
 #pragma unroll
   for (int s = 0; s < NSP; s++) x[NSP * i + s] = v[s];
 }
@@ -1342,13 +1420,13 @@ int chem_ls_solve(long n, const double *LU, const unsigned long long *piv, const
 __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, double &dTs,
                           const DirkDev &o, double h, double (&y)[NSP], double *Ys, long n,
                           long i) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double yn[NSP], z[NSP], f[NSP], F[ADJ_MAXSTAGE][NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) yn[s] = z[s] = y[s];
-  cell_rhs<true>(cc, c, Ts, dTs, yn, o.rhs_scale, f);      // refresh Ts at y_n for J
   double a[NSP][NSP];
   unsigned long long pv = 0;
+  cell_rhs<true>(cc, c, Ts, dTs, yn, o.rhs_scale, f);      // refresh Ts at y_n for J
   bool ok = true;
   double crate = 1.0, delp = 0.0;                     // Newton rate estimate, last norm
 #pragma unroll
@@ -1357,7 +1435,7 @@ __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, doub
       const double hg = h * o.A[st * MAXSTAGE + st];
       if (st == 0) {
         cell_matrix_regs(cc, c, Ts, dTs, yn, hg, o.rhs_scale, a);
-        pv = lu_factor_regs(a);
+        pv = lu_factor_regs<true>(a);
       }
       double r[NSP];
 #pragma unroll
@@ -1388,12 +1466,12 @@ __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, doub
         if (++setups > o.max_setups) { ok = false; break; }
         cell_rhs<true>(cc, c, Ts, dTs, z, o.rhs_scale, f);   // temperature at the iterate
         cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a);
-        pv = lu_factor_regs(a);
+        pv = lu_factor_regs<true>(a);
         crate = 1.0;
         it = 0;
       }
 #pragma unroll
-      for (int s = 0; s < NSP; s++) F[st][s] = (z[s] - r[s]) / hg;
+      for (int s = 0; s < NSP; s++) F[st][s] = (z[s] - r[s]) * (1.0 / hg);
       if (Ys)
 #pragma unroll
         for (int s = 0; s < NSP; s++) Ys[(long)(st * NSP + s) * n + i] = z[s];
@@ -1442,7 +1520,7 @@ __device__ inline void stage_adjoint_matrix(const ChemConst &cc, const CellIn &c
                                             const double (&Y)[NSP], double srhs, double h,
                                             double hg, const double (&w)[NSP],
                                             double (&Mt)[NSP][NSP], double (&yb)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double ya[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = Y[s] * c.s(s);
@@ -1475,7 +1553,7 @@ __global__ void __launch_bounds__(256)
 chem_adjoint_backward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, int nsteps, int K,
                       const int *order, const double *ck, double *Te, double *Ys,
                       const double *lamT, double *lam0) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const long u = (long)blockIdx.x * blockDim.x + threadIdx.x;   // as in chem_adjoint_forward
   if (u >= n) return;
   const long i = order ? order[u] : u;
@@ -1522,7 +1600,7 @@ chem_adjoint_backward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, in
           }
           double Mt[NSP][NSP], yb[NSP];
           stage_adjoint_matrix(cc, c, Ts, Y, o.rhs_scale, h, h * o.A[k * MAXSTAGE + k], w, Mt, yb);
-          const unsigned long long pv = lu_factor_regs(Mt);
+          const unsigned long long pv = lu_factor_regs<true>(Mt);
           lu_solve_regs(Mt, pv, yb);
 #pragma unroll
           for (int s = 0; s < NSP; s++) nu[k][s] = yb[s];

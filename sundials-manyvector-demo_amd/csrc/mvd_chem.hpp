@@ -10,6 +10,7 @@
 // streaming 736 bytes per cell through HBM.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "mvd_device.hpp"
 
 namespace mvd {
 
@@ -72,16 +73,55 @@ double *chem_state_ptr(ChemState &s, int which);
 void chem_free(ChemState &s);
 
 // -------------------------------------------------------------------------------------
-// device functions (reference operation order, no FMA contraction)
+// device functions: the reference's expressions. Products and sums of one expression are
+// contracted to FMAs by the front end (contract(on), the same way wherever a function is
+// inlined, so the solvers that share these functions agree bit for bit), and the divides of
+// the inner loops use fast_div / fast_rcp (about 0.5 and 1 ulp). At one wave per SIMD the
+// implicit kernels are bound by the instructions they issue: the uncontracted form with
+// IEEE divides and the library logarithm had 2800 separate FP64 multiplies and adds and 81
+// divides of 11 instructions in the batched step.
 // -------------------------------------------------------------------------------------
 
-// (int)(idbin*(log T - lb)) clamped to [0, nbins-1] (raja_primordial_network.cpp:953-958)
+// log(x) by the reduction and reassembly of Sun's fdlibm (K. C. Ng, 1993), x = 2^k (1 + f),
+// sqrt(1/2) <= 1 + f < sqrt(2), s = f / (2 + f), log(1 + f) = f - (f^2/2 - s (f^2/2 + R(s^2))),
+// with R the degree-6 interpolant (Chebyshev nodes, error 9e-18) of 2 (atanh(s)/s - 1).
+// Within 1 ulp; not above 0 or infinite: NaN. About half the library's instructions (no
+// extended precision).
+__device__ inline double chem_log(double x) {
+#pragma clang fp contract(off)
+  const double m0 = __builtin_amdgcn_frexp_mant(x);        // [1/2, 1)
+  const bool low = m0 < 0.70710678118654752440;
+  const double m = low ? m0 + m0 : m0;
+  const double k = (double)(__builtin_amdgcn_frexp_exp(x) - (low ? 1 : 0));
+  const double f = m - 1.0;
+  const double s = fast_div(f, m + 1.0), z = s * s;
+  double R = 0.14616449685043406;
+  R = fma(R, z, 0.15331721600556042);
+  R = fma(R, z, 0.18182889125261723);
+  R = fma(R, z, 0.2222221113479508);
+  R = fma(R, z, 0.28571428625975487);
+  R = fma(R, z, 0.39999999999899505);
+  R = fma(R, z, 0.666666666666667);
+  R *= z;
+  const double h = 0.5 * f * f;
+  const double ln2_hi = 6.93147180369123816490e-01, ln2_lo = 1.90821492927058770002e-10;
+  const double lo = fma(s, h + R, k * ln2_lo);
+  const double v = fma(k, ln2_hi, f - (h - lo));
+  return x > 0.0 && x < __builtin_inf() ? v : __builtin_nan("");
+}
+
+// Table position of log T: bin b = (int)(idbin*(log T - lb)) clamped to [0, nbins-1]
+// (raja_primordial_network.cpp:953-958; NaN: 0) and the distance Tdef = (log T - t_b) /
+// (t_{b+1} - t_b) from the bin's lower node in bins (one FMA on the uniform grid; the
+// difference of the two node temperatures loses more digits).
 __device__ inline int chem_bin(const ChemConst &c, double logT) {
-  const double x = c.idbin * (logT - c.lb);
-  int b = (x == x) ? (int)fmin(fmax(x, -1.0), 2.0e9) : 0;
-  if (b <= 0) b = 0;
-  else if (b >= c.nbins) b = c.nbins - 1;
-  return b;
+  return (int)fmin(fmax(c.idbin * (logT - c.lb), 0.0), (double)(c.nbins - 1));
+}
+
+__device__ inline int chem_locate(const ChemConst &c, double logT, double &Tdef) {
+  const double b = trunc(fmin(fmax(c.idbin * (logT - c.lb), 0.0), (double)(c.nbins - 1)));
+  Tdef = fma(c.idbin, logT - c.lb, -b);
+  return (int)b;
 }
 
 // The four gamma tables of the temperature solve (gH2_1, dgH2_1, gH2_2, dgH2_2), read
@@ -100,37 +140,40 @@ __device__ inline GammaTabs gamma_tabs(const ChemConst &c) {
 
 // Mass density (in hydrogen masses) of the temperature solve
 __device__ inline double temperature_density(const double (&y)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   return 2.0 * y[0] + 2.0 * y[1] + 1.0079400000000001 * y[2] + 1.0079400000000001 * y[3] +
          1.0079400000000001 * y[4] + 4.0026020000000004 * y[5] + 4.0026020000000004 * y[6] +
          4.0026020000000004 * y[7];
 }
 
-// One Newton step of the temperature solve from the input T (density `dm` = density * mH):
+// One Newton step of the temperature solve from the input T (kdm = kb / (density * mH)):
 // returns the next iterate and sets dge_dT at T (raja_primordial_network.cpp:943-990).
 __device__ inline double temperature_step(const ChemConst &c, const GammaTabs &gt,
-                                          const double (&y)[NSP], double dm, double T,
-                                          double &dge_dT) {
-#pragma clang fp contract(off)
-  const double kb = 1.3806504e-16;
-  const double gamma = 5.e0 / 3.e0;
-  const double gm1 = 1.0 / (gamma - 1);
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
+                                          const double (&y)[NSP], double kdm, double nmono,
+                                          double T, double &dge_dT) {
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
   const double gH2_2 = gt.g2[b] + Tdef * (gt.g2[b + 1] - gt.g2[b]);
   const double dgH2_2 = gt.dg2[b] + Tdef * (gt.dg2[b + 1] - gt.dg2[b]);
   const double gH2_1 = gt.g1[b] + Tdef * (gt.g1[b + 1] - gt.g1[b]);
   const double dgH2_1 = gt.dg1[b] + Tdef * (gt.dg1[b + 1] - gt.dg1[b]);
-  const double g1 = 1.0 / (gH2_1 - 1.0);
-  const double g2 = 1.0 / (gH2_2 - 1.0);
-  const double nsum = y[0] * g1 + y[1] * g2 + y[2] * gm1 + y[3] * gm1 + y[4] * gm1 +
-                      y[5] * gm1 + y[6] * gm1 + y[7] * gm1 + gm1 * y[8];
-  dge_dT = T * kb * ((-y[0]) * g1 * g1 * dgH2_1 - y[1] * g2 * g2 * dgH2_2) / dm + kb * nsum / dm;
-  const double dge = T * kb * nsum / dm - y[9];
-  return T - dge / dge_dT;
+  const double g1 = fast_rcp(gH2_1 - 1.0);
+  const double g2 = fast_rcp(gH2_2 - 1.0);
+  const double a1 = y[0] * g1, a2 = y[1] * g2;
+  const double knum = kdm * (a1 + a2 + nmono);             // kb nsum / dm
+  const double slope = a1 * g1 * dgH2_1 + a2 * g2 * dgH2_2;
+  dge_dT = knum - T * kdm * slope;
+  const double dge = T * knum - y[9];
+  return T - fast_div(dge, dge_dT);
+}
+
+// kb / (density * mH) and the monatomic species' share of nsum, constant over a solve
+__device__ inline void temperature_consts(const double (&y)[NSP], double &kdm, double &nmono) {
+#pragma clang fp contract(on)
+  const double kb = 1.3806504e-16, gm1 = 1.0 / (5.e0 / 3.e0 - 1);
+  kdm = kb / (temperature_density(y) * 1.67e-24);
+  nmono = gm1 * (y[2] + y[3] + y[4] + y[5] + y[6] + y[7] + y[8]);
 }
 
 // Longest cycle of the temperature iteration that ends the loop early.
@@ -150,15 +193,16 @@ constexpr int TCYCLE = 4;
 // makes near some roots, otherwise run the full ten steps and hold up their whole wave.
 __device__ inline void chem_temperature(const ChemConst &c, const GammaTabs &gt,
                                         const double (&y)[NSP], double &Ts, double &dTs_ge) {
-#pragma clang fp contract(off)
-  const double dm = temperature_density(y) * 1.67e-24;
+#pragma clang fp contract(on)
+  double kdm, nmono;
+  temperature_consts(y, kdm, nmono);
   double Tnew = Ts * 1.1, dge_dT = 0.0;
   double xh[TCYCLE], dh[TCYCLE];        // x_k, d_k of the last steps, newest first
 #pragma unroll
   for (int q = 0; q < TCYCLE; q++) xh[q] = dh[q] = 0.0;
   for (int it = 0; it < 10; it++) {
     const double T = Ts;
-    Tnew = temperature_step(c, gt, y, dm, T, dge_dT);
+    Tnew = temperature_step(c, gt, y, kdm, nmono, T, dge_dT);
     Ts = Tnew;
 #pragma unroll
     for (int q = TCYCLE - 1; q > 0; q--) {
@@ -191,23 +235,24 @@ __device__ inline void chem_temperature(const ChemConst &c, const GammaTabs &gt,
   Ts = Tnew;
   if (Ts < c.tmin) Ts = c.tmin;
   else if (Ts > c.tmax) Ts = c.tmax;
-  dTs_ge = 1.0 / dge_dT;
+  dTs_ge = fast_rcp(dge_dT);
 }
 
 // The ten steps without the early exit (the self-check of the exit compares the two)
 __device__ inline void chem_temperature_ten(const ChemConst &c, const double (&y)[NSP],
                                             double &Ts, double &dTs_ge) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const GammaTabs gt = gamma_tabs(c);
-  const double dm = temperature_density(y) * 1.67e-24;
+  double kdm, nmono;
+  temperature_consts(y, kdm, nmono);
   double Tnew = Ts * 1.1, dge_dT = 0.0;
   for (int it = 0; it < 10; it++) {
-    Tnew = temperature_step(c, gt, y, dm, Ts, dge_dT);
+    Tnew = temperature_step(c, gt, y, kdm, nmono, Ts, dge_dT);
     Ts = Tnew;
   }
   if (Ts < c.tmin) Ts = c.tmin;
   else if (Ts > c.tmax) Ts = c.tmax;
-  dTs_ge = 1.0 / dge_dT;
+  dTs_ge = fast_rcp(dge_dT);
 }
 
 __device__ inline void chem_temperature(const ChemConst &c, const double (&y)[NSP], double &Ts,
@@ -219,13 +264,10 @@ __device__ inline void chem_temperature(const ChemConst &c, const double (&y)[NS
 // (raja_primordial_network.cpp:1046-1245)
 __device__ inline void chem_rates(const ChemConst &c, double T, double (&k)[NRATE],
                                   double (&dk)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
-  const double Tfactor = (1.0 / T) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
+  const double Tfactor = fast_rcp(T) * c.idbin;
 #pragma unroll
   for (int r = 0; r < NRATE; r++) {
     const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
@@ -238,13 +280,10 @@ __device__ inline void chem_rates(const ChemConst &c, double T, double (&k)[NRAT
 template <int R0, int R1>
 __device__ inline void chem_rates_range(const ChemConst &c, double T, double (&k)[NRATE],
                                         double (&dk)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
-  const double Tfactor = (1.0 / T) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
+  const double Tfactor = fast_rcp(T) * c.idbin;
 #pragma unroll
   for (int r = R0; r < R1; r++) {
     const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
@@ -256,12 +295,9 @@ __device__ inline void chem_rates_range(const ChemConst &c, double T, double (&k
 // Rate values of tables [R0, R1) only.
 template <int R0, int R1>
 __device__ inline void chem_rates_only_range(const ChemConst &c, double T, double (&k)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
 #pragma unroll
   for (int r = R0; r < R1; r++) {
     const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
@@ -274,13 +310,10 @@ __device__ inline void chem_rates_only_range(const ChemConst &c, double T, doubl
 template <int R0, int R1>
 __device__ inline void chem_rates_pairs(const ChemConst &c, double T, double (&k)[NRATE],
                                         double (&dk)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
-  const double Tfactor = (1.0 / T) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
+  const double Tfactor = fast_rcp(T) * c.idbin;
   const double2 *row = c.tabp + (long)b * NRATE;
 #pragma unroll
   for (int r = R0; r < R1; r++) {
@@ -292,12 +325,9 @@ __device__ inline void chem_rates_pairs(const ChemConst &c, double T, double (&k
 
 template <int R0, int R1>
 __device__ inline void chem_rates_only_pairs(const ChemConst &c, double T, double (&k)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
   const double2 *row = c.tabp + (long)b * NRATE;
 #pragma unroll
   for (int r = R0; r < R1; r++) {
@@ -308,12 +338,9 @@ __device__ inline void chem_rates_only_pairs(const ChemConst &c, double T, doubl
 
 // Only the rate values (no derivatives).
 __device__ inline void chem_rates_only(const ChemConst &c, double T, double (&k)[NRATE]) {
-#pragma clang fp contract(off)
-  const double lT = log(T);
-  const int b = chem_bin(c, lT);
-  const double t1 = c.lb + (double)b * c.dbin;
-  const double t2 = c.lb + (double)(b + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
+#pragma clang fp contract(on)
+  double Tdef;
+  const int b = chem_locate(c, chem_log(T), Tdef);
 #pragma unroll
   for (int r = 0; r < NRATE; r++) {
     const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
@@ -334,7 +361,7 @@ struct Reactions {
 };
 
 __device__ inline Reactions chem_reactions(const double (&y)[NSP], const double (&k)[NRATE]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const double H2_1 = y[0], H2_2 = y[1], H_1 = y[2], H_2 = y[3], H_m0 = y[4], He_1 = y[5],
                He_2 = y[6], He_3 = y[7], de = y[8];
   Reactions R;
@@ -369,7 +396,7 @@ __device__ inline Reactions chem_reactions(const double (&y)[NSP], const double 
 // gas-energy row only the 25 cooling rates.
 __device__ inline void chem_rhs_species(const double (&y)[NSP], const double (&k)[NRATE],
                                         double (&f)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const Reactions R = chem_reactions(y, k);
   f[0] = R.r08 + R.r10 - R.r11 - R.r12 - R.r13 + R.r19 + R.r21 + R.r22;
   f[1] = R.r09 - R.r10 + R.r11 + R.r17 - R.r18 - R.r19;
@@ -387,7 +414,7 @@ __device__ inline void chem_rhs_species(const double (&y)[NSP], const double (&k
 template <class R>
 __device__ inline R chem_rhs_energy_t(const R (&y)[NSP], const R (&k)[NRATE], R T, double z,
                                       const CellAux &ax) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const R H2_1 = y[0], H_1 = y[2], H_2 = y[3], He_1 = y[5], He_2 = y[6], He_3 = y[7],
           de = y[8];
   const double cie = ax.cie, h2o = ax.h2o;
@@ -397,7 +424,7 @@ __device__ inline R chem_rhs_energy_t(const R (&y)[NSP], const R (&k)[NRATE], R 
   const double zp1 = z + 1.0;
   const double zp4 = (zp1 * zp1) * (zp1 * zp1);
   return -2.0158800000000001 * H2_1 * k[C_CIECO] * cie * ax.mdensity -
-         H2_1 * cie * k[C_H2LTE] * h2o / (k[C_H2LTE] / gS + 1.0) - H_1 * k[C_CEHI] * cie * de -
+         fast_div(H2_1 * cie * k[C_H2LTE] * h2o * gS, k[C_H2LTE] + gS) - H_1 * k[C_CEHI] * cie * de -
          H_1 * k[C_CIHI] * cie * de - H_2 * cie * de * k[C_REHII] -
          He_1 * k[C_CIHEI] * cie * de - He_2 * k[C_CEHEII] * cie * de -
          He_2 * k[C_CEHEI] * cie * (de * de) - He_2 * k[C_CIHEII] * cie * de -
@@ -405,7 +432,7 @@ __device__ inline R chem_rhs_energy_t(const R (&y)[NSP], const R (&k)[NRATE], R 
          He_2 * cie * de * k[C_REHEII2] - He_3 * cie * de * k[C_REHEIII] -
          k[C_BREM] * cie * de * (H_2 + He_2 + 4.0 * He_3) -
          cie * k[C_COMPTON] * de * zp4 * (T - 2.73 * z - 2.73) +
-         0.5 * 1.0 / (k[C_NCRN] / ncrD + 1.0) *
+         fast_div(0.5 * ncrD, k[C_NCRN] + ncrD) *
              ((-H2_1) * H_1 * k[C_H2MCOOL] + (H_1 * H_1 * H_1) * k[C_H2MHEAT]);
 }
 
@@ -421,7 +448,7 @@ __device__ inline double chem_rhs_energy(const double (&y)[NSP], const double (&
 __device__ inline void chem_energy_grad(const double (&y)[NSP], const double (&k)[NRATE],
                                         const double (&dk)[NRATE], double T, double z,
                                         const CellAux &ax, double (&g)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const double H2_1 = y[0], H_1 = y[2], H_2 = y[3], He_1 = y[5], He_2 = y[6], He_3 = y[7],
                de = y[8];
   const double c = ax.cie, h2o = ax.h2o, md = ax.mdensity;
@@ -436,12 +463,12 @@ __device__ inline void chem_energy_grad(const double (&y)[NSP], const double (&k
   {
     const double gS = H2_1 * k[C_GAH2] + H_1 * k[C_GAHI] + H_2 * k[C_GAHP] + He_1 * k[C_GAHE] +
                       de * k[C_GAEL];
-    const double D = k[C_H2LTE] / gS + 1.0, iD = 1.0 / D;
-    const double N = H2_1 * c * k[C_H2LTE] * h2o;
-    const double Db = N * iD * iD;                  // d(-N/D)/dD
-    const double gSb = Db * (-k[C_H2LTE] / (gS * gS));
+    // -N / D with D = k / gS + 1, 1/D = gS / (k + gS)
+    const double ikg = fast_rcp(k[C_H2LTE] + gS), iD = gS * ikg;
+    const double q = H2_1 * c * h2o, kq = k[C_H2LTE] * ikg;
+    const double gSb = -q * kq * kq;                // N / D^2 (-k / gS^2)
     b0 += -(c * k[C_H2LTE] * h2o) * iD;
-    kb[C_H2LTE] += -(H2_1 * c * h2o) * iD + Db / gS;
+    kb[C_H2LTE] += -q * iD * iD;                    // -(q / D) + N / (D^2 gS)
     b0 += gSb * k[C_GAH2];  kb[C_GAH2] += gSb * H2_1;
     b2 += gSb * k[C_GAHI];  kb[C_GAHI] += gSb * H_1;
     b3 += gSb * k[C_GAHP];  kb[C_GAHP] += gSb * H_2;
@@ -489,11 +516,12 @@ __device__ inline void chem_energy_grad(const double (&y)[NSP], const double (&k
   // H2 formation heating / cooling: 0.5 / (k_NCRN / ncrD + 1) Q
   {
     const double ncrD = H2_1 * k[C_NCRD2] + H_1 * k[C_NCRD1];
-    const double E = k[C_NCRN] / ncrD + 1.0, iE = 1.0 / E;
+    // 0.5 Q / E with E = k / ncrD + 1, 1/E = ncrD / (k + ncrD)
+    const double ike = fast_rcp(k[C_NCRN] + ncrD), iE = ncrD * ike;
     const double Q = (-H2_1) * H_1 * k[C_H2MCOOL] + (H_1 * H_1 * H_1) * k[C_H2MHEAT];
-    const double Qb = 0.5 * iE, Eb = -0.5 * Q * iE * iE;
-    const double ncrDb = Eb * (-k[C_NCRN] / (ncrD * ncrD));
-    kb[C_NCRN] += Eb / ncrD;
+    const double Qb = 0.5 * iE, Eb = -0.5 * Q * ike;
+    const double ncrDb = -Eb * (k[C_NCRN] * ike);
+    kb[C_NCRN] += Eb * iE;
     b0 += Qb * (-H_1 * k[C_H2MCOOL]) + ncrDb * k[C_NCRD2];
     b2 += Qb * (-H2_1 * k[C_H2MCOOL] + 3.0 * (H_1 * H_1) * k[C_H2MHEAT]) + ncrDb * k[C_NCRD1];
     kb[C_H2MCOOL] += Qb * (-H2_1 * H_1);
@@ -555,7 +583,7 @@ struct ChemVjpPre {
 template <bool PAIRS>
 __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NSP], double T,
                                         bool clamped, const CellAux &ax, ChemVjpPre &P) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   double k[NRATE], dk[NRATE];
   if (PAIRS) chem_rates_pairs<0, NRATE>(c, T, k, dk);
   else chem_rates(c, T, k, dk);
@@ -575,18 +603,15 @@ __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NS
   // temperature path
   const double kb = 1.3806504e-16, mh = 1.67e-24;
   const double gm1 = 1.0 / (5.e0 / 3.e0 - 1);
-  const double lT = log(T);
-  const int bn = chem_bin(c, lT);
-  const double t1 = c.lb + (double)bn * c.dbin;
-  const double t2 = c.lb + (double)(bn + 1) * c.dbin;
-  const double Tdef = (lT - t1) / (t2 - t1);
-  const double Tfactor = (1.0 / T) / (t2 - t1);
+  double Tdef;
+  const int bn = chem_locate(c, chem_log(T), Tdef);
+  const double Tfactor = fast_rcp(T) * c.idbin;
   const double *g1t = c.tab + G_GH2_1 * TLEN, *g2t = c.tab + G_GH2_2 * TLEN;
   const double gH2_1 = g1t[bn] + Tdef * (g1t[bn + 1] - g1t[bn]);
   const double gH2_2 = g2t[bn] + Tdef * (g2t[bn + 1] - g2t[bn]);
   const double sl1 = (g1t[bn + 1] - g1t[bn]) * Tfactor;       // d gamma_H2_1 / dT
   const double sl2 = (g2t[bn + 1] - g2t[bn]) * Tfactor;
-  const double g1 = 1.0 / (gH2_1 - 1.0), g2 = 1.0 / (gH2_2 - 1.0);
+  const double g1 = fast_rcp(gH2_1 - 1.0), g2 = fast_rcp(gH2_2 - 1.0);
   const double cs[NSP - 1] = {g1, g2, gm1, gm1, gm1, gm1, gm1, gm1, gm1};
   const double ws[NSP - 1] = {2.0, 2.0, 1.0079400000000001, 1.0079400000000001,
                               1.0079400000000001, 4.0026020000000004, 4.0026020000000004,
@@ -597,17 +622,17 @@ __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NS
     nsum += y[s] * cs[s];
     density += ws[s] * y[s];
   }
-  const double dm = density * mh;
-  P.dgdT = kb * nsum / dm + T * kb * ((-y[0]) * g1 * g1 * sl1 - y[1] * g2 * g2 * sl2) / dm;
+  const double idn = fast_rcp(density), kdm = kb / mh * idn;
+  P.dgdT = kdm * (nsum - T * (y[0] * g1 * g1 * sl1 + y[1] * g2 * g2 * sl2));
+  const double td = T * kdm, nd = nsum * idn;
 #pragma unroll
-  for (int s = 0; s < NSP - 1; s++)
-    P.dgdy[s] = T * kb / mh * (cs[s] * density - nsum * ws[s]) / (density * density);
+  for (int s = 0; s < NSP - 1; s++) P.dgdy[s] = td * (cs[s] - nd * ws[s]);
 }
 
 // The temperature path's share of yab for the T-cotangent Tb.
 __device__ inline void chem_vjp_temperature(const ChemVjpPre &P, double Tb,
                                             double (&yab)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   if (P.clamped) return;
   const double TbT = Tb / P.dgdT;
 #pragma unroll
@@ -617,7 +642,7 @@ __device__ inline void chem_vjp_temperature(const ChemVjpPre &P, double Tb,
 
 __device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP],
                                       const double (&vp)[NSP], double (&yab)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
 #pragma unroll
   for (int s = 0; s < NSP; s++) yab[s] = 0.0;
   double Tb = 0.0;
@@ -647,7 +672,7 @@ __device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP
 // rows, all zero, are left out.
 __device__ inline void chem_vjp_row(const ChemVjpPre &P, const double (&y)[NSP], int r,
                                     double v, double (&row)[NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
 #pragma unroll
   for (int s = 0; s < NSP; s++) row[s] = 0.0;
   double Tb = 0.0;
@@ -698,7 +723,7 @@ __device__ inline void chem_rhs_physical(const double (&y)[NSP], const double (&
 __device__ inline void chem_jac_species(const double (&y)[NSP], const double (&k)[NRATE],
                                         const double (&rk)[NRATE], double Tge,
                                         double (&J)[NSP][NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const double H2_1 = y[0], H2_2 = y[1], H_1 = y[2], H_2 = y[3], H_m0 = y[4], He_1 = y[5],
                He_2 = y[6], He_3 = y[7], de = y[8];
   const double k01 = k[K01], k02 = k[K02], k03 = k[K03], k04 = k[K04], k05 = k[K05],
@@ -788,7 +813,7 @@ __device__ inline void chem_jac_species(const double (&y)[NSP], const double (&k
 __device__ inline void chem_jac_energy(const double (&y)[NSP], const double (&k)[NRATE],
                                        const double (&rk)[NRATE], double T, double z,
                                        double Tge, const CellAux &ax, double (&J)[NSP][NSP]) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const double H2_1 = y[0], H_1 = y[2], H_2 = y[3], He_1 = y[5], He_2 = y[6], He_3 = y[7],
                de = y[8];
   const double H1sq = H_1 * H_1;
@@ -800,23 +825,24 @@ __device__ inline void chem_jac_energy(const double (&y)[NSP], const double (&k)
                h2mheat = k[C_H2MHEAT], ncrd1 = k[C_NCRD1], ncrd2 = k[C_NCRD2], ncrn = k[C_NCRN],
                reHeII1 = k[C_REHEII1], reHeII2 = k[C_REHEII2], reHeIII = k[C_REHEIII],
                reHII = k[C_REHII];
-  const double inv_md = 1.0 / ax.mdensity;
+  const double inv_md = fast_rcp(ax.mdensity);
   const double h2o = ax.h2o;
   const double S = H2_1 * gaH2 + H_1 * gaHI + H_2 * gaHp + He_1 * gaHe + de * gael;
   const double Dn = H2_1 * ncrd2 + H_1 * ncrd1;
-  const double gden = h2lte / S + 1.0;
-  const double nden = ncrn / Dn + 1.0;
-  const double nden_m2 = 1.0 / (nden * nden);
+  // gden = h2lte / S + 1 and nden = ncrn / Dn + 1 enter through their reciprocals
+  // S / (h2lte + S) and Dn / (ncrn + Dn), and gden S = h2lte + S, nden Dn = ncrn + Dn
+  const double ig = fast_rcp(h2lte + S), in = fast_rcp(ncrn + Dn);
+  const double igden = S * ig, inden = Dn * in;
   const double Y = (-H2_1) * H_1 * h2mcool + (H_1 * H_1 * H_1) * h2mheat;
-  const double gq = (h2lte * h2lte) * h2o / ((gden * gden) * (S * S));
+  const double gq = (h2lte * ig) * (h2lte * ig) * h2o;
+  const double nq = 0.5 * ncrn * Y * (in * in);
   const double zp1 = z + 1.0;
   const double zp4 = (zp1 * zp1) * (zp1 * zp1);
-  J[9][0] = ((-H2_1) * gaH2 * gq - 0.5 * H_1 * h2mcool * 1.0 / nden -
-             2.0158800000000001 * cieco * ax.mdensity - h2lte * h2o / gden +
-             0.5 * ncrd2 * ncrn * nden_m2 * Y / (Dn * Dn)) * inv_md;
+  J[9][0] = ((-H2_1) * gaH2 * gq - 0.5 * H_1 * h2mcool * inden -
+             2.0158800000000001 * cieco * ax.mdensity - h2lte * h2o * igden + ncrd2 * nq) * inv_md;
   J[9][2] = ((-H2_1) * gaHI * gq - ceHI * de - ciHI * de +
-             0.5 * ncrd1 * ncrn * nden_m2 * Y / (Dn * Dn) +
-             0.5 * ((-H2_1) * h2mcool + 3.0 * H1sq * h2mheat) * 1.0 / nden) * inv_md;
+             ncrd1 * nq +
+             0.5 * ((-H2_1) * h2mcool + 3.0 * H1sq * h2mheat) * inden) * inv_md;
   J[9][3] = ((-H2_1) * gaHp * gq - brem * de - de * reHII) * inv_md;
   J[9][5] = ((-H2_1) * gaHe * gq - ciHeI * de) * inv_md;
   J[9][6] = ((-brem) * de - ceHeII * de - ceHeI * (de * de) - ciHeII * de -
@@ -829,12 +855,11 @@ __device__ inline void chem_jac_energy(const double (&y)[NSP], const double (&k)
   const double Rg = (-H2_1) * rk[C_GAH2] - H_1 * rk[C_GAHI] - H_2 * rk[C_GAHP] -
                     He_1 * rk[C_GAHE] - de * rk[C_GAEL];
   const double adhoc =
-      (-H2_1) * h2lte * h2o * ((-h2lte) * Rg / (S * S) - rk[C_H2LTE] / S) / (gden * gden) -
-      H2_1 * h2o * rk[C_H2LTE] / gden +
-      0.5 * nden_m2 * Y *
-          (-1.0 * ncrn * ((-H2_1) * rk[C_NCRD2] - H_1 * rk[C_NCRD1]) / (Dn * Dn) -
-           1.0 * rk[C_NCRN] / Dn) +
-      0.5 * 1.0 / nden * ((-H2_1) * H_1 * rk[C_H2MCOOL] + (H_1 * H_1 * H_1) * rk[C_H2MHEAT]);
+      H2_1 * h2o * (h2lte * ig) * (h2lte * Rg * ig + rk[C_H2LTE] * igden) -
+      H2_1 * h2o * rk[C_H2LTE] * igden +
+      0.5 * in * Y *
+          (ncrn * (H2_1 * rk[C_NCRD2] + H_1 * rk[C_NCRD1]) * in - rk[C_NCRN] * inden) +
+      0.5 * inden * ((-H2_1) * H_1 * rk[C_H2MCOOL] + (H_1 * H_1 * H_1) * rk[C_H2MHEAT]);
   J[9][9] = adhoc * inv_md * Tge;
 }
 
