@@ -463,7 +463,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     // live in LDS: in registers across the matrix set-up they cost 170 spilled VGPRs. With
     // the contracted arithmetic (mvd_chem.hpp) and the even chunks, against lanes that ran
     // on alone and evaluated the RHS again after a setup: 4096 cells, 167 forced
-    // seven-stage steps 72.4 -> 39.0 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
+    // seven-stage steps 72.4 -> 19.7 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
     // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included).
     // the next chunk's queue position, requested once the cell's loads are in flight (lane
     // 0 is active whenever the chunk is; the substepping variants request it at the chunk's
@@ -1108,13 +1108,17 @@ static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, boo
   p.block = dirk_fit_block(block, o.nstage, fa.sharedSizeBytes, (size_t)lim, o.esdirk != 0);
   if (p.block == 0) return -1;
   p.wpb = p.block / 64;
-  // Cells per wave and turn: up to 64, spread evenly over the waves of the grid and the turns
-  // each of them takes. A batch of fewer than 64 cells per wave of the device then runs on
-  // all waves with fewer cells each, so that fewer cells wait for a wave's slowest one and a
-  // wave pays for fewer cells' setups and retries.
+  // Cells per wave and turn: 32 to 64, spread evenly over the waves of the grid and the turns
+  // each of them takes, so that a batch that does not fill every lane of the device's waves
+  // leaves fewer cells waiting for a wave's slowest one (one multirate slow step of 32^3
+  // cells: 30.9 ms with 32 cells per wave, 32.4 with 64). Fewer than 32 cost more than they
+  // give, since then twice the CUs and their shared instruction caches run the same long
+  // code (167 forced seven-stage steps of 4096 cells: 36.4 ms with 4 cells per wave, 23.2
+  // with 16, 19.7 with 32, 19.3 with 64).
   const long want = grid_waves > 0 ? grid_waves : 1;
   const long turns = (n + 64 * want - 1) / (64 * want);
   p.chunk = (int)((n + turns * want - 1) / (turns * want));
+  if (p.chunk < 32) p.chunk = 32;
   const long chunks = (n + p.chunk - 1) / p.chunk;
   const long waves = want < chunks ? want : chunks;
   p.grid = (waves + p.wpb - 1) / p.wpb;
