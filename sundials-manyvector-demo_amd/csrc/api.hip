@@ -104,6 +104,7 @@ int mvd_create(const mvd_params *p, void *stream, mvd_context **out) {
   c->g.nchem = p->nchem;
   for (int i = 0; i < 6; i++) c->g.bc[i] = p->bc[i];
   c->g.gamma = p->gamma;
+  c->g.igm = 1.0 / (p->gamma - 1.0);
   c->g.dx = (p->xr - p->xl) / p->nx;   // SetupDecomp, euler3D.hpp:412-414
   c->g.dy = (p->yr - p->yl) / p->ny;
   c->g.dz = (p->zr - p->zl) / p->nz;

@@ -9,10 +9,9 @@
 //   fe_xyface_div  : x- and y-faces of 16 x 15-cell plane tiles from one LDS staging of the
 //                    tile and its x/y halos, and their part of the divergence into wdot
 //                    (the x and y face fluxes stay in LDS); the legal-state check;
-//   fe_zface_div_xy: z-faces (tiles of 16 x-cells by 32 faces, two per thread, their
-//                    primitives staged in LDS), and the divergence of the 31 cells between
-//                    a tile's 32 faces (tiles overlap by one face), adding the x/y part
-//                    read from wdot at the kernel's start.
+//   fe_zface_div_xy: z-faces (blocks walk up columns of 16 x-cells 16 faces at a time, their
+//                    primitives staged in LDS) and the divergence of the cells between
+//                    them, adding the x/y part read from wdot.
 // Fast path with tracers (three launches):
 //   fe_xyface_div<NC>: as without tracers, then the tracers on the same x- and y-faces
 //                    (their values staged in LDS as [tracer][point] after the fluid phase)
@@ -146,21 +145,18 @@ fe_plain_div(Grid g, const double *Fx, const double *Fy, const double *Fz, Field
 // fast path
 // ------------------------------------------------------------------------------------
 
-// Raw conserved state of a stencil point, converted to direction-local order with the
-// ghost signs applied.
+// Raw conserved state of a stencil point of a z line with the ghost signs applied.
 struct RawPt {
-  double r, mn, m1, m2, e;
+  double r, mx, my, mz, e;
 };
 
-template <int D>
-__device__ inline RawPt load_raw(const Fields &f, int c, double sa, double sn) {
-  const double r = f.w[0][c], mx = f.w[1][c], my = f.w[2][c], mz = f.w[3][c], e = f.w[4][c];
+__device__ inline RawPt load_raw_z(const Fields &f, int c, double sa, double sn) {
   RawPt q;
-  q.r = r * sa;
-  q.e = e * sa;
-  if (D == 0) { q.mn = mx * sn; q.m1 = my * sa; q.m2 = mz * sa; }
-  else if (D == 1) { q.mn = my * sn; q.m1 = mx * sa; q.m2 = mz * sa; }
-  else { q.mn = mz * sn; q.m1 = my * sa; q.m2 = mx * sa; }
+  q.r = f.w[0][c] * sa;
+  q.mx = f.w[1][c] * sa;
+  q.my = f.w[2][c] * sa;
+  q.mz = f.w[3][c] * sn;
+  q.e = f.w[4][c] * sa;
   return q;
 }
 
@@ -180,10 +176,6 @@ __device__ inline int line_cell(const Grid &g, int base, int stride, int n, int 
   return base + m.src * stride;
 }
 
-__device__ inline Pt to_point(const RawPt &q, double gamma) {
-  return make_point(q.r, q.mn, q.m1, q.m2, q.e, gamma);
-}
-
 // local (rho, m_normal, m_t1, m_t2, e) flux of direction D into global component order
 template <int D>
 __device__ inline void to_global(const double (&Fl)[5], double *Fg) {
@@ -197,7 +189,7 @@ __device__ inline void to_global(const double (&Fl)[5], double *Fg) {
 // out.chem (the fluid z-faces are fe_zface_div_xy's). A block of 16 x 16 threads covers 16
 // x-cells of row j and 16 consecutive z-faces, i.e. the 15 cells between them. Per point
 // of the tile (21 per column) LDS holds the normal velocity w, the wave speed |w| + c
-// (make_point's, so the face's alpha is the fluid flux's bit for bit) and the NC tracer
+// (store_point's c, so the face's alpha is the fluid flux's bit for bit) and the NC tracer
 // values; each thread forms its face's alpha and split factors once and then the NC
 // tracer fluxes. Without the fluid flux's registers the kernel runs at a higher occupancy
 // than a fused fluid + tracer z kernel.
@@ -243,7 +235,7 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       if (!use[r]) continue;
-      raw[r] = load_raw<2>(f, cs[r], sa[r], sn[r]);
+      raw[r] = load_raw_z(f, cs[r], sa[r], sn[r]);
 #pragma unroll
       for (int v = 0; v < NC; v++) tv[r][v] = f.chem[(long)NC * cs[r] + v] * sa[r];
     }
@@ -251,9 +243,12 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
     for (int r = 0; r < NR; r++) {
       if (!use[r]) continue;
       const int s = t + 256 * r;
-      const Pt P = to_point(raw[r], g.gamma);
-      s_buf[s] = P.mn * P.ir;
-      s_buf[NPT + s] = P.a;
+      const RawPt &q = raw[r];
+      const double ir = fast_rcp(q.r);
+      const double p = (g.gamma - 1.0) * (q.e - 0.5 * (q.mx * q.mx + q.my * q.my + q.mz * q.mz) * ir);
+      const double un = q.mz * ir;
+      s_buf[s] = un;
+      s_buf[NPT + s] = fabs(un) + fast_sqrt(g.gamma * p * ir);
 #pragma unroll
       for (int v = 0; v < NC; v++) s_buf[(2 + v) * NPT + s] = tv[r][v];
     }
@@ -292,123 +287,129 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
   }
 }
 
-// z-faces without tracers (nchem = 0), adding their part to the x/y part that
-// fe_xyface_div left in out. A block of 16 x 16 threads covers 16 x-cells of row j and
-// ZF = 16 FPT consecutive z-faces (FPT per thread, 16 apart), i.e. the ZF - 1 cells between
-// them; the ZF + 5 points of each column are converted once into LDS. The x/y part of the
-// thread's cells is loaded at the start, so that its latency is spent under the staging and
-// the face fluxes instead of after them.
-template <int FPT>
-__global__ void __launch_bounds__(256)
-fe_zface_div_xy(Grid g, Fields f, FieldsOut out, double idz) {
-  constexpr int TX = 16, ZF = 16 * FPT, TPTS = ZF + 5, TC = ZF - 1;
-  constexpr int FS = TPTS * TX;
-  __shared__ double s_pt[9 * FS];
-  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-  const int nxc = (g.nx + TX - 1) / TX, ncc = (g.nz + TC - 1) / TC;
+// z-faces of the fluid fields, adding their part to the x/y part that fe_xyface_div left in
+// out. A block of 16 x 16 threads walks up a segment of `len` cells of the columns of 16
+// x-cells of row j, ZC faces at a time (one per thread). Each chunk's points (its faces' and
+// five more rows) are in LDS as primitive values; the next chunk's 16 new rows and the x/y
+// part of the cells it completes are loaded while the fluxes are formed, so only a segment's
+// first loads are waited for, no point is loaded or converted twice within a segment, and
+// the last five rows and the last face's flux are carried over. A kernel that loaded 37
+// rows for 32 faces and then computed them issued 65% of the time; at 256^3 the z faces went
+// from 0.72 to 0.55 ms with this form (0.74 at four waves per SIMD, where it spills).
+constexpr int ZX = 16, ZC = 16, ZROWS = ZC + 5;
+__global__ void __launch_bounds__(256, 3)
+fe_zface_div_xy(Grid g, Fields f, FieldsOut out, double idz, int nseg, int len) {
+  constexpr int FS = ZROWS * ZX;                        // points per field
+  constexpr int FF = (ZC + 1) * ZX;                     // fluxes per field (one carried row)
+  __shared__ double s_pt[PT_NF * FS], s_f[5 * FF];
+  const int t = threadIdx.x, tx = t % ZX, ty = t / ZX;
+  const int nxc = (g.nx + ZX - 1) / ZX;
   int b = blockIdx.x;
   const int xc = b % nxc;
   b /= nxc;
-  const int cc = b % ncc;
-  const int j = b / ncc;
-  const int k0 = cc * TC;
-  const int i = xc * TX + tx;
-  const long plane = (long)g.nx * g.ny;
-  // x/y part of the thread's cells (k0 + ty + 16 q)
-  double dxy[FPT][5];
-#pragma unroll
-  for (int q = 0; q < FPT; q++) {
-    const int c = ty + 16 * q, k = k0 + c;
-    const long cell = i + (long)g.nx * j + plane * k;
-    const bool own = c < TC && i < g.nx && k < g.nz;
-#pragma unroll
-    for (int a = 0; a < 5; a++) dxy[q][a] = own ? out.w[a][cell] : 0.0;
-  }
-  // points k0 - 3 .. k0 + ZF + 1 of the 16 columns; a thread's points (s = t + 256 n) are
-  // located first and all their loads issued before any is converted
+  const int seg = b % nseg;
+  const int j = b / nseg;
+  const int ks = seg * len, ke = min(ks + len, g.nz);   // cells [ks, ke), faces ks..ke
+  const int i = xc * ZX + tx;
+  const int plane = g.nx * g.ny;
+  const int col = i + g.nx * j;
+  const bool iok = i < g.nx;
+  // point (row e, this thread's column) or nothing
+  const auto load = [&](int e, RawPt &q) {
+    const bool use = iok && e <= g.nz + 2;
+    double sa = 1.0, sn = 1.0;
+    const int c = use ? line_cell<2>(g, col, plane, g.nz, e, sa, sn) : 0;
+    if (use) q = load_raw_z(f, c, sa, sn);
+    return use;
+  };
+  const auto store = [&](int row, const RawPt &q) {
+    (void)store_point(s_pt + row * ZX + tx, FS, q.r, q.mx, q.my, q.mz, q.e, g.gamma);
+  };
   {
-    constexpr int NR = (TPTS * TX + 255) / 256;
-    const int stride = g.nx * g.ny;
-    int cs[NR];
-    double sa[NR], sn[NR];
-    bool use[NR];
+    RawPt q0, q1;                                       // rows ty, and 16 + ty of the first chunk
+    const bool u0 = load(ks - 3 + ty, q0);
+    const bool u1 = ty < ZROWS - 16 && load(ks - 3 + 16 + ty, q1);
+    if (u0) store(ty, q0);
+    if (u1) store(16 + ty, q1);
+  }
+  for (int f0 = ks;; f0 += ZC) {
+    const bool more = f0 + ZC <= ke;
+    RawPt qn;
+    bool un = false;
+    if (more) un = load(f0 + ZC + 2 + ty, qn);          // row 5 + ty of the next chunk
+    const int k = f0 - 1 + ty;                          // the cell this chunk's faces complete
+    const bool own = iok && k >= ks && k < ke;
+    const int cell = col + plane * k;
+    double dxy[5];
+#pragma unroll
+    for (int a = 0; a < 5; a++) dxy[a] = own ? out.w[a][cell] : 0.0;
+    __syncthreads();                                    // the chunk's points are there
+    if (iok && f0 + ty <= ke) {
+      double Fl[5], Fz[5];
+      const double *base = s_pt + ty * ZX + tx;
+      face_flux_lds<PT_W, PT_V, PT_U>(base, FS, ZX, g.gamma, g.igm,
+                                      face_alpha<PT_W>(base, FS, ZX), Fl);
+      to_global<2>(Fl, Fz);
+#pragma unroll
+      for (int a = 0; a < 5; a++) s_f[a * FF + (ty + 1) * ZX + tx] = Fz[a];
+    }
+    __syncthreads();                                    // fluxes there, points read
+    if (own) {
+#pragma unroll
+      for (int a = 0; a < 5; a++) {
+        const double *F = s_f + a * FF + ty * ZX + tx;
+        out.w[a][cell] = 0.0 - (dxy[a] + (F[ZX] - F[0]) * idz);
+      }
+    }
+    if (!more) break;
+    // carry rows 16..20 of every field to rows 0..4 and the last face's flux to row 0
+    constexpr int NP = PT_NF * 5 * ZX, NALL = NP + 5 * ZX, NR = (NALL + 255) / 256;
+    double cv[NR];
 #pragma unroll
     for (int n = 0; n < NR; n++) {
-      const int s = threadIdx.x + 256 * n;
-      const int r = s / TX, x = s - r * TX;
-      const int e = k0 - 3 + r;
-      use[n] = s < TPTS * TX && xc * TX + x < g.nx && e <= g.nz + 2;
-      cs[n] = use[n] ? line_cell<2>(g, xc * TX + x + g.nx * j, stride, g.nz, e, sa[n], sn[n]) : 0;
+      const int e = t + 256 * n;
+      const int fp = e / (5 * ZX), pp = e % (5 * ZX), ef = e - NP;
+      cv[n] = e < NP ? s_pt[fp * FS + ZC * ZX + pp]
+                     : e < NALL ? s_f[(ef / ZX) * FF + ZC * ZX + ef % ZX] : 0.0;
     }
-    RawPt raw[NR];
-#pragma unroll
-    for (int n = 0; n < NR; n++)
-      if (use[n]) raw[n] = load_raw<2>(f, cs[n], sa[n], sn[n]);
+    __syncthreads();
 #pragma unroll
     for (int n = 0; n < NR; n++) {
-      if (!use[n]) continue;
-      const Pt P = to_point(raw[n], g.gamma);
-      double *pt = s_pt + threadIdx.x + 256 * n;
-      pt[0 * FS] = P.r;  pt[1 * FS] = P.mn; pt[2 * FS] = P.m1;
-      pt[3 * FS] = P.m2; pt[4 * FS] = P.e;  pt[5 * FS] = P.p;
-      pt[6 * FS] = P.ir; pt[7 * FS] = P.a;  pt[8 * FS] = P.sr;
+      const int e = t + 256 * n;
+      const int fp = e / (5 * ZX), pp = e % (5 * ZX), ef = e - NP;
+      if (e < NP) s_pt[fp * FS + pp] = cv[n];
+      else if (e < NALL) s_f[(ef / ZX) * FF + ef % ZX] = cv[n];
     }
-  }
-  __syncthreads();
-  double Fz[FPT][5];
-#pragma unroll
-  for (int q = 0; q < FPT; q++) {
-    const int fz = ty + 16 * q;
-    if (i < g.nx && k0 + fz <= g.nz) {
-      double Fl[5], alpha;
-      face_flux_lds(s_pt + fz * TX + tx, FS, TX, g.gamma, Fl, alpha);
-      to_global<2>(Fl, Fz[q]);
-    }
-  }
-  __syncthreads();   // the point tile is dead; its LDS takes the face fluxes [comp][face][x]
-#pragma unroll
-  for (int q = 0; q < FPT; q++) {
-    const int fz = ty + 16 * q;
-    if (i < g.nx && k0 + fz <= g.nz) {
-#pragma unroll
-      for (int a = 0; a < 5; a++) s_pt[(a * ZF + fz) * TX + tx] = Fz[q][a];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < FPT; q++) {
-    const int c = ty + 16 * q, k = k0 + c;
-    if (c >= TC || i >= g.nx || k >= g.nz) continue;
-    const long cell = i + (long)g.nx * j + plane * k;
-#pragma unroll
-    for (int a = 0; a < 5; a++) {
-      const double dz = (s_pt[(a * ZF + c + 1) * TX + tx] - s_pt[(a * ZF + c) * TX + tx]) * idz;
-      out.w[a][cell] = 0.0 - (dxy[q][a] + dz);
-    }
+    if (un) store(5 + ty, qn);
   }
 }
 
 // x- and y-faces of one z-plane tile together: a block covers XY_TX x XY_TY cells of plane k
 // and forms (Fx[i+1]-Fx[i])/dx + (Fy[j+1]-Fy[j])/dy for them into out (the z kernel then
 // adds the z part), so the x and y face fluxes never go to HBM. The points of the tile and
-// of its x and y halos (a cross, 3 deep) are converted once into LDS, keeping mx and my in
-// place and both wave speeds |u|+c and |v|+c, so that every point serves both directions;
-// x-faces (XY_TX+1 per row) and y-faces (XY_TY+1 per column) are 255 and 256 with the
-// 16 x 15 tile: one of each per thread.
+// of its x and y halos (a cross, 3 deep) are converted once into LDS and serve both
+// directions; x-faces (XY_TX+1 per row) and y-faces (XY_TY+1 per column) are 255 and 256
+// with the 16 x 15 tile: one of each per thread.
 //
-// With NC tracers a second phase follows on the same faces: the tracer values of the cross
-// (each point's NC values one contiguous AoS read, issued before the fluid divergence) go
-// to LDS as [tracer][point], where the fluid points were; the normal velocities of the stencil points (u on the tile's rows, v
-// on its columns) are kept aside from the fluid staging, and each face's fluid alpha stays
-// in a register; each thread then forms its x- and y-face's tracer fluxes from LDS, and
-// the divergence goes through LDS in passes of at most XY_TP tracers.
+// With NC tracers further phases follow on the same faces, at most XY_TP tracers at a time:
+// their values on the cross (issued before the previous divergence) go to LDS where dead
+// point fields were, one tracer per field; u, v and c stay, for the faces' split factors;
+// each thread forms its x- and y-face's tracer fluxes from LDS. The kernel is bound by its
+// FP64 instructions: 8 point fields and the y fluxes (40 KB) let four blocks share a CU, so
+// that four waves per SIMD hide the LDS and dependency latency (128 registers, 84% of the
+// issue rate). At 256^3: 0.92 ms, 1.26 before (three waves per SIMD, ten point fields, 786
+// FP64 instructions per face where there are now 557).
 constexpr int XY_TX = 16, XY_TY = 15;
 constexpr int XY_PX = XY_TX + 6, XY_PY = XY_TY + 6;      // point window 22 x 21
 constexpr int XY_NP = XY_PX * XY_PY;
-constexpr int XY_NF = 10;     // r, mx, my, mz, e, p, 1/r, |u|+c, sqrt(r), |v|+c
 constexpr int XY_NXF = (XY_TX + 1) * XY_TY, XY_NYF = XY_TX * (XY_TY + 1);   // 255, 256
-constexpr int XY_LDS = XY_NF * XY_NP + 5 * XY_NYF;          // points + y-face fluxes
-constexpr int XY_TP = XY_LDS / (XY_NXF + XY_NYF);           // tracers per divergence pass: 11
+constexpr int XY_LDS = PT_NF * XY_NP + 5 * XY_NYF;          // points + y-face fluxes
+constexpr int XY_TP = 5;     // fields per divergence pass: the fluid's, or at most as many tracers
+// the x-face fluxes go over dead point fields, from PT_W on; u, v (PT_U, PT_V) and c survive
+static_assert(PT_W * XY_NP + XY_TP * XY_NXF <= PT_C * XY_NP, "x fluxes over w, p, sr, c2");
+
+// LDS field that holds tracer v of a pass (the fields a tracer phase may overwrite)
+__device__ constexpr int xy_slot(int v) { return v < 4 ? PT_W + v : PT_R; }
 
 // Point q of the cross of the tile at (x0, y0) in plane k: its cell, ghost signs (all
 // fields, mx, my) and whether it is used (inside the cross and the extended grid) and a
@@ -448,17 +449,21 @@ __device__ inline XYPoint xy_point(const Grid &g, int x0, int y0, int k, int q) 
   return P;
 }
 
+// (Fx[i+1]-Fx[i])/dx + (Fy[j+1]-Fy[j])/dy of field a of a pass, cell (ci, cj) of the tile
+__device__ inline double xy_div(const double *sfx, const double *sfy, int a, int ci, int cj,
+                                double idx, double idy) {
+  const double *fx = sfx + (a * XY_TY + cj) * (XY_TX + 1) + ci;
+  const double *fy = sfy + (a * (XY_TY + 1) + cj) * XY_TX + ci;
+  return (fx[1] - fx[0]) * idx + (fy[XY_TX] - fy[0]) * idy;
+}
+
 template <int NC>
-__global__ void __launch_bounds__(256, 3)
+__global__ void __launch_bounds__(256, 4)
 fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned *flag) {
-  // points [XY_NF][XY_NP], then the y-face fluxes [5][XY_TY+1][XY_TX]; one array, so that the
-  // tracer phase can use all of it
-  __shared__ double lds[XY_LDS];
-  double *const sh = lds, *const sfy = lds + XY_NF * XY_NP;
-  // tracer stencils' normal velocities: u of the row points [XY_TY][XY_PX], then v of the
-  // column points [XY_PY][XY_TX]
-  constexpr int UN_X = XY_TY * XY_PX, UN_N = UN_X + XY_PY * XY_TX;
-  __shared__ double sun[NC > 0 ? UN_N : 1];
+  // points [PT_NF][XY_NP], then the y-face fluxes [5][XY_TY+1][XY_TX]
+  __shared__ double sh[XY_LDS];
+  double *const sfy = sh + PT_NF * XY_NP;
+  double *const sfx = sh + PT_W * XY_NP;     // [5][XY_TY][XY_TX+1], once the points are dead
   const int t = threadIdx.x;
   const int nxb = (g.nx + XY_TX - 1) / XY_TX, nyb = (g.ny + XY_TY - 1) / XY_TY;
   // The hardware deals blocks to the 8 XCDs in turn, and each XCD has its own L2. Tiles are
@@ -477,170 +482,149 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
   // A thread's points (q = t + 256 r) are located first and all their loads issued before
   // any is converted, so that their latencies overlap.
   constexpr int NR = (XY_NP + 255) / 256;
-  XYPoint pt[NR];
+  {
+    XYPoint pt[NR];
 #pragma unroll
-  for (int r = 0; r < NR; r++) pt[r] = xy_point(g, x0, y0, k, t + 256 * r);
-  double raw[NR][5];
+    for (int r = 0; r < NR; r++) pt[r] = xy_point(g, x0, y0, k, t + 256 * r);
+    double raw[NR][5];
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
+    for (int r = 0; r < NR; r++) {
 #pragma unroll
-    for (int a = 0; a < 5; a++) raw[r][a] = pt[r].use ? f.w[a][pt[r].cell] : 1.0;
-  }
-#pragma unroll
-  for (int r = 0; r < NR; r++) {
-    if (!pt[r].use) continue;
-    const double rr = raw[r][0] * pt[r].s_all, mx = raw[r][1] * pt[r].s_mx;
-    const double my = raw[r][2] * pt[r].s_my;
-    const double mz = raw[r][3] * pt[r].s_all, e = raw[r][4] * pt[r].s_all;
-    const double ir = fast_rcp(rr);
-    const double p = (g.gamma - 1.0) * (e - 0.5 * (mx * mx + my * my + mz * mz) * ir);
-    const double cs = sun_sqrt(g.gamma * p * ir);
-    const int q = t + 256 * r;
-    double *pp = sh + q;
-    pp[0 * XY_NP] = rr; pp[1 * XY_NP] = mx; pp[2 * XY_NP] = my;
-    pp[3 * XY_NP] = mz; pp[4 * XY_NP] = e;  pp[5 * XY_NP] = p;
-    pp[6 * XY_NP] = ir; pp[7 * XY_NP] = fabs(mx * ir) + cs;
-    pp[8 * XY_NP] = sun_sqrt(rr);
-    pp[9 * XY_NP] = fabs(my * ir) + cs;
-    if (NC > 0) {
-      const int yy = q / XY_PX, xx = q - yy * XY_PX;
-      if (pt[r].row) sun[(yy - 3) * XY_PX + xx] = mx * ir;
-      if (pt[r].col) sun[UN_X + yy * XY_TX + (xx - 3)] = my * ir;
+      for (int a = 0; a < 5; a++) raw[r][a] = pt[r].use ? f.w[a][pt[r].cell] : 1.0;
     }
-    if (pt[r].own) {
-      unsigned bits = 0;
-      if (!(rr > 0.0)) bits |= 1u;
-      if (!(e > 0.0)) bits |= 2u;
-      if (!(p > 0.0)) bits |= 4u;
-      if (bits) atomicOr(flag, bits);
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+      if (!pt[r].use) continue;
+      const double rr = raw[r][0] * pt[r].s_all, mx = raw[r][1] * pt[r].s_mx;
+      const double my = raw[r][2] * pt[r].s_my;
+      const double mz = raw[r][3] * pt[r].s_all, e = raw[r][4] * pt[r].s_all;
+      const double p = store_point(sh + t + 256 * r, XY_NP, rr, mx, my, mz, e, g.gamma);
+      if (pt[r].own) {
+        unsigned bits = 0;
+        if (!(rr > 0.0)) bits |= 1u;
+        if (!(e > 0.0)) bits |= 2u;
+        if (!(p > 0.0)) bits |= 4u;
+        if (bits) atomicOr(flag, bits);
+      }
     }
   }
   __syncthreads();
   // y-face t: column cx, faces between rows y0+fy-1 and y0+fy (points yy = fy..fy+5)
   const int cx = t % XY_TX, fy = t / XY_TX;
-  const bool yok = x0 + cx < g.nx && y0 + fy <= g.ny && fy <= XY_TY;
+  const bool yok = x0 + cx < g.nx && y0 + fy <= g.ny;
+  const double *const yb0 = sh + fy * XY_PX + cx + 3;
   // x-face t: row ry, faces between columns x0+fx-1 and x0+fx (points xx = fx..fx+5)
   const int ry = t / (XY_TX + 1), fx = t % (XY_TX + 1);
   const bool xok = t < XY_NXF && y0 + ry < g.ny && x0 + fx <= g.nx;
+  const double *const xb0 = sh + (ry + 3) * XY_PX + fx;
   if (yok) {
-    double Fl[5], Fy[5], alpha_y;
-    face_flux_lds_f<2, 1, 9>(sh + fy * XY_PX + cx + 3, XY_NP, XY_PX, g.gamma, Fl, alpha_y);
+    double Fl[5], Fy[5];
+    face_flux_lds<PT_V, PT_U, PT_W>(yb0, XY_NP, XY_PX, g.gamma, g.igm,
+                                    face_alpha<PT_V>(yb0, XY_NP, XY_PX), Fl);
     to_global<1>(Fl, Fy);
 #pragma unroll
     for (int a = 0; a < 5; a++) sfy[(a * (XY_TY + 1) + fy) * XY_TX + cx] = Fy[a];
   }
   double Fx[5];
-  if (xok) {
-    double alpha_x;
-    face_flux_lds_f<1, 2, 7>(sh + (ry + 3) * XY_PX + fx, XY_NP, 1, g.gamma, Fx, alpha_x);
-  }
+  if (xok)
+    face_flux_lds<PT_U, PT_V, PT_W>(xb0, XY_NP, 1, g.gamma, g.igm,
+                                    face_alpha<PT_U>(xb0, XY_NP, 1), Fx);
   __syncthreads();                    // points dead: their LDS takes the x-face fluxes
-  double *sfx = sh;                   // [5][XY_TY][XY_TX+1] (over fields 0-2)
   if (xok)
 #pragma unroll
     for (int a = 0; a < 5; a++) sfx[(a * XY_TY + ry) * (XY_TX + 1) + fx] = Fx[a];
   __syncthreads();
-  // the faces' alpha for the tracers, formed again (as the fluid flux forms it) from the
-  // wave speeds, which the x-face fluxes did not overwrite, rather than held through the
-  // fluid fluxes
-  double alpha_y = 0.0, alpha_x = 0.0;
-  if (NC > 0) {
-#pragma unroll
-    for (int l = 0; l < 6; l++) {
-      alpha_y = fmax(alpha_y, sh[9 * XY_NP + (fy + l) * XY_PX + cx + 3]);
-      alpha_x = fmax(alpha_x, sh[7 * XY_NP + (ry + 3) * XY_PX + fx + l]);
-    }
-  }
-  // the tracer values of the thread's cross points, loaded now so that their latency
-  // passes under the fluid divergence
-  double tv[NC > 0 ? NR : 1][NC > 0 ? NC : 1];
-  if (NC > 0) {
-    // the points are located again rather than kept from the staging: made opaque, the
-    // tile origin keeps the compiler from holding the staging's values across the fluxes
-    int ox = x0, oy = y0, ok = k;
-    __asm__ volatile("" : "+s"(ox), "+s"(oy), "+s"(ok));
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-      const XYPoint P = xy_point(g, ox, oy, ok, t + 256 * r);
-#pragma unroll
-      for (int v = 0; v < NC; v++)
-        tv[r][v] = P.use ? f.chem[(long)NC * P.cell + v] * P.s_all : 0.0;
-    }
-  }
   const int ci = t % XY_TX, cj = t / XY_TX;
   const bool cok = cj < XY_TY && x0 + ci < g.nx && y0 + cj < g.ny;
   const long cell = (x0 + ci) + (long)g.nx * ((y0 + cj) + (long)g.ny * k);
-  if (cok) {
+  if constexpr (NC == 0) {
+    if (cok)
 #pragma unroll
-    for (int a = 0; a < 5; a++) {
-      const double dx = (sfx[(a * XY_TY + cj) * (XY_TX + 1) + ci + 1] -
-                         sfx[(a * XY_TY + cj) * (XY_TX + 1) + ci]) * idx;
-      const double dy = (sfy[(a * (XY_TY + 1) + cj + 1) * XY_TX + ci] -
-                         sfy[(a * (XY_TY + 1) + cj) * XY_TX + ci]) * idy;
-      out.w[a][cell] = dx + dy;
-    }
-  }
-  if (NC == 0) return;
-  __syncthreads();                    // fluid fluxes read: LDS takes the tracer values
+      for (int a = 0; a < 5; a++) out.w[a][cell] = xy_div(sfx, sfy, a, ci, cj, idx, idy);
+  } else {
+    // the faces' alpha for the tracers, formed again (as the fluid flux forms it) rather
+    // than held through the fluid fluxes
+    double alpha_y = 0.0, alpha_x = 0.0;
+    if (yok) alpha_y = face_alpha<PT_V>(yb0, XY_NP, XY_PX);
+    if (xok) alpha_x = face_alpha<PT_U>(xb0, XY_NP, 1);
+    constexpr int NPASS = (NC + XY_TP - 1) / XY_TP, TP = (NC + NPASS - 1) / NPASS;
+#pragma unroll 1
+    for (int v0 = 0; v0 < NC; v0 += TP) {
+      // the pass's tracer values of the thread's cross points, loaded now so that their
+      // latency passes under the divergence of the previous pass. The points are located
+      // again rather than kept: made opaque, the tile origin keeps the compiler from
+      // holding the staging's values.
+      double tv[NR][TP];
+      {
+        int ox = x0, oy = y0, ok = k;
+        __asm__ volatile("" : "+s"(ox), "+s"(oy), "+s"(ok));
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
-    const int q = t + 256 * r;
-    if (q < XY_NP)
+        for (int r = 0; r < NR; r++) {
+          const XYPoint P = xy_point(g, ox, oy, ok, t + 256 * r);
 #pragma unroll
-      for (int v = 0; v < NC; v++) sh[v * XY_NP + q] = tv[r][v];
-  }
-  __syncthreads();
-  double Fxt[NC > 0 ? NC : 1], Fyt[NC > 0 ? NC : 1];
-  if (yok) {
-    double un[6], hp[5], hm[5];
-#pragma unroll
-    for (int l = 0; l < 6; l++) un[l] = sun[UN_X + (fy + l) * XY_TX + cx];
-    tracer_split(un, alpha_y, hp, hm);
-#pragma unroll
-    for (int v = 0; v < NC; v++) {
-      const double *c0 = sh + v * XY_NP + fy * XY_PX + cx + 3;
-      double cv[6];
-#pragma unroll
-      for (int l = 0; l < 6; l++) cv[l] = c0[l * XY_PX];
-      Fyt[v] = tracer_face_flux(cv, hp, hm);
-    }
-  }
-  if (xok) {
-    double un[6], hp[5], hm[5];
-#pragma unroll
-    for (int l = 0; l < 6; l++) un[l] = sun[ry * XY_PX + fx + l];
-    tracer_split(un, alpha_x, hp, hm);
-#pragma unroll
-    for (int v = 0; v < NC; v++) {
-      const double *c0 = sh + v * XY_NP + (ry + 3) * XY_PX + fx;
-      double cv[6];
-#pragma unroll
-      for (int l = 0; l < 6; l++) cv[l] = c0[l];
-      Fxt[v] = tracer_face_flux(cv, hp, hm);
-    }
-  }
-  // divergence in passes of XY_TP tracers (one pass for up to 11): pass fluxes
-  // [v][x-faces | y-faces] in LDS, so that each cell's tracers are written together
-#pragma unroll
-  for (int v0 = 0; v0 < NC; v0 += XY_TP) {
-    __syncthreads();                  // tracer values (first pass) / last pass's fluxes read
-#pragma unroll
-    for (int v = v0; v < NC && v < v0 + XY_TP; v++) {
-      double *fl = sh + (v - v0) * (XY_NXF + XY_NYF);
-      if (xok) fl[ry * (XY_TX + 1) + fx] = Fxt[v];
-      if (yok) fl[XY_NXF + fy * XY_TX + cx] = Fyt[v];
-    }
-    __syncthreads();
-    if (cok) {
-#pragma unroll
-      for (int v = v0; v < NC && v < v0 + XY_TP; v++) {
-        const double *fl = sh + (v - v0) * (XY_NXF + XY_NYF);
-        const double dx = (fl[cj * (XY_TX + 1) + ci + 1] - fl[cj * (XY_TX + 1) + ci]) * idx;
-        const double dy = (fl[XY_NXF + (cj + 1) * XY_TX + ci] -
-                           fl[XY_NXF + cj * XY_TX + ci]) * idy;
-        out.chem[(long)NC * cell + v] = dx + dy;
+          for (int v = 0; v < TP; v++)
+            tv[r][v] = P.use && v0 + v < NC ? f.chem[(long)NC * P.cell + v0 + v] * P.s_all : 0.0;
+        }
       }
+      if (cok) {
+        if (v0 == 0) {
+#pragma unroll
+          for (int a = 0; a < 5; a++) out.w[a][cell] = xy_div(sfx, sfy, a, ci, cj, idx, idy);
+        } else {
+#pragma unroll
+          for (int v = 0; v < TP; v++)
+            out.chem[(long)NC * cell + v0 - TP + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
+        }
+      }
+      __syncthreads();                  // the previous pass's fluxes are read
+#pragma unroll
+      for (int r = 0; r < NR; r++) {
+        const int q = t + 256 * r;
+        if (q < XY_NP)
+#pragma unroll
+          for (int v = 0; v < TP; v++) sh[xy_slot(v) * XY_NP + q] = tv[r][v];
+      }
+      __syncthreads();
+      double Fxt[TP];
+      if (yok) {
+        double un[6], hp[5], hm[5];
+#pragma unroll
+        for (int l = 0; l < 6; l++) un[l] = yb0[PT_V * XY_NP + l * XY_PX];
+        tracer_split(un, alpha_y, hp, hm);
+#pragma unroll
+        for (int v = 0; v < TP; v++) {
+          double cv[6];
+#pragma unroll
+          for (int l = 0; l < 6; l++) cv[l] = yb0[xy_slot(v) * XY_NP + l * XY_PX];
+          sfy[(v * (XY_TY + 1) + fy) * XY_TX + cx] = tracer_face_flux(cv, hp, hm);
+        }
+      }
+      if (xok) {
+        double un[6], hp[5], hm[5];
+#pragma unroll
+        for (int l = 0; l < 6; l++) un[l] = xb0[PT_U * XY_NP + l];
+        tracer_split(un, alpha_x, hp, hm);
+#pragma unroll
+        for (int v = 0; v < TP; v++) {
+          double cv[6];
+#pragma unroll
+          for (int l = 0; l < 6; l++) cv[l] = xb0[xy_slot(v) * XY_NP + l];
+          Fxt[v] = tracer_face_flux(cv, hp, hm);
+        }
+      }
+      __syncthreads();                  // tracer values dead
+      if (xok)
+#pragma unroll
+        for (int v = 0; v < TP; v++) sfx[(v * XY_TY + ry) * (XY_TX + 1) + fx] = Fxt[v];
+      __syncthreads();
     }
+    if (cok)
+#pragma unroll
+      for (int v = 0; v < TP; v++) {
+        constexpr int v0 = (NPASS - 1) * TP;
+        if (v0 + v < NC)
+          out.chem[(long)NC * cell + v0 + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
+      }
   }
 }
 
@@ -653,7 +637,6 @@ __global__ void reset_flag(unsigned *flag) { *flag = 0u; }
 static inline unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 constexpr int TILE_X = 16, TILE_F = 16;   // fe_zface_tracers' tile
-constexpr int ZFPT = 2;     // z-faces per thread in fe_zface_div_xy
 
 template <int NC>
 static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
@@ -683,10 +666,13 @@ static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScrat
                      1.0 / g.dx, 1.0 / g.dy, flag);
   tm.end(PROF_XYFACE_DIV, st);
   tm.begin(PROF_ZFACE_DIV, st);
-  constexpr int ZC = 16 * ZFPT - 1;                        // cells per z tile
-  hipLaunchKernelGGL(fe_zface_div_xy<ZFPT>,
-                     dim3((unsigned)(nxc * ((g.nz + ZC - 1) / ZC) * g.ny)), dim3(256), 0, st,
-                     g, f, o, 1.0 / g.dz);
+  // column segments: whole columns when they fill the device with four blocks per CU, else
+  // as many segments (of 16 m - 1 cells, the cells between 16 m faces) as that takes
+  const long want = (4L * 256 + nxc * g.ny - 1) / (nxc * g.ny);
+  const int zlen = ZC * (int)(((g.nz + want - 1) / want + ZC) / ZC) - 1;
+  const int nseg = (g.nz + zlen - 1) / zlen;
+  hipLaunchKernelGGL(fe_zface_div_xy, dim3((unsigned)(nxc * nseg * g.ny)), dim3(256), 0, st, g,
+                     f, o, 1.0 / g.dz, nseg, zlen);
   if constexpr (NC > 0)
     hipLaunchKernelGGL(fe_zface_tracers<NC>,
                        dim3((unsigned)(nxc * ((g.nz + TF - 2) / (TF - 1)) * g.ny)),

@@ -8,11 +8,11 @@
 //   face_flux_ref  - the reference recipe (utilities.cpp:270-479) operation by operation,
 //                    with FMA contraction disabled; used by the plain comparator kernels
 //                    and reproducible bit for bit against a non-FMA CPU build.
-//   face_flux_lds  - the same mathematics rearranged for the FP64 pipes: per-point
-//                    primitive values computed once per point (staged in LDS), 1/rho
-//                    instead of repeated divides, the left eigenvector product factored
-//                    into a handful of FMAs, the WENO weights over one common
-//                    denominator and one divide per component for both split sides.
+//   face_flux_lds  - the same mathematics rearranged for the FP64 pipes: primitive values
+//                    computed once per point (staged in LDS), the characteristic projection
+//                    taken relative to the Roe velocity, the smoothness indicators as
+//                    completed squares, the WENO weights over one common denominator and
+//                    one reciprocal per component for both split sides.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -28,6 +28,7 @@ struct Grid {
   int nx, ny, nz, nchem;
   int bc[6];               // xl, xr, yl, yr, zl, zr
   double gamma, dx, dy, dz;
+  double igm;              // 1 / (gamma - 1)
 };
 
 __host__ __device__ inline int extent(const Grid &g, int d) {
@@ -81,6 +82,19 @@ __device__ inline double fast_div(double n, double d) {
   r = fma(r, fma(-d, r, 1.0), r);
   const double q = n * r;
   return fma(fma(-d, q, n), r, q);
+}
+
+// sqrt(x) for normal x > 0, 0 for x <= 0 (SUNRsqrt's rule): Goldschmidt's iteration from
+// v_rsq_f64 with a residual correction, within 1 ulp in half the library's instructions
+// (no scaling of denormals).
+__device__ inline double fast_sqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double gq = x * y, h = 0.5 * y;
+  const double e = fma(-h, gq, 0.5);
+  gq = fma(gq, e, gq);
+  h = fma(h, e, h);
+  gq = fma(fma(-gq, gq, x), h, gq);
+  return x <= 0.0 ? 0.0 : gq;
 }
 
 // ---------------------------------------------------------------------------------
@@ -197,179 +211,210 @@ __device__ inline void face_flux_ref(double (&s)[6][5 + NC], double gamma, doubl
 // Fast face flux.
 // ---------------------------------------------------------------------------------
 
-// Per-point values along the sweep direction (direction-local momentum order).
-struct Pt {
-  double r, mn, m1, m2, e;   // conserved: rho, normal momentum, transverse momenta, energy
-  double p, ir, a, sr;       // pressure, 1/rho, |u_n| + c, sqrt(rho)
-};
+// A stencil point as the face fluxes read it from LDS, field q at base[q * FS]: the
+// primitive state, sqrt(rho), c^2 = gamma p / rho (signed) and c.
+enum { PT_R = 0, PT_U, PT_V, PT_W, PT_P, PT_SR, PT_C2, PT_C, PT_NF };
 
-__device__ inline Pt make_point(double r, double mn, double m1, double m2, double e,
-                                double gamma) {
-  Pt q;
-  q.r = r; q.mn = mn; q.m1 = m1; q.m2 = m2; q.e = e;
-  q.ir = fast_rcp(r);
-  q.p = (gamma - 1.0) * (e - 0.5 * (mn * mn + m1 * m1 + m2 * m2) * q.ir);
-  const double un = mn * q.ir;
-  q.a = fabs(un) + sun_sqrt(gamma * q.p * q.ir);
-  q.sr = sun_sqrt(r);
-  return q;
+// Converts a conserved state; returns p.
+__device__ inline double store_point(double *pp, int FS, double r, double mx, double my,
+                                     double mz, double e, double gamma) {
+  const double ir = fast_rcp(r);
+  const double p = (gamma - 1.0) * (e - 0.5 * (mx * mx + my * my + mz * mz) * ir);
+  const double c2 = gamma * p * ir;
+  pp[PT_R * FS] = r;
+  pp[PT_U * FS] = mx * ir;
+  pp[PT_V * FS] = my * ir;
+  pp[PT_W * FS] = mz * ir;
+  pp[PT_P * FS] = p;
+  pp[PT_SR * FS] = fast_sqrt(r);
+  pp[PT_C2 * FS] = c2;
+  pp[PT_C * FS] = fast_sqrt(c2);
+  return p;
 }
 
-// WENO5-JS numerator/denominator pair for one component, with three algebraic savings:
-//  * beta_k = (13/12) x_k^2 + (1/4) y_k^2 = (13/12) (x_k^2 + (3/13) y_k^2); the common factor
-//    (13/12)^2 of every (eps + beta_k)^2 cancels in the weight ratio, so the weights use
-//    (eps*12/13 + x_k^2 + (3/13) y_k^2)^2, formed as two FMAs around one product;
-//  * over the common denominator s1 s2 s3 (s_k = (eps + beta_k)^2) the weights are
-//    d_k prod_{m != k} s_m, so the linear weights d_k multiply the candidate stencils
-//    (constant coefficients) instead of the products;
-//  * the candidate stencils' 1/6 is folded into the same coefficients, and each stencil is
-//    written as its f2 part plus differences already formed for the smoothness indicators.
-// Returns the reconstructed value as num/den. epsb is eps*12/13 for the values as given;
-// WENO5 is homogeneous in the sense WENO(l f; eps) = l WENO(f; eps / l^2), so a caller
-// that reconstructs f / l passes WENO_EPSB / l^2 and multiplies the result by l.
-constexpr double WENO_EPSB = 1e-6 * 12.0 / 13.0;
-template <bool PLUS>
-__device__ inline void weno5_nd(double f0, double f1, double f2, double f3, double f4,
-                                double epsb, double &num, double &den) {
-  const double c = 3.0 / 13.0;
-  const double d01 = f1 - f0, d12 = f2 - f1, d23 = f3 - f2, d34 = f4 - f3;
-  const double x1 = d34 - d23, x2 = d23 - d12, x3 = d12 - d01;
-  const double y1 = x1 - 2.0 * d23;         // 3 f2 - 4 f3 + f4
-  const double y2 = d12 + d23;              // -(f1 - f3)
-  const double y3 = x3 + 2.0 * d12;         // f0 - 4 f1 + 3 f2
-  const double b1 = fma(x1, x1, fma(c * y1, y1, epsb));
-  const double b2 = fma(x2, x2, fma(c * y2, y2, epsb));
-  const double b3 = fma(x3, x3, fma(c * y3, y3, epsb));
-  const double s1 = b1 * b1, s2 = b2 * b2, s3 = b3 * b3;
-  const double s23 = s2 * s3, s13 = s1 * s3, s12 = s1 * s2;
-  // d_k / 6 times the candidate stencils, each written as (6 d_k / 6) f2 plus differences:
-  // the f2 terms add up to f2 den, so num = f2 den + sum_k q'_k prod_{m != k} s_m
-  double q1, q2, q3;
-  if (PLUS) {               // d = (3, 6, 1) / 10
-    q1 = fma(0.2, d23, -0.05 * d34);                       // (2 f2 + 5 f3 - f4) / 20
-    q2 = fma(0.1, d12, 0.2 * d23);                         // (-f1 + 5 f2 + 2 f3) / 10
-    q3 = fma(1.0 / 12.0, d12, (-1.0 / 30.0) * d01);        // (2 f0 - 7 f1 + 11 f2) / 60
-    den = fma(0.3, s23, fma(0.6, s13, 0.1 * s12));
-  } else {                  // d = (1, 6, 3) / 10
-    q1 = fma(-1.0 / 12.0, d23, (1.0 / 30.0) * d34);        // (11 f2 - 7 f3 + 2 f4) / 60
-    q2 = fma(-0.2, d12, -0.1 * d23);                       // (2 f1 + 5 f2 - f3) / 10
-    q3 = fma(-0.2, d12, 0.05 * d01);                       // (-f0 + 5 f1 + 2 f2) / 20
-    den = fma(0.1, s23, fma(0.6, s13, 0.3 * s12));
-  }
-  num = fma(f2, den, fma(q1, s23, fma(q2, s13, q3 * s12)));
+// WENO5-JS over f0..f4 (the f+ formula; the f- one is the same function of the reversed
+// values): the reconstruction is f2 + (2/3) S / den. With the differences a, b, c, d of
+// neighbouring values the smoothness indicators are completed squares,
+//   beta_3 = 4/3 ((a - 11/8 b)^2 + 39/64 b^2), beta_2 = 4/3 ((b - 5/8 c)^2 + 39/64 c^2),
+//   beta_1 = 4/3 ((d - 11/8 c)^2 + 39/64 c^2),
+// whose second squares are shared; the common factor (4/3)^2 cancels in the weight ratio, so
+// eps enters as 3/4 eps. Over the common denominator the weights are d_k times products of
+// the other two (eps + beta)^2; den = (10/3) sum of them, and the candidate stencils are
+// written relative to f2: c - d/4, c + b/2, 5/12 b - a/6 (times 2/3 and the linear weights'
+// ratios 1, 2, 1/3). 29 operations. epsb is 3/4 eps for the values as given; WENO5 is
+// homogeneous in the sense WENO(l f; eps) = l WENO(f; eps / l^2), so a caller that
+// reconstructs f / l passes WENO_EPSB / l^2 and multiplies the result by l.
+constexpr double WENO_EPSB = 0.75e-6;
+
+// A constant in a scalar register pair. Given as a literal the compiler puts it into a
+// two-address FMA and copies the addend it would overwrite (40 64-bit moves per face).
+__device__ inline double scalar_const(double v) {
+  __asm__("" : "+s"(v));
+  return v;
 }
 
-// Sum of the f+ and f- reconstructions of one component with a single divide:
-//   n+/d+ + n-/d- = (n+ d- + n- d+) / (d+ d-)
-// (d+ d- is a product of four (eps+beta)^2 factors: finite for |beta| < 1e38).
-__device__ inline double weno5_pair(const double (&fp)[5], const double (&fm)[5]) {
-  double np, dp, nm, dm;
-  weno5_nd<true>(fp[0], fp[1], fp[2], fp[3], fp[4], WENO_EPSB, np, dp);
-  weno5_nd<false>(fm[0], fm[1], fm[2], fm[3], fm[4], WENO_EPSB, nm, dm);
-  return fast_div(fma(np, dm, nm * dp), dp * dm);
+__device__ inline void weno5_sd(double f0, double f1, double f2, double f3, double f4,
+                                double epsb, double &S, double &den) {
+  const double a = f1 - f0, b = f2 - f1, c = f3 - f2, d = f4 - f3;
+  const double c1375 = scalar_const(-1.375), c0625 = scalar_const(-0.625);
+  const double c025 = scalar_const(-0.25);
+  const double t3 = fma(c1375, b, a), t2 = fma(c0625, c, b), t1 = fma(c1375, c, d);
+  const double wb = fma(0.609375 * b, b, epsb), wc = fma(0.609375 * c, c, epsb);
+  const double b1 = fma(t1, t1, wc), b2 = fma(t2, t2, wc), b3 = fma(t3, t3, wb);
+  const double p1 = b2 * b3, p2 = b1 * b3, p3 = b1 * b2;
+  const double s1 = p1 * p1, s2 = p2 * p2, s3 = p3 * p3;
+  const double q1 = fma(c025, d, c), q2 = fma(0.5, b, c);
+  const double q3 = fma(-1.0 / 6.0, a, (5.0 / 12.0) * b);
+  S = fma(q1, s1, fma(q2, s2, q3 * s3));
+  den = fma(1.0 / 3.0, s3, fma(2.0, s2, s1));
+}
+
+// The corrections of the f+ and f- reconstructions together, with a single reciprocal:
+//   q = S+ / den+ + S- / den-,   f+ + f- = f2+ + f2- + (2/3) q
+// (den+ den- is a product of eight (eps + beta) factors: finite for |beta| < 1e38).
+// fp: f+ at points 0..4; fm: f- at points 5..1 (reversed).
+__device__ inline double weno5_q(const double (&fp)[5], const double (&fm)[5], double epsb) {
+  double Sp, dp, Sm, dm;
+  weno5_sd(fp[0], fp[1], fp[2], fp[3], fp[4], epsb, Sp, dp);
+  weno5_sd(fm[0], fm[1], fm[2], fm[3], fm[4], epsb, Sm, dm);
+  return fma(Sp, dm, Sm * dp) * fast_rcp(dp * dm);
+}
+
+__device__ inline double weno5_both(const double (&fp)[5], const double (&fm)[5], double epsb) {
+  return fma(2.0 / 3.0, weno5_q(fp, fm, epsb), fp[2] + fm[2]);
+}
+
+// Lax-Friedrichs speed of a face: the largest |u_n| + c of its six points.
+template <int UN>
+__device__ inline double face_alpha(const double *base, int FS, int LS) {
+  double alpha = 0.0;
+#pragma unroll
+  for (int l = 0; l < 6; l++)
+    alpha = fmax(alpha, fabs(base[UN * FS + l * LS]) + base[PT_C * FS + l * LS]);
+  return alpha;
 }
 
 // Face flux with the 6-point stencil read from LDS as it is needed (point l, field q at
-// base[q*FS + l*LS]), one split side at a time, so only one side's 25 projected values are
-// live. Fields: 0 r, FMN the normal momentum, FM1 the first transverse one, 3 the second,
-// 4 e, 5 p, 6 1/r, FA |u_n| + c, 8 sqrt(r) (Pt order is FMN = 1, FM1 = 2, FA = 7; a point
-// shared by x- and y-faces keeps mx, my in 1, 2 and both speeds, in 7 and 9).
-template <int FMN, int FM1, int FA>
-__device__ inline void face_flux_lds_f(const double *base, int FS, int LS, double gamma,
-                                       double (&F)[5], double &alpha_out) {
-  const double gm = gamma - 1.0;
-  double alpha = 0.0;
-#pragma unroll
-  for (int l = 0; l < 6; l++) alpha = fmax(alpha, base[FA * FS + l * LS]);
-  double u, v, w, H;
+// base[q*FS + l*LS]), one split side at a time. UN, U1, U2: the normal and transverse velocity fields; F in direction-local order.
+// The split flux of a point is (F +- alpha U) / 2 with, for x0 = rho (u +- alpha),
+//   mass x0, normal momentum x0 u + p, transverse x0 v, x0 w, energy x0 E + u p,
+// and its products with the left eigenvectors, taken in the frame of the Roe velocity
+// (du, dv, dw the velocity differences, D = du^2 + dv^2 + dw^2), are
+//   A = x0 du + p,  K = p (u +- alpha + (gamma-1) du) + (gamma-1)/2 x0 D,
+//   K - A, x0 dv, x0 dw, x0 - K / cs, K + A
+// up to constant factors: no cancellation of the mean flow, five fields per point. The Roe
+// cs (the reference's csnd, the squared sound speed) is the weighted mean of the points' c^2
+// plus (gamma-1)/2 w_L w_R |V_L - V_R|^2.
+template <int UN, int U1, int U2>
+__device__ inline void face_flux_lds(const double *base, int FS, int LS, double gamma,
+                                     double igm, double alpha, double (&F)[5]) {
+  const double gm = gamma - 1.0, gmh = 0.5 * gm;
+  double u, v, w, cs;
   {
     const double *L = base + 2 * LS, *R = base + 3 * LS;
-    const double Lsr = L[8 * FS], Rsr = R[8 * FS];
+    const double Lsr = L[PT_SR * FS], Rsr = R[PT_SR * FS];
     const double iden = fast_rcp(Lsr + Rsr);
-    const double wl = Lsr * L[6 * FS], wr = Rsr * R[6 * FS];
-    u = (L[FMN * FS] * wl + R[FMN * FS] * wr) * iden;
-    v = (L[FM1 * FS] * wl + R[FM1 * FS] * wr) * iden;
-    w = (L[3 * FS] * wl + R[3 * FS] * wr) * iden;
-    H = ((L[5 * FS] + L[4 * FS]) * wl + (R[5 * FS] + R[4 * FS]) * wr) * iden;
+    const double wl = Lsr * iden, wr = Rsr * iden;
+    const double uL = L[UN * FS], vL = L[U1 * FS], zL = L[U2 * FS];
+    const double uR = R[UN * FS], vR = R[U1 * FS], zR = R[U2 * FS];
+    u = fma(uL, wl, uR * wr);
+    v = fma(vL, wl, vR * wr);
+    w = fma(zL, wl, zR * wr);
+    const double du = uR - uL, dv = vR - vL, dw = zR - zL;
+    cs = fma(L[PT_C2 * FS], wl, R[PT_C2 * FS] * wr) +
+         gmh * (wl * wr) * fma(du, du, fma(dv, dv, dw * dw));
   }
-  const double qsq = u * u + v * v + w * w;
-  const double hq = 0.5 * qsq;
-  const double cs = gm * (H - hq);
   const double ci = fast_rcp(cs);
-  const double hci = 0.25 * ci;
-  // K = (gamma-1)(q^2/2 x0 - u x1 - v x2 - w x3 + x4) with the factor folded in
-  const double gh = gm * hq, gu = gm * u, gv = gm * v, gw = gm * w;
-  // The characteristic values are reconstructed without their constant factors (hci for
-  // components 0 and 4, 1/2 for 1..3), with eps scaled to match (1 / hci^2 = 16 cs^2).
-  const double eps04 = (16.0 * WENO_EPSB) * (cs * cs), eps13 = 4.0 * WENO_EPSB;
-  double nps[5], dps[5], ff[5];
+  // The characteristic values are reconstructed without their constant factors (hci = 1/(4
+  // cs) for components 0 and 4, 1/2 for 1..3), with eps scaled to match (1 / hci^2 = 16
+  // cs^2).
+  // ff1, ff2, ff3: the shear and entropy components (times 1/2); h04 and d04: half the sum
+  // and half the difference of the acoustic ones (times hci), formed from K and A so that
+  // the pressure-sized parts of K - A and K + A never meet in a rounded sum
+  double ff1, ff2, ff3, h04, d04, xp[5], xm[5], D[6];            // xp[l]: point l, xm[l]: point 5 - l
+  {
+    double dv[6], dw[6];
 #pragma unroll
-  for (int side = 0; side < 2; side++) {
-    __builtin_amdgcn_sched_barrier(0);
-    double pr[5][5];
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      const double *q = base + (l + side) * LS;
-      const double r = q[0], mn = q[FMN * FS], m1 = q[FM1 * FS], m2 = q[3 * FS],
-                   e = q[4 * FS];
-      const double p = q[5 * FS];
-      const double ul = mn * q[6 * FS];
-      const double sa = side == 0 ? alpha : -alpha;
-      const double us = ul + sa;
-      const double x0 = fma(sa, r, mn);
-      const double x1 = fma(us, mn, p);
-      const double x2 = us * m1;
-      const double x3 = us * m2;
-      const double x4 = fma(us, e, ul * p);
-      const double K = fma(gm, x4, fma(-gw, x3, fma(-gv, x2, fma(-gu, x1, gh * x0))));
-      const double A = fma(u, x0, -x1);
-      pr[l][0] = A + K;                  // times hci
-      pr[l][1] = fma(-v, x0, x2);        // times 1/2
-      pr[l][2] = fma(-w, x0, x3);        // times 1/2
-      pr[l][3] = fma(-ci, K, x0);        // times 1/2
-      pr[l][4] = K - A;                  // times hci
+    for (int l = 0; l < 6; l++) {
+      const double *q = base + l * LS;
+      const double un = q[UN * FS], r = q[PT_R * FS];
+      if (l < 5) xp[l] = r * (un + alpha);
+      if (l > 0) xm[5 - l] = r * (un - alpha);
+      const double du = un - u;
+      dv[l] = q[U1 * FS] - v;
+      dw[l] = q[U2 * FS] - w;
+      D[l] = gmh * fma(du, du, fma(dv[l], dv[l], dw[l] * dw[l]));
     }
+    // the shear components (times 1/2)
+    const double eps13 = 4.0 * WENO_EPSB;
+    double fp[5], fm[5];
 #pragma unroll
-    for (int c = 0; c < 5; c++) {
-      const double eps = (c == 0 || c == 4) ? eps04 : eps13;
-      if (side == 0) {
-        weno5_nd<true>(pr[0][c], pr[1][c], pr[2][c], pr[3][c], pr[4][c], eps, nps[c], dps[c]);
-      } else {
-        double nm, dm;
-        weno5_nd<false>(pr[0][c], pr[1][c], pr[2][c], pr[3][c], pr[4][c], eps, nm, dm);
-        ff[c] = fast_div(fma(nps[c], dm, nm * dps[c]), dps[c] * dm);
+    for (int l = 0; l < 5; l++) { fp[l] = xp[l] * dv[l]; fm[l] = xm[l] * dv[5 - l]; }
+    ff1 = weno5_both(fp, fm, eps13);
+    __asm__ volatile("" : "+v"(ff1));
+#pragma unroll
+    for (int l = 0; l < 5; l++) { fp[l] = xp[l] * dw[l]; fm[l] = xm[l] * dw[5 - l]; }
+    ff2 = weno5_both(fp, fm, eps13);
+    __asm__ volatile("" : "+v"(ff2));
+  }
+  // an offset the compiler does not know to be zero: the points are read again here instead
+  // of being kept in registers through the shear components
+  int again = 0;
+  __asm__ volatile("" : "+v"(again));
+  {
+    double Kp[5], Km[5], Ap[5], Am[5], fp[5], fm[5];
+    const double tp = fma(-gm, u, alpha), tm = fma(-gm, u, -alpha);
+#pragma unroll
+    for (int l = 0; l < 6; l++) {
+      const double *q = base + l * LS + again;
+      const double un = q[UN * FS], p = q[PT_P * FS];
+      const double du = un - u;
+      if (l < 5) {
+        Kp[l] = fma(p, fma(gamma, un, tp), xp[l] * D[l]);
+        Ap[l] = fma(xp[l], du, p);
+      }
+      if (l > 0) {
+        Km[5 - l] = fma(p, fma(gamma, un, tm), xm[5 - l] * D[l]);
+        Am[5 - l] = fma(xm[5 - l], du, p);
       }
     }
+    // the entropy component (times 1/2), then the acoustic ones (times hci)
+#pragma unroll
+    for (int l = 0; l < 5; l++) { fp[l] = fma(-ci, Kp[l], xp[l]); fm[l] = fma(-ci, Km[l], xm[l]); }
+    ff3 = weno5_both(fp, fm, 4.0 * WENO_EPSB);
+    __asm__ volatile("" : "+v"(ff3));
+    const double eps04 = (16.0 * WENO_EPSB) * (cs * cs);
+#pragma unroll
+    for (int l = 0; l < 5; l++) { fp[l] = Kp[l] - Ap[l]; fm[l] = Km[l] - Am[l]; }
+    double q0 = weno5_q(fp, fm, eps04);
+    __asm__ volatile("" : "+v"(q0));
+#pragma unroll
+    for (int l = 0; l < 5; l++) { fp[l] = Kp[l] + Ap[l]; fm[l] = Km[l] + Am[l]; }
+    const double q4 = weno5_q(fp, fm, eps04);
+    h04 = fma(1.0 / 3.0, q0 + q4, Kp[2] + Km[2]);
+    d04 = fma(1.0 / 3.0, q4 - q0, Ap[2] + Am[2]);
   }
-  __builtin_amdgcn_sched_barrier(0);
-  // the factors back: hci on 0 and 4 (cs hci = 1/4), 1/2 on 1..3
-  const double s04 = hci * (ff[0] + ff[4]);
-  const double d40 = 0.25 * (ff[4] - ff[0]);
-  const double f1 = 0.5 * ff[1], f2 = 0.5 * ff[2], f3 = 0.5 * ff[3];
-  F[0] = s04 + f3;
-  F[1] = u * F[0] + d40;
-  F[2] = v * F[0] + f1;
-  F[3] = w * F[0] + f2;
-  F[4] = H * s04 + u * d40 + v * f1 + w * f2 + hq * f3;
-  alpha_out = alpha;
-}
-
-__device__ inline void face_flux_lds(const double *base, int FS, int LS, double gamma,
-                                     double (&F)[5], double &alpha_out) {
-  face_flux_lds_f<1, 2, 7>(base, FS, LS, gamma, F, alpha_out);
+  // the factors back (cs hci = 1/4); H = cs / (gamma-1) + q^2/2
+  const double d40 = 0.5 * d04, f1 = 0.5 * ff1, f2t = 0.5 * ff2;
+  const double hq = 0.5 * fma(u, u, fma(v, v, w * w));
+  F[0] = 0.5 * fma(ci, h04, ff3);
+  F[1] = fma(u, F[0], d40);
+  F[2] = fma(v, F[0], f1);
+  F[3] = fma(w, F[0], f2t);
+  F[4] = fma(0.5 * igm, h04, fma(hq, F[0], fma(u, d40, fma(v, f1, w * f2t))));
 }
 
 // Species (passive tracer) face flux for one component from its 6 point values c[l]
 // (utilities.cpp:376-377,395,439,473): component-wise WENO5 of the split fluxes
 // (u c +- alpha c) / 2, no characteristic projection. The split fluxes are formed as
-// c[l] hp[l] and c[l+1] hm[l] with the face's split factors hp[l] = (u_l + alpha) / 2 and
-// hm[l] = (u_{l+1} - alpha) / 2 (tracer_split), which every tracer of the face shares.
+// c[l] hp[l] and c[5-l] hm[l] with the face's split factors hp[l] = (u_l + alpha) / 2 and
+// hm[l] = (u_{5-l} - alpha) / 2 (tracer_split), which every tracer of the face shares.
 __device__ inline void tracer_split(const double (&un)[6], double alpha, double (&hp)[5],
                                     double (&hm)[5]) {
 #pragma unroll
   for (int l = 0; l < 5; l++) {
     hp[l] = 0.5 * (un[l] + alpha);
-    hm[l] = 0.5 * (un[l + 1] - alpha);
+    hm[l] = 0.5 * (un[5 - l] - alpha);
   }
 }
 
@@ -379,9 +424,9 @@ __device__ inline double tracer_face_flux(const double (&c)[6], const double (&h
 #pragma unroll
   for (int l = 0; l < 5; l++) {
     fp[l] = c[l] * hp[l];
-    fm[l] = c[l + 1] * hm[l];
+    fm[l] = c[5 - l] * hm[l];
   }
-  return weno5_pair(fp, fm);
+  return weno5_both(fp, fm, WENO_EPSB);
 }
 
 }  // namespace mvd
