@@ -99,9 +99,10 @@ int mvd_max_wave_speed(mvd_context *ctx, const double *const *w, double *alpha);
 int mvd_stability(mvd_context *ctx, const double *const *w, double t, double *dt_stab);
 
 /* fslow (multirate_chem_hydro_main.cpp:996-1083) / fexpl (imex_chem_hydro_main.cpp:910-1000):
- * scales chem by the Dengo scale, overwrites w[4] (et) from the gas energy and kinetic
- * energy, calls fe(), moves etdot into the gas-energy slot of wdot[5], zeroes wdot[4] and
- * unscales chem. Requires nchem > 0 and mvd_chem_setup. */
+ * overwrites w[4] (et) from the scaled gas energy and kinetic energy, evaluates fe() of the
+ * species times their Dengo scale, moves etdot into the gas-energy slot of wdot[5] and zeroes
+ * wdot[4]. w[5] is left as it is (the reference scales it in place and back, which may change
+ * its last bit). Requires nchem = 10 and mvd_chem_setup. */
 int mvd_fslow(mvd_context *ctx, double t, double *const *w, double *const *wdot);
 /* PostprocessStep of the IMEX driver (imex_chem_hydro_main.cpp:1002-1050): apply the Dengo
  * scaling to w[5] in place, rebuild et = ge / EnergyUnits + |m|^2 / (2 rho) from the gas

@@ -294,13 +294,10 @@ int mvd_fslow(mvd_context *ctx, double t, double *const *w, double *const *wdot)
   if (rc) return rc;
   if (ctx->chem.n != (long)ctx->g.nx * ctx->g.ny * ctx->g.nz || ctx->g.nchem != mvd::NSP)
     return MVD_BAD_ARGUMENT;
-  if (mvd::fslow_prepare_launch(ctx->g, w, ctx->chem.scale, 1.0 / ctx->energy_units, ctx->stream))
-    return MVD_DEVICE_ERROR;
-  rc = fe_common(ctx, (const double *const *)w, wdot, false, false);
-  if (rc) return rc;
-  if (mvd::fslow_finish_launch(ctx->g, wdot, ctx->stream)) return MVD_DEVICE_ERROR;
-  const long nch = ctx->chem.n * mvd::NSP;
-  if (mvd::chem_scale_launch(nch, w[5], ctx->chem.scale, 0, ctx->stream)) return MVD_DEVICE_ERROR;
+  rc = mvd::fslow_launch(ctx->g, w, wdot, ctx->chem.scale, 1.0 / ctx->energy_units, false, ctx->fe,
+                         ctx->stream);
+  if (rc == -2) return MVD_UNSUPPORTED;
+  if (rc) return MVD_DEVICE_ERROR;
   if (!dev_ok(hipMemcpyAsync(ctx->host_flag, ctx->fe.flag, sizeof(unsigned),
                              hipMemcpyDeviceToHost, ctx->stream)) ||
       !dev_ok(hipStreamSynchronize(ctx->stream)))
@@ -365,9 +362,8 @@ int mvd_postprocess_step(mvd_context *ctx, double, double *const *w) {
   const int rc = check_ptrs(ctx, (const double *const *)w);
   if (rc) return rc;
   // apply_Dengo_scaling, et from the gas energy and the kinetic energy, unapply
-  if (mvd::fslow_prepare_launch(ctx->g, w, ctx->chem.scale, 1.0 / ctx->energy_units,
-                                ctx->stream) ||
-      mvd::chem_scale_launch(ctx->chem.n * mvd::NSP, w[5], ctx->chem.scale, 0, ctx->stream) ||
+  if (mvd::postprocess_launch(ctx->g, w, ctx->chem.scale, 1.0 / ctx->energy_units,
+                              ctx->stream) ||
       !dev_ok(hipStreamSynchronize(ctx->stream)))
     return MVD_DEVICE_ERROR;
   return MVD_SUCCESS;

@@ -193,9 +193,15 @@ __device__ inline void to_global(const double (&Fl)[5], double *Fg) {
 // values; each thread forms its face's alpha and split factors once and then the NC
 // tracer fluxes. Without the fluid flux's registers the kernel runs at a higher occupancy
 // than a fused fluid + tracer z kernel.
-template <int NC>
+//
+// ST: doubles per cell record of f.chem and out.chem. MODE (fslow's rates, NC = 9 species of
+// records of 10): 1 also moves the total-energy rate out.w[4] (final: the fluid kernels have
+// run) into the record's tenth slot and leaves zero there; 2 in addition converts the whole
+// record to the scaled variables (FeSlow).
+enum { TR_PLAIN = 0, TR_SLOW, TR_SLOW_SCALED };
+template <int NC, int ST, int MODE>
 __global__ void __launch_bounds__(256)
-fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
+fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz, FeSlow slow) {
   constexpr int TX = 16, TF = 16, TPTS = TF + 5, TC = TF - 1, NPT = TPTS * TX;
   constexpr int NR = (NPT + 255) / 256;
   constexpr int PT_SZ = (2 + NC) * NPT, FL_SZ = NC * TF * TX;
@@ -214,7 +220,9 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
   const long cell = i + (long)g.nx * (j + (long)g.ny * k);
   double dxy[NC];
 #pragma unroll
-  for (int v = 0; v < NC; v++) dxy[v] = cell_ok ? out.chem[(long)NC * cell + v] : 0.0;
+  for (int v = 0; v < NC; v++) dxy[v] = cell_ok ? out.chem[(long)ST * cell + v] : 0.0;
+  double erate = 0.0;
+  if (MODE != TR_PLAIN && cell_ok) erate = out.w[4][cell];
   // points k0 - 3 .. k0 + TF + 1 of the 16 columns: located, loaded, then converted
   {
     const int stride = g.nx * g.ny;
@@ -237,7 +245,7 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
       if (!use[r]) continue;
       raw[r] = load_raw_z(f, cs[r], sa[r], sn[r]);
 #pragma unroll
-      for (int v = 0; v < NC; v++) tv[r][v] = f.chem[(long)NC * cs[r] + v] * sa[r];
+      for (int v = 0; v < NC; v++) tv[r][v] = f.chem[(long)ST * cs[r] + v] * sa[r];
     }
 #pragma unroll
     for (int r = 0; r < NR; r++) {
@@ -280,10 +288,16 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz) {
   }
   __syncthreads();
   if (!cell_ok) return;
+  const double *const sc = MODE == TR_SLOW_SCALED ? slow.scale + (long)ST * cell : nullptr;
 #pragma unroll
   for (int v = 0; v < NC; v++) {
     const double dz = (s_buf[(v * TF + ty + 1) * TX + tx] - s_buf[(v * TF + ty) * TX + tx]) * idz;
-    out.chem[(long)NC * cell + v] = 0.0 - (dxy[v] + dz);
+    const double r = 0.0 - (dxy[v] + dz);
+    out.chem[(long)ST * cell + v] = MODE == TR_SLOW_SCALED ? r / sc[v] : r;
+  }
+  if (MODE != TR_PLAIN) {
+    out.chem[(long)ST * cell + NC] = MODE == TR_SLOW_SCALED ? erate * slow.eunits / sc[NC] : erate;
+    out.w[4][cell] = 0.0;
   }
 }
 
@@ -457,7 +471,7 @@ __device__ inline double xy_div(const double *sfx, const double *sfy, int a, int
   return (fx[1] - fx[0]) * idx + (fy[XY_TX] - fy[0]) * idy;
 }
 
-template <int NC>
+template <int NC, int ST>
 __global__ void __launch_bounds__(256, 4)
 fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned *flag) {
   // points [PT_NF][XY_NP], then the y-face fluxes [5][XY_TY+1][XY_TX]
@@ -563,7 +577,7 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
           const XYPoint P = xy_point(g, ox, oy, ok, t + 256 * r);
 #pragma unroll
           for (int v = 0; v < TP; v++)
-            tv[r][v] = P.use && v0 + v < NC ? f.chem[(long)NC * P.cell + v0 + v] * P.s_all : 0.0;
+            tv[r][v] = P.use && v0 + v < NC ? f.chem[(long)ST * P.cell + v0 + v] * P.s_all : 0.0;
         }
       }
       if (cok) {
@@ -573,7 +587,7 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
         } else {
 #pragma unroll
           for (int v = 0; v < TP; v++)
-            out.chem[(long)NC * cell + v0 - TP + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
+            out.chem[(long)ST * cell + v0 - TP + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
         }
       }
       __syncthreads();                  // the previous pass's fluxes are read
@@ -623,7 +637,7 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
       for (int v = 0; v < TP; v++) {
         constexpr int v0 = (NPASS - 1) * TP;
         if (v0 + v < NC)
-          out.chem[(long)NC * cell + v0 + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
+          out.chem[(long)ST * cell + v0 + v] = xy_div(sfx, sfy, v, ci, cj, idx, idy);
       }
   }
 }
@@ -638,14 +652,15 @@ static inline unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) 
 
 constexpr int TILE_X = 16, TILE_F = 16;   // fe_zface_tracers' tile
 
-template <int NC>
+// NC tracers in records of ST doubles
+template <int NC, int ST = NC, int MODE = TR_PLAIN>
 static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
-                     hipStream_t st, bool plain, unsigned *accum) {
+                     hipStream_t st, bool plain, unsigned *accum, const FeSlow &slow = {}) {
   const long nxp = g.nx + 1, nyp = g.ny + 1, nzp = g.nz + 1;
   unsigned *const flag = accum ? accum : s.flag;
   if (!accum) hipLaunchKernelGGL(reset_flag, dim3(1), dim3(1), 0, st, s.flag);
   KernelTimer &tm = s.timer;
-  if (plain) {
+  if constexpr (MODE == TR_PLAIN) if (plain) {
     tm.begin(PROF_PLAIN_FACES, st);
     hipLaunchKernelGGL(fe_plain_faces<NC>, dim3(nblocks(nxp * nyp * nzp, 256)), dim3(256), 0, st,
                        g, f, s.Fx, s.Fy, s.Fz, flag);
@@ -662,7 +677,7 @@ static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScrat
   const long nxc = (g.nx + TX - 1) / TX;
   const long nxyb = ((long)(g.nx + XY_TX - 1) / XY_TX) * ((g.ny + XY_TY - 1) / XY_TY) * g.nz;
   tm.begin(PROF_XYFACE_DIV, st);
-  hipLaunchKernelGGL(fe_xyface_div<NC>, dim3((unsigned)nxyb), dim3(256), 0, st, g, f, o,
+  hipLaunchKernelGGL((fe_xyface_div<NC, ST>), dim3((unsigned)nxyb), dim3(256), 0, st, g, f, o,
                      1.0 / g.dx, 1.0 / g.dy, flag);
   tm.end(PROF_XYFACE_DIV, st);
   tm.begin(PROF_ZFACE_DIV, st);
@@ -674,17 +689,28 @@ static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScrat
   hipLaunchKernelGGL(fe_zface_div_xy, dim3((unsigned)(nxc * nseg * g.ny)), dim3(256), 0, st, g,
                      f, o, 1.0 / g.dz, nseg, zlen);
   if constexpr (NC > 0)
-    hipLaunchKernelGGL(fe_zface_tracers<NC>,
+    hipLaunchKernelGGL((fe_zface_tracers<NC, ST, MODE>),
                        dim3((unsigned)(nxc * ((g.nz + TF - 2) / (TF - 1)) * g.ny)),
-                       dim3(TX * TF), 0, st, g, f, o, 1.0 / g.dz);
+                       dim3(TX * TF), 0, st, g, f, o, 1.0 / g.dz, slow);
   tm.end(PROF_ZFACE_DIV, st);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// 32-bit cell indices in the fast kernels
+static bool fe_too_large(const Grid &g) {
+  return (long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1) >= (1L << 31) / 16;
+}
+
+int fe_slow_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
+                   hipStream_t st, unsigned *accum, const FeSlow &slow) {
+  if (fe_too_large(g) || g.nchem != 10) return -2;
+  return slow.scale ? launch_fe<9, 10, TR_SLOW_SCALED>(g, f, o, s, st, false, accum, slow)
+                    : launch_fe<9, 10, TR_SLOW>(g, f, o, s, st, false, accum, slow);
+}
+
 int fe_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
               hipStream_t st, bool plain, unsigned *accum) {
-  // 32-bit cell indices in the fast kernels
-  if ((long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1) >= (1L << 31) / 16) return -2;
+  if (fe_too_large(g)) return -2;
   switch (g.nchem) {
     case 0: return launch_fe<0>(g, f, o, s, st, plain, accum);
     case 1: return launch_fe<1>(g, f, o, s, st, plain, accum);

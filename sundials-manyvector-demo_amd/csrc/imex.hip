@@ -144,23 +144,9 @@ int imex_evolve(const Grid &g, FeScratch &fe, ChemState &ch, double eunit_inv, I
       // Fe_i = fexpl(z_i)
       double *Fp[6];
       sub_ptrs(Fei, n, Fp);
-      if (fslow_prepare_launch(g, Zp, ch.scale, eunit_inv, st)) { rc = -1; break; }
-      Fields fz;
-      for (int q = 0; q < 5; q++) fz.w[q] = Zp[q];
-      fz.chem = Zp[5];
-      FieldsOut fo;
-      for (int q = 0; q < 5; q++) fo.w[q] = Fp[q];
-      fo.chem = Fp[5];
-      const int frc = fe_launch(g, fz, fo, fe, st, false, m.flag);   // bits into the run's flag
-      if (frc) { rc = frc; break; }
-      if (fslow_finish_launch(g, Fp, st) || chem_scale_launch(nc, Zp[5], ch.scale, 0, st)) {
-        rc = -1;
-        break;
-      }
-      if (consistent && chem_forcing_to_scaled_launch(n, Fp[5], ch.scale, 1.0 / eunit_inv, st)) {
-        rc = -1;
-        break;
-      }
+      // (its legal-state bits into the run's flag)
+      rc = fslow_launch(g, Zp, Fp, ch.scale, eunit_inv, consistent, fe, st, m.flag);
+      if (rc) break;
     }
     if (rc) break;
     // y_{n+1}, in place on Yn
@@ -179,8 +165,7 @@ int imex_evolve(const Grid &g, FeScratch &fe, ChemState &ch, double eunit_inv, I
     }
     if (linear_combination_launch(1 + S, cf, Xf, Yn, 5 * n, st) ||
         linear_combination_launch(1 + 2 * S, cc, Xc, Yn + 5 * n, nc, st) ||
-        fslow_prepare_launch(g, Ynp, ch.scale, eunit_inv, st) ||        // PostprocessStep
-        chem_scale_launch(nc, Ynp[5], ch.scale, 0, st))
+        postprocess_launch(g, Ynp, ch.scale, eunit_inv, st))
       rc = -1;
   }
   fe.timer.on = timer_on;

@@ -81,20 +81,10 @@ int enqueue_slow_step(const Grid &g, FeScratch &fe, ChemState &ch, double eunit_
   for (int i = 1; i < 4; i++) {
     double *Fi[6];
     sub_ptrs(m.F + (long)(i - 1) * len, n, g.nchem, Fi);
-    // fslow(Y) -> F_{i-1}: scaling, et overwrite, fe(), etdot -> chemdot[9], unscaling
-    if (fslow_prepare_launch(g, Y, ch.scale, eunit_inv, st)) return -1;
-    Fields fy;
-    for (int q = 0; q < 5; q++) fy.w[q] = Y[q];
-    fy.chem = Y[5];
-    FieldsOut fo;
-    for (int q = 0; q < 5; q++) fo.w[q] = Fi[q];
-    fo.chem = Fi[5];
-    const int rc = fe_launch(g, fy, fo, fe, st, false, m.flag);  // bits into the run's flag
+    // fslow(Y) -> F_{i-1}: et overwrite, fe() of the scaled species, etdot -> chemdot[9]
+    // (its legal-state bits into the run's flag)
+    const int rc = fslow_launch(g, Y, Fi, ch.scale, eunit_inv, consistent, fe, st, m.flag);
     if (rc) return rc;
-    if (fslow_finish_launch(g, Fi, st)) return -1;
-    if (chem_scale_launch(n * g.nchem, Y[5], ch.scale, 0, st)) return -1;
-    if (consistent && chem_forcing_to_scaled_launch(n, Fi[5], ch.scale, 1.0 / eunit_inv, st))
-      return -1;
     // forcing r_i over the whole ManyVector
     const double dc = KW_C[i] - KW_C[i - 1];
     double coef[3];

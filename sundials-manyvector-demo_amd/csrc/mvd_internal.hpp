@@ -62,21 +62,35 @@ struct FeScratch {
 int fe_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
               hipStream_t st, bool plain, unsigned *accum = nullptr);
 bool fe_nchem_supported(int nchem);
+// fe() as the slow right-hand side takes it (records of 10 species): the gas energy is not
+// advected as a tracer (its slot's rate is overwritten), the total-energy rate goes into its
+// slot of o.chem and o.w[4] becomes 0. With a scale ([cell][10]) the record is converted to
+// the scaled variables: species rates divided by their scale, the energy rate times eunits
+// divided by the gas energy's.
+struct FeSlow {
+  const double *scale = nullptr;
+  double eunits = 1.0;
+};
+int fe_slow_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
+                   hipStream_t st, unsigned *accum, const FeSlow &slow);
 
 // CFL wave speed: max over cells of |mx/rho| + c (stability, utilities.cpp:483-528).
 int max_wave_speed_launch(const Grid &g, const Fields &f, FeScratch &s, hipStream_t st,
                           double *host_out);
 
-// fslow pieces (multirate_chem_hydro_main.cpp:1024-1068)
-int fslow_prepare_launch(const Grid &g, double *const *w, const double *scale,
-                         double eunit_inv, hipStream_t st);
-int fslow_finish_launch(const Grid &g, double *const *wdot, hipStream_t st);
+// fslow (multirate_chem_hydro_main.cpp:996-1083), queued: et of w rebuilt from the gas energy,
+// wdot its rates; converted: the chemistry rates in the scaled variables (as FeSlow). accum as
+// for fe_launch. Returns 0, -2 (unsupported grid) or -1.
+int fslow_launch(const Grid &g, double *const *w, double *const *wdot, const double *scale,
+                 double eunit_inv, bool converted, FeScratch &s, hipStream_t st,
+                 unsigned *accum = nullptr);
+// PostprocessStep (imex_chem_hydro_main.cpp:1002-1050): et from the gas energy, and the
+// chemistry through its scaling and back (x * s / s)
+int postprocess_launch(const Grid &g, double *const *w, const double *scale, double eunit_inv,
+                       hipStream_t st);
 int chem_scale_launch(long n, double *chem, const double *scale, int apply, hipStream_t st);
 // N_VConst: z[0..len) = c
 int const_launch(double c, double *z, long len, hipStream_t st);
-// n cells, 10 species each: species rates / scale, energy slot * eunits / scale
-int chem_forcing_to_scaled_launch(long n, double *Fc, const double *scale, double eunits,
-                                  hipStream_t st);
 
 // fe() vector-Jacobian product (fe_vjp.hip); buf holds fe_vjp_buffer_doubles(g) doubles
 size_t fe_vjp_buffer_doubles(const Grid &g);
