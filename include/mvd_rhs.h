@@ -182,7 +182,7 @@ int mvd_erk_bs3(mvd_erk_table *tab);
 /* Fixed-step explicit evolution of fEuler (euler3D_main.cpp:194 ARKStepCreate with fEuler
  * explicit, :280 ARKStepSetFixedStep, :357 ARKStepEvolve): nsteps steps of size h, in place
  * on w (device arrays of the ManyVector). Stages z_i = y + sum_{j<i} h a_ij F_j, F_i = fe(z_i),
- * y <- y + sum_i h b_i F_i; one step is captured as a device graph and replayed. Returns 0,
+ * y <- y + sum_i h b_i F_i; all steps are queued without waiting in between. Returns 0,
  * or MVD_ILLEGAL_STATE when any stage met an illegal state (w then holds the state after
  * nsteps steps, as an unchecked fixed-step run would), or an error code. */
 int mvd_erk_evolve(mvd_context *ctx, const mvd_erk_table *tab, double t0, double h, int nsteps,

@@ -5,6 +5,9 @@
 //                    (plus the domain's upper boundary faces) with the reference-order
 //                    face flux, into SoA face-flux buffers;
 //   fe_plain_div   : one thread per cell forms the divergence in the reference order.
+// Small grids without tracers (one launch; also a Runge-Kutta stage with its combination):
+//   fe_box         : faces of all three directions of a box of 8 x 4 x 4 cells, one per
+//                    thread, and the divergence.
 // Fast path without tracers (two launches):
 //   fe_xyface_div  : x- and y-faces of 16 x 15-cell plane tiles from one LDS staging of the
 //                    tile and its x/y halos, and their part of the divergence into wdot
@@ -14,7 +17,8 @@
 //                    them, adding the x/y part read from wdot.
 // Fast path with tracers (three launches):
 //   fe_xyface_div<NC>: as without tracers, then the tracers on the same x- and y-faces
-//                    (their values staged in LDS as [tracer][point] after the fluid phase)
+//                    (their values staged in LDS, up to five tracers at a time, after the
+//                    fluid phase)
 //                    and their part of the divergence into wdot;
 //   fe_zface_div_xy: the fluid z-faces, as without tracers;
 //   fe_zface_tracers: the tracer z-faces (tiles of 16 x-cells by 16 faces; per point the
@@ -642,6 +646,201 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
   }
 }
 
+// ------------------------------------------------------------------------------------
+// one-launch fe() of small grids without tracers
+// ------------------------------------------------------------------------------------
+
+// fe() of a grid too small to fill the device is bound by latency: each launch costs its
+// start, its staging and one face flux per thread in turn (Sod's 128x3x3 cells: 7 us for the
+// x/y kernel, which forms two fluxes per thread, then 4 us for z and 2 us for the stage's
+// linear combination). Here a block of 512 threads does all of it for a box of 8 x 4 x 4
+// cells: the 464 faces of the three directions, one per thread. The box's points and their
+// 3-deep halos are staged line by line, once per direction, with the velocities in
+// direction-local order, so that every thread runs the same code whatever its face's
+// direction. A Runge-Kutta stage's linear combination is formed while the points are loaded,
+// and its value, or the step's, is stored by the cells' own threads. Faces and points are
+// recomputed between boxes (464 against 384 faces, 608 points for 128 cells).
+constexpr int BX = 8, BY = 4, BZ = 4, BCELLS = BX * BY * BZ;
+constexpr int BPX = 15, BPY = 11;                       // padded lines of 14 and 10 points
+constexpr int BOFY = BY * BZ * BPX, BOFZ = BOFY + BX * BZ * BPY, BFS = BOFZ + BX * BY * BPY;
+constexpr int BNFX = BY * BZ * (BX + 1), BNFY = BX * BZ * (BY + 1), BNFZ = BX * BY * (BZ + 1);
+constexpr int BNF = BNFX + BNFY + BNFZ;                 // 464
+constexpr int BNP = BCELLS + 6 * (BY * BZ + BX * BZ + BX * BY);   // 608
+static_assert(BNF <= 512 && 5 * BNF <= PT_NF * BFS, "one face per thread; fluxes over points");
+
+// Point p of the staging of the box at (x0, y0, z0): its local coordinates, the cell it is
+// read from, its signs, and which lines it belongs to.
+struct BoxPoint {
+  int lx, ly, lz, cell;
+  double sa, sx, sy, sz;
+  bool use, core, ox, oy, oz;
+};
+
+__device__ inline BoxPoint box_point(const Grid &g, int x0, int y0, int z0, int p) {
+  BoxPoint P;
+  // local coordinates: the box's cells, then the halos of the x, y and z lines
+  if (p < BCELLS) {
+    P.lx = p % BX; P.ly = p / BX % BY; P.lz = p / (BX * BY);
+  } else if (p < BCELLS + 6 * BY * BZ) {
+    const int q = p - BCELLS, h = q % 6;
+    P.lx = h < 3 ? h - 3 : BX - 3 + h; P.ly = q / 6 % BY; P.lz = q / (6 * BY);
+  } else if (p < BCELLS + 6 * (BY * BZ + BX * BZ)) {
+    const int q = p - (BCELLS + 6 * BY * BZ), h = q / BX % 6;
+    P.lx = q % BX; P.ly = h < 3 ? h - 3 : BY - 3 + h; P.lz = q / (6 * BX);
+  } else {
+    const int q = p - (BCELLS + 6 * (BY * BZ + BX * BZ)), h = q / (BX * BY);
+    P.lx = q % BX; P.ly = q / BX % BY; P.lz = h < 3 ? h - 3 : BZ - 3 + h;
+  }
+  const int ex = x0 + P.lx, ey = y0 + P.ly, ez = z0 + P.lz;
+  // which dimension the point lies outside the grid in: none, or one (a ghost of lines along
+  // it); a point outside in two, or past the third ghost, is not used
+  P.ox = ex < 0 || ex >= g.nx;
+  P.oy = ey < 0 || ey >= g.ny;
+  P.oz = ez < 0 || ez >= g.nz;
+  P.use = p < BNP && P.ox + P.oy + P.oz <= 1 && ex <= g.nx + 2 && ey <= g.ny + 2 &&
+          ez <= g.nz + 2;
+  P.core = P.use && p < BCELLS && !P.ox && !P.oy && !P.oz;   // a cell of the box
+  int i = ex, j = ey, k = ez;
+  P.sa = P.sx = P.sy = P.sz = 1.0;
+  if (P.ox) {
+    const GhostMap m = ghost_map(g, 0, ex);
+    i = m.src; P.sa = P.sy = P.sz = m.sgn_all; P.sx = m.sgn_norm;
+  } else if (P.oy) {
+    const GhostMap m = ghost_map(g, 1, ey);
+    j = m.src; P.sa = P.sx = P.sz = m.sgn_all; P.sy = m.sgn_norm;
+  } else if (P.oz) {
+    const GhostMap m = ghost_map(g, 2, ez);
+    k = m.src; P.sa = P.sx = P.sy = m.sgn_all; P.sz = m.sgn_norm;
+  }
+  P.cell = P.use ? i + g.nx * (j + g.ny * k) : 0;
+  return P;
+}
+
+template <int NT>
+__global__ void __launch_bounds__(512, 2)
+fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, double idz,
+       unsigned *flag) {
+  __shared__ double sh[PT_NF * BFS];
+  const int t = threadIdx.x;
+  const int nbx = (g.nx + BX - 1) / BX, nby = (g.ny + BY - 1) / BY;
+  int b = blockIdx.x;
+  const int x0 = (b % nbx) * BX;
+  b /= nbx;
+  const int y0 = (b % nby) * BY, z0 = (b / nby) * BZ;
+  const int ncell = g.nx * g.ny * g.nz;
+  // all loads of the thread's one or two points are issued before any is used
+  constexpr int NR = (BNP + 511) / 512;
+  BoxPoint P[NR];
+#pragma unroll
+  for (int n = 0; n < NR; n++) P[n] = box_point(g, x0, y0, z0, t + 512 * n);
+  double raw[NR][5], Kv[NR][NT > 0 ? NT : 1][5];
+#pragma unroll
+  for (int n = 0; n < NR; n++) {
+    if (!P[n].use) continue;
+#pragma unroll
+    for (int q = 0; q < 5; q++) raw[n][q] = y.w[q][P[n].cell];
+#pragma unroll
+    for (int m = 0; m < NT; m++)
+#pragma unroll
+      for (int q = 0; q < 5; q++) Kv[n][m][q] = s.K[m][q * ncell + P[n].cell];
+  }
+#pragma unroll
+  for (int n = 0; n < NR; n++) {
+    const BoxPoint &Q = P[n];
+    if (!Q.use) continue;
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int m = 0; m < NT; m++)
+#pragma unroll
+        for (int q = 0; q < 5; q++) raw[n][q] += s.c[m] * Kv[n][m][q];
+    }
+    if (Q.core && s.z) {
+#pragma unroll
+      for (int q = 0; q < 5; q++) s.z[q * ncell + Q.cell] = raw[n][q];
+    }
+    const double r = raw[n][0] * Q.sa, e = raw[n][4] * Q.sa;
+    const double mx = raw[n][1] * Q.sx, my = raw[n][2] * Q.sy, mz = raw[n][3] * Q.sz;
+    double pt[PT_NF];
+    const double pr = store_point(pt, 1, r, mx, my, mz, e, g.gamma);
+    if (Q.core) {
+      unsigned bits = 0;
+      if (!(r > 0.0)) bits |= 1u;
+      if (!(e > 0.0)) bits |= 2u;
+      if (!(pr > 0.0)) bits |= 4u;
+      if (bits) atomicOr(flag, bits);
+    }
+    const bool inx = Q.lx >= 0 && Q.lx < BX, iny = Q.ly >= 0 && Q.ly < BY;
+    const bool inz = Q.lz >= 0 && Q.lz < BZ;
+    const auto put = [&](int at, double un, double u1, double u2) {
+      double *d = sh + at;
+      d[PT_R * BFS] = pt[PT_R]; d[PT_U * BFS] = un; d[PT_V * BFS] = u1; d[PT_W * BFS] = u2;
+      d[PT_P * BFS] = pt[PT_P]; d[PT_SR * BFS] = pt[PT_SR]; d[PT_C2 * BFS] = pt[PT_C2];
+      d[PT_C * BFS] = pt[PT_C];
+    };
+    if (iny && inz && !Q.oy && !Q.oz)
+      put((Q.ly + BY * Q.lz) * BPX + Q.lx + 3, pt[PT_U], pt[PT_V], pt[PT_W]);
+    if (inx && inz && !Q.ox && !Q.oz)
+      put(BOFY + (Q.lx + BX * Q.lz) * BPY + Q.ly + 3, pt[PT_V], pt[PT_U], pt[PT_W]);
+    if (inx && iny && !Q.ox && !Q.oy)
+      put(BOFZ + (Q.lx + BX * Q.ly) * BPY + Q.lz + 3, pt[PT_W], pt[PT_V], pt[PT_U]);
+  }
+  __syncthreads();
+  // face t: lines of BX + 1, BY + 1, BZ + 1 faces
+  int at = 0;
+  bool ok = false;
+  if (t < BNFX) {
+    const int f = t % (BX + 1), line = t / (BX + 1);
+    at = line * BPX + f;
+    ok = x0 + f <= g.nx && y0 + line % BY < g.ny && z0 + line / BY < g.nz;
+  } else if (t < BNFX + BNFY) {
+    const int q = t - BNFX, f = q % (BY + 1), line = q / (BY + 1);
+    at = BOFY + line * BPY + f;
+    ok = y0 + f <= g.ny && x0 + line % BX < g.nx && z0 + line / BX < g.nz;
+  } else if (t < BNF) {
+    const int q = t - (BNFX + BNFY), f = q % (BZ + 1), line = q / (BZ + 1);
+    at = BOFZ + line * BPY + f;
+    ok = z0 + f <= g.nz && x0 + line % BX < g.nx && y0 + line / BX < g.ny;
+  }
+  double F[5];
+  if (ok)
+    face_flux_lds<PT_U, PT_V, PT_W>(sh + at, BFS, 1, g.gamma, g.igm, face_alpha<PT_U>(sh + at, BFS, 1),
+                                    F);
+  __syncthreads();                    // points dead: their LDS takes the fluxes [comp][face]
+  if (ok) {
+#pragma unroll
+    for (int a = 0; a < 5; a++) sh[a * BNF + t] = F[a];
+  }
+  __syncthreads();
+  // one value per thread and turn: field a of cell q
+  for (int n = t; n < 5 * BCELLS; n += 512) {
+    const int a = n / BCELLS, q = n % BCELLS;
+    const int lx = q % BX, ly = q / BX % BY, lz = q / (BX * BY);
+    if (x0 + lx >= g.nx || y0 + ly >= g.ny || z0 + lz >= g.nz) continue;
+    const int ay = a == 1 ? 2 : a == 2 ? 1 : a, az = a == 1 ? 3 : a == 3 ? 1 : a;
+    const double *Fx = sh + a * BNF + (ly + BY * lz) * (BX + 1) + lx;
+    const double *Fy = sh + ay * BNF + BNFX + (lx + BX * lz) * (BY + 1) + ly;
+    const double *Fz = sh + az * BNF + BNFX + BNFY + (lx + BX * ly) * (BZ + 1) + lz;
+    const double dxy = (Fx[1] - Fx[0]) * idx + (Fy[1] - Fy[0]) * idy;
+    const double rate = 0.0 - (dxy + (Fz[1] - Fz[0]) * idz);
+    const int c = (x0 + lx) + g.nx * ((y0 + ly) + g.ny * (z0 + lz));
+    // (selected, not indexed: an index that is not constant would copy the arguments to
+    // scratch memory)
+    double *o = out.w[0];
+    const double *ya = y.w[0];
+#pragma unroll
+    for (int m = 1; m < 5; m++)
+      if (a == m) { o = out.w[m]; ya = y.w[m]; }
+    o[c] = rate;
+    if (s.y1) {
+#pragma clang fp contract(off)
+      double v = ya[c];
+      for (int m = 0; m < s.nb; m++) v += s.b[m] * s.Kb[m][a * ncell + c];
+      s.y1[a * ncell + c] = v + s.blast * rate;
+    }
+  }
+}
+
 __global__ void reset_flag(unsigned *flag) { *flag = 0u; }
 
 // ------------------------------------------------------------------------------------
@@ -708,9 +907,31 @@ int fe_slow_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch
                     : launch_fe<9, 10, TR_SLOW>(g, f, o, s, st, false, accum, slow);
 }
 
+bool fe_box_fits(const Grid &g) {
+  return g.nchem == 0 && (long)g.nx * g.ny * g.nz <= FE_BOX_MAX;
+}
+
+int fe_box_launch(const Grid &g, const Fields &y, const BoxStage &bs, const FieldsOut &o,
+                  hipStream_t st, unsigned *flag) {
+  const long nb = (long)((g.nx + BX - 1) / BX) * ((g.ny + BY - 1) / BY) * ((g.nz + BZ - 1) / BZ);
+  const auto kern = bs.nt == 0   ? fe_box<0>
+                    : bs.nt == 1 ? fe_box<1>
+                    : bs.nt == 2 ? fe_box<2>
+                    : bs.nt == 3 ? fe_box<3>
+                    : bs.nt == 4 ? fe_box<4>
+                                 : fe_box<5>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), 0, st, g, y, bs, o, 1.0 / g.dx,
+                     1.0 / g.dy, 1.0 / g.dz, flag);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int fe_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
               hipStream_t st, bool plain, unsigned *accum) {
   if (fe_too_large(g)) return -2;
+  if (!plain && fe_box_fits(g) && !s.timer.on) {
+    if (!accum) hipLaunchKernelGGL(reset_flag, dim3(1), dim3(1), 0, st, s.flag);
+    return fe_box_launch(g, f, BoxStage{}, o, st, accum ? accum : s.flag);
+  }
   switch (g.nchem) {
     case 0: return launch_fe<0>(g, f, o, s, st, plain, accum);
     case 1: return launch_fe<1>(g, f, o, s, st, plain, accum);
