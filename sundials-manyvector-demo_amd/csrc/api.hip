@@ -395,7 +395,7 @@ int mvd_chem_lsetup(mvd_context *ctx, double gamma, const double *J) {
   if (!std::isfinite(gamma)) return MVD_BAD_ARGUMENT;
   const long n = ctx->chem.n;
   if (!ctx->ls_lu) {
-    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * n)) ||
+    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * ((n + 63) / 64 * 64))) ||
         !dev_ok(hipMalloc(&ctx->ls_piv, sizeof(unsigned long long) * n)) ||
         !dev_ok(hipMalloc(&ctx->ls_nsing, sizeof(int))))
       return MVD_DEVICE_ERROR;
@@ -417,7 +417,7 @@ int mvd_chem_lsetup_matrix(mvd_context *ctx, const double *A) {
   if (!ctx->chem.ready) return MVD_NOT_READY;
   const long n = ctx->chem.n;
   if (!ctx->ls_lu) {
-    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * n)) ||
+    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * ((n + 63) / 64 * 64))) ||
         !dev_ok(hipMalloc(&ctx->ls_piv, sizeof(unsigned long long) * n)) ||
         !dev_ok(hipMalloc(&ctx->ls_nsing, sizeof(int))))
       return MVD_DEVICE_ERROR;

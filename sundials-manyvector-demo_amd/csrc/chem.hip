@@ -153,12 +153,16 @@ chem_temperature_check_kernel(long n, ChemConst cc, const double *scale, const d
 }
 
 // calculate_jacobian_cvklu (raja_primordial_network.cpp:1393-1965): dense column-major
-// blocks, each entry times inv_scale[row]*scale[col].
-__global__ void __launch_bounds__(256)
+// blocks, each entry times inv_scale[row]*scale[col]. One wave per block; the lanes' blocks
+// go out through LDS (blk_store). Bound by the 800 bytes written per cell: 64^3 cells 92 ->
+// 70 us.
+__global__ void __launch_bounds__(64)
 chem_jac_kernel(long n, ChemConst cc, ChemPtrs p, const double *yd, double *J, double sjac) {
 #pragma clang fp contract(off)
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  __shared__ double lds[BLK_LDS];
+  const long base = (long)blockIdx.x * 64;
+  const int ncell = (int)min(n - base, 64L);
+  const long i = base + min((int)threadIdx.x, ncell - 1);   // spare lanes repeat the last cell
   double y[NSP], sc[NSP], isc[NSP];
 #pragma unroll
   for (int v = 0; v < NSP; v++) {
@@ -172,11 +176,11 @@ chem_jac_kernel(long n, ChemConst cc, ChemPtrs p, const double *yd, double *J, d
   const CellAux ax{p.md[i], p.imd[i], p.cie[i], p.h2o[i]};
   double Jp[NSP][NSP];
   chem_jac_physical(y, k, dk, T, cc.z, p.dTs[i], ax, Jp);
-  double *blk = J + (long)NSP * NSP * i;
 #pragma unroll
   for (int c = 0; c < NSP; c++)
 #pragma unroll
-    for (int r = 0; r < NSP; r++) blk[NSP * c + r] = Jp[r][c] * (isc[r] * sc[c]) * sjac;
+    for (int r = 0; r < NSP; r++) Jp[r][c] = Jp[r][c] * (isc[r] * sc[c]) * sjac;
+  blk_store(J + (long)BLK * base, ncell, lds, Jp);
 }
 
 static ChemPtrs ptrs_of(ChemState &s) {
@@ -260,8 +264,8 @@ int chem_rhs(ChemState &s, const double *y, double *ydot, hipStream_t st, bool s
 
 int chem_jac(ChemState &s, const double *y, double *J, hipStream_t st, bool sync,
              double sjac) {
-  hipLaunchKernelGGL(chem_jac_kernel, dim3(nb(s.n)), dim3(256), 0, st, s.n, s.cc, ptrs_of(s), y,
-                     J, sjac);
+  hipLaunchKernelGGL(chem_jac_kernel, dim3((unsigned)((s.n + 63) / 64)), dim3(64), 0, st, s.n, s.cc,
+                     ptrs_of(s), y, J, sjac);
   if (hipGetLastError() != hipSuccess) return MVD_DEVICE_ERROR;
   if (!sync) return MVD_SUCCESS;
   return hipStreamSynchronize(st) == hipSuccess ? MVD_SUCCESS : MVD_DEVICE_ERROR;

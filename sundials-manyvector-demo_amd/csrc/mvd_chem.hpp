@@ -73,6 +73,88 @@ double *chem_state_ptr(ChemState &s, int which);
 void chem_free(ChemState &s);
 
 // -------------------------------------------------------------------------------------
+// one wave's 10x10 blocks between memory and registers
+// -------------------------------------------------------------------------------------
+
+// The matrices of the C ABI are one column-major block of 800 bytes per cell. Lanes that read
+// or write their own cells' blocks touch 64 lines per instruction and return to each of them
+// eight times, with more lines in use than the L1 holds. A wave therefore moves the blocks
+// of 32 cells at a time through LDS: memory side as one contiguous run of 16-byte accesses,
+// register side one block per lane, rows padded to an odd number of doubles (no bank
+// conflicts). 26 KB per wave. One-wave blocks; every lane of the wave calls these.
+constexpr int BLK = NSP * NSP, BLK_PITCH = BLK + 1, BLK_HALF = 32;
+constexpr int BLK_LDS = BLK_HALF * BLK_PITCH;           // doubles of LDS
+struct __attribute__((aligned(8))) Pair8 { double x, y; };   // 16 bytes at 8-byte alignment
+
+__device__ inline void blk_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Element (pair) e of a half's run: its place in LDS.
+__device__ inline int blk_place(int e) {
+  const int cell = e / (BLK / 2);
+  return cell * BLK_PITCH + 2 * (e - cell * (BLK / 2));
+}
+
+// a[r][q] = element 10 q + r of the lane's block; `ncell` (>= 1) cells of the wave exist,
+// lanes past them get nothing. src: the wave's first block.
+__device__ inline void blk_load(const double *src, int ncell, double *lds, double (&a)[NSP][NSP]) {
+  const int lane = threadIdx.x & 63;
+  for (int half = 0; half < 2; half++) {
+    const int nc = min(ncell - half * BLK_HALF, BLK_HALF);
+    if (nc <= 0) break;
+    const Pair8 *p = reinterpret_cast<const Pair8 *>(src + (long)half * BLK_HALF * BLK);
+    const int np = nc * (BLK / 2);
+    constexpr int NL = BLK_HALF * (BLK / 2) / 64;       // 25 loads in flight
+    Pair8 v[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) v[i] = p[min(i * 64 + lane, np - 1)];
+    blk_sync();                                         // the previous half is read
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+      const int at = blk_place(i * 64 + lane);
+      lds[at] = v[i].x;
+      lds[at + 1] = v[i].y;
+    }
+    blk_sync();
+    if ((lane >> 5) == half) {
+      const double *b = lds + (lane & 31) * BLK_PITCH;
+#pragma unroll
+      for (int q = 0; q < NSP; q++)
+#pragma unroll
+        for (int r = 0; r < NSP; r++) a[r][q] = b[NSP * q + r];
+    }
+  }
+}
+
+// The reverse: the lanes' blocks to dst.
+__device__ inline void blk_store(double *dst, int ncell, double *lds, const double (&a)[NSP][NSP]) {
+  const int lane = threadIdx.x & 63;
+  for (int half = 0; half < 2; half++) {
+    const int nc = min(ncell - half * BLK_HALF, BLK_HALF);
+    if (nc <= 0) break;
+    blk_sync();                                         // the previous half is stored
+    if ((lane >> 5) == half) {
+      double *b = lds + (lane & 31) * BLK_PITCH;
+#pragma unroll
+      for (int q = 0; q < NSP; q++)
+#pragma unroll
+        for (int r = 0; r < NSP; r++) b[NSP * q + r] = a[r][q];
+    }
+    blk_sync();
+    Pair8 *p = reinterpret_cast<Pair8 *>(dst + (long)half * BLK_HALF * BLK);
+    const int np = nc * (BLK / 2);
+#pragma unroll 5
+    for (int i = 0; i < BLK_HALF * (BLK / 2) / 64; i++) {
+      const int e = i * 64 + lane, at = blk_place(e);
+      if (e < np) p[e] = Pair8{lds[at], lds[at + 1]};
+    }
+  }
+}
+
+// -------------------------------------------------------------------------------------
 // device functions: the reference's expressions. Products and sums of one expression are
 // contracted to FMAs by the front end (contract(on), the same way wherever a function is
 // inlined, so the solvers that share these functions agree bit for bit), and the divides of

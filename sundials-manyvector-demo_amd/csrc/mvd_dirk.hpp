@@ -57,7 +57,7 @@ int chem_adjoint_run(ChemState &s, const DirkDev &o, double h, int nsteps, int K
                      const double *lamT, double *lam0, double *scratch, hipStream_t st,
                      int *host_fail);
 // block linear solver of the chemistry subvector (A = I - gamma J, batched LU); formed:
-// J already holds A (gamma unused)
+// J already holds A (gamma unused); LU: 100 doubles per cell, cells rounded up to 64
 int chem_ls_setup(long n, double gamma, const double *J, double *LU, unsigned long long *piv,
                   int *nsing, hipStream_t st, bool formed = false);
 int chem_ls_solve(long n, const double *LU, const unsigned long long *piv, const double *b,
