@@ -14,9 +14,13 @@
 //   fe_vjp_fix_x/_yz - add the contributions that left a line or segment (ghost points,
 //                      rows of neighbouring segments), held in a small side buffer.
 // The x sweep stores wbar, the others add. No atomics: the result is deterministic.
-// The tracers of w and wbar are handled tracer-major inside (cells_to_planes /
-// planes_to_cells around the sweeps); the cotangent's, read at two cells per face, stay
-// cell-major; the interface keeps the cell-major layout.
+// Tracers have a kernel of their own per direction (fe_vjp_tracers), run before the fluid
+// sweep, which takes over the velocity and wave-speed adjoints that the tracers produce. In
+// one kernel the 15 components left one wave per SIMD (38 KB of LDS, 480 registers) waiting on
+// its loads; apart, with the tracer-major copies of w and wbar gone, 128^3 with ten tracers
+// takes 2.28 instead of 2.77 ms.
+#include <algorithm>
+
 #include "mvd_device.hpp"
 #include "mvd_internal.hpp"
 #include "../../include/mvd_rhs.h"
@@ -104,38 +108,6 @@ __device__ inline void face_prim(const double (&s)[6][5], double gamma, FacePrim
     P.ul[l] = s[l][1] * P.ir[l];
     const double a = fabs(P.ul[l]) + sun_sqrt(gamma * P.p[l] * P.ir[l]);
     if (P.alpha < a) { P.alpha = a; P.lstar = l; }
-  }
-}
-
-// One tracer: t[6] the stencil values, Fbc its flux cotangent; tb[6] receives the tracer
-// adjoint, ulb and alphab accumulate. The split flux fs = (ul t +- alpha t) / 2 is formed as
-// t hs with the point's split factor hs = (ul +- alpha) / 2 (ha = alpha / 2), whose
-// derivatives are hs (t), t / 2 (ul) and +-t / 2 (alpha).
-__device__ inline void tracer_vjp(const double (&t)[6], double Fbc, const FacePrim &P,
-                                  double ha, double (&tb)[6], double (&ulb)[6],
-                                  double &alphab) {
-#pragma unroll
-  for (int l = 0; l < 6; l++) tb[l] = 0.0;
-#pragma unroll
-  for (int sd = 0; sd < 2; sd++) {
-    double fa[5], hs[5], g[5];
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      const int pt = l + sd;
-      hs[l] = fma(0.5, P.ul[pt], sd == 0 ? ha : -ha);
-      fa[l] = t[pt] * hs[l];
-    }
-    (void)weno5_grad(fa, sd, g);
-    const double sg = sd == 0 ? 0.5 : -0.5;
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      const int pt = l + sd;
-      const double fsb = Fbc * g[l];
-      const double ft = fsb * t[pt];
-      ulb[pt] += 0.5 * ft;
-      alphab += sg * ft;
-      tb[pt] += fsb * hs[l];
-    }
   }
 }
 
@@ -342,14 +314,13 @@ __device__ inline int gcomp(int d, int a) {
 }  // namespace
 
 // One face's stencil adjoint, handed to a sink with the ghost rule's signs applied, one
-// component at a time: the tracers first (the fluid part needs the velocity and
-// wave-speed adjoints they produce), then the fluid in global component order. For each
-// component the sink's pre(q) is called before the adjoint is computed (to start the
-// loads its put needs) and put(q, x[6], pre) after. The next tracer's stencil is loaded
-// while the current one is swept. Face (i, j, k) along d lies between cells c-1 and c.
-template <int NC, class Sink>
-__device__ inline void face_vjp(const Grid &g, const Fields &w, const Fields &vc, int d, int i,
-                                int j, int k, Sink &sink) {
+// fluid component at a time in global order. For each component the sink's pre(q) is
+// called before (to start the loads its put needs) and put(q, x[6], pre) after. ulb3 and
+// alphab: the tracers' adjoints of the velocity of the cell right of the face and of the
+// Lax-Friedrichs speed. Face (i, j, k) along d lies between cells c-1 and c.
+template <class Sink>
+__device__ inline void face_vjp(const Grid &g, const Fields &w, const Fields &vc, const double *ub,
+                                double alphab, int d, int i, int j, int k, Sink &sink) {
   const int n = extent(g, d);
   const int c0 = d == 0 ? i : d == 1 ? j : k;
   const double idelta = 1.0 / (d == 0 ? g.dx : d == 1 ? g.dy : g.dz);
@@ -377,53 +348,7 @@ __device__ inline void face_vjp(const Grid &g, const Fields &w, const Fields &vc
   FacePrim P;
   face_prim(s, g.gamma, P);
   double ulb[6] = {0, 0, 0, 0, 0, 0};
-  double alphab = 0.0;
-  if (NC > 0) {
-    // software pipeline: the stencil and sink loads of tracer c + PD are issued before
-    // tracer c is swept (the empty asm statement keeps the compiler from sinking them);
-    // PD = 1 measured fastest (2 and 3 were 1-2% slower at 128^3 with 10 tracers)
-    constexpr int PD = 1;
-    struct Tr { double t[6], r, l; };
-    const long ncell = (long)g.nx * g.ny * g.nz;
-    auto load_tracer = [&](Tr &x, int c) {
-      const long pl = (long)c * ncell;
-#pragma unroll
-      for (int l = 0; l < 6; l++) x.t[l] = w.chem[pl + cell[l]];
-      x.r = vc.chem[(long)NC * cr + c];   // the cotangent stays cell-major (two cells a face)
-      x.l = vc.chem[(long)NC * cl + c];
-    };
-    using Pre = decltype(sink.pre(5));
-    Tr buf[PD];
-    Pre pb[PD];
-#pragma unroll
-    for (int k = 0; k < PD; k++) {
-      pb[k] = sink.pre(5 + k);
-      load_tracer(buf[k], k);
-    }
-#pragma unroll 1
-    for (int c0 = 0; c0 < NC; c0 += PD) {
-#pragma unroll
-      for (int k = 0; k < PD; k++) {
-        const int c = c0 + k;
-        if (c < NC) {
-          double t[6], tb[6];
-#pragma unroll
-          for (int l = 0; l < 6; l++) t[l] = flip(buf[k].t[l], (na >> l) & 1u);
-          const double Fbc = (mr * buf[k].r - ml * buf[k].l) * idelta;
-          const Pre pre = pb[k];
-          if (c + PD < NC) {
-            pb[k] = sink.pre(5 + c + PD);
-            load_tracer(buf[k], c + PD);
-          }
-          __asm__ volatile("" ::: "memory");
-          tracer_vjp(t, Fbc, P, 0.5 * P.alpha, tb, ulb, alphab);
-#pragma unroll
-          for (int l = 0; l < 6; l++) tb[l] = flip(tb[l], (na >> l) & 1u);
-          sink.put(5 + c, tb, pre);
-        }
-      }
-    }
-  }
+  if (ub != nullptr && hr) ulb[3] = ub[cr];
   double Fb[5];
 #pragma unroll
   for (int a = 0; a < 5; a++) {
@@ -449,9 +374,264 @@ __device__ inline void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline void out_put(const FieldsOut &o, long ncell, int q, long cell, double v,
-                               bool add) {
-  double *p = q < 5 ? &o.w[q][cell] : &o.chem[(long)(q - 5) * ncell + cell];
+// The adjoint of a WENO5 reconstruction over f0..f4 (the f+ formula; the f- one is the same
+// function of the reversed values): x_i = y d(weno)/d f_i for the cotangent y. weno =
+// f2 + (2/3) Q with Q = sum o_k q_k over the normalised weights o_k = d_k e_k^-2 / sum, in the
+// differences a, b, c, d of neighbouring values and the completed squares e_k of weno5_sd:
+//   dQ = sum o_k dq_k - 2 sum (o_k / e_k) (q_k - Q) de_k,
+//   de_1 = 2 t1 dt1 + (39/32) c dc and so on.
+// One reciprocal (of the common denominator times e_1 e_2 e_3: seven factors, finite for
+// |beta| < 1e43); 77 operations. Returns Q.
+__device__ inline double weno5_adj(double f0, double f1, double f2, double f3, double f4,
+                                   double epsb, double y, double (&x)[5]) {
+  const double a = f1 - f0, b = f2 - f1, c = f3 - f2, d = f4 - f3;
+  const double c1375 = scalar_const(-1.375), c0625 = scalar_const(-0.625);
+  const double c025 = scalar_const(-0.25), c025p = scalar_const(0.25);
+  const double c125 = scalar_const(1.25), c13 = scalar_const(1.0 / 3.0);
+  const double t3 = fma(c1375, b, a), t2 = fma(c0625, c, b), t1 = fma(c1375, c, d);
+  const double hb = 0.609375 * b, hc = 0.609375 * c;
+  const double wb = fma(hb, b, epsb), wc = fma(hc, c, epsb);
+  const double e1 = fma(t1, t1, wc), e2 = fma(t2, t2, wc), e3 = fma(t3, t3, wb);
+  const double p1 = e2 * e3, p2 = e1 * e3, p3 = e1 * e2;
+  const double s1 = p1 * p1, s2 = 2.0 * (p2 * p2), s3 = c13 * (p3 * p3);
+  const double q1 = fma(c025, d, c), q2 = fma(c025p, b, 0.5 * c), q3 = fma(-0.5, a, c125 * b);
+  const double den = s1 + s2 + s3, E = p1 * e1;
+  const double r = fast_rcp(den * E);
+  const double iden = E * r, iE = (-4.0 * den) * r;
+  const double Q = fma(q1, s1, fma(q2, s2, q3 * s3)) * iden;
+  const double yd = ((2.0 / 3.0) * y) * iden;
+  const double o1 = s1 * yd, o2 = s2 * yd, o3 = s3 * yd;
+  const double m1 = (o1 * (p1 * iE)) * (q1 - Q), m2 = (o2 * (p2 * iE)) * (q2 - Q);
+  const double m3 = (o3 * (p3 * iE)) * (q3 - Q);
+  const double u1 = m1 * t1, u2 = m2 * t2, u3 = m3 * t3;
+  const double ga = fma(-0.5, o3, u3), gd = fma(c025, o1, u1);
+  const double gb = fma(m3, hb, fma(c1375, u3, fma(c125, o3, fma(c025p, o2, u2))));
+  const double gc = fma(m1 + m2, hc, fma(c0625, u2, fma(c1375, u1, fma(0.5, o2, o1))));
+  x[0] = -ga;
+  x[1] = ga - gb;
+  x[2] = y + (gb - gc);
+  x[3] = gc - gd;
+  x[4] = gd;
+  return Q;
+}
+
+// ------------------------------------------------------------------------------------
+// Tracers. With u_l the normal velocities and alpha the Lax-Friedrichs speed of a face, a
+// tracer's flux reconstructs t_l (u_l +- alpha) / 2; its adjoint goes to the tracer, to the
+// velocities and to alpha. A lane walks one tracer of one column along D over the rows
+// [c0, c1), the lanes of a wave being consecutive (column, tracer) pairs: cell-major tracer
+// rows along y and z are read as they lie. The stencil and the open rows' adjoints slide
+// through registers (six faces per round, so that every index is a constant); a row is
+// written out with its last face. Segments do the faces that reach into them again instead
+// of exchanging rows, ghost rows are added to their source rows in the lane: no side
+// buffer and no fix-up pass. The velocity adjoint of each cell and the alpha adjoint of each
+// face are summed over a cell's tracers (in tracer order) once per round and handed to the
+// fluid sweep in ub [cell] and alb [face]; so are the velocities and alphas that the lanes
+// of a cell share, which one lane computes for all. 128^3 with ten tracers: 0.28 ms per
+// direction, about 210 FP64 instructions per face and tracer (0.15 ms to issue) at two to three
+// waves per SIMD.
+// ------------------------------------------------------------------------------------
+struct TrWalk {
+  const double *r, *m0, *m1, *m2, *e, *mn;   // fluid; mn: the momentum along the walk
+  const double *t, *v;
+  double *out, *ub, *alb;
+  long rs, bs_in, bs_out, ncol;  // row stride; column col starts at (col % nin) bs_in + (col / nin) bs_out
+  long afs, acs;                 // alb strides of a face and of a column
+  int nin, n, ncb, nseg, per, add;
+  double sa_lo, su_lo, sa_hi, su_hi;   // ghost signs: all fields, normal velocity
+  double idelta, gamma;
+};
+
+// Row of extended index e: wrapped, mirrored or shifted (ghost_map); rows further out than
+// the ghosts, which no face reads, are clamped.
+__device__ inline int walk_row(const TrWalk &k, int e, double &sa, double &su) {
+  sa = su = 1.0;
+  const int n = k.n;
+  if (e >= 0 && e < n) return e;
+  if (k.per) {
+    e = e < 0 ? e + n : e - n;
+    return e < 0 ? e + n : e >= n ? e - n : e;
+  }
+  if (e < 0) { sa = k.sa_lo; su = k.su_lo; return min(-1 - e, n - 1); }
+  sa = k.sa_hi; su = k.su_hi;
+  return min(e - 3, n - 1);
+}
+
+template <int NC>
+__global__ void __launch_bounds__(64, 2)
+fe_vjp_tracers(TrWalk k) {
+  constexpr int GPW = 64 / NC;                 // columns per wave
+  __shared__ double ring_u[12][GPW], ring_a[12][GPW], alpha[6][GPW];
+  __shared__ double red[6][2][GPW * NC + 4], held[3][2][64];
+  const int lane = threadIdx.x, n = k.n;
+  const int blk = blockIdx.x % k.ncb, seg = blockIdx.x / k.ncb;
+  const int c0 = (int)((long)seg * n / k.nseg), c1 = (int)((long)(seg + 1) * n / k.nseg);
+  const int fa = k.per ? c0 - 2 : max(c0 - 2, 0);       // first face
+  const int fend = c1 + 2, fb = k.per ? fend : min(fend, n);   // faces past fb only close rows
+  const int grp = min(lane / NC, GPW - 1), c = lane % NC;
+  const long col0 = (long)blk * GPW;
+  const bool act = lane < GPW * NC && col0 + grp < k.ncol;
+  const auto cell_of = [&](long col) {
+    const unsigned q = (unsigned)col / (unsigned)k.nin;
+    return (long)((unsigned)col - q * (unsigned)k.nin) * k.bs_in + (long)q * k.bs_out;
+  };
+  const long base = cell_of(min(col0 + grp, k.ncol - 1));
+  const double *tp = k.t + base * NC + c, *vp = k.v + base * NC + c;
+  double *op = k.out + base * NC + c;
+  // velocities and wave speeds of rows ra .. ra+cnt-1 into ring slots rho, rho+1, ...
+  const auto fill = [&](int ra, int rho, int cnt) {
+    for (int i = lane; i < cnt * GPW; i += 64) {
+      const int rr = i / GPW, gg = i - rr * GPW;
+      double sa, su;
+      const long cc = cell_of(min(col0 + gg, k.ncol - 1)) +
+                      walk_row(k, min(ra + rr, fend + 2), sa, su) * k.rs;
+      const double m0 = k.m0[cc], m1 = k.m1[cc], m2 = k.m2[cc];
+      const double ir = fast_rcp(k.r[cc]);
+      const double p = (k.gamma - 1.0) * (k.e[cc] - 0.5 * (m0 * m0 + m1 * m1 + m2 * m2) * ir);
+      const double u = k.mn[cc] * ir;
+      const int sl = (rho + rr) % 12;
+      ring_u[sl][gg] = 0.5 * su * u;
+      ring_a[sl][gg] = fabs(u) + fast_sqrt(k.gamma * p * ir);
+    }
+  };
+  const auto row_ptr = [&](int e, double &sa) {
+    double su;
+    return (long)walk_row(k, min(e, fend + 2), sa, su) * k.rs * NC;
+  };
+  fill(fa - 3, 0, 11);
+  wave_sync_lds();
+  // window slot (j + l) % 6 holds point l of the round's face j: tracer, half velocity and
+  // the adjoints so far
+  double tw[6], hu[6], at[6], au[6], tn[6], vn[6], on[6];
+#pragma unroll
+  for (int l = 0; l < 6; l++) at[l] = au[l] = tw[l] = hu[l] = 0.0;
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    double sa;
+    const long o = row_ptr(fa - 3 + l, sa);
+    tw[l] = sa * tp[o];
+    hu[l] = ring_u[l][grp];
+  }
+  const auto load_face = [&](int f, double &t, double &v, double &o) {
+    double sa;
+    t = tp[row_ptr(f + 2, sa)] * sa;
+    v = vp[row_ptr(f, sa)];
+    o = k.add ? op[row_ptr(f - 3 >= c0 && f - 3 < c1 ? f - 3 : c0, sa)] : 0.0;
+  };
+#pragma unroll
+  for (int j = 0; j < 6; j++) load_face(fa + j, tn[j], vn[j], on[j]);
+  double vprev = 0.0;
+  if (fa > 0 || k.per) { double sa; vprev = vp[row_ptr(fa - 1, sa)]; }
+  int par = 0;                                  // this round's ring offset: 0 or 6
+  for (int f0 = fa; f0 <= fend; f0 += 6) {
+    for (int i = lane; i < 6 * GPW; i += 64) {
+      const int j = i / GPW, gg = i - j * GPW;
+      double a = 0.0;
+#pragma unroll
+      for (int l = 0; l < 6; l++) a = fmax(a, ring_a[(par + j + l) % 12][gg]);
+      alpha[j][gg] = a;
+    }
+    wave_sync_lds();
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+      const int f = f0 + j;
+      double alphab = 0.0, vu = 0.0;
+      tw[(j + 5) % 6] = tn[j];
+      hu[(j + 5) % 6] = ring_u[(par + j + 5) % 12][grp];
+      at[(j + 5) % 6] = au[(j + 5) % 6] = 0.0;
+      const double vcur = (f < n || k.per) ? vn[j] : 0.0;
+      const double old = on[j];
+      const double y = (vcur - vprev) * k.idelta;
+      vprev = vcur;
+      load_face(f + 6, tn[j], vn[j], on[j]);
+      if (f <= fb) {
+        const double ha = 0.5 * alpha[j][grp];
+        double xp[5], xm[5], hp[5], hm[5];
+        {
+          double fp[5];
+#pragma unroll
+          for (int l = 0; l < 5; l++) {
+            hp[l] = hu[(j + l) % 6] + ha;
+            fp[l] = tw[(j + l) % 6] * hp[l];
+          }
+          (void)weno5_adj(fp[0], fp[1], fp[2], fp[3], fp[4], WENO_EPSB, y, xp);
+#pragma unroll
+          for (int l = 0; l < 5; l++) at[(j + l) % 6] = fma(xp[l], hp[l], at[(j + l) % 6]);
+        }
+        {
+          double fm[5];                          // point 5 - l
+#pragma unroll
+          for (int l = 0; l < 5; l++) {
+            hm[l] = hu[(j + 5 - l) % 6] - ha;
+            fm[l] = tw[(j + 5 - l) % 6] * hm[l];
+          }
+          (void)weno5_adj(fm[0], fm[1], fm[2], fm[3], fm[4], WENO_EPSB, y, xm);
+#pragma unroll
+          for (int l = 0; l < 5; l++)
+            at[(j + 5 - l) % 6] = fma(xm[l], hm[l], at[(j + 5 - l) % 6]);
+        }
+        // u_l: half of t (x+ + x-), alpha: half of the sum of t (x+ - x-)
+#pragma unroll
+        for (int l = 0; l < 6; l++) {
+          const double t = tw[(j + l) % 6];
+          const double xs = l == 0 ? xp[0] : l == 5 ? xm[0] : xp[l] + xm[5 - l];
+          const double xd = l == 0 ? xp[0] : l == 5 ? -xm[0] : xp[l] - xm[5 - l];
+          au[(j + l) % 6] = fma(t, xs, au[(j + l) % 6]);
+          alphab = fma(t, xd, alphab);
+        }
+      }
+      // row f-3 is complete; ghosts go to their source rows
+      const int e = f - 3;
+      double vt = at[j];
+      vu = au[j];
+      if (!k.per) {
+        if (e < 0) {
+          held[e + 3][0][lane] = k.sa_lo * vt;
+          held[e + 3][1][lane] = k.su_lo * vu;
+        } else if (e < 3) {
+          vt += held[2 - e][0][lane];
+          vu += held[2 - e][1][lane];
+        }
+        if (e >= n - 3) {
+          vt = fma(k.sa_hi, at[(j + 3) % 6], vt);
+          vu = fma(k.su_hi, au[(j + 3) % 6], vu);
+        }
+      }
+      if (e >= c0 && e < c1 && act) op[(long)e * k.rs * NC] = k.add ? old + vt : vt;
+      if (lane < GPW * NC) {
+        red[j][0][lane] = vu;
+        red[j][1][lane] = alphab;
+      }
+    }
+    wave_sync_lds();
+    // sums over the tracers; each face's alpha adjoint is written by the segment it opens
+    // (face n by the last one, as zero if it is face 0 again)
+    for (int i = lane; i < 12 * GPW; i += 64) {
+      const int j = i / (2 * GPW), q = (i / GPW) & 1, gg = i - (i / GPW) * GPW;
+      double a = red[j][q][gg * NC];
+#pragma unroll
+      for (int cc = 1; cc < NC; cc++) a += red[j][q][gg * NC + cc];
+      a *= 0.5;
+      const long col = col0 + gg;
+      if (col < k.ncol) {
+        const int f = f0 + j, e = f - 3;
+        if (q == 0) {
+          if (e >= c0 && e < c1) k.ub[cell_of(col) + e * k.rs] = a;
+        } else if (f >= c0 && (f < c1 || (f == n && c1 == n))) {
+          k.alb[f * k.afs + col * k.acs] = k.per && f == n ? 0.0 : a;
+        }
+      }
+    }
+    fill(f0 + 8, par + 11, 6);
+    par = 6 - par;
+    wave_sync_lds();
+  }
+}
+
+constexpr int NV = 5;      // fluid components
+
+__device__ inline void out_put(const FieldsOut &o, int q, long cell, double v, bool add) {
+  double *p = &o.w[q][cell];
   *p = add ? *p + v : v;
 }
 
@@ -478,7 +658,6 @@ __device__ inline int xghost_pair(int n, int f, int l) {
 // The six points go in as six no-return LDS adds, one point per instruction: within one
 // instruction the lanes hit distinct slots, and a wave's LDS operations complete in
 // order, so the sum order (point 0 first) is fixed.
-template <int NV>
 struct XSink {
   double *ring;            // [NV][128]
   double *side;            // [(pair * NV + q) * nlines + line]
@@ -496,11 +675,10 @@ struct XSink {
   }
 };
 
-template <int NC>
 __global__ void __launch_bounds__(64)
-fe_vjp_sweep_x(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int lps, int add) {
-  constexpr int NV = 5 + NC;
-  __shared__ double ring[NV * 128];
+fe_vjp_sweep_x(Grid g, Fields w, Fields vc, const double *ub, const double *alb, FieldsOut out,
+               double *side, int lps, int add) {
+    __shared__ double ring[NV * 128];
   const int lane = threadIdx.x;
   const int nx = g.nx, nxp = g.nx + 1;
   const int nlines = g.ny * g.nz;
@@ -508,7 +686,6 @@ fe_vjp_sweep_x(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int lps
   const int L1 = min(L0 + lps, nlines);
   if (L0 >= nlines) return;
   const long Q0 = (long)L0 * nxp, Q1 = (long)L1 * nxp;
-  const long ncell = (long)nx * nlines;
   for (int s = lane; s < NV * 128; s += 64) ring[s] = 0.0;
   wave_sync_lds();
   long done = Q0;          // first slot not yet written out
@@ -516,8 +693,8 @@ fe_vjp_sweep_x(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int lps
     const long q = B + lane;
     if (q < Q1) {
       const int line = (int)(q / nxp), f = (int)(q - (long)line * nxp);
-      XSink<NV> sink{ring, side, q, f, nx, line, nlines};
-      face_vjp<NC>(g, w, vc, 0, f, line % g.ny, line / g.ny, sink);
+      XSink sink{ring, side, q, f, nx, line, nlines};
+      face_vjp(g, w, vc, ub, alb ? alb[q] : 0.0, 0, f, line % g.ny, line / g.ny, sink);
     }
     wave_sync_lds();
     const long hi = (B + 64 >= Q1) ? Q1 - 1 : B + 60;
@@ -527,7 +704,7 @@ fe_vjp_sweep_x(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int lps
       if (e < nx) {
         const long cell = e + (long)nx * line;
 #pragma unroll 1
-        for (int qq = 0; qq < NV; qq++) out_put(out, ncell, qq, cell, ring[qq * 128 + slot], add);
+        for (int qq = 0; qq < NV; qq++) out_put(out, qq, cell, ring[qq * 128 + slot], add);
       }
 #pragma unroll 1
       for (int qq = 0; qq < NV; qq++) ring[qq * 128 + slot] = 0.0;
@@ -542,16 +719,13 @@ fe_vjp_sweep_x(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int lps
 // distinct source cells (lines of six cells or more), each source takes its pairs' sums in
 // registers, in the pairs' order, and is read and written once (all loads issued
 // together): the same sums as one read-modify-write per pair.
-template <int NC>
 __global__ void __launch_bounds__(256)
 fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
-  constexpr int NV = 5 + NC;
-  const int nlines = g.ny * g.nz;
+    const int nlines = g.ny * g.nz;
   const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (tid >= (long)nlines * NV) return;
   const int line = (int)(tid % nlines), qq = (int)(tid / nlines);
   const int n = g.nx;
-  const long ncell = (long)n * nlines;
   int src[6];
 #pragma unroll
   for (int e = 0; e < 6; e++) src[e] = ghost_map(g, 0, e < 3 ? e - 3 : n + (e - 3)).src;
@@ -577,7 +751,7 @@ fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
 #pragma unroll
     for (int e = 0; e < 6; e++) {
       cell[e] = src[e] + (long)n * line;
-      old[e] = qq < 5 ? out.w[qq][cell[e]] : out.chem[(long)(qq - 5) * ncell + cell[e]];
+      old[e] = out.w[qq][cell[e]];
     }
     double v[6];
     v[0] = old[0] + add[0];
@@ -588,8 +762,7 @@ fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
     v[5] = old[5] + add[5];
 #pragma unroll
     for (int e = 0; e < 6; e++) {
-      if (qq < 5) out.w[qq][cell[e]] = v[e];
-      else out.chem[(long)(qq - 5) * ncell + cell[e]] = v[e];
+      out.w[qq][cell[e]] = v[e];
     }
     return;
   }
@@ -600,7 +773,7 @@ fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
       const int pr = xghost_pair(n, f, l);
       if (pr < 0) continue;
       const long cell = ghost_map(g, 0, f - 3 + l).src + (long)n * line;
-      out_put(out, (long)n * nlines, qq, cell, side[((long)pr * NV + qq) * nlines + line], true);
+      out_put(out, qq, cell, side[((long)pr * NV + qq) * nlines + line], true);
     }
   }
 }
@@ -614,14 +787,12 @@ fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
 // either side that belong to neighbouring segments) go to the side buffer
 // [((seg * 6 + k) * NV + q) * ncol + col] and are added by fe_vjp_fix_yz.
 // ------------------------------------------------------------------------------------
-template <int NV>
 struct ColSink {
   double *ring;            // this wave's [5][NV][64]
   double *side;
   FieldsOut out;
   int lane, slot0;         // slot0: ring slot of row f-3 (slot of row f-3+l is (slot0+l)%5)
   int e0, c0, c1, seg;
-  long ncell;
   long col, ncol;
   long cell0;              // cell of row f-3 when it lies in [c0, c1)
   long cbase;              // cell of the column's row 0
@@ -629,7 +800,7 @@ struct ColSink {
   __device__ int slot(int l) const { const int s = slot0 + l; return s >= 5 ? s - 5 : s; }
   __device__ bool owned() const { return e0 >= c0 && e0 < c1; }
   __device__ double *dst(int comp) const {
-    return comp < 5 ? &out.w[comp][cell0] : &out.chem[(long)(comp - 5) * ncell + cell0];
+    return &out.w[comp][cell0];
   }
   struct Pre { double r0, w0; };
   // row f-3 so far, and the value already in wbar where this sweep adds to it (read
@@ -637,7 +808,7 @@ struct ColSink {
   // looked at in put, so that the loads stay in flight meanwhile)
   __device__ Pre pre(int comp) const {
     const long c = add && owned() ? cell0 : cbase;
-    const double w0 = comp < 5 ? out.w[comp][c] : out.chem[(long)(comp - 5) * ncell + c];
+    const double w0 = out.w[comp][c];
     return Pre{ring[((long)slot0 * NV + comp) * 64 + lane], w0};
   }
   __device__ void put(int comp, const double (&x)[6], const Pre &p) {
@@ -653,11 +824,11 @@ struct ColSink {
   }
 };
 
-template <int D, int NC>
+template <int D>
 __global__ void __launch_bounds__(64)
-fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int nseg, int add) {
-  constexpr int NV = 5 + NC;
-  __shared__ double ring[5 * NV * 64];
+fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, const double *ub, const double *alb, FieldsOut out,
+                double *side, int nseg, int add) {
+    __shared__ double ring[5 * NV * 64];
   const int lane = threadIdx.x;
   const int nxb = (g.nx + 63) / 64;
   const int nt = D == 1 ? g.nz : g.ny;
@@ -673,15 +844,15 @@ fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int ns
   for (int s = 0; s < 5 * NV; s++) ring[s * 64 + lane] = 0.0;
   const long rstride = D == 1 ? g.nx : (long)g.nx * g.ny;
   const long cbase = D == 1 ? i + (long)g.nx * g.ny * t : i + (long)g.nx * t;
-  const long ncell = (long)g.nx * g.ny * g.nz;
-  ColSink<NV> sink{ring, side, out, lane, 0, 0, c0, c1, seg, ncell, col, ncol, 0, cbase,
+  ColSink sink{ring, side, out, lane, 0, 0, c0, c1, seg, col, ncol, 0, cbase,
                    add != 0};
   for (int f = c0; f <= flast; f++) {
     sink.slot0 = (f - c0) % 5;
     sink.e0 = f - 3;
     sink.cell0 = cbase + (long)(f - 3) * rstride;
-    if (D == 1) face_vjp<NC>(g, w, vc, 1, i, f, t, sink);
-    else face_vjp<NC>(g, w, vc, 2, i, t, f, sink);
+    const double ab = alb ? alb[f * ncol + col] : 0.0;
+    if (D == 1) face_vjp(g, w, vc, ub, ab, 1, i, f, t, sink);
+    else face_vjp(g, w, vc, ub, ab, 2, i, t, f, sink);
   }
   // rows flast-2 .. flast+2 are complete
   for (int r = 0; r < 5; r++) {
@@ -689,7 +860,7 @@ fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int ns
     const int sl = (flast + 1 - c0 + r) % 5;
     for (int qq = 0; qq < NV; qq++) {
       const double v = ring[((long)sl * NV + qq) * 64 + lane];
-      if (e >= c0 && e < c1) out_put(out, ncell, qq, cbase + (long)e * rstride, v, add != 0);
+      if (e >= c0 && e < c1) out_put(out, qq, cbase + (long)e * rstride, v, add != 0);
       else {
         const int k = e < c0 ? e - (c0 - 3) : 3 + (e - c1);
         side[(((long)seg * 6 + k) * NV + qq) * ncol + col] = v;
@@ -703,11 +874,10 @@ fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, FieldsOut out, double *side, int ns
 // Side rows of every segment of a column into their cells (one thread per column and
 // component, segments and rows in a fixed order): rows of neighbouring segments directly,
 // ghost rows through the ghost rule's source (their signs were applied at the faces).
-template <int D, int NC>
+template <int D>
 __global__ void __launch_bounds__(256)
 fe_vjp_fix_yz(Grid g, const double *side, FieldsOut out, int nseg) {
-  constexpr int NV = 5 + NC;
-  const int nt = D == 1 ? g.nz : g.ny;
+    const int nt = D == 1 ? g.nz : g.ny;
   const int n = D == 1 ? g.ny : g.nz;
   const long ncol = (long)g.nx * nt;
   const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -717,7 +887,6 @@ fe_vjp_fix_yz(Grid g, const double *side, FieldsOut out, int nseg) {
   const int i = (int)(col % g.nx), t = (int)(col / g.nx);
   const long rstride = D == 1 ? g.nx : (long)g.nx * g.ny;
   const long cbase = D == 1 ? i + (long)g.nx * g.ny * t : i + (long)g.nx * t;
-  const long ncell = (long)g.nx * g.ny * g.nz;
   for (int seg = 0; seg < nseg; seg++) {
     const int c0 = (int)((long)seg * n / nseg), c1 = (int)((long)(seg + 1) * n / nseg);
     // when a segment's six side rows land in six distinct cells (segments of at least
@@ -737,12 +906,11 @@ fe_vjp_fix_yz(Grid g, const double *side, FieldsOut out, int nseg) {
       for (int k = 0; k < 6; k++) {
         cell[k] = cbase + (long)src[k] * rstride;
         add[k] = side[(((long)seg * 6 + k) * NV + qq) * ncol + col];
-        old[k] = qq < 5 ? out.w[qq][cell[k]] : out.chem[(long)(qq - 5) * ncell + cell[k]];
+        old[k] = out.w[qq][cell[k]];
       }
 #pragma unroll
       for (int k = 0; k < 6; k++) {
-        if (qq < 5) out.w[qq][cell[k]] = old[k] + add[k];
-        else out.chem[(long)(qq - 5) * ncell + cell[k]] = old[k] + add[k];
+        out.w[qq][cell[k]] = old[k] + add[k];
       }
       continue;
     }
@@ -751,41 +919,14 @@ fe_vjp_fix_yz(Grid g, const double *side, FieldsOut out, int nseg) {
       const int e = k < 3 ? c0 - 3 + k : c1 + (k - 3);
       const int src = ghost_map(g, D, e).src;
       const long cell = cbase + (long)src * rstride;
-      out_put(out, ncell, qq, cell, side[(((long)seg * 6 + k) * NV + qq) * ncol + col], true);
+      out_put(out, qq, cell, side[(((long)seg * 6 + k) * NV + qq) * ncol + col], true);
     }
   }
 }
 
-// Tracer layout: the C ABI holds tracers cell-major ([cell][nchem]); the sweeps read
-// and write them tracer-major ([nchem][cell]) so that every tracer access of a wave is one
-// contiguous 512-byte run. 256 cells per block through an LDS tile, both sides coalesced.
-template <int NC>
-__global__ void __launch_bounds__(256) cells_to_planes(const double *a, double *p, long ncell) {
-  __shared__ double t[(NC > 0 ? NC : 1) * 257];
-  const long base = (long)blockIdx.x * 256;
-  const long lim = (ncell - base) * NC;
-  for (int k = threadIdx.x; k < NC * 256; k += 256)
-    if (k < lim) t[(k % NC) * 257 + k / NC] = a[base * NC + k];
-  __syncthreads();
-  const long cell = base + threadIdx.x;
-  if (cell < ncell)
-#pragma unroll
-    for (int c = 0; c < NC; c++) p[(long)c * ncell + cell] = t[c * 257 + threadIdx.x];
-}
-
-template <int NC>
-__global__ void __launch_bounds__(256) planes_to_cells(const double *p, double *a, long ncell) {
-  __shared__ double t[(NC > 0 ? NC : 1) * 257];
-  const long base = (long)blockIdx.x * 256;
-  const long cell = base + threadIdx.x;
-  if (cell < ncell)
-#pragma unroll
-    for (int c = 0; c < NC; c++) t[c * 257 + threadIdx.x] = p[(long)c * ncell + cell];
-  __syncthreads();
-  const long lim = (ncell - base) * NC;
-  for (int k = threadIdx.x; k < NC * 256; k += 256)
-    if (k < lim) a[base * NC + k] = t[(k % NC) * 257 + k / NC];
-}
+// Waves that the tracer walk of one direction is split into at least, where columns allow:
+// four per SIMD.
+constexpr long TRACER_WAVES = 4096;
 
 // Launch shape: one wave per SIMD over the device (4 per CU) where the grid allows.
 struct VjpPlan {
@@ -799,7 +940,7 @@ static VjpPlan vjp_plan(const Grid &g) {
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const long target = 4L * (ncu > 0 ? ncu : 256);
-  const long nv = 5 + g.nchem;
+  const long nv = NV;
   VjpPlan p{};
   const long nlines = (long)g.ny * g.nz;
   p.lps = (int)((nlines + target - 1) / target);
@@ -819,60 +960,106 @@ static VjpPlan vjp_plan(const Grid &g) {
   return p;
 }
 
-// Scratch: the side buffer, then (with tracers) tracer planes of w and wbar.
+// One direction: the tracers (with NC > 0), then the fluid sweep and its fix-up.
 template <int NC>
-static int fe_vjp_run(const Grid &g, const Fields &w, const Fields &v, const FieldsOut &out,
-                      double *buf, hipStream_t st) {
-  const VjpPlan p = vjp_plan(g);
-  const long nlines = (long)g.ny * g.nz;
-  const long ncell = (long)g.nx * nlines;
-  const int nxb = (g.nx + 63) / 64;
-  constexpr long NV = 5 + NC;
-  double *side = buf;
-  Fields wp = w, vp = v;
-  FieldsOut op = out;
-  const unsigned tb = (unsigned)((ncell + 255) / 256);
-  if constexpr (NC > 0) {
-    double *pw = buf + p.side, *po = pw + NC * ncell;
-    hipLaunchKernelGGL(cells_to_planes<NC>, dim3(tb), dim3(256), 0, st, w.chem, pw, ncell);
-    wp.chem = pw;
-    op.chem = po;
-  }
-  hipLaunchKernelGGL(fe_vjp_sweep_x<NC>, dim3((unsigned)((nlines + p.lps - 1) / p.lps)),
-                     dim3(64), 0, st, g, wp, vp, op, side, p.lps, 0);
-  hipLaunchKernelGGL(fe_vjp_fix_x<NC>, dim3((unsigned)((nlines * NV + 255) / 256)), dim3(256), 0,
-                     st, g, (const double *)side, op);
-  hipLaunchKernelGGL((fe_vjp_sweep_yz<1, NC>), dim3((unsigned)(nxb * g.nz * p.nseg[1])), dim3(64),
-                     0, st, g, wp, vp, op, side, p.nseg[1], 1);
-  hipLaunchKernelGGL((fe_vjp_fix_yz<1, NC>),
-                     dim3((unsigned)(((long)g.nx * g.nz * NV + 255) / 256)), dim3(256), 0, st, g,
-                     (const double *)side, op, p.nseg[1]);
-  hipLaunchKernelGGL((fe_vjp_sweep_yz<2, NC>), dim3((unsigned)(nxb * g.ny * p.nseg[2])), dim3(64),
-                     0, st, g, wp, vp, op, side, p.nseg[2], 1);
-  hipLaunchKernelGGL((fe_vjp_fix_yz<2, NC>),
-                     dim3((unsigned)(((long)g.nx * g.ny * NV + 255) / 256)), dim3(256), 0, st, g,
-                     (const double *)side, op, p.nseg[2]);
-  if constexpr (NC > 0)
-    hipLaunchKernelGGL(planes_to_cells<NC>, dim3(tb), dim3(256), 0, st, (const double *)op.chem,
-                       out.chem, ncell);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+static void tracers_launch(const Grid &g, int d, const Fields &w, const double *v, double *out,
+                           double *ub, double *alb, hipStream_t st) {
+  constexpr long GPW = 64 / NC;
+  const long nx = g.nx, nxy = nx * g.ny;
+  TrWalk k{};
+  k.r = w.w[0]; k.m0 = w.w[1]; k.m1 = w.w[2]; k.m2 = w.w[3]; k.e = w.w[4]; k.mn = w.w[1 + d];
+  k.t = w.chem; k.v = v; k.out = out; k.ub = ub; k.alb = alb;
+  k.n = extent(g, d);
+  k.ncol = nxy * g.nz / k.n;
+  k.nin = (int)(d == 0 ? 1 : d == 1 ? nx : nxy);
+  k.bs_in = d == 0 ? 0 : 1;
+  k.bs_out = d == 0 ? nx : nxy;
+  k.rs = d == 0 ? 1 : d == 1 ? nx : nxy;
+  k.afs = d == 0 ? 1 : k.ncol;
+  k.acs = d == 0 ? k.n + 1 : 1;
+  k.per = g.bc[2 * d] == BC_PERIODIC;
+  k.add = d != 0;
+  const int lo = g.bc[2 * d], hi = g.bc[2 * d + 1];
+  k.sa_lo = lo == BC_DIRICHLET ? -1.0 : 1.0;
+  k.sa_hi = hi == BC_DIRICHLET ? -1.0 : 1.0;
+  k.su_lo = lo == BC_REFLECTING ? -1.0 : 1.0;      // Dirichlet negates m and rho: u stays
+  k.su_hi = hi == BC_REFLECTING ? -1.0 : 1.0;
+  k.idelta = 1.0 / (d == 0 ? g.dx : d == 1 ? g.dy : g.dz);
+  k.gamma = g.gamma;
+  k.ncb = (int)((k.ncol + GPW - 1) / GPW);
+  const long maxseg = k.n >= 16 ? k.n / 8 : 1;
+  k.nseg = (int)std::min(maxseg, (TRACER_WAVES + k.ncb - 1) / k.ncb);
+  hipLaunchKernelGGL(fe_vjp_tracers<NC>, dim3((unsigned)(k.ncb * k.nseg)), dim3(64), 0, st, k);
 }
 
+static int tracers_run(const Grid &g, int d, const Fields &w, const double *v, double *out,
+                       double *ub, double *alb, hipStream_t st) {
+  switch (g.nchem) {
+    case 1: tracers_launch<1>(g, d, w, v, out, ub, alb, st); return 0;
+    case 2: tracers_launch<2>(g, d, w, v, out, ub, alb, st); return 0;
+    case 4: tracers_launch<4>(g, d, w, v, out, ub, alb, st); return 0;
+    case 6: tracers_launch<6>(g, d, w, v, out, ub, alb, st); return 0;
+    case 10: tracers_launch<10>(g, d, w, v, out, ub, alb, st); return 0;
+    default: return MVD_UNSUPPORTED;
+  }
+}
+
+static long max_faces(const Grid &g) {
+  const long nx = g.nx, ny = g.ny, nz = g.nz;
+  return std::max({(nx + 1) * ny * nz, nx * (ny + 1) * nz, nx * ny * (nz + 1)});
+}
+
+// Scratch: the side buffer; with tracers also ub (cells), alb (faces of a direction) and a
+// tracer array for calls whose wbar tracers overlap an input's.
 size_t fe_vjp_buffer_doubles(const Grid &g) {
-  return vjp_plan(g).side + (size_t)2 * g.nchem * g.nx * g.ny * g.nz;
+  const long ncell = (long)g.nx * g.ny * g.nz;
+  return vjp_plan(g).side + (g.nchem ? (size_t)(1 + g.nchem) * ncell + max_faces(g) : 0);
 }
 
 int fe_vjp_launch(const Grid &g, const Fields &w, const Fields &v, const FieldsOut &out,
                   double *buf, hipStream_t st) {
-  switch (g.nchem) {
-    case 0: return fe_vjp_run<0>(g, w, v, out, buf, st);
-    case 1: return fe_vjp_run<1>(g, w, v, out, buf, st);
-    case 2: return fe_vjp_run<2>(g, w, v, out, buf, st);
-    case 4: return fe_vjp_run<4>(g, w, v, out, buf, st);
-    case 6: return fe_vjp_run<6>(g, w, v, out, buf, st);
-    case 10: return fe_vjp_run<10>(g, w, v, out, buf, st);
-    default: return MVD_UNSUPPORTED;
+  constexpr long NV = 5;
+  const VjpPlan p = vjp_plan(g);
+  const long nlines = (long)g.ny * g.nz, ncell = g.nx * nlines;
+  const int nxb = (g.nx + 63) / 64;
+  double *side = buf, *ub = nullptr, *alb = nullptr, *tr = nullptr;
+  if (g.nchem) {
+    ub = buf + p.side;
+    alb = ub + ncell;
+    const long nt = g.nchem * ncell;
+    const auto overlaps = [&](const double *a) { return a < out.chem + nt && out.chem < a + nt; };
+    tr = overlaps(w.chem) || overlaps(v.chem) ? alb + max_faces(g) : out.chem;
   }
+  for (int d = 0; d < 3; d++) {
+    if (g.nchem) {
+      const int rc = tracers_run(g, d, w, v.chem, tr, ub, alb, st);
+      if (rc) return rc;
+    }
+    if (d == 0) {
+      hipLaunchKernelGGL(fe_vjp_sweep_x, dim3((unsigned)((nlines + p.lps - 1) / p.lps)), dim3(64),
+                         0, st, g, w, v, (const double *)ub, (const double *)alb, out, side, p.lps,
+                         0);
+      hipLaunchKernelGGL(fe_vjp_fix_x, dim3((unsigned)((nlines * NV + 255) / 256)), dim3(256), 0,
+                         st, g, (const double *)side, out);
+    } else if (d == 1) {
+      hipLaunchKernelGGL(fe_vjp_sweep_yz<1>, dim3((unsigned)(nxb * g.nz * p.nseg[1])), dim3(64), 0,
+                         st, g, w, v, (const double *)ub, (const double *)alb, out, side,
+                         p.nseg[1], 1);
+      hipLaunchKernelGGL(fe_vjp_fix_yz<1>, dim3((unsigned)(((long)g.nx * g.nz * NV + 255) / 256)),
+                         dim3(256), 0, st, g, (const double *)side, out, p.nseg[1]);
+    } else {
+      hipLaunchKernelGGL(fe_vjp_sweep_yz<2>, dim3((unsigned)(nxb * g.ny * p.nseg[2])), dim3(64), 0,
+                         st, g, w, v, (const double *)ub, (const double *)alb, out, side,
+                         p.nseg[2], 1);
+      hipLaunchKernelGGL(fe_vjp_fix_yz<2>, dim3((unsigned)(((long)g.nx * g.ny * NV + 255) / 256)),
+                         dim3(256), 0, st, g, (const double *)side, out, p.nseg[2]);
+    }
+  }
+  if (tr != out.chem &&
+      hipMemcpyAsync(out.chem, tr, sizeof(double) * g.nchem * ncell, hipMemcpyDeviceToDevice,
+                     st) != hipSuccess)
+    return -1;
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 }  // namespace mvd
