@@ -71,10 +71,8 @@ int mvd_last_state_flags(mvd_context *ctx);
 /* Vector-Jacobian product of fe() (no counterpart in the reference, which has no adjoint;
  * for adjoint/sensitivity callers): wbar = (d wdot / d w)^T v, v and wbar in the layout of
  * wdot. The derivative of the Lax-Friedrichs speed max() follows its first maximum.
- * Keeps no face buffer. On first use it allocates its scratch: a side buffer for the stencil
- * adjoints that leave an x-line or a y/z column segment (60 doubles per x-line, 30 per column
- * segment) and, with tracers, two doubles per cell and a tracer array (for a call whose wbar
- * tracers overlap an input's tracers). */
+ * Keeps no face buffer. With tracers it allocates its scratch on first use: two doubles per
+ * cell and a tracer array (for a call whose wbar tracers overlap an input's tracers). */
 int mvd_fe_vjp(mvd_context *ctx, double t, const double *const *w, const double *const *v,
                double *const *wbar);
 

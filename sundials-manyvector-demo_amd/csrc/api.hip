@@ -21,7 +21,7 @@ struct mvd_context {
   mvd::ChemState chem;
   int dirk_block = 256;   // batched DIRK launch shape (set by mvd_chem_dirk_tune)
   int dirk_waves = 0;     // resident waves of the persistent grid (0: one per SIMD)
-  double *vjp_buf = nullptr;   // fe() VJP scratch: side buffer, tracer planes (first use)
+  double *vjp_buf = nullptr;   // fe() VJP scratch of the tracers (first use)
   // block linear solver of the chemistry subvector (allocated by the first lsetup)
   double *ls_lu = nullptr;
   unsigned long long *ls_piv = nullptr;
@@ -192,8 +192,8 @@ int mvd_fe_vjp(mvd_context *ctx, double, const double *const *w, const double *c
   if (!rc) rc = check_ptrs(ctx, v);
   if (!rc) rc = check_ptrs(ctx, (const double *const *)wbar);
   if (rc) return rc;
-  if (!ctx->vjp_buf &&
-      !dev_ok(hipMalloc(&ctx->vjp_buf, sizeof(double) * mvd::fe_vjp_buffer_doubles(ctx->g))))
+  const size_t nbuf = mvd::fe_vjp_buffer_doubles(ctx->g);
+  if (nbuf && !ctx->vjp_buf && !dev_ok(hipMalloc(&ctx->vjp_buf, sizeof(double) * nbuf)))
     return MVD_DEVICE_ERROR;
   rc = mvd::fe_vjp_launch(ctx->g, fields_of(ctx, w), fields_of(ctx, v), fields_out(ctx, wbar),
                           ctx->vjp_buf, ctx->stream);

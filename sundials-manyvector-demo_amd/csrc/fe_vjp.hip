@@ -3,22 +3,18 @@
 // fe(w) = -div F with every face flux a function of its 6-point stencil, so
 //   Fbar(face between cells c-1 | c) = (v_c - v_{c-1}) / delta   (no cell: 0)
 // and each face's stencil adjoint sbar = (dF/ds)^T Fbar goes back to the stencil's source
-// cells (ghost points are +-copies of interior cells). Every face recomputes its flux (the
-// reference recipe, utilities.cpp:270-479) and sweeps it in reverse (WENO5-JS weights,
-// Lax-Friedrichs split, characteristic projections, Roe average and eigenvectors, point
-// fluxes, wave speeds, EOS). No face buffer: one sweep kernel per direction adds the
-// contributions into the cells as it walks along the lines, through a ring of open rows
-// in LDS, and writes each cell once its last face is in:
-//   fe_vjp_sweep_x   - a wave walks whole x-lines 64 faces at a time (lanes along x);
-//   fe_vjp_sweep_yz  - each lane walks its own column along y or z (lanes along x);
-//   fe_vjp_fix_x/_yz - add the contributions that left a line or segment (ghost points,
-//                      rows of neighbouring segments), held in a small side buffer.
-// The x sweep stores wbar, the others add. No atomics: the result is deterministic.
-// Tracers have a kernel of their own per direction (fe_vjp_tracers), run before the fluid
-// sweep, which takes over the velocity and wave-speed adjoints that the tracers produce. In
-// one kernel the 15 components left one wave per SIMD (38 KB of LDS, 480 registers) waiting on
-// its loads; apart, with the tracer-major copies of w and wbar gone, 128^3 with ten tracers
-// takes 2.28 instead of 2.77 ms.
+// cells (ghost points are +-copies of interior cells). Every face recomputes its flux in the
+// form of face_flux_lds and sweeps it in reverse. No face buffer: per direction a kernel walks
+// along the lines and writes each cell once its last face is in:
+//   fe_vjp_tracers - tracers, each lane its own (column, tracer), any direction;
+//   fe_vjp_lines   - fluid along x: a wave walks whole x-lines 64 faces at a time;
+//   fe_vjp_walk    - fluid along y or z: each lane its own column.
+// The x kernels store wbar, the others add. No atomics between waves: the result is
+// deterministic. The tracer kernel of a direction runs before the fluid one, which takes over
+// the velocity and wave-speed adjoints that the tracers produce. 128^3 with ten tracers: per
+// direction 0.28 (tracers) and 0.24 ms (fluid), 1.55 ms in all; one kernel for both, with tracer-
+// major copies of w and wbar and the reference's formula order, took 2.77 ms at one wave per
+// SIMD (480 registers, 38 KB of LDS).
 #include <algorithm>
 
 #include "mvd_device.hpp"
@@ -28,351 +24,6 @@
 namespace mvd {
 
 namespace {
-
-constexpr double W_BC = 1.083333333333333333333333333333333333333;   // 13/12
-constexpr double W_EPS = 1e-6;
-constexpr double W_C13 = 0.3333333333333333333333333333333333333333;
-constexpr double W_C56 = 0.8333333333333333333333333333333333333333;
-constexpr double W_C16 = 0.1666666666666666666666666666666666666667;
-constexpr double W_C76 = 1.166666666666666666666666666666666666667;
-constexpr double W_C116 = 1.833333333333333333333333333333333333333;
-
-// WENO5-JS reconstruction from f[0..4] (side 0: the f+ formula over points i-3..i+1,
-// side 1: the mirrored f- formula over points i-2..i+2) and its gradient g = dr/df.
-// With the normalised weights o_k = w_k / sum w: r = sum o_k q_k and
-//   dr/df = sum o_k dq_k/df + sum_k kap_k db_k/df,   kap_k = -2 o_k (q_k - r) / e_k,
-// db_k/df = 2 (13/12) A_k dA_k/df + (B_k / 2) dB_k/df; the gradient is written out term by
-// term (no products with the zero entries of the stencil derivatives).
-__device__ inline double weno5_grad(const double (&f)[5], int side, double (&g)[5]) {
-  const double A1 = f[2] - 2.0 * f[3] + f[4], B1 = 3.0 * f[2] - 4.0 * f[3] + f[4];
-  const double A2 = f[1] - 2.0 * f[2] + f[3], B2 = f[1] - f[3];
-  const double A3 = f[0] - 2.0 * f[1] + f[2], B3 = f[0] - 4.0 * f[1] + 3.0 * f[2];
-  const double b1 = W_BC * A1 * A1 + 0.25 * B1 * B1;
-  const double b2 = W_BC * A2 * A2 + 0.25 * B2 * B2;
-  const double b3 = W_BC * A3 * A3 + 0.25 * B3 * B3;
-  const double d1 = side == 0 ? 0.3 : 0.1, d3 = side == 0 ? 0.1 : 0.3;
-  const double e1 = W_EPS + b1, e2 = W_EPS + b2, e3 = W_EPS + b3;
-  const double ie1 = fast_rcp(e1), ie2 = fast_rcp(e2), ie3 = fast_rcp(e3);
-  const double w1 = d1 * ie1 * ie1, w2 = 0.6 * ie2 * ie2, w3 = d3 * ie3 * ie3;
-  // candidate stencils q_k and their coefficients (dq_k/df over the points they use)
-  double q1, q2, q3;
-  double c10, c11, c12, c21, c22, c23, c32, c33, c34;   // dq3/df0..2, dq2/df1..3, dq1/df2..4
-  if (side == 0) {
-    c10 = W_C13; c11 = -W_C76; c12 = W_C116;
-    c21 = -W_C16; c22 = W_C56; c23 = W_C13;
-    c32 = W_C13; c33 = W_C56; c34 = -W_C16;
-  } else {
-    c10 = -W_C16; c11 = W_C56; c12 = W_C13;
-    c21 = W_C13; c22 = W_C56; c23 = -W_C16;
-    c32 = W_C116; c33 = -W_C76; c34 = W_C13;
-  }
-  q1 = c32 * f[2] + c33 * f[3] + c34 * f[4];
-  q2 = c21 * f[1] + c22 * f[2] + c23 * f[3];
-  q3 = c10 * f[0] + c11 * f[1] + c12 * f[2];
-  const double iS = fast_rcp(w1 + w2 + w3);
-  const double o1 = w1 * iS, o2 = w2 * iS, o3 = w3 * iS;
-  const double r = q1 * o1 + q2 * o2 + q3 * o3;
-  const double k1 = -2.0 * o1 * ie1 * (q1 - r);
-  const double k2 = -2.0 * o2 * ie2 * (q2 - r);
-  const double k3 = -2.0 * o3 * ie3 * (q3 - r);
-  // kap_k db_k/df = a_k dA_k/df + c_k dB_k/df
-  const double a1 = (2.0 * W_BC) * k1 * A1, h1 = 0.5 * k1 * B1;   // dA1 (0,0,1,-2,1), dB1 (0,0,3,-4,1)
-  const double a2 = (2.0 * W_BC) * k2 * A2, h2 = 0.5 * k2 * B2;   // dA2 (0,1,-2,1,0), dB2 (0,1,0,-1,0)
-  const double a3 = (2.0 * W_BC) * k3 * A3, h3 = 0.5 * k3 * B3;   // dA3 (1,-2,1,0,0), dB3 (1,-4,3,0,0)
-  g[0] = o3 * c10 + a3 + h3;
-  g[1] = o2 * c21 + o3 * c11 + a2 + h2 - 2.0 * a3 - 4.0 * h3;
-  g[2] = o1 * c32 + o2 * c22 + o3 * c12 + a1 + 3.0 * h1 - 2.0 * a2 + a3 + 3.0 * h3;
-  g[3] = o1 * c33 + o2 * c23 - 2.0 * a1 - 4.0 * h1 + a2 - h2;
-  g[4] = o1 * c34 + a1 + h1;
-  return r;
-}
-
-// Adjoint of one face flux for the five fluid components, plus what the tracers need:
-// s, Fb, sb in direction-local order (rho, m_normal, m_t1, m_t2, et). The tracer part of
-// the reverse sweep (tracer_vjp) runs first and hands over the adjoints of the point
-// velocities (ulb) and of the Lax-Friedrichs speed (alphab) it produced.
-struct FacePrim {
-  double p[6], ul[6], ir[6];   // pressure, normal velocity, 1/rho per stencil point
-  double alpha;
-  int lstar;                   // the point that sets alpha
-};
-
-__device__ inline void face_prim(const double (&s)[6][5], double gamma, FacePrim &P) {
-  const double gm = gamma - 1.0;
-  P.alpha = 0.0;
-  P.lstar = -1;
-#pragma unroll
-  for (int l = 0; l < 6; l++) {
-    P.ir[l] = fast_rcp(s[l][0]);
-    P.p[l] = gm * (s[l][4] - (s[l][1] * s[l][1] + s[l][2] * s[l][2] + s[l][3] * s[l][3]) * 0.5 * P.ir[l]);
-    P.ul[l] = s[l][1] * P.ir[l];
-    const double a = fabs(P.ul[l]) + sun_sqrt(gamma * P.p[l] * P.ir[l]);
-    if (P.alpha < a) { P.alpha = a; P.lstar = l; }
-  }
-}
-
-__device__ inline void fluid_vjp(const double (&s)[6][5], double gamma, const FacePrim &P,
-                                 const double (&Fb)[5], double (&ulb)[6], double alphab,
-                                 double (&sb)[6][5]) {
-  const double gm = gamma - 1.0;
-  const double alpha = P.alpha;
-  const double sL = sun_sqrt(s[2][0]), sR = sun_sqrt(s[3][0]);
-  const double isL = fast_rcp(sL), isR = fast_rcp(sR);
-  const double sbar = 0.5 * (sL + sR), isbar = fast_rcp(sbar);
-  const double u = 0.5 * (s[2][1] * isL + s[3][1] * isR) * isbar;
-  const double v = 0.5 * (s[2][2] * isL + s[3][2] * isR) * isbar;
-  const double w = 0.5 * (s[2][3] * isL + s[3][3] * isR) * isbar;
-  const double H = 0.5 * ((P.p[2] + s[2][4]) * isL + (P.p[3] + s[3][4]) * isR) * isbar;
-  const double qsq = u * u + v * v + w * w;
-  const double cs = gm * (H - 0.5 * qsq);
-  const double ci = fast_rcp(cs);
-  const double LV[5][5] = {
-      {0.5 * ci * (u + 0.5 * gm * qsq), -0.5 * ci * (gm * u + 1.0), -0.5 * v * gm * ci,
-       -0.5 * w * gm * ci, 0.5 * gm * ci},
-      {-v, 0.0, 1.0, 0.0, 0.0},
-      {-w, 0.0, 0.0, 1.0, 0.0},
-      {(-gm) * ci * (qsq - H), u * gm * ci, v * gm * ci, w * gm * ci, (-gm) * ci},
-      {-0.5 * ci * (u - 0.5 * gm * qsq), -0.5 * ci * (gm * u - 1.0), -0.5 * v * gm * ci,
-       -0.5 * w * gm * ci, 0.5 * gm * ci}};
-  auto flux = [&](int l, int c) -> double {
-    if (c == 0) return s[l][1];
-    if (c == 1) return P.ul[l] * s[l][1] + P.p[l];
-    if (c == 4) return P.ul[l] * (s[l][4] + P.p[l]);
-    return P.ul[l] * s[l][c];
-  };
-  auto split = [&](int sd, int l, int c) -> double {
-    const int pt = l + sd;
-    return sd == 0 ? 0.5 * (flux(pt, c) + alpha * s[pt][c])
-                   : 0.5 * (flux(pt, c) - alpha * s[pt][c]);
-  };
-  // ---- reverse ----
-#pragma unroll
-  for (int l = 0; l < 6; l++)
-#pragma unroll
-    for (int c = 0; c < 5; c++) sb[l][c] = 0.0;
-  double pb[6] = {0, 0, 0, 0, 0, 0};
-  auto flux_adj = [&](int pt, int c, double fb) {
-    if (c == 0) { sb[pt][1] += fb; return; }
-    if (c == 1) { ulb[pt] += fb * s[pt][1]; sb[pt][1] += fb * P.ul[pt]; pb[pt] += fb; return; }
-    if (c == 4) {
-      ulb[pt] += fb * (s[pt][4] + P.p[pt]);
-      sb[pt][4] += fb * P.ul[pt];
-      pb[pt] += fb * P.ul[pt];
-      return;
-    }
-    ulb[pt] += fb * s[pt][c];
-    sb[pt][c] += fb * P.ul[pt];
-  };
-  // back-projection F = RV ff: ffb = RV^T Fb does not depend on ff, so the forward
-  // reconstruction and its reverse share one WENO pass per side
-  double ffb[5];
-  ffb[0] = Fb[0] + (u - cs) * Fb[1] + v * Fb[2] + w * Fb[3] + (H - u * cs) * Fb[4];
-  ffb[1] = Fb[2] + v * Fb[4];
-  ffb[2] = Fb[3] + w * Fb[4];
-  ffb[3] = Fb[0] + u * Fb[1] + v * Fb[2] + w * Fb[3] + 0.5 * qsq * Fb[4];
-  ffb[4] = Fb[0] + (u + cs) * Fb[1] + v * Fb[2] + w * Fb[3] + (H + u * cs) * Fb[4];
-  double ff[5] = {0, 0, 0, 0, 0};
-  double ub = 0.0, vb = 0.0, wb = 0.0, Hb = 0.0, cib = 0.0, qsqb = 0.0;
-#pragma unroll
-  for (int sd = 0; sd < 2; sd++) {
-    // fc[a][l]: characteristic split flux, then (in place) its adjoint ffb[a] * dW_a/dfc
-    double fc[5][5];
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      double fs[5];
-#pragma unroll
-      for (int b = 0; b < 5; b++) fs[b] = split(sd, l, b);
-#pragma unroll
-      for (int a = 0; a < 5; a++)
-        fc[a][l] = LV[a][0] * fs[0] + LV[a][1] * fs[1] + LV[a][2] * fs[2] +
-                   LV[a][3] * fs[3] + LV[a][4] * fs[4];
-    }
-#pragma unroll
-    for (int a = 0; a < 5; a++) {
-      double g[5];
-      ff[a] += weno5_grad(fc[a], sd, g);
-#pragma unroll
-      for (int l = 0; l < 5; l++) fc[a][l] = ffb[a] * g[l];
-    }
-    // per stencil point: LV-entry adjoints (LVb[a][b] = sum_l fc[a][l] fs[l][b]) folded
-    // straight into the Roe-state adjoints, and fsb = LV^T fc[.][l] into the split
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      double fs[5];
-#pragma unroll
-      for (int b = 0; b < 5; b++) fs[b] = split(sd, l, b);
-      const double e0 = fc[0][l], e3 = fc[3][l], e4 = fc[4][l];
-      const double e04p = e0 + e4;
-      cib += 0.5 * (u + 0.5 * gm * qsq) * e0 * fs[0] - 0.5 * (gm * u + 1.0) * e0 * fs[1] -
-             0.5 * gm * e04p * (v * fs[2] + w * fs[3] - fs[4]) - gm * (qsq - H) * e3 * fs[0] +
-             gm * e3 * (u * fs[1] + v * fs[2] + w * fs[3] - fs[4]) -
-             0.5 * (u - 0.5 * gm * qsq) * e4 * fs[0] - 0.5 * (gm * u - 1.0) * e4 * fs[1];
-      ub += 0.5 * ci * (e0 - e4) * fs[0] - 0.5 * ci * gm * e04p * fs[1] + gm * ci * e3 * fs[1];
-      qsqb += 0.25 * ci * gm * e04p * fs[0] - gm * ci * e3 * fs[0];
-      vb += -0.5 * gm * ci * e04p * fs[2] - fc[1][l] * fs[0] + gm * ci * e3 * fs[2];
-      wb += -0.5 * gm * ci * e04p * fs[3] - fc[2][l] * fs[0] + gm * ci * e3 * fs[3];
-      Hb += gm * ci * e3 * fs[0];
-      const int pt = l + sd;
-      const double sg = sd == 0 ? 0.5 : -0.5;
-#pragma unroll
-      for (int b = 0; b < 5; b++) {
-        const double fsb = LV[0][b] * fc[0][l] + LV[1][b] * fc[1][l] + LV[2][b] * fc[2][l] +
-                           LV[3][b] * fc[3][l] + LV[4][b] * fc[4][l];
-        flux_adj(pt, b, 0.5 * fsb);
-        sb[pt][b] += sg * alpha * fsb;
-        alphab += sg * fsb * s[pt][b];
-      }
-    }
-  }
-  // RV entries -> Roe state
-  double csb;
-  {
-    const double R10 = Fb[1] * ff[0], R14 = Fb[1] * ff[4];
-    const double R40 = Fb[4] * ff[0], R44 = Fb[4] * ff[4];
-    ub += R10 + Fb[1] * ff[3] + R14 + (R44 - R40) * cs;
-    csb = R14 - R10 + (R44 - R40) * u;
-    vb += Fb[2] * (ff[0] + ff[3] + ff[4]) + Fb[4] * ff[1];
-    wb += Fb[3] * (ff[0] + ff[3] + ff[4]) + Fb[4] * ff[2];
-    Hb += R40 + R44;
-    qsqb += 0.5 * Fb[4] * ff[3];
-  }
-  csb += -cib * ci * ci;
-  Hb += gm * csb;
-  qsqb += -0.5 * gm * csb;
-  ub += 2.0 * u * qsqb;
-  vb += 2.0 * v * qsqb;
-  wb += 2.0 * w * qsqb;
-  double sLb = 0.0, sRb = 0.0, sbarb = 0.0;
-  {
-    const double Aub = 0.5 * ub * isbar, Avb = 0.5 * vb * isbar, Awb = 0.5 * wb * isbar,
-                 AHb = 0.5 * Hb * isbar;
-    sbarb -= (ub * u + vb * v + wb * w + Hb * H) * isbar;
-    sb[2][1] += Aub * isL; sb[3][1] += Aub * isR;
-    sb[2][2] += Avb * isL; sb[3][2] += Avb * isR;
-    sb[2][3] += Awb * isL; sb[3][3] += Awb * isR;
-    sb[2][4] += AHb * isL; sb[3][4] += AHb * isR;
-    pb[2] += AHb * isL; pb[3] += AHb * isR;
-    sLb -= (Aub * s[2][1] + Avb * s[2][2] + Awb * s[2][3] + AHb * (P.p[2] + s[2][4])) * isL * isL;
-    sRb -= (Aub * s[3][1] + Avb * s[3][2] + Awb * s[3][3] + AHb * (P.p[3] + s[3][4])) * isR * isR;
-  }
-  sLb += 0.5 * sbarb;
-  sRb += 0.5 * sbarb;
-  if (s[2][0] > 0.0) sb[2][0] += 0.5 * sLb * isL;
-  if (s[3][0] > 0.0) sb[3][0] += 0.5 * sRb * isR;
-  // Lax-Friedrichs speed: alpha = |u_l*| + sqrt(gamma p_l* / rho_l*)
-  {
-    double ulS = 0.0, pS = 0.0, irS = 0.0;
-#pragma unroll
-    for (int l = 0; l < 6; l++)
-      if (l == P.lstar) { ulS = P.ul[l]; pS = P.p[l]; irS = P.ir[l]; }
-    const double X = gamma * pS * irS;
-    const double ulbS = ulS < 0.0 ? -alphab : alphab;
-    double pbS = 0.0, rbS = 0.0;
-    if (X > 0.0) {
-      const double Xb = 0.5 * alphab * fast_rcp(sun_sqrt(X));
-      pbS = Xb * gamma * irS;
-      rbS = -Xb * X * irS;
-    }
-#pragma unroll
-    for (int l = 0; l < 6; l++)
-      if (l == P.lstar) { ulb[l] += ulbS; pb[l] += pbS; sb[l][0] += rbS; }
-  }
-  // ul = m / rho, p = gm (et - |m|^2 / (2 rho))
-#pragma unroll
-  for (int l = 0; l < 6; l++) {
-    const double ir = P.ir[l];
-    sb[l][1] += ulb[l] * ir;
-    sb[l][0] -= ulb[l] * P.ul[l] * ir;
-    const double K = s[l][1] * s[l][1] + s[l][2] * s[l][2] + s[l][3] * s[l][3];
-    sb[l][4] += gm * pb[l];
-    const double Kb = -gm * pb[l] * 0.5 * ir;
-    sb[l][1] += 2.0 * s[l][1] * Kb;
-    sb[l][2] += 2.0 * s[l][2] * Kb;
-    sb[l][3] += 2.0 * s[l][3] * Kb;
-    sb[l][0] += gm * pb[l] * K * 0.5 * ir * ir;
-  }
-}
-
-__device__ inline long cell_idx(const Grid &g, long i, long j, long k) {
-  return i + (long)g.nx * (j + (long)g.ny * k);
-}
-
-// x times -1 when neg (the sign bit flipped: bitwise x * -1.0), else x
-__device__ inline double flip(double x, unsigned neg) {
-  return __longlong_as_double(__double_as_longlong(x) ^ ((long long)neg << 63));
-}
-
-// direction-local component a -> global field index
-__device__ inline int gcomp(int d, int a) {
-  if (a == 1) return 1 + d;
-  if (a == 1 + d) return 1;
-  return a;
-}
-
-
-
-}  // namespace
-
-// One face's stencil adjoint, handed to a sink with the ghost rule's signs applied, one
-// fluid component at a time in global order. For each component the sink's pre(q) is
-// called before (to start the loads its put needs) and put(q, x[6], pre) after. ulb3 and
-// alphab: the tracers' adjoints of the velocity of the cell right of the face and of the
-// Lax-Friedrichs speed. Face (i, j, k) along d lies between cells c-1 and c.
-template <class Sink>
-__device__ inline void face_vjp(const Grid &g, const Fields &w, const Fields &vc, const double *ub,
-                                double alphab, int d, int i, int j, int k, Sink &sink) {
-  const int n = extent(g, d);
-  const int c0 = d == 0 ? i : d == 1 ? j : k;
-  const double idelta = 1.0 / (d == 0 ? g.dx : d == 1 ? g.dy : g.dz);
-  // cells either side of the face; a missing one reads the other and counts as zero (the
-  // loads stay unconditional, which keeps the compiler's waits on them precise)
-  const bool hr = c0 < n, hl = c0 > 0;
-  const long cr = cell_idx(g, i - (d == 0 && !hr), j - (d == 1 && !hr), k - (d == 2 && !hr));
-  const long cl = hl ? cell_idx(g, i - (d == 0), j - (d == 1), k - (d == 2)) : cr;
-  const double mr = hr ? 1.0 : 0.0, ml = hl ? 1.0 : 0.0;
-  long cell[6];
-  unsigned na = 0, nn = 0;     // bit l: point l's ghost sign is -1 (all / normal)
-  double s[6][5];
-#pragma unroll
-  for (int l = 0; l < 6; l++) {
-    const GhostMap m = ghost_map(g, d, c0 - 3 + l);
-    int ii = i, jj = j, kk = k;
-    if (d == 0) ii = m.src; else if (d == 1) jj = m.src; else kk = m.src;
-    cell[l] = cell_idx(g, ii, jj, kk);
-    na |= (m.sgn_all < 0.0 ? 1u : 0u) << l;
-    nn |= (m.sgn_norm < 0.0 ? 1u : 0u) << l;
-#pragma unroll
-    for (int a = 0; a < 5; a++)
-      s[l][a] = flip(w.w[gcomp(d, a)][cell[l]], ((a == 1 ? nn : na) >> l) & 1u);
-  }
-  FacePrim P;
-  face_prim(s, g.gamma, P);
-  double ulb[6] = {0, 0, 0, 0, 0, 0};
-  if (ub != nullptr && hr) ulb[3] = ub[cr];
-  double Fb[5];
-#pragma unroll
-  for (int a = 0; a < 5; a++) {
-    const int q = gcomp(d, a);
-    Fb[a] = (mr * vc.w[q][cr] - ml * vc.w[q][cl]) * idelta;
-  }
-  double sb[6][5];
-  fluid_vjp(s, g.gamma, P, Fb, ulb, alphab, sb);
-#pragma unroll
-  for (int a = 0; a < 5; a++) {
-    const int q = gcomp(d, a);
-    const auto pre = sink.pre(q);
-    double x[6];
-#pragma unroll
-    for (int l = 0; l < 6; l++) x[l] = flip(sb[l][a], ((a == 1 ? nn : na) >> l) & 1u);
-    sink.put(q, x, pre);
-  }
-}
-
-__device__ inline void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The adjoint of a WENO5 reconstruction over f0..f4 (the f+ formula; the f- one is the same
 // function of the reversed values): x_i = y d(weno)/d f_i for the cotangent y. weno =
@@ -415,36 +66,31 @@ __device__ inline double weno5_adj(double f0, double f1, double f2, double f3, d
   return Q;
 }
 
-// ------------------------------------------------------------------------------------
-// Tracers. With u_l the normal velocities and alpha the Lax-Friedrichs speed of a face, a
-// tracer's flux reconstructs t_l (u_l +- alpha) / 2; its adjoint goes to the tracer, to the
-// velocities and to alpha. A lane walks one tracer of one column along D over the rows
-// [c0, c1), the lanes of a wave being consecutive (column, tracer) pairs: cell-major tracer
-// rows along y and z are read as they lie. The stencil and the open rows' adjoints slide
-// through registers (six faces per round, so that every index is a constant); a row is
-// written out with its last face. Segments do the faces that reach into them again instead
-// of exchanging rows, ghost rows are added to their source rows in the lane: no side
-// buffer and no fix-up pass. The velocity adjoint of each cell and the alpha adjoint of each
-// face are summed over a cell's tracers (in tracer order) once per round and handed to the
-// fluid sweep in ub [cell] and alb [face]; so are the velocities and alphas that the lanes
-// of a cell share, which one lane computes for all. 128^3 with ten tracers: 0.28 ms per
-// direction, about 210 FP64 instructions per face and tracer (0.15 ms to issue) at two to three
-// waves per SIMD.
-// ------------------------------------------------------------------------------------
-struct TrWalk {
-  const double *r, *m0, *m1, *m2, *e, *mn;   // fluid; mn: the momentum along the walk
-  const double *t, *v;
-  double *out, *ub, *alb;
+// The lines of cells along a direction D ("columns"), the rows of a line and its ghosts.
+struct Walk {
   long rs, bs_in, bs_out, ncol;  // row stride; column col starts at (col % nin) bs_in + (col / nin) bs_out
   long afs, acs;                 // alb strides of a face and of a column
   int nin, n, ncb, nseg, per, add;
-  double sa_lo, su_lo, sa_hi, su_hi;   // ghost signs: all fields, normal velocity
-  double idelta, gamma;
+  double sa_lo, su_lo, sa_hi, su_hi;   // ghost signs: all conserved fields, normal velocity
+  double idelta, gamma, igm;
+};
+
+struct TrWalk : Walk {
+  const double *r, *m0, *m1, *m2, *e, *mn;   // fluid; mn: the momentum along the walk
+  const double *t, *v;
+  double *out, *ub, *alb;
+};
+
+// Fluid fields in direction-local order: rho, m_normal, m_t1, m_t2, et.
+struct FlWalk : Walk {
+  const double *w[5], *v[5];
+  double *out[5];
+  const double *ub, *alb;        // of the tracers, or null
 };
 
 // Row of extended index e: wrapped, mirrored or shifted (ghost_map); rows further out than
 // the ghosts, which no face reads, are clamped.
-__device__ inline int walk_row(const TrWalk &k, int e, double &sa, double &su) {
+__device__ inline int walk_row(const Walk &k, int e, double &sa, double &su) {
   sa = su = 1.0;
   const int n = k.n;
   if (e >= 0 && e < n) return e;
@@ -457,12 +103,42 @@ __device__ inline int walk_row(const TrWalk &k, int e, double &sa, double &su) {
   return min(e - 3, n - 1);
 }
 
+__device__ inline long walk_cell(const Walk &k, long col) {
+  const unsigned q = (unsigned)col / (unsigned)k.nin;
+  return (long)((unsigned)col - q * (unsigned)k.nin) * k.bs_in + (long)q * k.bs_out;
+}
+
+__device__ inline void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ------------------------------------------------------------------------------------
+// Tracers. With u_l the normal velocities and alpha the Lax-Friedrichs speed of a face, a
+// tracer's flux reconstructs t_l (u_l +- alpha) / 2; its adjoint goes to the tracer, to the
+// velocities and to alpha. A lane walks one tracer of one column along D over the rows
+// [c0, c1), the lanes of a wave being consecutive (column, tracer) pairs: cell-major tracer
+// rows along y and z are read as they lie. The stencil and the open rows' adjoints slide
+// through registers (six faces per round, so that every index is a constant); a row is
+// written out with its last face. Segments do the faces that reach into them again instead
+// of exchanging rows, ghost rows are added to their source rows in the lane: no side
+// buffer and no fix-up pass. The velocity adjoint of each cell and the alpha adjoint of each
+// face are summed over a cell's tracers (in tracer order) once per round and handed to the
+// fluid sweep in ub [cell] and alb [face]; so are the velocities and alphas that the lanes
+// of a cell share, which one lane computes for all. About 280 instructions per
+// face and tracer, 216 of them FP64 (0.2 ms to issue at 128^3 with ten tracers; 0.28 ms taken at
+// three waves per SIMD, 0.31 at two; the row offsets come from LDS, computed in the scalar unit
+// they spilled).
+// ------------------------------------------------------------------------------------
 template <int NC>
-__global__ void __launch_bounds__(64, 2)
+__global__ void __launch_bounds__(64, 3)
 fe_vjp_tracers(TrWalk k) {
   constexpr int GPW = 64 / NC;                 // columns per wave
+  constexpr int STEP = 64 / GPW;               // lanes lane / GPW + STEP * pass take the rows
   __shared__ double ring_u[12][GPW], ring_a[12][GPW], alpha[6][GPW];
-  __shared__ double red[6][2][GPW * NC + 4], held[3][2][64];
+  __shared__ double red[6][2][GPW * NC + 4], rsign[24];
+  __shared__ long roff[24];
   const int lane = threadIdx.x, n = k.n;
   const int blk = blockIdx.x % k.ncb, seg = blockIdx.x / k.ncb;
   const int c0 = (int)((long)seg * n / k.nseg), c1 = (int)((long)(seg + 1) * n / k.nseg);
@@ -471,20 +147,27 @@ fe_vjp_tracers(TrWalk k) {
   const int grp = min(lane / NC, GPW - 1), c = lane % NC;
   const long col0 = (long)blk * GPW;
   const bool act = lane < GPW * NC && col0 + grp < k.ncol;
-  const auto cell_of = [&](long col) {
-    const unsigned q = (unsigned)col / (unsigned)k.nin;
-    return (long)((unsigned)col - q * (unsigned)k.nin) * k.bs_in + (long)q * k.bs_out;
-  };
-  const long base = cell_of(min(col0 + grp, k.ncol - 1));
-  const double *tp = k.t + base * NC + c, *vp = k.v + base * NC + c;
-  double *op = k.out + base * NC + c;
-  // velocities and wave speeds of rows ra .. ra+cnt-1 into ring slots rho, rho+1, ...
-  const auto fill = [&](int ra, int rho, int cnt) {
-    for (int i = lane; i < cnt * GPW; i += 64) {
-      const int rr = i / GPW, gg = i - rr * GPW;
+  const long base = walk_cell(k, min(col0 + grp, k.ncol - 1)) * NC + c;
+  const double *tp = k.t + base, *vp = k.v + base;
+  double *op = k.out + base;
+  // what the lanes of a cell share: one lane per (row, column) of a round
+  const int gg = lane % GPW, gr = lane / GPW;
+  const bool gact = col0 + gg < k.ncol;
+  const long gbase = walk_cell(k, min(col0 + gg, k.ncol - 1));
+  // offsets and signs of rows ra, ra+1, ... (cnt <= 64) into slots rho, rho+1, ... of 24
+  const auto fill_rows = [&](int ra, int rho, int cnt) {
+    if (lane < cnt) {
       double sa, su;
-      const long cc = cell_of(min(col0 + gg, k.ncol - 1)) +
-                      walk_row(k, min(ra + rr, fend + 2), sa, su) * k.rs;
+      const int sl = (rho + lane) % 24;
+      roff[sl] = (long)walk_row(k, min(ra + lane, fend + 2), sa, su) * k.rs * NC;
+      rsign[sl] = sa;
+    }
+  };
+  // velocities and wave speeds of rows ra, ra+1, ... into ring slots rho, rho+1, ... of 12
+  const auto fill = [&](int ra, int rho, int cnt) {
+    for (int rr = gr; rr < cnt; rr += STEP) {
+      double sa, su;
+      const long cc = gbase + walk_row(k, min(ra + rr, fend + 2), sa, su) * k.rs;
       const double m0 = k.m0[cc], m1 = k.m1[cc], m2 = k.m2[cc];
       const double ir = fast_rcp(k.r[cc]);
       const double p = (k.gamma - 1.0) * (k.e[cc] - 0.5 * (m0 * m0 + m1 * m1 + m2 * m2) * ir);
@@ -494,10 +177,7 @@ fe_vjp_tracers(TrWalk k) {
       ring_a[sl][gg] = fabs(u) + fast_sqrt(k.gamma * p * ir);
     }
   };
-  const auto row_ptr = [&](int e, double &sa) {
-    double su;
-    return (long)walk_row(k, min(e, fend + 2), sa, su) * k.rs * NC;
-  };
+  fill_rows(fa - 3, 0, 17);
   fill(fa - 3, 0, 11);
   wave_sync_lds();
   // window slot (j + l) % 6 holds point l of the round's face j: tracer, half velocity and
@@ -507,43 +187,43 @@ fe_vjp_tracers(TrWalk k) {
   for (int l = 0; l < 6; l++) at[l] = au[l] = tw[l] = hu[l] = 0.0;
 #pragma unroll
   for (int l = 0; l < 5; l++) {
-    double sa;
-    const long o = row_ptr(fa - 3 + l, sa);
-    tw[l] = sa * tp[o];
+    tw[l] = rsign[l] * tp[roff[l]];
     hu[l] = ring_u[l][grp];
   }
-  const auto load_face = [&](int f, double &t, double &v, double &o) {
-    double sa;
-    t = tp[row_ptr(f + 2, sa)] * sa;
-    v = vp[row_ptr(f, sa)];
-    o = k.add ? op[row_ptr(f - 3 >= c0 && f - 3 < c1 ? f - 3 : c0, sa)] : 0.0;
+  // face f's new tracer row f+2, cotangent row f and open row f-3; rt: slot of row f-3
+  const auto load_face = [&](int f, int rt, double &t, double &v, double &o) {
+    t = tp[roff[(rt + 5) % 24]];
+    v = vp[roff[(rt + 3) % 24]];
+    if (k.add) o = f - 3 >= c0 && f - 3 < c1 ? op[roff[rt % 24]] : 0.0;
   };
 #pragma unroll
-  for (int j = 0; j < 6; j++) load_face(fa + j, tn[j], vn[j], on[j]);
-  double vprev = 0.0;
-  if (fa > 0 || k.per) { double sa; vprev = vp[row_ptr(fa - 1, sa)]; }
-  int par = 0;                                  // this round's ring offset: 0 or 6
+  for (int j = 0; j < 6; j++) on[j] = 0.0;
+#pragma unroll
+  for (int j = 0; j < 6; j++) load_face(fa + j, j, tn[j], vn[j], on[j]);
+  double vprev = fa > 0 || k.per ? vp[roff[2]] : 0.0;
+  int par = 0, rt = 0;              // this round's slots of row f0-3: 0 or 6 of 12; of 24
+#pragma unroll 1
   for (int f0 = fa; f0 <= fend; f0 += 6) {
-    for (int i = lane; i < 6 * GPW; i += 64) {
-      const int j = i / GPW, gg = i - j * GPW;
+    for (int jj = gr; jj < 6; jj += STEP) {
       double a = 0.0;
 #pragma unroll
-      for (int l = 0; l < 6; l++) a = fmax(a, ring_a[(par + j + l) % 12][gg]);
-      alpha[j][gg] = a;
+      for (int l = 0; l < 6; l++) a = fmax(a, ring_a[(par + jj + l) % 12][gg]);
+      alpha[jj][gg] = a;
     }
+    fill_rows(f0 + 14, rt + 17, 6);
     wave_sync_lds();
 #pragma unroll
     for (int j = 0; j < 6; j++) {
       const int f = f0 + j;
       double alphab = 0.0, vu = 0.0;
-      tw[(j + 5) % 6] = tn[j];
+      tw[(j + 5) % 6] = tn[j] * rsign[(rt + j + 5) % 24];
       hu[(j + 5) % 6] = ring_u[(par + j + 5) % 12][grp];
       at[(j + 5) % 6] = au[(j + 5) % 6] = 0.0;
       const double vcur = (f < n || k.per) ? vn[j] : 0.0;
       const double old = on[j];
       const double y = (vcur - vprev) * k.idelta;
       vprev = vcur;
-      load_face(f + 6, tn[j], vn[j], on[j]);
+      load_face(f + 6, rt + j + 6, tn[j], vn[j], on[j]);
       if (f <= fb) {
         const double ha = 0.5 * alpha[j][grp];
         double xp[5], xm[5], hp[5], hm[5];
@@ -580,395 +260,533 @@ fe_vjp_tracers(TrWalk k) {
           alphab = fma(t, xd, alphab);
         }
       }
-      // row f-3 is complete; ghosts go to their source rows
+      // row f-3 is complete; ghost rows are added to their source rows: -1-e (faces 0..2,
+      // which only a column's first round has) and e-3
       const int e = f - 3;
-      double vt = at[j];
-      vu = au[j];
       if (!k.per) {
-        if (e < 0) {
-          held[e + 3][0][lane] = k.sa_lo * vt;
-          held[e + 3][1][lane] = k.su_lo * vu;
-        } else if (e < 3) {
-          vt += held[2 - e][0][lane];
-          vu += held[2 - e][1][lane];
+        if (j < 3 && f == j) {
+          at[(j + 5 - 2 * j) % 6] = fma(k.sa_lo, at[j], at[(j + 5 - 2 * j) % 6]);
+          au[(j + 5 - 2 * j) % 6] = fma(k.su_lo, au[j], au[(j + 5 - 2 * j) % 6]);
         }
-        if (e >= n - 3) {
-          vt = fma(k.sa_hi, at[(j + 3) % 6], vt);
-          vu = fma(k.su_hi, au[(j + 3) % 6], vu);
+        if (f >= n) {
+          at[j] = fma(k.sa_hi, at[(j + 3) % 6], at[j]);
+          au[j] = fma(k.su_hi, au[(j + 3) % 6], au[j]);
         }
       }
-      if (e >= c0 && e < c1 && act) op[(long)e * k.rs * NC] = k.add ? old + vt : vt;
+      if (e >= c0 && e < c1 && act) op[roff[(rt + j) % 24]] = k.add ? old + at[j] : at[j];
       if (lane < GPW * NC) {
-        red[j][0][lane] = vu;
+        red[j][0][lane] = au[j];
         red[j][1][lane] = alphab;
       }
     }
     wave_sync_lds();
     // sums over the tracers; each face's alpha adjoint is written by the segment it opens
     // (face n by the last one, as zero if it is face 0 again)
-    for (int i = lane; i < 12 * GPW; i += 64) {
-      const int j = i / (2 * GPW), q = (i / GPW) & 1, gg = i - (i / GPW) * GPW;
-      double a = red[j][q][gg * NC];
+    for (int jq = gr; jq < 12; jq += STEP) {
+      const int f = f0 + (jq >> 1), e = f - 3, q = jq & 1;
+      const double *r = &red[jq >> 1][q][gg * NC];
+      double a = r[0];
 #pragma unroll
-      for (int cc = 1; cc < NC; cc++) a += red[j][q][gg * NC + cc];
+      for (int cc = 1; cc < NC; cc++) a += r[cc];
       a *= 0.5;
-      const long col = col0 + gg;
-      if (col < k.ncol) {
-        const int f = f0 + j, e = f - 3;
+      if (gact) {
         if (q == 0) {
-          if (e >= c0 && e < c1) k.ub[cell_of(col) + e * k.rs] = a;
+          if (e >= c0 && e < c1) k.ub[gbase + e * k.rs] = a;
         } else if (f >= c0 && (f < c1 || (f == n && c1 == n))) {
-          k.alb[f * k.afs + col * k.acs] = k.per && f == n ? 0.0 : a;
+          k.alb[f * k.afs + (col0 + gg) * k.acs] = k.per && f == n ? 0.0 : a;
         }
       }
     }
     fill(f0 + 8, par + 11, 6);
     par = 6 - par;
+    rt = rt == 18 ? 0 : rt + 6;
     wave_sync_lds();
   }
 }
 
-constexpr int NV = 5;      // fluid components
+// ------------------------------------------------------------------------------------
+// Fluid. The adjoint of face_flux_lds: with G = W / (4 cs) for the acoustic reconstructions
+// W (K -+ A), S = G4 + G0, T = G4 - G0 and half the shear and entropy ones g1, g2, g3,
+//   F0 = S + g3, F1 = u F0 + cs T, F2 = v F0 + g1, F3 = w F0 + g2,
+//   F4 = cs S / (gamma-1) + (u^2 + v^2 + w^2)/2 F0 + u cs T + v g1 + w g2.
+// The cotangents of the reconstructions need only the Roe state, so one pass forms each
+// reconstruction and its adjoint, one split side at a time. W depends on cs through its eps,
+// which is the derivative of a homogeneous function: d(G)/d(1/(4 cs)) = sum f dW/df.
+// Adjoints are those of the points' (rho, u_n, u_t1, u_t2, p); a cell's go back to the
+// conserved fields once all of its faces are in (fluid_store). Bound by issue at two waves per
+// SIMD: 0.15 ms of instructions in 0.23 - 0.24 ms per direction at 128^3 (the reference's
+// formula order with the tracers taken out: 0.46 ms at one wave per SIMD).
+// ------------------------------------------------------------------------------------
+enum { Q_R = 0, Q_U, Q_V, Q_W, Q_P, Q_A };     // Q_A: |u_n| + c
 
-__device__ inline void out_put(const FieldsOut &o, int q, long cell, double v, bool add) {
-  double *p = &o.w[q][cell];
-  *p = add ? *p + v : v;
+// Waits for a before b is used: keeps the compiler from starting on the next reconstruction
+// (and from reading its points) while the registers of the current one are taken.
+__device__ inline void then_on(const double (&a)[5], double (&b)[5]) {
+  __asm__ volatile("" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4])
+                   : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]));
+}
+__device__ inline int then_at(const double (&a)[5], int o) {
+  __asm__ volatile("" : "+v"(o) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]));
+  return o;
 }
 
-// Ghost-point contributions of an x-line: the (face, point) pairs whose extended index
-// lies outside the line, 6 on each end. Index of pair (f, l), or -1 for an interior point.
-__device__ inline int xghost_pair(int n, int f, int l) {
-  const int e = f - 3 + l;
-  if (e < 0) return f == 0 ? l : f == 1 ? 3 + l : 5;
-  if (e >= n) {
-    const int b = n - f;
-    return b == 0 ? 3 + l : b == 1 ? 5 + l : 11;   // l in 3..5 / 4..5 / 5
+// Forms the sums here and not where they are used next (the compiler moves them into a later
+// block and keeps both terms in registers until then).
+__device__ inline void hold(double (&acc)[6][5]) {
+#pragma unroll
+  for (int l = 0; l < 6; l++)
+    __asm__ volatile("" : "+v"(acc[l][0]), "+v"(acc[l][1]), "+v"(acc[l][2]), "+v"(acc[l][3]), "+v"(acc[l][4]));
+}
+
+// Stencil point l, field q at P[off[l] + q * FS]. lstar: the first point with the largest
+// |u_n| + c. acc[l] += the adjoint of point l. About 1250 FP64 instructions; the points are read
+// again from LDS wherever they are used, which is what makes it fit into 256 registers.
+template <int FS>
+__device__ inline void face_adjoint(const double *P, const int (&off)[6], double gamma, double igm,
+                                    double alpha, int lstar, const double (&Fb)[5], double alphab,
+                                    double (&acc)[6][5]) {
+  const double gm = gamma - 1.0, gmh = 0.5 * gm;
+  double u, v, w, cs, wl, wr;
+  {
+    const double *L = P + off[2], *R = P + off[3];
+    const double rL = L[Q_R * FS], rR = R[Q_R * FS], sL = fast_sqrt(rL), sR = fast_sqrt(rR);
+    const double iden = fast_rcp(sL + sR);
+    wl = sL * iden;
+    wr = sR * iden;
+    const double uL = L[Q_U * FS], vL = L[Q_V * FS], zL = L[Q_W * FS];
+    const double uR = R[Q_U * FS], vR = R[Q_V * FS], zR = R[Q_W * FS];
+    u = fma(uL, wl, uR * wr);
+    v = fma(vL, wl, vR * wr);
+    w = fma(zL, wl, zR * wr);
+    const double du = uR - uL, dv = vR - vL, dw = zR - zL;
+    const double cL = gamma * L[Q_P * FS] * fast_rcp(rL), cR = gamma * R[Q_P * FS] * fast_rcp(rR);
+    cs = fma(cL, wl, cR * wr) + gmh * (wl * wr) * fma(du, du, fma(dv, dv, dw * dw));
   }
-  return -1;
-}
-
-// ------------------------------------------------------------------------------------
-// x sweep: one wave walks a run of whole x-lines 64 faces at a time (faces consecutive in
-// memory, lines back to back); the contributions go to a 128-slot ring indexed by the
-// flattened position line * (nx+1) + e of their target. Lanes share slots, so the six
-// stencil points are added in six ordered passes. A slot is final once the faces up to
-// three beyond it are in; it is then written out and cleared. Ghost points go to the side
-// buffer per (line, pair) and are added by fe_vjp_fix_x.
-// ------------------------------------------------------------------------------------
-// The six points go in as six no-return LDS adds, one point per instruction: within one
-// instruction the lanes hit distinct slots, and a wave's LDS operations complete in
-// order, so the sum order (point 0 first) is fixed.
-struct XSink {
-  double *ring;            // [NV][128]
-  double *side;            // [(pair * NV + q) * nlines + line]
-  long q;                  // flattened face
-  int f, n, line, nlines;
-  __device__ int pre(int) const { return 0; }
-  __device__ void put(int comp, const double (&x)[6], int) {
+  const double ci = fast_rcp(cs), hci = 0.25 * ci;
+  const double tb = fma(u, Fb[4], Fb[1]), y1 = 0.5 * fma(v, Fb[4], Fb[2]);
+  const double y2 = 0.5 * fma(w, Fb[4], Fb[3]);
+  double y0, y4, y3;
+  {
+    const double hq = 0.5 * fma(u, u, fma(v, v, w * w));
+    const double B0 = fma(hq, Fb[4], fma(u, Fb[1], fma(v, Fb[2], fma(w, Fb[3], Fb[0]))));
+    const double Sb = fma(igm * cs, Fb[4], B0), Tb = cs * tb;
+    y0 = hci * (Sb - Tb);
+    y4 = hci * (Sb + Tb);
+    y3 = 0.5 * B0;
+  }
+  const double eps04 = (16.0 * WENO_EPSB) * (cs * cs), eps13 = 4.0 * WENO_EPSB;
+  double W0 = 0.0, W1 = 0.0, W2 = 0.0, W3 = 0.0, W4 = 0.0;
+  double sfx = 0.0, skx = 0.0, ub = 0.0, vb = 0.0, wb = 0.0;
+  double X[5] = {y0, y1, y2, y3, y4};
+#pragma unroll
+  for (int sd = 0; sd < 2; sd++) {
+    const double al = sd == 0 ? alpha : -alpha;
+    const double tt = fma(-gm, u, al);
+    const auto pt = [&](int l, int o) { return P + off[sd == 0 ? l : 5 - l] + o; };
+    double x[5], K[5], D[5], Kb[5], Ab[5], f[5];
+    int o = then_at(X, 0);
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      const double *q = pt(l, o);
+      const double un = q[Q_U * FS], p = q[Q_P * FS], du = un - u;
+      const double dv = q[Q_V * FS] - v, dw = q[Q_W * FS] - w;
+      x[l] = q[Q_R * FS] * (un + al);
+      D[l] = gmh * fma(du, du, fma(dv, dv, dw * dw));
+      K[l] = fma(p, fma(gamma, un, tt), x[l] * D[l]);
+      f[l] = K[l] - fma(x[l], du, p);
+    }
+    {
+      const double Q0 = weno5_adj(f[0], f[1], f[2], f[3], f[4], eps04, y0, Ab);
+      W0 += fma(2.0 / 3.0, Q0, f[2]);
+#pragma unroll
+      for (int l = 0; l < 5; l++) sfx = fma(f[l], Ab[l], sfx);
+      __asm__ volatile("" : "+v"(sfx), "+v"(W0));
+    }
+    o = then_at(Ab, 0);
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      const double *q = pt(l, o);
+      f[l] = K[l] + fma(x[l], q[Q_U * FS] - u, q[Q_P * FS]);
+    }
+    {
+      double x4[5];
+      const double Q4 = weno5_adj(f[0], f[1], f[2], f[3], f[4], eps04, y4, x4);
+      W4 += fma(2.0 / 3.0, Q4, f[2]);
+#pragma unroll
+      for (int l = 0; l < 5; l++) {
+        sfx = fma(f[l], x4[l], sfx);
+        Kb[l] = Ab[l] + x4[l];
+        Ab[l] = x4[l] - Ab[l];
+      }
+      __asm__ volatile("" : "+v"(sfx), "+v"(W4));
+    }
+#pragma unroll
+    for (int l = 0; l < 5; l++) f[l] = fma(-ci, K[l], x[l]);
+    then_on(Ab, f);
+    {
+      const double Q3 = weno5_adj(f[0], f[1], f[2], f[3], f[4], eps13, y3, X);
+      W3 += fma(2.0 / 3.0, Q3, f[2]);
+      __asm__ volatile("" : "+v"(W3));
+    }
+    o = then_at(X, 0);
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      const int a = sd == 0 ? l : 5 - l;
+      const double *q = pt(l, o);
+      const double un = q[Q_U * FS], p = q[Q_P * FS], du = un - u;
+      skx = fma(K[l], X[l], skx);
+      Kb[l] = fma(-ci, X[l], Kb[l]);
+      X[l] = fma(Kb[l], D[l], fma(Ab[l], du, X[l]));
+      acc[a][4] += fma(Kb[l], fma(gamma, un, tt), Ab[l]);
+      const double pk = p * Kb[l];
+      K[l] = gm * (Kb[l] * x[l]);                 // the adjoint of D, times gamma - 1
+      const double dub = fma(Ab[l], x[l], du * K[l]);
+      acc[a][1] += fma(gamma, pk, dub);
+      ub -= fma(gm, pk, dub);
+      alphab += sd == 0 ? pk : -pk;
+    }
+    hold(acc);
+    then_on(X, K);
+    // the shear components
+#pragma unroll
+    for (int c = 2; c < 4; c++) {
+      double xs[5], d[5];
+      o = then_at(X, 0);
+#pragma unroll
+      for (int l = 0; l < 5; l++) {
+        d[l] = pt(l, o)[c * FS] - (c == 2 ? v : w);
+        f[l] = x[l] * d[l];
+      }
+      const double Q = weno5_adj(f[0], f[1], f[2], f[3], f[4], eps13, c == 2 ? y1 : y2, xs);
+      (c == 2 ? W1 : W2) += fma(2.0 / 3.0, Q, f[2]);
+#pragma unroll
+      for (int l = 0; l < 5; l++) {
+        const double b = fma(xs[l], x[l], d[l] * K[l]);
+        X[l] = fma(xs[l], d[l], X[l]);
+        acc[sd == 0 ? l : 5 - l][c] += b;
+        (c == 2 ? vb : wb) -= b;
+      }
+      hold(acc);
+    }
+    o = then_at(X, 0);
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      const int a = sd == 0 ? l : 5 - l;
+      const double *q = pt(l, o);
+      const double xr = X[l] * q[Q_R * FS];
+      acc[a][0] = fma(X[l], q[Q_U * FS] + al, acc[a][0]);
+      acc[a][1] += xr;
+      alphab += sd == 0 ? xr : -xr;
+    }
+    hold(acc);
+    __asm__ volatile("" : "+v"(skx), "+v"(W1), "+v"(W2));
+    X[0] = alphab; X[1] = ub; X[2] = vb; X[3] = wb; X[4] = sfx;
+  }
+  // the Roe state: from the back-projection, then to the two points
+  double csb;
+  {
+    const double S = hci * (W4 + W0), T = hci * (W4 - W0), F0 = fma(0.5, W3, S);
+    csb = fma(ci, fma(ci, skx, -sfx), fma(igm * Fb[4], S, T * tb));
+    ub += fma(Fb[1], F0, Fb[4] * fma(u, F0, cs * T));
+    vb += fma(Fb[2], F0, Fb[4] * fma(v, F0, 0.5 * W1));
+    wb += fma(Fb[3], F0, Fb[4] * fma(w, F0, 0.5 * W2));
+  }
+  {
+    const int o = then_at(X, 0);
+    const double *L = P + off[2] + o, *R = P + off[3] + o;
+    const double rL = L[Q_R * FS], irL = fast_rcp(rL), cL = gamma * L[Q_P * FS] * irL;
+    const double rR = R[Q_R * FS], irR = fast_rcp(rR), cR = gamma * R[Q_P * FS] * irR;
+    const double du = R[Q_U * FS] - L[Q_U * FS], dv = R[Q_V * FS] - L[Q_V * FS];
+    const double dw = R[Q_W * FS] - L[Q_W * FS];
+    const double Qb = gmh * csb, Qv = fma(du, du, fma(dv, dv, dw * dw)), ww = wl * wr;
+    // the adjoint of w_L minus that of w_R
+    const double wd = fma(Qb * Qv, wr - wl, csb * (cL - cR)) - fma(ub, du, fma(vb, dv, wb * dw));
+    const double q2 = 2.0 * Qb * ww;
+    acc[2][1] += fma(ub, wl, -q2 * du);
+    acc[3][1] += fma(ub, wr, q2 * du);
+    acc[2][2] += fma(vb, wl, -q2 * dv);
+    acc[3][2] += fma(vb, wr, q2 * dv);
+    acc[2][3] += fma(wb, wl, -q2 * dw);
+    acc[3][3] += fma(wb, wr, q2 * dw);
+    // dw_L = w_L w_R / 2 (drho_L / rho_L - drho_R / rho_R); c^2 = gamma p / rho
+    const double h = 0.5 * wd * ww, cl = csb * wl * irL, cr = csb * wr * irR;
+    acc[2][0] += fma(-cl, cL, rL > 0.0 ? h * irL : 0.0);
+    acc[3][0] -= fma(cr, cR, rR > 0.0 ? h * irR : 0.0);
+    acc[2][4] = fma(gamma, cl, acc[2][4]);
+    acc[3][4] = fma(gamma, cr, acc[3][4]);
+  }
+  hold(acc);
+  // Lax-Friedrichs speed: alpha = |u_l*| + c_l*
+  {
+    int o = off[0];
+#pragma unroll
+    for (int l = 1; l < 6; l++) o = l == lstar ? off[l] : o;
+    const double uS = P[o + Q_U * FS], pS = P[o + Q_P * FS], ir = fast_rcp(P[o + Q_R * FS]);
+    const double c2 = gamma * pS * ir;
+    const double cc = c2 > 0.0 ? 0.5 * ir * fast_rcp(fast_sqrt(c2)) : 0.0;
+    const double kp = gamma * cc, kr = -c2 * cc, ku = uS < 0.0 ? -1.0 : 1.0;
 #pragma unroll
     for (int l = 0; l < 6; l++) {
-      const int pr = xghost_pair(n, f, l);
-      if (pr < 0) atomicAdd(&ring[comp * 128 + (int)((q - 3 + l) & 127)], x[l]);
-      else side[((long)pr * NV + comp) * nlines + line] = x[l];
-      wave_sync_lds();
+      const double ab = l == lstar ? alphab : 0.0;
+      acc[l][0] = fma(kr, ab, acc[l][0]);
+      acc[l][1] = fma(ku, ab, acc[l][1]);
+      acc[l][4] = fma(kp, ab, acc[l][4]);
     }
   }
-};
+}
 
-__global__ void __launch_bounds__(64)
-fe_vjp_sweep_x(Grid g, Fields w, Fields vc, const double *ub, const double *alb, FieldsOut out,
-               double *side, int lps, int add) {
-    __shared__ double ring[NV * 128];
-  const int lane = threadIdx.x;
-  const int nx = g.nx, nxp = g.nx + 1;
-  const int nlines = g.ny * g.nz;
-  const int L0 = blockIdx.x * lps;
-  const int L1 = min(L0 + lps, nlines);
-  if (L0 >= nlines) return;
-  const long Q0 = (long)L0 * nxp, Q1 = (long)L1 * nxp;
-  for (int s = lane; s < NV * 128; s += 64) ring[s] = 0.0;
-  wave_sync_lds();
-  long done = Q0;          // first slot not yet written out
-  for (long B = Q0; B < Q1; B += 64) {
-    const long q = B + lane;
-    if (q < Q1) {
-      const int line = (int)(q / nxp), f = (int)(q - (long)line * nxp);
-      XSink sink{ring, side, q, f, nx, line, nlines};
-      face_vjp(g, w, vc, ub, alb ? alb[q] : 0.0, 0, f, line % g.ny, line / g.ny, sink);
+// A conserved state as a stencil point, with its ghost signs.
+template <int FS>
+__device__ inline void put_point(const Walk &k, const double (&x)[5], double sa, double su,
+                                 double *q) {
+  const double ir = fast_rcp(x[0]), u = x[1] * ir;
+  const double p = (k.gamma - 1.0) * (x[4] - 0.5 * (x[1] * x[1] + x[2] * x[2] + x[3] * x[3]) * ir);
+  q[Q_R * FS] = sa * x[0];
+  q[Q_U * FS] = su * u;
+  q[Q_V * FS] = x[2] * ir;
+  q[Q_W * FS] = x[3] * ir;
+  q[Q_P * FS] = sa * p;
+  q[Q_A * FS] = fabs(u) + fast_sqrt(k.gamma * p * ir);
+}
+
+// Adjoint of a cell's (rho, u, p) back to its conserved fields, into wbar (local order).
+__device__ inline void fluid_store(const FlWalk &k, long cell, const double (&b)[5], double r,
+                                   double u, double v, double w) {
+  double old[5];
+#pragma unroll
+  for (int a = 0; a < 5; a++) old[a] = k.add ? k.out[a][cell] : 0.0;
+  const double ir = fast_rcp(r), pb = (k.gamma - 1.0) * b[4];
+  double x[5];
+  x[0] = fma(0.5 * pb, fma(u, u, fma(v, v, w * w)), b[0]) -
+         fma(b[1], u, fma(b[2], v, b[3] * w)) * ir;
+  x[1] = fma(-pb, u, b[1] * ir);
+  x[2] = fma(-pb, v, b[2] * ir);
+  x[3] = fma(-pb, w, b[3] * ir);
+  x[4] = pb;
+#pragma unroll
+  for (int a = 0; a < 5; a++) k.out[a][cell] = k.add ? old[a] + x[a] : x[a];
+}
+
+// y and z: each lane walks its own column over the rows [c0, c1) of a segment, with the
+// stencil in an LDS ring of six rows and the open rows' adjoints in registers. Segments do
+// the five faces that reach into them from outside again, ghost rows are added to their
+// source rows in the lane. The loads for the next face are issued between the split sides and
+// the Roe state, where registers are free.
+__global__ void __launch_bounds__(64, 2)
+fe_vjp_walk(FlWalk k) {
+  constexpr int FS = 64, LS = 6 * 64;
+  __shared__ double P[6 * LS];
+  const int lane = threadIdx.x, n = k.n;
+  const int blk = blockIdx.x % k.ncb, seg = blockIdx.x / k.ncb;
+  const int c0 = (int)((long)seg * n / k.nseg), c1 = (int)((long)(seg + 1) * n / k.nseg);
+  const int fa = k.per ? c0 - 2 : max(c0 - 2, 0);
+  const int fend = c1 + 2, fb = k.per ? fend : min(fend, n);
+  const long col0 = (long)blk * 64 + lane;
+  const bool act = col0 < k.ncol;
+  const long col = act ? col0 : k.ncol - 1, base = walk_cell(k, col);
+  double nw[5], nv[5], vl[5], nal = 0.0, acc[6][5];
+  const auto load_row = [&](int e) {
+    double sa, su;
+    const long c = base + walk_row(k, min(e, fend + 2), sa, su) * k.rs;
+#pragma unroll
+    for (int a = 0; a < 5; a++) nw[a] = k.w[a][c];
+  };
+  const auto put_row = [&](int e, int slot) {
+    double sa, su;
+    (void)walk_row(k, min(e, fend + 2), sa, su);
+    put_point<FS>(k, nw, sa, su, P + slot * LS + lane);
+  };
+  // the cotangents of the cells either side of face f, and its alpha adjoint
+  const auto load_v = [&](int f) {
+    double sa, su;
+    f = min(f, fend + 2);
+    const int row = walk_row(k, f, sa, su);
+    const long cr = base + row * k.rs;
+    const long cl = base + walk_row(k, k.per ? f - 1 : max(f - 1, 0), sa, su) * k.rs;
+#pragma unroll
+    for (int a = 0; a < 5; a++) { nv[a] = k.v[a][cr]; vl[a] = k.v[a][cl]; }
+    if (k.alb) nal = k.alb[(k.per ? row : min(f, n)) * k.afs + col * k.acs];
+  };
+#pragma unroll
+  for (int l = 0; l < 6; l++)
+#pragma unroll
+    for (int a = 0; a < 5; a++) acc[l][a] = 0.0;
+#pragma unroll 1
+  for (int l = 0; l < 5; l++) {
+    load_row(fa - 3 + l);
+    put_row(fa - 3 + l, l);
+  }
+  load_v(fa);
+  load_row(fa + 2);
+  int s0 = 0;
+#pragma unroll 1
+  for (int f = fa; f <= fend; f++) {
+    const int e = f - 3;
+    const bool own = e >= c0 && e < c1;
+    put_row(f + 2, s0 >= 1 ? s0 - 1 : 5);
+    int off[6];
+#pragma unroll
+    for (int l = 0; l < 6; l++) off[l] = (s0 + l >= 6 ? s0 + l - 6 : s0 + l) * LS + lane;
+    if (f <= fb) {
+      double Fb[5], alpha = 0.0;
+      const double mr = f < n || k.per ? k.idelta : 0.0, ml = f > 0 || k.per ? k.idelta : 0.0;
+#pragma unroll
+      for (int a = 0; a < 5; a++)
+        Fb[a] = mr == ml ? (nv[a] - vl[a]) * k.idelta : mr != 0.0 ? nv[a] * mr : -(vl[a] * ml);
+      int lstar = -1;
+#pragma unroll
+      for (int l = 0; l < 6; l++) {
+        const double a = P[off[l] + Q_A * FS];
+        if (alpha < a) { alpha = a; lstar = l; }
+      }
+      face_adjoint<FS>(P, off, k.gamma, k.igm, alpha, lstar, Fb, nal, acc);
+    }
+    load_row(f + 3);
+    load_v(f + 1);
+    // row f-3 is complete; ghost rows: -1-e and e-3 are their source rows
+    if (!k.per) {
+      const auto fold = [&](int to, int from, double sa, double su) {
+        acc[to][0] = fma(sa, acc[from][0], acc[to][0]);
+        acc[to][1] = fma(su, acc[from][1], acc[to][1]);
+        acc[to][2] += acc[from][2];
+        acc[to][3] += acc[from][3];
+        acc[to][4] = fma(sa, acc[from][4], acc[to][4]);
+      };
+      if (f == 0) fold(5, 0, k.sa_lo, k.su_lo);
+      else if (f == 1) fold(3, 0, k.sa_lo, k.su_lo);
+      else if (f == 2) fold(1, 0, k.sa_lo, k.su_lo);
+      if (f >= n) fold(0, 3, k.sa_hi, k.su_hi);
+    }
+    if (own && act) {
+      const long cell = base + e * k.rs;
+      const double *q = P + off[0];
+      if (k.ub) acc[0][1] += k.ub[cell];
+      fluid_store(k, cell, acc[0], q[Q_R * FS], q[Q_U * FS], q[Q_V * FS], q[Q_W * FS]);
+    }
+#pragma unroll
+    for (int l = 0; l < 5; l++)
+#pragma unroll
+      for (int a = 0; a < 5; a++) acc[l][a] = acc[l + 1][a];
+#pragma unroll
+    for (int a = 0; a < 5; a++) acc[5][a] = 0.0;
+    s0 = s0 == 5 ? 0 : s0 + 1;
+  }
+}
+
+// x: a wave walks whole lines 64 faces at a time, the lanes along x; lines follow one
+// another, each with its ghost points (and, if periodic, with the faces around its ends done
+// again) at consecutive positions, whose points and adjoints live in a ring of RING positions.
+// The six points of a face are added with six LDS adds per component: within one
+// instruction the lanes hit distinct positions and a wave's LDS operations complete in order,
+// so the order of the sums is fixed. A position is final once the faces up to three beyond it
+// are in. RING holds the positions of 64 faces and the six below them: 64 + 5 per line begun
+// + 6, 128 for lines of eight faces or more.
+template <int RING>
+__global__ void __launch_bounds__(64, 2)
+fe_vjp_lines(FlWalk k, int lps) {
+  constexpr int FS = RING;
+  __shared__ double P[6 * RING], A[5 * RING];
+  const int lane = threadIdx.x, n = k.n;
+  const int fa = k.per ? -2 : 0, nf = k.per ? n + 5 : n + 1, np = nf + 5;
+  // faces and positions are counted from the wave's first line
+  const long line0 = (long)blockIdx.x * lps;
+  const int nl = (int)min((long)lps, k.ncol - line0);
+  const double inf = 1.0 / nf, inp = 1.0 / np;
+  const auto div = [](int a, double inv) { return (int)(((double)a + 0.5) * inv); };   // exact below 2^31
+  const int Q1 = nl * nf;
+  int loaded = 0, done = 0;                        // next position to load, to write out
+#pragma unroll 1
+  for (int B = 0; B < Q1; B += 64) {
+    const int qe = min(B + 64, Q1) - 1;            // last face of this pass
+    const int le = div(qe, inf), last = qe + le * (np - nf) + 5;
+    for (int p = loaded + lane; p <= last; p += 64) {
+      const int line = div(p, inp), e = p - line * np + fa - 3;
+      const int slot = p & (RING - 1);
+      double sa, su;
+      const long c = (line0 + line) * n + walk_row(k, e, sa, su);
+      double x[5];
+#pragma unroll
+      for (int a = 0; a < 5; a++) x[a] = k.w[a][c];
+      put_point<FS>(k, x, sa, su, P + slot);
+#pragma unroll
+      for (int a = 0; a < 5; a++) A[a * RING + slot] = 0.0;
+    }
+    loaded = last + 1;
+    wave_sync_lds();
+    const int q = min(B + lane, qe);
+    const bool mine = B + lane <= qe;
+    const int line = div(q, inf), f = q - line * nf + fa;
+    int off[6];
+#pragma unroll
+    for (int l = 0; l < 6; l++) off[l] = (q + line * (np - nf) + l) & (RING - 1);
+    double acc[6][5];
+    {
+      double Fb[5], alphab = 0.0, alpha = 0.0;
+      double sa, su;
+      const bool hr = k.per || f < n, hl = k.per || f > 0;
+      const long cr = (line0 + line) * n + walk_row(k, hr ? f : n - 1, sa, su);
+      const long cl = (line0 + line) * n + walk_row(k, hl ? f - 1 : 0, sa, su);
+#pragma unroll
+      for (int a = 0; a < 5; a++) {
+        const double vr = k.v[a][cr], vl = k.v[a][cl];
+        Fb[a] = ((hr ? vr : 0.0) - (hl ? vl : 0.0)) * k.idelta;
+      }
+      if (k.alb) alphab = k.alb[(k.per ? walk_row(k, f, sa, su) : f) + (line0 + line) * (n + 1)];
+      int lstar = -1;
+#pragma unroll
+      for (int l = 0; l < 6; l++) {
+        const double a = P[Q_A * FS + off[l]];
+        if (alpha < a) { alpha = a; lstar = l; }
+#pragma unroll
+        for (int b = 0; b < 5; b++) acc[l][b] = 0.0;
+      }
+      face_adjoint<FS>(P, off, k.gamma, k.igm, alpha, lstar, Fb, alphab, acc);
+    }
+    if (mine) {
+#pragma unroll
+      for (int l = 0; l < 6; l++) {
+#pragma unroll
+        for (int a = 0; a < 5; a++) atomicAdd(&A[a * RING + off[l]], acc[l][a]);
+        wave_sync_lds();
+      }
     }
     wave_sync_lds();
-    const long hi = (B + 64 >= Q1) ? Q1 - 1 : B + 60;
-    for (long P = done + lane; P <= hi; P += 64) {
-      const int line = (int)(P / nxp), e = (int)(P - (long)line * nxp);
-      const int slot = (int)(P & 127);
-      if (e < nx) {
-        const long cell = e + (long)nx * line;
-#pragma unroll 1
-        for (int qq = 0; qq < NV; qq++) out_put(out, qq, cell, ring[qq * 128 + slot], add);
-      }
-#pragma unroll 1
-      for (int qq = 0; qq < NV; qq++) ring[qq * 128 + slot] = 0.0;
+    // positions below the next face's stencil are final
+    const int hi = qe + 1 + div(qe + 1, inf) * (np - nf);
+    for (int p = done + lane; p < hi; p += 64) {
+      const int ln = div(p, inp), e = p - ln * np + fa - 3;
+      if (e < 0 || e >= n) continue;
+      const int slot = p & (RING - 1);
+      const long cell = (line0 + ln) * n + e;
+      double b[5];
+#pragma unroll
+      for (int a = 0; a < 5; a++) b[a] = A[a * RING + slot];
+      const auto ghost = [&](int pg, double sa, double su) {
+        const int sl = pg & (RING - 1);
+        b[0] = fma(sa, A[sl], b[0]);
+        b[1] = fma(su, A[RING + sl], b[1]);
+        b[2] += A[2 * RING + sl];
+        b[3] += A[3 * RING + sl];
+        b[4] = fma(sa, A[4 * RING + sl], b[4]);
+      };
+      if (!k.per && e < 3) ghost(p - 2 * e - 1, k.sa_lo, k.su_lo);
+      if (!k.per && e >= n - 3) ghost(p + 3, k.sa_hi, k.su_hi);
+      if (k.ub) b[1] += k.ub[cell];
+      fluid_store(k, cell, b, P[Q_R * FS + slot], P[Q_U * FS + slot], P[Q_V * FS + slot],
+                  P[Q_W * FS + slot]);
     }
-    done = hi + 1;
+    done = hi;
     wave_sync_lds();
   }
 }
 
-// Ghost contributions of each x-line into their source cells (one thread per line and
-// component, pairs in a fixed order). When the six ghost points e = -3..-1, n..n+2 have six
-// distinct source cells (lines of six cells or more), each source takes its pairs' sums in
-// registers, in the pairs' order, and is read and written once (all loads issued
-// together): the same sums as one read-modify-write per pair.
-__global__ void __launch_bounds__(256)
-fe_vjp_fix_x(Grid g, const double *side, FieldsOut out) {
-    const int nlines = g.ny * g.nz;
-  const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= (long)nlines * NV) return;
-  const int line = (int)(tid % nlines), qq = (int)(tid / nlines);
-  const int n = g.nx;
-  int src[6];
-#pragma unroll
-  for (int e = 0; e < 6; e++) src[e] = ghost_map(g, 0, e < 3 ? e - 3 : n + (e - 3)).src;
-  bool distinct = n >= 6;
-#pragma unroll
-  for (int a = 0; a < 6; a++)
-#pragma unroll
-    for (int b = a + 1; b < 6; b++) distinct = distinct && src[a] != src[b];
-  if (distinct) {
-    // ghost e = f - 3 + l: e = -3 (0,0); -2 (0,1) (1,0); -1 (0,2) (1,1) (2,0);
-    // n (n-2,5) (n-1,4) (n,3); n+1 (n-1,5) (n,4); n+2 (n,5), in pair order
-    const auto sv = [&](int f, int l) {
-      return side[((long)xghost_pair(n, f, l) * NV + qq) * nlines + line];
-    };
-    double add[6];
-    add[0] = sv(0, 0);
-    add[1] = sv(0, 1); add[2] = sv(0, 2);
-    const double a10 = sv(1, 0), a11 = sv(1, 1), a20 = sv(2, 0);
-    add[3] = sv(n - 2, 5); add[4] = sv(n - 1, 5); add[5] = sv(n, 5);
-    const double b14 = sv(n - 1, 4), b03 = sv(n, 3), b04 = sv(n, 4);
-    long cell[6];
-    double old[6];
-#pragma unroll
-    for (int e = 0; e < 6; e++) {
-      cell[e] = src[e] + (long)n * line;
-      old[e] = out.w[qq][cell[e]];
-    }
-    double v[6];
-    v[0] = old[0] + add[0];
-    v[1] = (old[1] + add[1]) + a10;
-    v[2] = ((old[2] + add[2]) + a11) + a20;
-    v[3] = ((old[3] + add[3]) + b14) + b03;
-    v[4] = (old[4] + add[4]) + b04;
-    v[5] = old[5] + add[5];
-#pragma unroll
-    for (int e = 0; e < 6; e++) {
-      out.w[qq][cell[e]] = v[e];
-    }
-    return;
-  }
-  for (int f = 0; f <= n; f++) {
-    if (f > 2 && f < n - 2) { f = n - 3; continue; }
-#pragma unroll 1
-    for (int l = 0; l < 6; l++) {
-      const int pr = xghost_pair(n, f, l);
-      if (pr < 0) continue;
-      const long cell = ghost_map(g, 0, f - 3 + l).src + (long)n * line;
-      out_put(out, qq, cell, side[((long)pr * NV + qq) * nlines + line], true);
-    }
-  }
-}
+// Waves that a direction's walk is split into at least, where columns allow: four per SIMD
+// for the tracers, two for the fluid (what its registers allow).
+constexpr long TRACER_WAVES = 4096, FLUID_WAVES = 2048;
 
-// ------------------------------------------------------------------------------------
-// y and z sweeps: each lane walks its own column (x = 64 * block + lane, fixed transverse
-// index t) over a segment [c0, c1) of faces along D; rows belong to that lane alone, so
-// no lane waits on another. The five rows f-2..f+2 still open live in an LDS ring
-// ([5][NV][64] per wave); row f-3 is complete with face f's first point and is written out
-// at once, its slot taking row f+2. Rows outside [c0, c1) (ghost rows and the three rows
-// either side that belong to neighbouring segments) go to the side buffer
-// [((seg * 6 + k) * NV + q) * ncol + col] and are added by fe_vjp_fix_yz.
-// ------------------------------------------------------------------------------------
-struct ColSink {
-  double *ring;            // this wave's [5][NV][64]
-  double *side;
-  FieldsOut out;
-  int lane, slot0;         // slot0: ring slot of row f-3 (slot of row f-3+l is (slot0+l)%5)
-  int e0, c0, c1, seg;
-  long col, ncol;
-  long cell0;              // cell of row f-3 when it lies in [c0, c1)
-  long cbase;              // cell of the column's row 0
-  bool add;
-  __device__ int slot(int l) const { const int s = slot0 + l; return s >= 5 ? s - 5 : s; }
-  __device__ bool owned() const { return e0 >= c0 && e0 < c1; }
-  __device__ double *dst(int comp) const {
-    return &out.w[comp][cell0];
-  }
-  struct Pre { double r0, w0; };
-  // row f-3 so far, and the value already in wbar where this sweep adds to it (read
-  // unconditionally, from the column's first row when f-3 is not an owned row, and only
-  // looked at in put, so that the loads stay in flight meanwhile)
-  __device__ Pre pre(int comp) const {
-    const long c = add && owned() ? cell0 : cbase;
-    const double w0 = out.w[comp][c];
-    return Pre{ring[((long)slot0 * NV + comp) * 64 + lane], w0};
-  }
-  __device__ void put(int comp, const double (&x)[6], const Pre &p) {
-    const double v = p.r0 + x[0];         // row f-3 is now complete
-    if (owned()) *dst(comp) = add ? p.w0 + v : v;
-    else {
-      const int k = e0 - (c0 - 3);        // e0 < c0 here
-      side[(((long)seg * 6 + k) * NV + comp) * ncol + col] = v;
-    }
-    ring[((long)slot0 * NV + comp) * 64 + lane] = x[5];   // the slot now holds row f+2
-#pragma unroll
-    for (int l = 1; l < 5; l++) atomicAdd(&ring[((long)slot(l) * NV + comp) * 64 + lane], x[l]);
-  }
-};
-
-template <int D>
-__global__ void __launch_bounds__(64)
-fe_vjp_sweep_yz(Grid g, Fields w, Fields vc, const double *ub, const double *alb, FieldsOut out,
-                double *side, int nseg, int add) {
-    __shared__ double ring[5 * NV * 64];
-  const int lane = threadIdx.x;
-  const int nxb = (g.nx + 63) / 64;
-  const int nt = D == 1 ? g.nz : g.ny;
-  const int n = D == 1 ? g.ny : g.nz;
-  const int xb = blockIdx.x % nxb;
-  const int rest = blockIdx.x / nxb;
-  const int t = rest % nt, seg = rest / nt;
-  const int i = xb * 64 + lane;
-  if (i >= g.nx) return;
-  const int c0 = (int)((long)seg * n / nseg), c1 = (int)((long)(seg + 1) * n / nseg);
-  const int flast = seg == nseg - 1 ? n : c1 - 1;
-  const long ncol = (long)g.nx * nt, col = i + (long)g.nx * t;
-  for (int s = 0; s < 5 * NV; s++) ring[s * 64 + lane] = 0.0;
-  const long rstride = D == 1 ? g.nx : (long)g.nx * g.ny;
-  const long cbase = D == 1 ? i + (long)g.nx * g.ny * t : i + (long)g.nx * t;
-  ColSink sink{ring, side, out, lane, 0, 0, c0, c1, seg, col, ncol, 0, cbase,
-                   add != 0};
-  for (int f = c0; f <= flast; f++) {
-    sink.slot0 = (f - c0) % 5;
-    sink.e0 = f - 3;
-    sink.cell0 = cbase + (long)(f - 3) * rstride;
-    const double ab = alb ? alb[f * ncol + col] : 0.0;
-    if (D == 1) face_vjp(g, w, vc, ub, ab, 1, i, f, t, sink);
-    else face_vjp(g, w, vc, ub, ab, 2, i, t, f, sink);
-  }
-  // rows flast-2 .. flast+2 are complete
-  for (int r = 0; r < 5; r++) {
-    const int e = flast - 2 + r;
-    const int sl = (flast + 1 - c0 + r) % 5;
-    for (int qq = 0; qq < NV; qq++) {
-      const double v = ring[((long)sl * NV + qq) * 64 + lane];
-      if (e >= c0 && e < c1) out_put(out, qq, cbase + (long)e * rstride, v, add != 0);
-      else {
-        const int k = e < c0 ? e - (c0 - 3) : 3 + (e - c1);
-        side[(((long)seg * 6 + k) * NV + qq) * ncol + col] = v;
-      }
-    }
-  }
-  if (flast + 2 < c1 + 2)      // an inner segment's last side row (c1 + 2) gets nothing
-    for (int qq = 0; qq < NV; qq++) side[(((long)seg * 6 + 5) * NV + qq) * ncol + col] = 0.0;
-}
-
-// Side rows of every segment of a column into their cells (one thread per column and
-// component, segments and rows in a fixed order): rows of neighbouring segments directly,
-// ghost rows through the ghost rule's source (their signs were applied at the faces).
-template <int D>
-__global__ void __launch_bounds__(256)
-fe_vjp_fix_yz(Grid g, const double *side, FieldsOut out, int nseg) {
-    const int nt = D == 1 ? g.nz : g.ny;
-  const int n = D == 1 ? g.ny : g.nz;
-  const long ncol = (long)g.nx * nt;
-  const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= ncol * NV) return;
-  const long col = tid % ncol;
-  const int qq = (int)(tid / ncol);
-  const int i = (int)(col % g.nx), t = (int)(col / g.nx);
-  const long rstride = D == 1 ? g.nx : (long)g.nx * g.ny;
-  const long cbase = D == 1 ? i + (long)g.nx * g.ny * t : i + (long)g.nx * t;
-  for (int seg = 0; seg < nseg; seg++) {
-    const int c0 = (int)((long)seg * n / nseg), c1 = (int)((long)(seg + 1) * n / nseg);
-    // when a segment's six side rows land in six distinct cells (segments of at least
-    // three rows away from short columns), all its reads are issued together
-    int src[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) src[k] = ghost_map(g, D, k < 3 ? c0 - 3 + k : c1 + (k - 3)).src;
-    bool distinct = true;
-#pragma unroll
-    for (int a = 0; a < 6; a++)
-#pragma unroll
-      for (int b = a + 1; b < 6; b++) distinct = distinct && src[a] != src[b];
-    if (distinct) {
-      long cell[6];
-      double add[6], old[6];
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-        cell[k] = cbase + (long)src[k] * rstride;
-        add[k] = side[(((long)seg * 6 + k) * NV + qq) * ncol + col];
-        old[k] = out.w[qq][cell[k]];
-      }
-#pragma unroll
-      for (int k = 0; k < 6; k++) {
-        out.w[qq][cell[k]] = old[k] + add[k];
-      }
-      continue;
-    }
-#pragma unroll 1
-    for (int k = 0; k < 6; k++) {
-      const int e = k < 3 ? c0 - 3 + k : c1 + (k - 3);
-      const int src = ghost_map(g, D, e).src;
-      const long cell = cbase + (long)src * rstride;
-      out_put(out, qq, cell, side[(((long)seg * 6 + k) * NV + qq) * ncol + col], true);
-    }
-  }
-}
-
-// Waves that the tracer walk of one direction is split into at least, where columns allow:
-// four per SIMD.
-constexpr long TRACER_WAVES = 4096;
-
-// Launch shape: one wave per SIMD over the device (4 per CU) where the grid allows.
-struct VjpPlan {
-  int lps;          // x-lines per wave
-  int nseg[3];      // segments per y / z column (index 1, 2)
-  size_t side;      // side-buffer doubles (the largest direction's)
-};
-
-static VjpPlan vjp_plan(const Grid &g) {
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  const long target = 4L * (ncu > 0 ? ncu : 256);
-  const long nv = NV;
-  VjpPlan p{};
-  const long nlines = (long)g.ny * g.nz;
-  p.lps = (int)((nlines + target - 1) / target);
-  size_t side = (size_t)nlines * 12 * nv;
-  for (int d = 1; d < 3; d++) {
-    const long n = d == 1 ? g.ny : g.nz, nt = d == 1 ? g.nz : g.ny;
-    const long waves = (long)((g.nx + 63) / 64) * nt;
-    long ns = (target + waves - 1) / waves;
-    const long maxseg = n >= 16 ? n / 8 : 1;
-    if (ns > maxseg) ns = maxseg;
-    if (ns < 1) ns = 1;
-    p.nseg[d] = (int)ns;
-    const size_t sd = (size_t)g.nx * nt * ns * 6 * nv;
-    if (sd > side) side = sd;
-  }
-  p.side = side;
-  return p;
-}
-
-// One direction: the tracers (with NC > 0), then the fluid sweep and its fix-up.
-template <int NC>
-static void tracers_launch(const Grid &g, int d, const Fields &w, const double *v, double *out,
-                           double *ub, double *alb, hipStream_t st) {
-  constexpr long GPW = 64 / NC;
+static Walk walk_of(const Grid &g, int d) {
   const long nx = g.nx, nxy = nx * g.ny;
-  TrWalk k{};
-  k.r = w.w[0]; k.m0 = w.w[1]; k.m1 = w.w[2]; k.m2 = w.w[3]; k.e = w.w[4]; k.mn = w.w[1 + d];
-  k.t = w.chem; k.v = v; k.out = out; k.ub = ub; k.alb = alb;
+  Walk k{};
   k.n = extent(g, d);
   k.ncol = nxy * g.nz / k.n;
   k.nin = (int)(d == 0 ? 1 : d == 1 ? nx : nxy);
@@ -986,9 +804,26 @@ static void tracers_launch(const Grid &g, int d, const Fields &w, const double *
   k.su_hi = hi == BC_REFLECTING ? -1.0 : 1.0;
   k.idelta = 1.0 / (d == 0 ? g.dx : d == 1 ? g.dy : g.dz);
   k.gamma = g.gamma;
-  k.ncb = (int)((k.ncol + GPW - 1) / GPW);
-  const long maxseg = k.n >= 16 ? k.n / 8 : 1;
-  k.nseg = (int)std::min(maxseg, (TRACER_WAVES + k.ncb - 1) / k.ncb);
+  k.igm = g.igm;
+  return k;
+}
+
+// Column blocks of gpw columns and the segments that give at least `waves` waves, of
+// minrows rows or more.
+static void walk_split(Walk &k, long gpw, long waves, int minrows) {
+  k.ncb = (int)((k.ncol + gpw - 1) / gpw);
+  const long maxseg = std::max(1, k.n / minrows);
+  k.nseg = (int)std::min(maxseg, (waves + k.ncb - 1) / k.ncb);
+}
+
+template <int NC>
+static void tracers_launch(const Grid &g, int d, const Fields &w, const double *v, double *out,
+                           double *ub, double *alb, hipStream_t st) {
+  TrWalk k{};
+  (Walk &)k = walk_of(g, d);
+  k.r = w.w[0]; k.m0 = w.w[1]; k.m1 = w.w[2]; k.m2 = w.w[3]; k.e = w.w[4]; k.mn = w.w[1 + d];
+  k.t = w.chem; k.v = v; k.out = out; k.ub = ub; k.alb = alb;
+  walk_split(k, 64 / NC, TRACER_WAVES, 8);
   hipLaunchKernelGGL(fe_vjp_tracers<NC>, dim3((unsigned)(k.ncb * k.nseg)), dim3(64), 0, st, k);
 }
 
@@ -1004,60 +839,63 @@ static int tracers_run(const Grid &g, int d, const Fields &w, const double *v, d
   }
 }
 
+static void fluid_run(const Grid &g, int d, const Fields &w, const Fields &v, const FieldsOut &out,
+                      const double *ub, const double *alb, hipStream_t st) {
+  FlWalk k{};
+  (Walk &)k = walk_of(g, d);
+  k.ub = ub;
+  k.alb = alb;
+  for (int a = 0; a < 5; a++) {
+    const int q = a == 1 ? 1 + d : a == 1 + d ? 1 : a;
+    k.w[a] = w.w[q];
+    k.v[a] = v.w[q];
+    k.out[a] = out.w[q];
+  }
+  if (d == 0) {
+    const int lps = (int)((k.ncol + FLUID_WAVES - 1) / FLUID_WAVES);
+    const dim3 grid((unsigned)((k.ncol + lps - 1) / lps));
+    if (k.n + (k.per ? 5 : 1) >= 8)
+      hipLaunchKernelGGL(fe_vjp_lines<128>, grid, dim3(64), 0, st, k, lps);
+    else hipLaunchKernelGGL(fe_vjp_lines<256>, grid, dim3(64), 0, st, k, lps);
+  } else {
+    walk_split(k, 64, FLUID_WAVES, 4);
+    hipLaunchKernelGGL(fe_vjp_walk, dim3((unsigned)(k.ncb * k.nseg)), dim3(64), 0, st, k);
+  }
+}
+
+}  // namespace
+
 static long max_faces(const Grid &g) {
   const long nx = g.nx, ny = g.ny, nz = g.nz;
   return std::max({(nx + 1) * ny * nz, nx * (ny + 1) * nz, nx * ny * (nz + 1)});
 }
 
-// Scratch: the side buffer; with tracers also ub (cells), alb (faces of a direction) and a
-// tracer array for calls whose wbar tracers overlap an input's.
+// Scratch, with tracers only: ub (cells), alb (faces of a direction) and a tracer array for
+// calls whose wbar tracers overlap an input's.
 size_t fe_vjp_buffer_doubles(const Grid &g) {
   const long ncell = (long)g.nx * g.ny * g.nz;
-  return vjp_plan(g).side + (g.nchem ? (size_t)(1 + g.nchem) * ncell + max_faces(g) : 0);
+  return g.nchem ? (size_t)(1 + g.nchem) * ncell + max_faces(g) : 0;
 }
 
 int fe_vjp_launch(const Grid &g, const Fields &w, const Fields &v, const FieldsOut &out,
                   double *buf, hipStream_t st) {
-  constexpr long NV = 5;
-  const VjpPlan p = vjp_plan(g);
-  const long nlines = (long)g.ny * g.nz, ncell = g.nx * nlines;
-  const int nxb = (g.nx + 63) / 64;
-  double *side = buf, *ub = nullptr, *alb = nullptr, *tr = nullptr;
+  const long ncell = (long)g.nx * g.ny * g.nz, nt = g.nchem * ncell;
+  double *ub = nullptr, *alb = nullptr, *tr = out.chem;
   if (g.nchem) {
-    ub = buf + p.side;
+    ub = buf;
     alb = ub + ncell;
-    const long nt = g.nchem * ncell;
     const auto overlaps = [&](const double *a) { return a < out.chem + nt && out.chem < a + nt; };
-    tr = overlaps(w.chem) || overlaps(v.chem) ? alb + max_faces(g) : out.chem;
+    if (overlaps(w.chem) || overlaps(v.chem)) tr = alb + max_faces(g);
   }
   for (int d = 0; d < 3; d++) {
     if (g.nchem) {
       const int rc = tracers_run(g, d, w, v.chem, tr, ub, alb, st);
       if (rc) return rc;
     }
-    if (d == 0) {
-      hipLaunchKernelGGL(fe_vjp_sweep_x, dim3((unsigned)((nlines + p.lps - 1) / p.lps)), dim3(64),
-                         0, st, g, w, v, (const double *)ub, (const double *)alb, out, side, p.lps,
-                         0);
-      hipLaunchKernelGGL(fe_vjp_fix_x, dim3((unsigned)((nlines * NV + 255) / 256)), dim3(256), 0,
-                         st, g, (const double *)side, out);
-    } else if (d == 1) {
-      hipLaunchKernelGGL(fe_vjp_sweep_yz<1>, dim3((unsigned)(nxb * g.nz * p.nseg[1])), dim3(64), 0,
-                         st, g, w, v, (const double *)ub, (const double *)alb, out, side,
-                         p.nseg[1], 1);
-      hipLaunchKernelGGL(fe_vjp_fix_yz<1>, dim3((unsigned)(((long)g.nx * g.nz * NV + 255) / 256)),
-                         dim3(256), 0, st, g, (const double *)side, out, p.nseg[1]);
-    } else {
-      hipLaunchKernelGGL(fe_vjp_sweep_yz<2>, dim3((unsigned)(nxb * g.ny * p.nseg[2])), dim3(64), 0,
-                         st, g, w, v, (const double *)ub, (const double *)alb, out, side,
-                         p.nseg[2], 1);
-      hipLaunchKernelGGL(fe_vjp_fix_yz<2>, dim3((unsigned)(((long)g.nx * g.ny * NV + 255) / 256)),
-                         dim3(256), 0, st, g, (const double *)side, out, p.nseg[2]);
-    }
+    fluid_run(g, d, w, v, out, ub, alb, st);
   }
   if (tr != out.chem &&
-      hipMemcpyAsync(out.chem, tr, sizeof(double) * g.nchem * ncell, hipMemcpyDeviceToDevice,
-                     st) != hipSuccess)
+      hipMemcpyAsync(out.chem, tr, sizeof(double) * nt, hipMemcpyDeviceToDevice, st) != hipSuccess)
     return -1;
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
