@@ -66,70 +66,114 @@ struct ChemPtrs {
   double *Ts, *dTs;
 };
 
-// calculate_rhs_cvklu (raja_primordial_network.cpp:1015-1389)
-__global__ void __launch_bounds__(256)
+// calculate_rhs_cvklu (raja_primordial_network.cpp:1015-1389). One wave per block; the vectors
+// pass through LDS (vec_load), the species rows and the gas-energy row take their rates one
+// after the other (150 registers). 64^3 cells: 48.5 -> 42.5 us (all rates at once: 48.4 at two
+// waves per SIMD, 79 spilled at four; this form at two 43.8, at four 48.4). The state and the
+// result are 18 us of memory time, the rest the latency of the temperature solve and of the
+// table gathers.
+__global__ void __launch_bounds__(64, 3)
 chem_rhs_kernel(long n, ChemConst cc, ChemPtrs p, const double *yd, double *ydot, double srhs) {
 #pragma clang fp contract(off)
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  __shared__ double lds[VEC_LDS];
+  const long base = (long)blockIdx.x * 64;
+  const int ncell = (int)min(n - base, 64L);
+  const bool mine = (int)threadIdx.x < ncell;
+  const long i = base + min((int)threadIdx.x, ncell - 1);   // spare lanes repeat the last cell
   double y[NSP];
+  vec_load(yd + NSP * base, p.scale + NSP * base, ncell, lds, y);
+  if (!mine) {                                              // (and its values)
 #pragma unroll
-  for (int v = 0; v < NSP; v++) y[v] = yd[NSP * i + v] * p.scale[NSP * i + v];
+    for (int v = 0; v < NSP; v++) y[v] = lds[(ncell - 1) * VEC_PITCH + v];
+  }
   double Ts = p.Ts[i], dTs;
   chem_temperature(cc, y, Ts, dTs);
-  p.Ts[i] = Ts;
-  p.dTs[i] = dTs;
-  double k[NRATE];
-  chem_rates_only_pairs<0, NRATE>(cc, Ts, k);
+  if (mine) {
+    p.Ts[i] = Ts;
+    p.dTs[i] = dTs;
+  }
   const CellAux ax{p.md[i], p.imd[i], p.cie[i], p.h2o[i]};
-  double f[NSP];
-  chem_rhs_physical(y, k, Ts, cc.z, ax, f);
-#pragma unroll
-  for (int v = 0; v < NSP; v++) f[v] *= p.iscale[NSP * i + v];
-  f[9] *= ax.inv_mdensity;
+  double Tdef, k[NRATE], f[NSP];
+  const double2 *row = cc.tabp + (long)chem_locate(cc, chem_log(Ts), Tdef) * NRATE;
+  chem_rates_only_at<0, C_BREM>(row, Tdef, k);
+  chem_rhs_species(y, k, f);
+  // an offset that the compiler does not know, so that it starts the second half's loads here
+  int zero = 0;
+  __asm__ volatile("" : "+v"(zero) : "v"(f[0]), "v"(f[2]), "v"(f[8]));
+  chem_rates_only_at<C_BREM, NRATE>(row + zero, Tdef, k);
+  f[9] = chem_rhs_energy(y, k, Ts, cc.z, ax);
   // times the caller's factor (TimeUnits for ffast/fimpl, N_VScale after the RHS; 1 exact)
-#pragma unroll
-  for (int v = 0; v < NSP; v++) ydot[NSP * i + v] = srhs * f[v];
+  vec_store(ydot + NSP * base, p.iscale + NSP * base, srhs, ax.inv_mdensity, ncell, lds, f);
 }
 
 // Vector-Jacobian product of calculate_rhs_cvklu in the scaled variables:
 // ybar = (d ydot / d y)^T v, with the temperature a function of y (solved from the warm start
-// like the RHS, which it also updates); optionally ydot itself. The rates come from the
-// rate-major tables, all of them in one batch of loads: with one wave per SIMD the kernel
-// is bound by the latency of these gathers, and for cells of unrelated temperatures this
-// form measured faster than the pair table.
-__global__ void __launch_bounds__(256)
+// like the RHS, which it also updates); optionally ydot itself. One wave per block, the vectors
+// through LDS. The reactions and the gas-energy row take their rates from the pair table one
+// after the other: all 46 rates and slopes at once need 320 registers, and with one wave per
+// SIMD the kernel waits for them. 128^3 cells of unrelated temperatures: 0.47 -> 0.33 ms (at
+// three waves per SIMD it spills: 0.48); memory takes 0.18.
+__global__ void __launch_bounds__(64, 2)
 chem_vjp_kernel(long n, ChemConst cc, ChemPtrs p, const double *yd, const double *v,
                 double *ybar, double *ydot) {
 #pragma clang fp contract(off)
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  __shared__ double lds[VEC_LDS];
+  const long base = (long)blockIdx.x * 64;
+  const int ncell = (int)min(n - base, 64L);
+  const bool mine = (int)threadIdx.x < ncell;
+  const long i = base + min((int)threadIdx.x, ncell - 1);   // spare lanes repeat the last cell
   double y[NSP];
+  vec_load(yd + NSP * base, p.scale + NSP * base, ncell, lds, y);
+  if (!mine) {                                              // (and its values)
 #pragma unroll
-  for (int s = 0; s < NSP; s++) y[s] = yd[NSP * i + s] * p.scale[NSP * i + s];
+    for (int s = 0; s < NSP; s++) y[s] = lds[(ncell - 1) * VEC_PITCH + s];
+  }
   double Ts = p.Ts[i], dTs;
   chem_temperature(cc, y, Ts, dTs);
-  p.Ts[i] = Ts;
-  p.dTs[i] = dTs;
+  if (mine) {
+    p.Ts[i] = Ts;
+    p.dTs[i] = dTs;
+  }
   const CellAux ax{p.md[i], p.imd[i], p.cie[i], p.h2o[i]};
   if (ydot) {
     double k[NRATE], f[NSP];
-    chem_rates_only(cc, Ts, k);
+    chem_rates_only_pairs<0, NRATE>(cc, Ts, k);
     chem_rhs_physical(y, k, Ts, cc.z, ax, f);
-#pragma unroll
-    for (int s = 0; s < NSP; s++) f[s] *= p.iscale[NSP * i + s];
-    f[9] *= ax.inv_mdensity;
-#pragma unroll
-    for (int s = 0; s < NSP; s++) ydot[NSP * i + s] = f[s];
+    vec_store(ydot + NSP * base, p.iscale + NSP * base, 1.0, ax.inv_mdensity, ncell, lds, f);
   }
-  double vp[NSP], yb[NSP];
-#pragma unroll
-  for (int s = 0; s < NSP; s++) vp[s] = v[NSP * i + s] * p.iscale[NSP * i + s];
+  double vp[NSP], yb[NSP], Tb = 0.0;
+  vec_load(v + NSP * base, p.iscale + NSP * base, ncell, lds, vp);
   vp[9] *= ax.inv_mdensity;
-  const bool clamped = !(Ts > cc.tmin && Ts < cc.tmax);
-  chem_vjp_physical<false>(cc, y, Ts, clamped, ax, vp, yb);
 #pragma unroll
-  for (int s = 0; s < NSP; s++) ybar[NSP * i + s] = yb[s] * p.scale[NSP * i + s];
+  for (int s = 0; s < NSP; s++) yb[s] = 0.0;
+  double Tdef;
+  const int bn = chem_locate(cc, chem_log(Ts), Tdef);
+  const double Tfactor = fast_rcp(Ts) * cc.idbin;
+  const double2 *row = cc.tabp + (long)bn * NRATE;
+  double k[NRATE], dk[NRATE];
+  chem_rates_at<0, C_BREM>(row, Tdef, Tfactor, k, dk);
+  chem_vjp_species(k, dk, y, vp, yb, Tb);
+#pragma unroll
+  for (int s = 0; s < NSP; s++) __asm__ volatile("" : "+v"(yb[s]));
+  // (an offset that the compiler does not know, so that it starts the second half's loads here)
+  int zero = 0;
+  __asm__ volatile("" : "+v"(zero) : "v"(yb[0]), "v"(Tb));
+  chem_rates_at<C_BREM, NRATE>(row + zero, Tdef, Tfactor, k, dk);
+  {
+#pragma clang fp contract(on)
+    double e9[NSP];
+    chem_energy_grad(y, k, dk, Ts, cc.z, ax, e9);
+#pragma unroll
+    for (int s = 0; s < NSP - 1; s++) yb[s] += vp[9] * e9[s];
+    Tb += vp[9] * e9[NSP - 1];
+  }
+  if (Ts > cc.tmin && Ts < cc.tmax) {              // not clamped
+    struct { double dgdT, dgdy[NSP - 1]; bool clamped; } P;
+    P.clamped = false;
+    chem_vjp_path(cc, y, Ts, bn, Tdef, Tfactor, P);
+    chem_vjp_temperature(P, Tb, yb);
+  }
+  vec_store(ybar + NSP * base, p.scale + NSP * base, 1.0, 1.0, ncell, lds, yb);
 }
 
 // Self-check of the temperature solve's early exit: the early form and the ten steps from
@@ -255,8 +299,8 @@ int chem_prepare(ChemState &s, double *chem, hipStream_t st) {
 
 int chem_rhs(ChemState &s, const double *y, double *ydot, hipStream_t st, bool sync,
              double srhs) {
-  hipLaunchKernelGGL(chem_rhs_kernel, dim3(nb(s.n)), dim3(256), 0, st, s.n, s.cc, ptrs_of(s), y,
-                     ydot, srhs);
+  hipLaunchKernelGGL(chem_rhs_kernel, dim3((unsigned)((s.n + 63) / 64)), dim3(64), 0, st, s.n, s.cc,
+                     ptrs_of(s), y, ydot, srhs);
   if (hipGetLastError() != hipSuccess) return MVD_DEVICE_ERROR;
   if (!sync) return MVD_SUCCESS;
   return hipStreamSynchronize(st) == hipSuccess ? MVD_SUCCESS : MVD_DEVICE_ERROR;
@@ -274,8 +318,8 @@ int chem_jac(ChemState &s, const double *y, double *J, hipStream_t st, bool sync
 int chem_vjp(ChemState &s, const double *y, const double *v, double *ybar, double *ydot,
              hipStream_t st, bool sync) {
   if (!s.ready) return MVD_NOT_READY;
-  hipLaunchKernelGGL(chem_vjp_kernel, dim3(nb(s.n)), dim3(256), 0, st, s.n, s.cc, ptrs_of(s), y,
-                     v, ybar, ydot);
+  hipLaunchKernelGGL(chem_vjp_kernel, dim3((unsigned)((s.n + 63) / 64)), dim3(64), 0, st, s.n, s.cc,
+                     ptrs_of(s), y, v, ybar, ydot);
   if (hipGetLastError() != hipSuccess) return MVD_DEVICE_ERROR;
   if (sync && hipStreamSynchronize(st) != hipSuccess) return MVD_DEVICE_ERROR;
   return MVD_SUCCESS;

@@ -1547,7 +1547,7 @@ __device__ inline void stage_adjoint_matrix(const ChemConst &cc, const CellIn &c
   chem_temperature(cc, ya, T, dT);
   const bool clamped = !(T > cc.tmin && T < cc.tmax);
   ChemVjpPre P;                  // rates, gas-energy tangents, temperature path: once
-  chem_vjp_prepare<true>(cc, ya, T, clamped, c.ax, P);
+  chem_vjp_prepare(cc, ya, T, clamped, c.ax, P);
   double acc[NSP];
 #pragma unroll
   for (int q = 0; q < NSP; q++) acc[q] = 0.0;

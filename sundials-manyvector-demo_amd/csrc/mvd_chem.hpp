@@ -154,6 +154,57 @@ __device__ inline void blk_store(double *dst, int ncell, double *lds, const doub
   }
 }
 
+// The same for vectors of ten values per cell: a[s] = x[s] * f[s] of the lane's cell, the
+// product taken on the way into LDS. 5.6 KB per wave; cells are padded to 11 doubles.
+constexpr int VEC_PITCH = NSP + 1, VEC_LDS = 64 * VEC_PITCH;
+
+__device__ inline void vec_load(const double *x, const double *f, int ncell, double *lds,
+                                double (&a)[NSP]) {
+  const int lane = threadIdx.x & 63, np = ncell * (NSP / 2);
+  const Pair8 *px = reinterpret_cast<const Pair8 *>(x), *pf = reinterpret_cast<const Pair8 *>(f);
+  Pair8 vx[NSP / 2], vf[NSP / 2];
+#pragma unroll
+  for (int i = 0; i < NSP / 2; i++) {
+    const int e = min(i * 64 + lane, np - 1);
+    vx[i] = px[e];
+    vf[i] = pf[e];
+  }
+  blk_sync();                                           // lds is free again
+#pragma unroll
+  for (int i = 0; i < NSP / 2; i++) {
+    const int e = i * 64 + lane, cell = e / (NSP / 2);
+    double *d = lds + cell * VEC_PITCH + 2 * (e - cell * (NSP / 2));
+    d[0] = vx[i].x * vf[i].x;
+    d[1] = vx[i].y * vf[i].y;
+  }
+  blk_sync();
+#pragma unroll
+  for (int s = 0; s < NSP; s++) a[s] = lds[lane * VEC_PITCH + s];
+}
+
+// dst[s] = c ((a[s] f[s]) m9), with the factor m9 of the lane's cell on the last value only.
+__device__ inline void vec_store(double *dst, const double *f, double c, double m9, int ncell,
+                                 double *lds, const double (&a)[NSP]) {
+  const int lane = threadIdx.x & 63, np = ncell * (NSP / 2);
+  const Pair8 *pf = reinterpret_cast<const Pair8 *>(f);
+  Pair8 *pd = reinterpret_cast<Pair8 *>(dst);
+  blk_sync();
+#pragma unroll
+  for (int s = 0; s < NSP; s++) lds[lane * VEC_PITCH + s] = a[s];
+  lds[lane * VEC_PITCH + NSP] = m9;
+  blk_sync();
+#pragma unroll
+  for (int i = 0; i < NSP / 2; i++) {
+    const int e = i * 64 + lane, cell = e / (NSP / 2), q = e - cell * (NSP / 2);
+    if (e < np) {
+      const double *d = lds + cell * VEC_PITCH;
+      const Pair8 b = pf[e];
+      const double m = q == NSP / 2 - 1 ? d[NSP] : 1.0;
+      pd[e] = Pair8{c * (d[2 * q] * b.x), c * (d[2 * q + 1] * b.y * m)};
+    }
+  }
+}
+
 // -------------------------------------------------------------------------------------
 // device functions: the reference's expressions. Products and sums of one expression are
 // contracted to FMAs by the front end (contract(on), the same way wherever a function is
@@ -405,6 +456,29 @@ __device__ inline void chem_rates_pairs(const ChemConst &c, double T, double (&k
   }
 }
 
+// The same at a table position already known (row: the bin's pairs).
+template <int R0, int R1>
+__device__ inline void chem_rates_at(const double2 *row, double Tdef, double Tfactor,
+                                     double (&k)[NRATE], double (&dk)[NRATE]) {
+#pragma clang fp contract(on)
+#pragma unroll
+  for (int r = R0; r < R1; r++) {
+    const double2 a = row[r];
+    k[r] = a.x + Tdef * (a.y - a.x);
+    dk[r] = (a.y - a.x) * Tfactor;
+  }
+}
+
+template <int R0, int R1>
+__device__ inline void chem_rates_only_at(const double2 *row, double Tdef, double (&k)[NRATE]) {
+#pragma clang fp contract(on)
+#pragma unroll
+  for (int r = R0; r < R1; r++) {
+    const double2 a = row[r];
+    k[r] = a.x + Tdef * (a.y - a.x);
+  }
+}
+
 template <int R0, int R1>
 __device__ inline void chem_rates_only_pairs(const ChemConst &c, double T, double (&k)[NRATE]) {
 #pragma clang fp contract(on)
@@ -415,18 +489,6 @@ __device__ inline void chem_rates_only_pairs(const ChemConst &c, double T, doubl
   for (int r = R0; r < R1; r++) {
     const double2 a = row[r];
     k[r] = a.x + Tdef * (a.y - a.x);
-  }
-}
-
-// Only the rate values (no derivatives).
-__device__ inline void chem_rates_only(const ChemConst &c, double T, double (&k)[NRATE]) {
-#pragma clang fp contract(on)
-  double Tdef;
-  const int b = chem_locate(c, chem_log(T), Tdef);
-#pragma unroll
-  for (int r = 0; r < NRATE; r++) {
-    const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
-    k[r] = a0 + Tdef * (a1 - a0);
   }
 }
 
@@ -661,33 +723,13 @@ struct ChemVjpPre {
   bool clamped;
 };
 
-// PAIRS: the rates from the bin-major pair table (same values).
-template <bool PAIRS>
-__device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NSP], double T,
-                                        bool clamped, const CellAux &ax, ChemVjpPre &P) {
+// The temperature path's dg/dT and dg/dy at table position (bn, Tdef).
+template <class Pre>
+__device__ inline void chem_vjp_path(const ChemConst &c, const double (&y)[NSP], double T, int bn,
+                                     double Tdef, double Tfactor, Pre &P) {
 #pragma clang fp contract(on)
-  double k[NRATE], dk[NRATE];
-  if (PAIRS) chem_rates_pairs<0, NRATE>(c, T, k, dk);
-  else chem_rates(c, T, k, dk);
-#pragma unroll
-  for (int j = 0; j < NREACT; j++) {
-    P.k[j] = k[j];
-    P.dk[j] = dk[j];
-  }
-  // gas-energy row: its gradient along H2_1, H_1, H_2, He_1, He_2, He_3, de and T (in
-  // slot 9: ge has none)
-  chem_energy_grad(y, k, dk, T, c.z, ax, P.e9);
-  P.clamped = clamped;
-  P.dgdT = 1.0;
-#pragma unroll
-  for (int s = 0; s < NSP - 1; s++) P.dgdy[s] = 0.0;
-  if (clamped) return;
-  // temperature path
   const double kb = 1.3806504e-16, mh = 1.67e-24;
   const double gm1 = 1.0 / (5.e0 / 3.e0 - 1);
-  double Tdef;
-  const int bn = chem_locate(c, chem_log(T), Tdef);
-  const double Tfactor = fast_rcp(T) * c.idbin;
   const double *g1t = c.tab + G_GH2_1 * TLEN, *g2t = c.tab + G_GH2_2 * TLEN;
   const double gH2_1 = g1t[bn] + Tdef * (g1t[bn + 1] - g1t[bn]);
   const double gH2_2 = g2t[bn] + Tdef * (g2t[bn + 1] - g2t[bn]);
@@ -711,8 +753,32 @@ __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NS
   for (int s = 0; s < NSP - 1; s++) P.dgdy[s] = td * (cs[s] - nd * ws[s]);
 }
 
+__device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NSP], double T,
+                                        bool clamped, const CellAux &ax, ChemVjpPre &P) {
+#pragma clang fp contract(on)
+  double k[NRATE], dk[NRATE];
+  chem_rates_pairs<0, NRATE>(c, T, k, dk);
+#pragma unroll
+  for (int j = 0; j < NREACT; j++) {
+    P.k[j] = k[j];
+    P.dk[j] = dk[j];
+  }
+  // gas-energy row: its gradient along H2_1, H_1, H_2, He_1, He_2, He_3, de and T (in
+  // slot 9: ge has none)
+  chem_energy_grad(y, k, dk, T, c.z, ax, P.e9);
+  P.clamped = clamped;
+  P.dgdT = 1.0;
+#pragma unroll
+  for (int s = 0; s < NSP - 1; s++) P.dgdy[s] = 0.0;
+  if (clamped) return;
+  double Tdef;
+  const int bn = chem_locate(c, chem_log(T), Tdef);
+  chem_vjp_path(c, y, T, bn, Tdef, fast_rcp(T) * c.idbin, P);
+}
+
 // The temperature path's share of yab for the T-cotangent Tb.
-__device__ inline void chem_vjp_temperature(const ChemVjpPre &P, double Tb,
+template <class Pre>
+__device__ inline void chem_vjp_temperature(const Pre &P, double Tb,
                                             double (&yab)[NSP]) {
 #pragma clang fp contract(on)
   if (P.clamped) return;
@@ -722,13 +788,12 @@ __device__ inline void chem_vjp_temperature(const ChemVjpPre &P, double Tb,
   yab[NSP - 1] += TbT;                                            // dg/dge = -1
 }
 
-__device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP],
-                                      const double (&vp)[NSP], double (&yab)[NSP]) {
+// The species rows' share: in reverse through r_j = k_j * prod(reactants).
+template <int N>
+__device__ inline void chem_vjp_species(const double (&k)[N], const double (&dk)[N],
+                                        const double (&y)[NSP], const double (&vp)[NSP],
+                                        double (&yab)[NSP], double &Tb) {
 #pragma clang fp contract(on)
-#pragma unroll
-  for (int s = 0; s < NSP; s++) yab[s] = 0.0;
-  double Tb = 0.0;
-  // species rows: reverse through r_j = k_j * prod(reactants)
 #pragma unroll
   for (int j = 0; j < NREACT; j++) {
     double rb = 0.0;
@@ -737,11 +802,20 @@ __device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP
       if (CHEM_STO[s][j] != 0) rb += (double)CHEM_STO[s][j] * vp[s];
     const int a = CHEM_REACTANTS[j][0], b = CHEM_REACTANTS[j][1], cc = CHEM_REACTANTS[j][2];
     const double ya = y[a], yb = y[b], yc = cc >= 0 ? y[cc] : 1.0;
-    yab[a] += rb * (P.k[j] * yb * yc);
-    yab[b] += rb * (P.k[j] * ya * yc);
-    if (cc >= 0) yab[cc] += rb * (P.k[j] * ya * yb);
-    Tb += rb * (P.dk[j] * ya * yb * yc);
+    yab[a] += rb * (k[j] * yb * yc);
+    yab[b] += rb * (k[j] * ya * yc);
+    if (cc >= 0) yab[cc] += rb * (k[j] * ya * yb);
+    Tb += rb * (dk[j] * ya * yb * yc);
   }
+}
+
+__device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP],
+                                      const double (&vp)[NSP], double (&yab)[NSP]) {
+#pragma clang fp contract(on)
+#pragma unroll
+  for (int s = 0; s < NSP; s++) yab[s] = 0.0;
+  double Tb = 0.0;
+  chem_vjp_species(P.k, P.dk, y, vp, yab, Tb);
   // gas-energy row
   constexpr int dirs[7] = {0, 2, 3, 5, 6, 7, 8};
 #pragma unroll
@@ -777,15 +851,6 @@ __device__ inline void chem_vjp_row(const ChemVjpPre &P, const double (&y)[NSP],
     Tb += v * P.e9[NSP - 1];
   }
   chem_vjp_temperature(P, Tb, row);
-}
-
-template <bool PAIRS>
-__device__ inline void chem_vjp_physical(const ChemConst &c, const double (&y)[NSP], double T,
-                                         bool clamped, const CellAux &ax,
-                                         const double (&vp)[NSP], double (&yab)[NSP]) {
-  ChemVjpPre P;
-  chem_vjp_prepare<PAIRS>(c, y, T, clamped, ax, P);
-  chem_vjp_apply(P, y, vp, yab);
 }
 
 __device__ inline void chem_rhs_physical(const double (&y)[NSP], const double (&k)[NRATE],
