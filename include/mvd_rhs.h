@@ -370,7 +370,7 @@ int mvd_imex_evolve(mvd_context *ctx, double t0, double h, int nsteps, const mvd
  * by a thread-per-cell run of the plain solver's per-cell algorithm, keeping the state every
  * ckpt_every steps; then lam0 = (d y_N / d y_0)^T lamT (both [cell][10]) for the stage
  * equations solved exactly along that trajectory, with the exact stage Jacobians; each
- * segment is recomputed once from its checkpoint, keeping its steps' stage values. o must
+ * segment but the last is recomputed once from its checkpoint, keeping its steps' stage values. o must
  * be an SDIRK table of at most 4 stages, stiffly accurate (the last row of A sums to 1, as
  * mvd_dirk_sdirk3; an ESDIRK table gives MVD_UNSUPPORTED). Ts/dTs end at the
  * forward run's final state. Returns 0, the number (> 0) of cells whose forward Newton
@@ -378,7 +378,7 @@ int mvd_imex_evolve(mvd_context *ctx, double t0, double h, int nsteps, const mvd
  * The cells run in the batched step's temperature order at y_0 (from 4096 cells on).
  * Device scratch held by the context: ceil(nsteps/ckpt_every) * 12
  * + ckpt_every * (10 * nstage + 1) doubles and 22 bytes (the cell order) per cell, and
- * 128 KiB. */
+ * 128 KiB; the second term counts twice for batches of at most two waves per CU (below 4 GiB). */
 int mvd_chem_dirk_adjoint(mvd_context *ctx, double t, double h, int nsteps, int ckpt_every,
                           const mvd_dirk_opts *o, double *y, const double *lamT, double *lam0);
 

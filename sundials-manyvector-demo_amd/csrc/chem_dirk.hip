@@ -1434,26 +1434,35 @@ int chem_ls_solve(long n, const double *LU, const unsigned long long *piv, const
 //              b = the last row of A (the stiffly accurate tables of mvd_chem_dirk_step).
 // The per-cell step is the plain solver's algorithm (modified Newton, J at y_n, refactor
 // after max_iters), thread-local, so that recomputation repeats the forward run bit for bit.
-// Scratch per cell (element-major, coalesced): nckpt x 12 + K x (nstage x 10 + 1) doubles.
+// Scratch per cell (element-major, coalesced): nckpt x 12 + K x (nstage x 10 + 1) doubles, the
+// second part twice where pairs of waves run (adj_pipe).
+// A wave's steps are one long dependent chain at one wave per SIMD, so what shortens it is work
+// taken out or handed to an idle SIMD: gamma tables, scales and stage derivatives in LDS, the last
+// segment kept by the forward run instead of recomputed, and for small batches a second
+// wave that recomputes ahead of the backward walk. 32^3 cells, 20 steps, K = 5: forward 1.02 ->
+// 0.79 ms, backward 2.43 -> 0.92 ms (1.05 with the nu_k in registers, which spilled).
 // ---------------------------------------------------------------------------------
-__device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, double &dTs,
-                          const DirkDev &o, double h, double (&y)[NSP], double *Ys, long n,
-                          long i) {
+__device__ bool cell_step(const ChemConst &cc, const GammaTabs &gt, const CellIn &c, double &Ts,
+                          double &dTs, const DirkDev &o, double h, double (&y)[NSP], double *Fl,
+                          double *Ys, long n, long i) {
 #pragma clang fp contract(on)
-  double yn[NSP], z[NSP], f[NSP], F[ADJ_MAXSTAGE][NSP];
+  double z[NSP], f[NSP];
 #pragma unroll
-  for (int s = 0; s < NSP; s++) yn[s] = z[s] = y[s];
+  for (int s = 0; s < NSP; s++) {
+    z[s] = y[s];
+    Fl[s * 64] = y[s];
+  }
   double a[NSP][NSP];
   unsigned long long pv = 0;
-  cell_rhs<true>(cc, c, Ts, dTs, yn, o.rhs_scale, f);      // refresh Ts at y_n for J
-  bool ok = true;
+  cell_rhs<true>(cc, gt, c, Ts, dTs, y, o.rhs_scale, f);       // refresh Ts at y_n for J
+  bool ok = true, fresh = true;      // fresh: Ts and dTs are those of z
   double crate = 1.0, delp = 0.0;                     // Newton rate estimate, last norm
 #pragma unroll
   for (int st = 0; st < ADJ_MAXSTAGE; st++) {
     if (st < o.nstage && ok) {
       const double hg = h * o.A[st * MAXSTAGE + st];
       if (st == 0) {
-        cell_matrix_regs(cc, c, Ts, dTs, yn, hg, o.rhs_scale, a);
+        cell_matrix_regs(cc, c, Ts, dTs, y, hg, o.rhs_scale, a);
         pv = lu_factor_regs<true>(a);
       }
       double r[NSP];
@@ -1461,15 +1470,16 @@ __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, doub
       for (int s = 0; s < NSP; s++) {
         double acc = 0.0;
 #pragma unroll
-        for (int j = 0; j < st; j++) acc += o.A[st * MAXSTAGE + j] * F[j][s];
-        r[s] = yn[s] + h * acc;
+        for (int j = 0; j < st; j++) acc += o.A[st * MAXSTAGE + j] * Fl[((j + 1) * NSP + s) * 64];
+        r[s] = Fl[s * 64] + h * acc;
       }
       // the stage's Newton iterations; after max_iters or a growing correction, a setup at
       // the iterate and the iterations start again (up to max_setups times). One loop: the
       // nested form of the same control flow made this kernel spill ~200 VGPRs.
       int setups = 0, it = 0;
       for (;;) {
-        cell_rhs<true>(cc, c, Ts, dTs, z, o.rhs_scale, f);
+        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !fresh);
+        fresh = false;
         double d[NSP];
 #pragma unroll
         for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * f[s] - r[s]);
@@ -1483,14 +1493,16 @@ __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, doub
         delp = del;
         if (++it < o.max_iters && !diverging) continue;
         if (++setups > o.max_setups) { ok = false; break; }
-        cell_rhs<true>(cc, c, Ts, dTs, z, o.rhs_scale, f);   // temperature at the iterate
+        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f);   // temperature at the iterate
         cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a);
         pv = lu_factor_regs<true>(a);
+        fresh = true;
         crate = 1.0;
         it = 0;
       }
+      if (st + 1 < ADJ_MAXSTAGE)
 #pragma unroll
-      for (int s = 0; s < NSP; s++) F[st][s] = (z[s] - r[s]) * (1.0 / hg);
+        for (int s = 0; s < NSP; s++) Fl[((st + 1) * NSP + s) * 64] = (z[s] - r[s]) * (1.0 / hg);
       if (Ys)
 #pragma unroll
         for (int s = 0; s < NSP; s++) Ys[(long)(st * NSP + s) * n + i] = z[s];
@@ -1503,14 +1515,39 @@ __device__ bool cell_step(const ChemConst &cc, const CellIn &c, double &Ts, doub
 
 constexpr int ADJ_REC = NSP + 2;     // y, Ts, dTs
 
+// LDS of an adjoint block: the gamma tables, then scale and inv_scale of each group of 64 cells
+// ([20][64]), which every RHS reads, y_n and the stage derivatives but the last
+// ([10 ADJ_MAXSTAGE][64]). 63.5 KB for 64 cells, 156 KB for 256; a pair of waves adds 15 KB
+// (two pairs per CU).
+constexpr int ADJ_CELLS = (2 + ADJ_MAXSTAGE) * NSP * 64;
+
+__device__ inline CellIn adj_cell(const ChemPtrsD &p, const ChemConst &cc, long i, int group,
+                                  int part, double *lds) {
+  for (int e = threadIdx.x; e < 4 * TLEN; e += blockDim.x) lds[e] = cc.tab[G_GH2_1 * TLEN + e];
+  double *q = lds + 4 * TLEN + group * ADJ_CELLS + (threadIdx.x & 63);
+  if (part == 0) {
+#pragma unroll
+    for (int s = 0; s < NSP; s++) {
+      q[s * 64] = p.scale[NSP * i + s];
+      q[(NSP + s) * 64] = p.iscale[NSP * i + s];
+    }
+  }
+  __syncthreads();
+  return CellIn{q, q + NSP * 64, 64, CellAux{p.md[i], p.imd[i], p.cie[i], p.h2o[i]}};
+}
+
 __global__ void __launch_bounds__(256)
 chem_adjoint_forward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, int nsteps, int K,
-                     const int *order, double *y, double *ck, int *nfail) {
+                     const int *order, double *y, double *ck, double *Te, double *Ys, int *nfail) {
+  extern __shared__ double lds[];
   // thread u takes the u-th cell of the temperature order; scratch is indexed by u
-  const long u = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n) return;
+  const long u0 = (long)blockIdx.x * blockDim.x + threadIdx.x, u = min(u0, n - 1);
   const long i = order ? order[u] : u;
-  const CellIn c = load_cell(p, i);
+  const CellIn c = adj_cell(p, cc, i, threadIdx.x >> 6, 0, lds);
+  const GammaTabs gt = gamma_tabs(lds);
+  double *Fl = lds + 4 * TLEN + (threadIdx.x >> 6) * ADJ_CELLS + 2 * NSP * 64 + (threadIdx.x & 63);
+  if (u0 >= n) return;
+  const int last = (nsteps - 1) / K * K;       // first step of the last segment
   double Ts = p.Ts[i], dTs = p.dTs[i];
   double z[NSP];
 #pragma unroll
@@ -1524,7 +1561,9 @@ chem_adjoint_forward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, int
       rec[NSP * n + u] = Ts;
       rec[(NSP + 1) * n + u] = dTs;
     }
-    ok = cell_step(cc, c, Ts, dTs, o, h, z, nullptr, n, u) && ok;
+    double *Yst = st >= last ? Ys + (long)(st - last) * o.nstage * NSP * n : nullptr;
+    ok = cell_step(cc, gt, c, Ts, dTs, o, h, z, Fl, Yst, n, u) && ok;
+    if (Yst) Te[(long)(st - last) * n + u] = Ts;
   }
 #pragma unroll
   for (int s = 0; s < NSP; s++) y[NSP * i + s] = z[s];
@@ -1535,7 +1574,8 @@ chem_adjoint_forward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, int
 
 // M^T = (I - hg J)^T of one stage from the exact Jacobian rows at the scaled state Y
 // (temperature solved from the warm start T); also yb = h J^T w.
-__device__ inline void stage_adjoint_matrix(const ChemConst &cc, const CellIn &c, double T,
+__device__ inline void stage_adjoint_matrix(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
+                                            double T,
                                             const double (&Y)[NSP], double srhs, double h,
                                             double hg, const double (&w)[NSP],
                                             double (&Mt)[NSP][NSP], double (&yb)[NSP]) {
@@ -1544,7 +1584,7 @@ __device__ inline void stage_adjoint_matrix(const ChemConst &cc, const CellIn &c
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = Y[s] * c.s(s);
   double dT;
-  chem_temperature(cc, ya, T, dT);
+  chem_temperature(cc, gt, ya, T, dT);
   const bool clamped = !(T > cc.tmin && T < cc.tmax);
   ChemVjpPre P;                  // rates, gas-energy tangents, temperature path: once
   chem_vjp_prepare(cc, ya, T, clamped, c.ax, P);
@@ -1568,72 +1608,120 @@ __device__ inline void stage_adjoint_matrix(const ChemConst &cc, const CellIn &c
   for (int q = 0; q < NSP; q++) yb[q] = h * acc[q];
 }
 
-__global__ void __launch_bounds__(256)
+// One segment's steps from its checkpoint: stage values and end temperatures.
+__device__ inline void adj_recompute(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
+                                     const DirkDev &o, double h, int nst, double *Fl,
+                                     const double *rec, double *Te, double *Ys, long n, long u) {
+  double z[NSP];
+#pragma unroll
+  for (int s = 0; s < NSP; s++) z[s] = rec[s * n + u];
+  double Ts = rec[NSP * n + u], dTs = rec[(NSP + 1) * n + u];
+  for (int st = 0; st < nst; st++) {
+    (void)cell_step(cc, gt, c, Ts, dTs, o, h, z, Fl, Ys + (long)st * o.nstage * NSP * n, n, u);
+    Te[(long)st * n + u] = Ts;   // the warm start of the step's stage solves
+  }
+}
+
+// One segment's steps backwards. Nl: the nu_k of the stages but the first, as Fl.
+__device__ inline void adj_backward(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
+                                    const DirkDev &o, double h, int nst, double *Nl,
+                                    const double *Te, const double *Ys, long n, long u, double (&lam)[NSP]) {
+#pragma clang fp contract(on)
+  const int ns = o.nstage;
+  for (int st = nst - 1; st >= 0; st--) {
+    const double Ts = Te[(long)st * n + u];
+    const double *Yst = Ys + (long)st * ns * NSP * n;
+    double nu0[NSP];
+#pragma unroll
+    for (int k = ADJ_MAXSTAGE - 1; k >= 0; k--) {
+      if (k < ns) {
+        double w[NSP], Y[NSP];
+#pragma unroll
+        for (int s = 0; s < NSP; s++) {
+          double acc = dirk_coef(o, ns - 1, k) * lam[s];
+          if (ns - 1 == 0) acc = o.A[k] * lam[s];
+#pragma unroll
+          for (int m = k + 1; m < ADJ_MAXSTAGE; m++)
+            if (m < ns) acc += dirk_coef(o, m, k) * Nl[((m - 1) * NSP + s) * 64];
+          w[s] = acc;
+          Y[s] = Yst[(long)(k * NSP + s) * n + u];
+        }
+        double Mt[NSP][NSP], yb[NSP];
+        stage_adjoint_matrix(cc, gt, c, Ts, Y, o.rhs_scale, h, h * o.A[k * MAXSTAGE + k], w, Mt,
+                             yb);
+        const unsigned long long pv = lu_factor_regs<true>(Mt);
+        lu_solve_regs(Mt, pv, yb);
+#pragma unroll
+        for (int s = 0; s < NSP; s++) {
+          if (k == 0) nu0[s] = yb[s];
+          else Nl[((k - 1) * NSP + s) * 64] = yb[s];
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < ADJ_MAXSTAGE; k++)
+      if (k < ns)
+#pragma unroll
+        for (int s = 0; s < NSP; s++) lam[s] += k == 0 ? nu0[s] : Nl[((k - 1) * NSP + s) * 64];
+  }
+}
+
+// The last segment's stage values are there already (chem_adjoint_forward keeps them).
+// PIPE: two waves per 64 cells, one walking segment sg backwards while the other recomputes
+// segment sg-1 into the second half of Te and Ys (blocks of 128 threads).
+template <bool PIPE>
+__global__ void __launch_bounds__(PIPE ? 128 : 256)
 chem_adjoint_backward(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, int nsteps, int K,
                       const int *order, const double *ck, double *Te, double *Ys,
                       const double *lamT, double *lam0) {
-#pragma clang fp contract(on)
-  const long u = (long)blockIdx.x * blockDim.x + threadIdx.x;   // as in chem_adjoint_forward
-  if (u >= n) return;
+  extern __shared__ double lds[];
+  const int role = PIPE ? threadIdx.x >> 6 : 0;
+  const long u0 = PIPE ? (long)blockIdx.x * 64 + (threadIdx.x & 63)
+                       : (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long u = min(u0, n - 1);                   // as in chem_adjoint_forward
   const long i = order ? order[u] : u;
-  const CellIn c = load_cell(p, i);
+  const CellIn c = adj_cell(p, cc, i, PIPE ? 0 : threadIdx.x >> 6, role, lds);
+  const GammaTabs gt = gamma_tabs(lds);
+  double *Fl = lds + 4 * TLEN + (PIPE ? 0 : threadIdx.x >> 6) * ADJ_CELLS + 2 * NSP * 64 +
+               (threadIdx.x & 63);
+  double *Nl = PIPE ? lds + 4 * TLEN + ADJ_CELLS + (threadIdx.x & 63) : Fl;
+  if (!PIPE && u0 >= n) return;                    // (spare lanes of a pair stay for the barriers)
   double lam[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) lam[s] = lamT[NSP * i + s];
-  const int ns = o.nstage;
   const int nseg = (nsteps + K - 1) / K;
+  const auto steps_of = [&](int sg) { return min(K, nsteps - sg * K); };
+  const long half = (long)K * n, halfY = half * o.nstage * NSP;
   for (int sg = nseg - 1; sg >= 0; sg--) {
-    const int n0 = sg * K, n1 = n0 + K < nsteps ? n0 + K : nsteps;
-    const double *rec = ck + (long)sg * ADJ_REC * n;
-    {
-      double z[NSP];
-#pragma unroll
-      for (int s = 0; s < NSP; s++) z[s] = rec[s * n + u];
-      double Ts = rec[NSP * n + u], dTs = rec[(NSP + 1) * n + u];
-      for (int st = n0; st < n1; st++) {
-        (void)cell_step(cc, c, Ts, dTs, o, h, z, Ys + (long)(st - n0) * ns * NSP * n, n, u);
-        Te[(long)(st - n0) * n + u] = Ts;   // the warm start of the step's stage solves
+    if (PIPE) {
+      if (role == 0) {
+        if (sg > 0 && u0 < n)
+          adj_recompute(cc, gt, c, o, h, K, Fl, ck + (long)(sg - 1) * ADJ_REC * n,
+                        Te + ((sg - 1) & 1) * half, Ys + ((sg - 1) & 1) * halfY, n, u);
+      } else if (u0 < n) {
+        adj_backward(cc, gt, c, o, h, steps_of(sg), Nl, Te + (sg & 1) * half, Ys + (sg & 1) * halfY,
+                     n, u, lam);
       }
-    }
-    for (int st = n1 - 1; st >= n0; st--) {
-      const double Ts = Te[(long)(st - n0) * n + u];
-      const double *Yst = Ys + (long)(st - n0) * ns * NSP * n;
-      double nu[ADJ_MAXSTAGE][NSP];
-#pragma unroll
-      for (int k = 0; k < ADJ_MAXSTAGE; k++)
-#pragma unroll
-        for (int s = 0; s < NSP; s++) nu[k][s] = 0.0;
-#pragma unroll
-      for (int k = ADJ_MAXSTAGE - 1; k >= 0; k--) {
-        if (k < ns) {
-          double w[NSP], Y[NSP];
-#pragma unroll
-          for (int s = 0; s < NSP; s++) {
-            double acc = dirk_coef(o, ns - 1, k) * lam[s];
-            if (ns - 1 == 0) acc = o.A[k] * lam[s];
-#pragma unroll
-            for (int m = k + 1; m < ADJ_MAXSTAGE; m++)
-              if (m < ns) acc += dirk_coef(o, m, k) * nu[m][s];
-            w[s] = acc;
-            Y[s] = Yst[(long)(k * NSP + s) * n + u];
-          }
-          double Mt[NSP][NSP], yb[NSP];
-          stage_adjoint_matrix(cc, c, Ts, Y, o.rhs_scale, h, h * o.A[k * MAXSTAGE + k], w, Mt, yb);
-          const unsigned long long pv = lu_factor_regs<true>(Mt);
-          lu_solve_regs(Mt, pv, yb);
-#pragma unroll
-          for (int s = 0; s < NSP; s++) nu[k][s] = yb[s];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < ADJ_MAXSTAGE; k++)
-        if (k < ns)
-#pragma unroll
-          for (int s = 0; s < NSP; s++) lam[s] += nu[k][s];
+      __syncthreads();
+    } else {
+      if (sg < nseg - 1)
+        adj_recompute(cc, gt, c, o, h, K, Fl, ck + (long)sg * ADJ_REC * n, Te, Ys, n, u);
+      adj_backward(cc, gt, c, o, h, steps_of(sg), Nl, Te, Ys, n, u, lam);
     }
   }
+  if ((!PIPE || role == 1) && u0 < n)
 #pragma unroll
-  for (int s = 0; s < NSP; s++) lam0[NSP * i + s] = lam[s];
+    for (int s = 0; s < NSP; s++) lam0[NSP * i + s] = lam[s];
+}
+
+// Pairs of waves where the cells fill at most half of the SIMDs and there is something to
+// recompute; the second set of stage values stays below 4 GiB.
+static bool adj_pipe(long n, int nsteps, int K, int nstage) {
+  int dev = 0, ncu = 256;
+  if (hipGetDevice(&dev) == hipSuccess)
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  return (n + 63) / 64 <= 2L * ncu && nsteps > K &&
+         (double)n * K * (nstage * NSP + 1) * sizeof(double) < 4.0 * (1 << 30);
 }
 
 // Scratch: checkpoints | end temperatures | stage values | the cell order (order, keys,
@@ -1647,16 +1735,18 @@ static size_t adj_order_doubles(long n) {
 
 size_t chem_adjoint_scratch_doubles(long n, int nsteps, int K, int nstage) {
   const long nckpt = (nsteps + K - 1) / K;
-  return (size_t)n * (nckpt * ADJ_REC + (long)K * (nstage * NSP + 1)) + adj_order_doubles(n);
+  const long sets = adj_pipe(n, nsteps, K, nstage) ? 2 : 1;
+  return (size_t)n * (nckpt * ADJ_REC + sets * K * (nstage * NSP + 1)) + adj_order_doubles(n);
 }
 
 int chem_adjoint_run(ChemState &s, const DirkDev &o, double h, int nsteps, int K, double *y,
                      const double *lamT, double *lam0, double *scratch, hipStream_t st,
                      int *host_fail) {
   const long n = s.n;
-  const unsigned nbk = (unsigned)((n + 255) / 256);
   const long nckpt = (nsteps + K - 1) / K;
-  double *ck = scratch, *Te = ck + nckpt * ADJ_REC * n, *Ys = Te + (long)K * n;
+  const bool pipe = adj_pipe(n, nsteps, K, o.nstage);
+  const long sets = pipe ? 2 : 1, keep = pipe ? (nckpt - 1) & 1 : 0;   // where the last segment lies
+  double *ck = scratch, *Te = ck + nckpt * ADJ_REC * n, *Ys = Te + sets * K * n;
   const ChemPtrsD p = ptrs_d(s);
   int *nfail = s.counters;
   hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, st, 1L, nfail, 0);
@@ -1664,7 +1754,7 @@ int chem_adjoint_run(ChemState &s, const DirkDev &o, double h, int nsteps, int K
   // cells of a wave take similar Newton paths; kept for the whole run
   int *order = nullptr;
   if (n >= TORD_MIN) {
-    const uintptr_t a = (uintptr_t)(Ys + (long)K * o.nstage * NSP * n);
+    const uintptr_t a = (uintptr_t)(Ys + sets * K * o.nstage * NSP * n);
     char *w = (char *)((a + 255) & ~(uintptr_t)255);
     order = (int *)w;
     unsigned short *key = (unsigned short *)(w + align256((size_t)n * sizeof(int)));
@@ -1678,10 +1768,21 @@ int chem_adjoint_run(ChemState &s, const DirkDev &o, double h, int nsteps, int K
     hipLaunchKernelGGL(tord_scatter, dim3((unsigned)((n + TORD_BLOCK - 1) / TORD_BLOCK)),
                        dim3(TORD_BLOCK), 0, st, n, (const unsigned short *)key, cnt, order);
   }
-  hipLaunchKernelGGL(chem_adjoint_forward, dim3(nbk), dim3(256), 0, st, n, s.cc, p, o, h, nsteps,
-                     K, (const int *)order, y, ck, nfail);
-  hipLaunchKernelGGL(chem_adjoint_backward, dim3(nbk), dim3(256), 0, st, n, s.cc, p, o, h,
-                     nsteps, K, (const int *)order, (const double *)ck, Te, Ys, lamT, lam0);
+  // one group of 64 cells per block while that spreads them over more CUs, else four
+  const int groups = pipe || (n + 63) / 64 <= 512 ? 1 : 4;
+  const unsigned nbk = (unsigned)((n + 64 * groups - 1) / (64 * groups));
+  const size_t shmem = sizeof(double) * (4 * TLEN + groups * ADJ_CELLS);
+  const size_t pairmem = sizeof(double) * (ADJ_MAXSTAGE - 1) * NSP * 64;   // Nl of a pair
+  hipLaunchKernelGGL(chem_adjoint_forward, dim3(nbk), dim3(64 * groups), shmem, st, n, s.cc, p, o, h,
+                     nsteps, K, (const int *)order, y, ck, Te + keep * K * n,
+                     Ys + keep * K * o.nstage * NSP * n, nfail);
+  if (pipe)
+    hipLaunchKernelGGL(chem_adjoint_backward<true>, dim3(nbk), dim3(128), shmem + pairmem, st, n, s.cc, p, o,
+                       h, nsteps, K, (const int *)order, (const double *)ck, Te, Ys, lamT, lam0);
+  else
+    hipLaunchKernelGGL(chem_adjoint_backward<false>, dim3(nbk), dim3(64 * groups), shmem, st, n,
+                       s.cc, p, o, h, nsteps, K, (const int *)order, (const double *)ck, Te, Ys,
+                       lamT, lam0);
   if (hipGetLastError() != hipSuccess) return -1;
   if (hipMemcpyAsync(host_fail, nfail, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
