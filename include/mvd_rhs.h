@@ -390,8 +390,8 @@ int mvd_chem_dirk_tune(mvd_context *ctx, double h, const mvd_dirk_opts *o, const
 /* Set the batched kernel's launch shape by hand (what mvd_chem_dirk_tune chooses): block
  * threads per block (64, 128 or 256; blocks whose LDS would not fit a CU are split at
  * launch) and waves resident waves of the persistent grid (0: one per SIMD of the device).
- * Each wave takes chunks of up to 64 cells (as few turns per wave as that allows, of even
- * size), the first by its index and the rest from the work queue, so waves smaller than the
+ * Each wave takes chunks of up to 64 cells (as few turns per wave as that allows; full ones
+ * when the cells need few waves), the first by its index and the rest from the work queue, so waves smaller than the
  * number of 64-cell chunks exercises the queue. The results do not
  * depend on the shape. get_shape returns the shape the next launch uses (waves resolved). */
 int mvd_chem_dirk_set_shape(mvd_context *ctx, int block, int waves);
@@ -404,7 +404,9 @@ int mvd_chem_dirk_set_shape(mvd_context *ctx, int block, int waves);
  * three stages and 64 with four; for tables of more than four stages (and
  * explicit-first-stage tables, which this call does not see) 54, the stage derivatives
  * going to a device buffer of 80 * (nstage - 1) bytes per thread of the persistent grid
- * instead. Halves the block until it fits; 0 when not even one wave fits. */
+ * instead. Halves the block until it fits; 0 when not even one wave fits. (A launch of at
+ * most two waves per CU keeps more in LDS, with blocks of as many waves: the forcing, the
+ * stage derivatives and, at one wave per CU, the rate pairs of each cell's table bin.) */
 int mvd_chem_dirk_fit_block(int block, int nstage, long static_lds, long lds_limit);
 int mvd_chem_dirk_get_shape(mvd_context *ctx, int *block, int *waves);
 

@@ -19,7 +19,9 @@
 // Jacobian from y_n, whose RHS evaluation is also the first iteration's, re-setup after
 // max_iters) and share their arithmetic, so they agree with each other bitwise and with the
 // CPU oracle iteration for iteration.
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include "mvd_chem.hpp"
 #include "mvd_dirk.hpp"
 #include "../../include/mvd_rhs.h"
@@ -44,11 +46,48 @@ __device__ inline CellIn load_cell(const ChemPtrsD &p, long i) {
 // calculate_rhs_cvklu for one cell in scaled variables, times srhs; updates Ts/dTs. The
 // temperature solve reads the gamma tables from gt (global memory or an LDS copy).
 // With solve_t false, Ts/dTs already hold the solution at y and the solve is skipped.
-// PAIRS: the rates come from the bin-major pair table (same values).
-template <bool PAIRS = false>
+// PAIRS: the rates come from the bin-major pair table (same values), or, where the caller
+// keeps a RateBin, from the lane's copy of its bin.
+struct NoRateBin {
+  static constexpr bool on = false;
+};
+
+// The pairs of the table bin a lane's temperature lies in, copied to LDS: pair r at
+// row[64 r], bin -1 when none is held. From one Newton iteration to the next the bin (1.1%
+// of T wide) hardly ever changes, and a read back costs 46 conflict-free 16-byte LDS loads
+// instead of as many gathers of up to 64 lines each.
+struct RateBin {
+  static constexpr bool on = true;
+  double2 *row;
+  int bin;
+  __device__ void hold(const ChemConst &cc, int b) {
+    if (b == bin) return;
+    bin = b;
+    const double2 *src = cc.tabp + (long)b * NRATE;
+    constexpr int PART = NRATE / 2;
+    static_assert(2 * PART == NRATE, "two parts");
+    copy<0, PART>(src);
+    __asm__ volatile("" ::: "memory");                     // bounds the loads in flight
+    copy<PART, NRATE>(src);
+  }
+  template <int R0, int R1>
+  __device__ void copy(const double2 *src) {
+    double a[R1 - R0], b[R1 - R0];
+#pragma unroll
+    for (int r = R0; r < R1; r++) {
+      const double2 v = src[r];
+      a[r - R0] = v.x;
+      b[r - R0] = v.y;
+    }
+#pragma unroll
+    for (int r = R0; r < R1; r++) row[r * 64] = make_double2(a[r - R0], b[r - R0]);
+  }
+};
+
+template <bool PAIRS = false, class Bin>
 __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
                                 double &Ts, double &dTs, const double (&y)[NSP], double srhs,
-                                double (&f)[NSP], bool solve_t = true) {
+                                double (&f)[NSP], bool solve_t, Bin &rb) {
 #pragma clang fp contract(on)
   double ya[NSP];
 #pragma unroll
@@ -59,11 +98,16 @@ __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const 
   double k[NRATE];
 #pragma unroll
   for (int r = 0; r < NRATE; r++) k[r] = 0.0;
-  if (PAIRS) chem_rates_only_pairs<0, C_BREM>(cc, Ts, k);
+  double Tdef = 0.0;
+  if constexpr (Bin::on) {
+    rb.hold(cc, chem_locate(cc, chem_log(Ts), Tdef));
+    chem_rates_only_at<0, C_BREM, 64>(rb.row, Tdef, k);
+  } else if (PAIRS) chem_rates_only_pairs<0, C_BREM>(cc, Ts, k);
   else chem_rates_only_range<0, C_BREM>(cc, Ts, k);
   chem_rhs_species(ya, k, f);
   __asm__ volatile("" ::: "memory");
-  if (PAIRS) chem_rates_only_pairs<C_BREM, NRATE>(cc, Ts, k);
+  if constexpr (Bin::on) chem_rates_only_at<C_BREM, NRATE, 64>(rb.row, Tdef, k);
+  else if (PAIRS) chem_rates_only_pairs<C_BREM, NRATE>(cc, Ts, k);
   else chem_rates_only_range<C_BREM, NRATE>(cc, Ts, k);
   f[9] = chem_rhs_energy(ya, k, Ts, cc.z, c.ax);
 #pragma unroll
@@ -71,6 +115,14 @@ __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const 
   f[9] *= c.ax.inv_mdensity;
 #pragma unroll
   for (int s = 0; s < NSP; s++) f[s] *= srhs;
+}
+
+template <bool PAIRS = false>
+__device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
+                                double &Ts, double &dTs, const double (&y)[NSP], double srhs,
+                                double (&f)[NSP], bool solve_t = true) {
+  NoRateBin none;
+  cell_rhs<PAIRS>(cc, gt, c, Ts, dTs, y, srhs, f, solve_t, none);
 }
 
 template <bool PAIRS = false>
@@ -273,10 +325,12 @@ __device__ constexpr bool CHEM_JNZ[NSP][NSP] = {
 // temperature: the species rows (reaction tables), then the gas-energy row (cooling tables),
 // so that both groups of rates never occupy registers at once. The rates come from the
 // rate-major tables here: with the factors held in registers, the pair table's wider loads
-// cost the batched kernel spills, and it measured faster this way.
+// cost the batched kernel spills, and it measured faster this way. (Where the lane keeps its
+// bin's pairs in LDS they come from there; the RHS evaluation at this Ts has set it.)
+template <class Bin>
 __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, double Ts,
                                         double dTs, const double (&y)[NSP], double hg,
-                                        double srhs, double (&M)[NSP][NSP]) {
+                                        double srhs, double (&M)[NSP][NSP], const Bin &rb) {
 #pragma clang fp contract(on)
   double ya[NSP];
 #pragma unroll
@@ -285,7 +339,12 @@ __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, do
 #pragma unroll
   for (int r = 0; r < NRATE; r++) k[r] = dk[r] = 0.0;
   const double hs = hg * srhs;
-  chem_rates_range<0, C_BREM>(cc, Ts, k, dk);
+  double Tdef = 0.0, Tfactor = 0.0;
+  if constexpr (Bin::on) {
+    chem_locate(cc, chem_log(Ts), Tdef);
+    Tfactor = fast_rcp(Ts) * cc.idbin;
+    chem_rates_at<0, C_BREM, 64>(rb.row, Tdef, Tfactor, k, dk);
+  } else chem_rates_range<0, C_BREM>(cc, Ts, k, dk);
   chem_jac_species(ya, k, dk, dTs, M);
 #pragma unroll
   for (int r = 0; r < NSP - 1; r++) {
@@ -296,7 +355,8 @@ __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, do
       M[r][q] = CHEM_JNZ[r][q] ? eye - row * (M[r][q] * c.s(q)) : eye;
     }
   }
-  chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
+  if constexpr (Bin::on) chem_rates_at<C_BREM, NRATE, 64>(rb.row, Tdef, Tfactor, k, dk);
+  else chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
   chem_jac_energy(ya, k, dk, Ts, cc.z, dTs, c.ax, M);
   const double row = hs * c.is(NSP - 1);
 #pragma unroll
@@ -304,6 +364,12 @@ __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, do
     const double eye = NSP - 1 == q ? 1.0 : 0.0;
     M[NSP - 1][q] = CHEM_JNZ[NSP - 1][q] ? eye - row * (M[NSP - 1][q] * c.s(q)) : eye;
   }
+}
+
+__device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, double Ts,
+                                        double dTs, const double (&y)[NSP], double hg,
+                                        double srhs, double (&M)[NSP][NSP]) {
+  cell_matrix_regs(cc, c, Ts, dTs, y, hg, srhs, M, NoRateBin());
 }
 
 // Solve with the factors of lu_factor_regs<true> (reciprocal diagonal). The row exchanges
@@ -343,23 +409,37 @@ constexpr int FST_LDS_MAX = 4;
 __host__ __device__ inline bool dirk_wide(int nstage, bool esdirk) {
   return esdirk || nstage > FST_LDS_MAX;
 }
-__host__ __device__ inline int dirk_wave_words(int nstage, bool wide) {
-  return CELL_WORDS + NSP + (wide || nstage <= 3 ? 2 : nstage - 1) * NSP;
+// What else a launch keeps in LDS when its waves leave room (DirkMem):
+//   MEM_SHARED  nothing: four waves share a block;
+//   MEM_STAGES  the forcing and the wide tables' stage derivatives (after the work slots):
+//               at most two waves per CU;
+//   MEM_RATES   these and the rate pairs of each cell's table bin (RateBin): one wave per CU.
+enum DirkMem { MEM_SHARED = 0, MEM_STAGES, MEM_RATES };
+__host__ __device__ inline int dirk_slot_words(int nstage, bool wide) {
+  return (wide || nstage <= 3 ? 2 : nstage - 1) * NSP;
+}
+__host__ __device__ inline int dirk_wave_words(int nstage, bool wide, int mem = MEM_SHARED) {
+  return CELL_WORDS + NSP + dirk_slot_words(nstage, wide) +
+         (mem >= MEM_STAGES ? NSP + (wide ? (nstage - 1) * NSP : 0) : 0) +
+         (mem >= MEM_RATES ? 2 * NRATE : 0);
 }
 // dynamic LDS of the batched kernel for `wpb` waves per block
-inline size_t dirk_lds_bytes(int wpb, int nstage, bool wide) {
-  return sizeof(double) * ((size_t)4 * TLEN + (size_t)wpb * dirk_wave_words(nstage, wide) * 64);
+inline size_t dirk_lds_bytes(int wpb, int nstage, bool wide, int mem = MEM_SHARED) {
+  return sizeof(double) *
+         ((size_t)4 * TLEN + (size_t)wpb * dirk_wave_words(nstage, wide, mem) * 64);
 }
 
 // Threads per block of a batched launch asked for `block` threads: blocks whose LDS (the
 // dynamic part for their waves plus the kernel's static part) would exceed the per-block
 // limit are halved (fewer waves then share one copy of the gamma tables); 0 when not even
 // one wave fits.
-int dirk_fit_block(int block, int nstage, size_t static_lds, size_t limit, bool esdirk) {
-  const bool wide = dirk_wide(nstage, esdirk);
+static int fit_block(int block, int nstage, size_t static_lds, size_t limit, bool wide, int mem) {
   for (; block >= 64; block /= 2)
-    if (dirk_lds_bytes(block / 64, nstage, wide) + static_lds <= limit) return block;
+    if (dirk_lds_bytes(block / 64, nstage, wide, mem) + static_lds <= limit) return block;
   return 0;
+}
+int dirk_fit_block(int block, int nstage, size_t static_lds, size_t limit, bool esdirk) {
+  return fit_block(block, nstage, static_lds, limit, dirk_wide(nstage, esdirk), MEM_SHARED);
 }
 
 // FORCED: y' = s_rhs f(y) + force, force constant over the step ([cell][10], the forcing an
@@ -379,7 +459,8 @@ int dirk_fit_block(int block, int nstage, size_t static_lds, size_t limit, bool 
 // WIDE: tables with an explicit first stage (ESDIRK) or more than FST_LDS_MAX stages (the
 // stage derivatives then in the global buffer fglob); the other instantiations are the
 // plain SDIRK form, without that code.
-template <bool FORCED, bool SUBSTEP, bool WIDE>
+// MEM: what is kept in LDS beyond the cells' constants and work slots (DirkMem).
+template <bool FORCED, bool SUBSTEP, bool WIDE, int MEM>
 __global__ void __launch_bounds__(256)
 chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double *y,
                   const double *force, const int *order, const double2 *tdt, int *queue,
@@ -403,13 +484,25 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
   __syncthreads();
   const GammaTabs gt = gamma_tabs(lds);
   const int lane = threadIdx.x & 63;
-  double *const cst = lds + 4 * TLEN + (threadIdx.x >> 6) * (dirk_wave_words(o.nstage, WIDE) * 64);
+  double *const cst =
+      lds + 4 * TLEN + (threadIdx.x >> 6) * (dirk_wave_words(o.nstage, WIDE, MEM) * 64);
   double *const yst = cst + CELL_WORDS * 64 + lane;        // y_n[s] at s*64
   double *const slots = yst + NSP * 64;                    // work slot k, element s: (10 k + s)*64
   // F_j[s] at (j*10 + s) * fstr: in the work slots (fstr 64), or for the wide tables in the
   // global buffer (one column per thread of the grid)
-  const long fstr = WIDE ? (long)gridDim.x * blockDim.x : 64;
-  double *const Fst = WIDE ? fglob + (long)blockIdx.x * blockDim.x + threadIdx.x : slots;
+  // (or, MEM_STAGES, in LDS behind the forcing)
+  constexpr bool FLDS = MEM >= MEM_STAGES;
+  double *const frc = slots + dirk_slot_words(o.nstage, WIDE) * 64;      // forcing s at s*64
+  const long fstr = WIDE && !FLDS ? (long)gridDim.x * blockDim.x : 64;
+  double *const Fst = !WIDE ? slots : FLDS ? frc + NSP * 64
+                                          : fglob + (long)blockIdx.x * blockDim.x + threadIdx.x;
+  typename std::conditional<MEM >= MEM_RATES, RateBin, NoRateBin>::type rb;
+  if constexpr (MEM >= MEM_RATES) {
+    const int at = CELL_WORDS + NSP + dirk_slot_words(o.nstage, WIDE) + NSP +
+                   (WIDE ? (o.nstage - 1) * NSP : 0);
+    rb.row = reinterpret_cast<double2 *>(cst + at * 64) + lane;
+    rb.bin = -1;
+  }
   // The first chunk of each wave is its global wave index; later ones come from the queue
   // (which starts after them), each fetched while the previous chunk is being solved: lane
   // 0 issues the atomic after the chunk's prologue loads and the wave reads its result at
@@ -450,7 +543,14 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
       cst[(2 * NSP + 1) * 64 + lane] = p.imd[i];
       cst[(2 * NSP + 2) * 64 + lane] = p.cie[i];
       cst[(2 * NSP + 3) * 64 + lane] = p.h2o[i];
+      if (FORCED && FLDS) {
+#pragma unroll
+        for (int s = 0; s < NSP; s++) frc[s * 64] = force[NSP * i + s];
+      }
     }
+    auto forcing = [&](long i, int s) -> double {
+      return FLDS ? frc[s * 64] : force[NSP * i + s];
+    };
     // One loop, one RHS evaluation per pass. A pass is one Newton iteration of the cell's
     // stage; where a setup is due (at y_n, or after max_iters without convergence) the pass
     // forms and factors the matrix at the iterate between that evaluation and the update,
@@ -487,7 +587,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     // of z - hg f(z) - r; the forcing is then read at stage changes only.
 #pragma unroll
     for (int s = 0; s < NSP; s++)
-      slots[s * 64] = FORCED ? z[s] + hg * force[NSP * (long)cell + s] : z[s];
+      slots[s * 64] = FORCED ? z[s] + hg * forcing(cell, s) : z[s];
     for (;;) {
       // The lane offset and cell index are made opaque on every pass so that the per-lane
       // addresses of the cell's inputs are formed where they are used instead of being held
@@ -502,7 +602,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
                        CellAux{cl[(2 * NSP) * 64], cl[(2 * NSP + 1) * 64],
                                cl[(2 * NSP + 2) * 64], cl[(2 * NSP + 3) * 64]}};
         double f[NSP];
-        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !solved);
+        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !solved, rb);
         solved = false;
         if (WIDE && o.esdirk && st == 0) {
           // explicit first stage (ESDIRK): its value is y_n and F_0 = f(y_n), this pass's
@@ -510,7 +610,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
           // stage's first Newton iteration, with this f at its predictor y_n.
 #pragma unroll
           for (int s = 0; s < NSP; s++) {
-            const double fo = FORCED ? force[NSP * i + s] : 0.0;
+            const double fo = FORCED ? forcing(i, s) : 0.0;
             const double F0 = FORCED ? f[s] + fo : f[s];
             Fst[s * fstr] = F0;
             double a = 0.0;
@@ -534,7 +634,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
 #pragma unroll
             for (int s = 0; s < NSP; s++) ds[s * 64] = d[s];
           }
-          cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, lu);
+          cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, lu, rb);
           pv = lu_factor_regs<true>(lu);
           nsetup++;
           setup = false;
@@ -577,7 +677,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
                 hg = hs * o.gamma;
 #pragma unroll
                 for (int s = 0; s < NSP; s++)
-                  slots[s * 64] = FORCED ? z[s] + hg * force[NSP * i + s] : z[s];
+                  slots[s * 64] = FORCED ? z[s] + hg * forcing(i, s) : z[s];
                 rslot = 0;
                 st = 0;
                 it = 0;
@@ -609,7 +709,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
 #pragma unroll
         for (int s = 0; s < NSP; s++) {
           const double F = (z[s] - rold[s * 64]) * ihg;
-          Fst[((st - 1) * NSP + s) * fstr] = FORCED ? F + force[NSP * i + s] : F;
+          Fst[((st - 1) * NSP + s) * fstr] = FORCED ? F + forcing(i, s) : F;
         }
         double a[NSP];
 #pragma unroll
@@ -644,7 +744,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
 #pragma unroll
         for (int s = 0; s < NSP; s++) {
           double rs = yst[s * 64] + hs * a[s];             // the (sub)step start
-          if (FORCED) rs += hg * force[NSP * i + s];
+          if (FORCED) rs += hg * forcing(i, s);
           rnew[s * 64] = rs;
         }
         it = 0;
@@ -674,7 +774,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
 #pragma unroll
       for (int s = 0; s < NSP; s++) {
         yst[s * 64] = z[s];
-        slots[s * 64] = FORCED ? z[s] + hg * force[NSP * i + s] : z[s];
+        slots[s * 64] = FORCED ? z[s] + hg * forcing(i, s) : z[s];
       }
       rslot = 0;
       start = true;
@@ -1067,13 +1167,30 @@ tord_scatter(long n, const unsigned short *key, int *cnt, int *order) {
   if (i < n) order[(k ? pre[k - 1] : 0) + res[k] + r] = (int)i;
 }
 
+using DirkKernel = void (*)(long, ChemConst, ChemPtrsD, DirkDev, double, double *, const double *,
+                            const int *, const double2 *, int *, int *, int, double *, int);
+
+template <bool FORCED, bool SUBSTEP>
+static DirkKernel dirk_kernel(bool wide, int mem) {
+  if (wide)
+    return mem == MEM_RATES    ? chem_dirk_batched<FORCED, SUBSTEP, true, MEM_RATES>
+           : mem == MEM_STAGES ? chem_dirk_batched<FORCED, SUBSTEP, true, MEM_STAGES>
+                               : chem_dirk_batched<FORCED, SUBSTEP, true, MEM_SHARED>;
+  return mem == MEM_RATES ? chem_dirk_batched<FORCED, SUBSTEP, false, MEM_RATES>
+                          : chem_dirk_batched<FORCED, SUBSTEP, false, MEM_SHARED>;
+}
+
+static DirkKernel dirk_kernel(bool forced, bool sub, bool wide, int mem) {
+  if (forced) return sub ? dirk_kernel<true, true>(wide, mem) : dirk_kernel<true, false>(wide, mem);
+  return sub ? dirk_kernel<false, true>(wide, mem) : dirk_kernel<false, false>(wide, mem);
+}
+
 // Launch plan of one batched step: kernel variant, block after the LDS split, grid, and the
 // layout of its work buffer (per-block statistics rows | cell order | bucket totals and
 // running offsets | keys | temperatures at y_n).
 struct BatchedPlan {
-  void (*kern)(long, ChemConst, ChemPtrsD, DirkDev, double, double *, const double *,
-               const int *, const double2 *, int *, int *, int, double *, int);
-  int block, wpb, chunk;
+  DirkKernel kern;
+  int block, wpb, chunk, mem;
   long grid, nrow;
   bool sorted;
   size_t b_rows, b_ord, b_cnt, b_key, b_tdt, b_fst;
@@ -1081,44 +1198,54 @@ struct BatchedPlan {
 };
 
 static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, bool forced,
-                        BatchedPlan &p) {
+                        int nsteps, BatchedPlan &p) {
   if (n <= 0 || n > (1L << 30)) return -1;
   if (block != 64 && block != 128 && block != 256) return -1;
   if (o.nstage < 1 || o.nstage > MAXSTAGE) return -1;
   const bool sub = o.max_halvings > 0;
   const bool wide = dirk_wide(o.nstage, o.esdirk != 0);
-  if (wide)
-    p.kern = forced ? (sub ? chem_dirk_batched<true, true, true>
-                           : chem_dirk_batched<true, false, true>)
-                    : (sub ? chem_dirk_batched<false, true, true>
-                           : chem_dirk_batched<false, false, true>);
-  else
-    p.kern = forced ? (sub ? chem_dirk_batched<true, true, false>
-                           : chem_dirk_batched<true, false, false>)
-                    : (sub ? chem_dirk_batched<false, true, false>
-                           : chem_dirk_batched<false, false, false>);
+  // LDS by the number of waves: one or two per CU leave room for more than four do.
+  // 167 forced seven-stage steps of 4096 cells: 19.7 ms without, 17.0 (as many full waves),
+  // 13.5 with MEM_RATES; one multirate slow step of 32^3 cells 31.0 -> 23.5 ms with
+  // MEM_STAGES; one seven-stage step of 20000 cells 270 -> 192 us.
+  int dev = 0, lim = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return -1;
+  const long want = grid_waves > 0 ? grid_waves : 1;
+  const long full = std::min<long>(want, (n + 63) / 64);   // waves with every lane taken
+  p.mem = full <= ncu ? MEM_RATES : wide && full <= 2L * ncu ? MEM_STAGES : MEM_SHARED;
   // blocks whose LDS would not fit are split: the kernel's static LDS as compiled and the
   // device's per-block limit, both asked of the runtime
-  hipFuncAttributes fa{};
-  int dev = 0, lim = 0;
-  if (hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(p.kern)) != hipSuccess ||
-      hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-    return -1;
-  p.block = dirk_fit_block(block, o.nstage, fa.sharedSizeBytes, (size_t)lim, o.esdirk != 0);
-  if (p.block == 0) return -1;
+  for (;; p.mem = MEM_SHARED) {
+    p.kern = dirk_kernel(forced, sub, wide, p.mem);
+    hipFuncAttributes fa{};
+    if (hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(p.kern)) != hipSuccess) return -1;
+    p.block = fit_block(block, o.nstage, fa.sharedSizeBytes, (size_t)lim, wide, p.mem);
+    // (MEM_STAGES in one-wave blocks would leave every second wave waiting for a CU)
+    if (p.block != 0 && (p.mem != MEM_STAGES || p.block >= 128)) break;
+    if (p.mem == MEM_SHARED) return -1;
+  }
   p.wpb = p.block / 64;
-  // Cells per wave and turn: 32 to 64, spread evenly over the waves of the grid and the turns
-  // each of them takes, so that a batch that does not fill every lane of the device's waves
-  // leaves fewer cells waiting for a wave's slowest one (one multirate slow step of 32^3
-  // cells: 30.9 ms with 32 cells per wave, 32.4 with 64). Fewer than 32 cost more than they
-  // give, since then twice the CUs and their shared instruction caches run the same long
-  // code (167 forced seven-stage steps of 4096 cells: 36.4 ms with 4 cells per wave, 23.2
-  // with 16, 19.7 with 32, 19.3 with 64).
-  const long want = grid_waves > 0 ? grid_waves : 1;
-  const long turns = (n + 64 * want - 1) / (64 * want);
-  p.chunk = (int)((n + turns * want - 1) / (turns * want));
+  // Cells per wave and turn. Four waves share a block: 32 to 64, spread evenly over the waves
+  // of the grid and the turns each of them takes, so that a batch that does not fill every
+  // lane of the device's waves leaves fewer cells waiting for a wave's slowest one.
+  // With more LDS per wave: full waves. Two neighbouring CUs share an instruction cache, and
+  // waves that do run this long code 15% slower (4096 cells, 167 steps: 64 full waves 13.5 ms,
+  // 128 half full ones 16.0). From half as many full waves as there are CUs on they share it
+  // anyhow, and the cells are spread over one wave per CU (9000 cells, 40 forced SDIRK3
+  // steps: 141 waves 3.85 ms, 256 waves 3.53). A single step of few cells, whose waves pull
+  // their cells from memory for most of its time, takes 32 to a wave (1500 cells: 115 -> 111
+  // us; 3000: 119 -> 122).
+  const long spread = p.mem == MEM_SHARED                      ? want
+                      : p.mem == MEM_RATES && 2 * full > ncu   ? std::min<long>(want, ncu)
+                                                               : full;
+  const long turns = (n + 64 * spread - 1) / (64 * spread);
+  p.chunk = (int)((n + turns * spread - 1) / (turns * spread));
   if (p.chunk < 32) p.chunk = 32;
+  if (p.mem != MEM_SHARED && full == spread && full < want)
+    p.chunk = nsteps == 1 && n <= 32 * 64 ? 32 : 64;
   const long chunks = (n + p.chunk - 1) / p.chunk;
   const long waves = want < chunks ? want : chunks;
   p.grid = (waves + p.wpb - 1) / p.wpb;
@@ -1130,7 +1257,7 @@ static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, boo
   p.b_key = p.sorted ? align256((size_t)n * sizeof(unsigned short)) : 0;
   p.b_tdt = p.sorted ? align256((size_t)n * sizeof(double2)) : 0;
   // stage derivatives of tables too long for LDS: one column per thread of the grid
-  p.b_fst = wide
+  p.b_fst = wide && p.mem == MEM_SHARED
                 ? align256((size_t)p.grid * p.block * (o.nstage - 1) * NSP * sizeof(double))
                 : 0;
   return 0;
@@ -1162,7 +1289,7 @@ static int batched_enqueue(const BatchedPlan &p, ChemState &s, const DirkDev &o,
   }
   if (!(p.sorted && !reuse_order))   // (else cleared with the bucket counters above)
     hipLaunchKernelGGL(fill_int, dim3(1), dim3(64), 0, st, (long)(2 + NSTAT), counters, 0);
-  const unsigned lds = (unsigned)dirk_lds_bytes(p.wpb, o.nstage, dirk_wide(o.nstage, o.esdirk != 0));
+  const unsigned lds = (unsigned)dirk_lds_bytes(p.wpb, o.nstage, dirk_wide(o.nstage, o.esdirk != 0), p.mem);
   const bool sub = o.max_halvings > 0;
   double *fglob =
       p.b_fst ? (double *)(work + p.b_rows + p.b_ord + p.b_cnt + p.b_key + p.b_tdt) : nullptr;
@@ -1178,7 +1305,7 @@ int dirk_batched_launch(ChemState &s, const DirkDev &o, double h, double *y, hip
                         int nsteps) {
   if (nsteps < 1) return -1;
   BatchedPlan p;
-  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, p)) return -1;
+  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, nsteps, p)) return -1;
   const void *work0 = s.work;
   if (ensure_work(s, p.bytes())) return -1;
   if (s.work != work0) reuse_order = false;                // a new buffer holds no order
@@ -1228,7 +1355,7 @@ int dirk_batched_launch_noalloc(ChemState &s, const DirkDev &o, double h, double
   if (s.n > NOALLOC_MAX_CELLS) return MVD_BAD_ARGUMENT;
   if (dirk_wide(o.nstage, o.esdirk != 0)) return MVD_UNSUPPORTED;   // no room for its stage buffer
   BatchedPlan p;
-  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, p)) return -1;
+  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, 1, p)) return -1;
   if (p.nrow > NOALLOC_MAX_ROWS || p.bytes() > NOALLOC_WORK) return MVD_BAD_ARGUMENT;
   unsigned char *base = dirk_noalloc_scratch();
   if (!base) return -1;

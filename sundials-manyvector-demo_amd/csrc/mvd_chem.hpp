@@ -456,25 +456,25 @@ __device__ inline void chem_rates_pairs(const ChemConst &c, double T, double (&k
   }
 }
 
-// The same at a table position already known (row: the bin's pairs).
-template <int R0, int R1>
+// The same at a table position already known (row: the bin's pairs, STRIDE apart).
+template <int R0, int R1, int STRIDE = 1>
 __device__ inline void chem_rates_at(const double2 *row, double Tdef, double Tfactor,
                                      double (&k)[NRATE], double (&dk)[NRATE]) {
 #pragma clang fp contract(on)
 #pragma unroll
   for (int r = R0; r < R1; r++) {
-    const double2 a = row[r];
+    const double2 a = row[r * STRIDE];
     k[r] = a.x + Tdef * (a.y - a.x);
     dk[r] = (a.y - a.x) * Tfactor;
   }
 }
 
-template <int R0, int R1>
+template <int R0, int R1, int STRIDE = 1>
 __device__ inline void chem_rates_only_at(const double2 *row, double Tdef, double (&k)[NRATE]) {
 #pragma clang fp contract(on)
 #pragma unroll
   for (int r = R0; r < R1; r++) {
-    const double2 a = row[r];
+    const double2 a = row[r * STRIDE];
     k[r] = a.x + Tdef * (a.y - a.x);
   }
 }
