@@ -48,6 +48,7 @@ __device__ inline CellIn load_cell(const ChemPtrsD &p, long i) {
 // With solve_t false, Ts/dTs already hold the solution at y and the solve is skipped.
 // PAIRS: the rates come from the bin-major pair table (same values), or, where the caller
 // keeps a RateBin, from the lane's copy of its bin.
+constexpr int RATE_BATCH = 25;        // pairs per wait: each group of tables at once
 struct NoRateBin {
   static constexpr bool on = false;
 };
@@ -92,22 +93,26 @@ __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const 
   double ya[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = y[s] * c.s(s);
-  if (solve_t) chem_temperature(cc, gt, ya, Ts, dTs);
+  if (solve_t) chem_temperature<true>(cc, gt, ya, Ts, dTs);
   // species rows from the reaction tables, then the energy row from the cooling tables;
   // the fence keeps the two groups of table loads from being scheduled together
   double k[NRATE];
 #pragma unroll
   for (int r = 0; r < NRATE; r++) k[r] = 0.0;
   double Tdef = 0.0;
+  const double2 *pairs = nullptr;
   if constexpr (Bin::on) {
     rb.hold(cc, chem_locate(cc, chem_log(Ts), Tdef));
-    chem_rates_only_at<0, C_BREM, 64>(rb.row, Tdef, k);
-  } else if (PAIRS) chem_rates_only_pairs<0, C_BREM>(cc, Ts, k);
+    chem_rates_only_batch<0, C_BREM, 64, RATE_BATCH>(rb.row, Tdef, k);
+  } else if (PAIRS) {
+    pairs = cc.tabp + (long)chem_locate(cc, chem_log(Ts), Tdef) * NRATE;
+    chem_rates_only_batch<0, C_BREM, 1, RATE_BATCH>(pairs, Tdef, k);
+  }
   else chem_rates_only_range<0, C_BREM>(cc, Ts, k);
   chem_rhs_species(ya, k, f);
   __asm__ volatile("" ::: "memory");
-  if constexpr (Bin::on) chem_rates_only_at<C_BREM, NRATE, 64>(rb.row, Tdef, k);
-  else if (PAIRS) chem_rates_only_pairs<C_BREM, NRATE>(cc, Ts, k);
+  if constexpr (Bin::on) chem_rates_only_batch<C_BREM, NRATE, 64, RATE_BATCH>(rb.row, Tdef, k);
+  else if (PAIRS) chem_rates_only_batch<C_BREM, NRATE, 1, RATE_BATCH>(pairs, Tdef, k);
   else chem_rates_only_range<C_BREM, NRATE>(cc, Ts, k);
   f[9] = chem_rhs_energy(ya, k, Ts, cc.z, c.ax);
 #pragma unroll
@@ -548,8 +553,14 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
         for (int s = 0; s < NSP; s++) frc[s * 64] = force[NSP * i + s];
       }
     }
-    auto forcing = [&](long i, int s) -> double {
-      return FLDS ? frc[s * 64] : force[NSP * i + s];
+    // the cell's forcing (0 without) in registers. Every loop below that writes LDS has its
+    // LDS reads taken out in front of it: the compiler must keep reads behind writes that may
+    // overlap them, and one by one each pays the latency (a stage change: 3300 cycles, 10 of
+    // them in turn at two places).
+    auto forcing = [&](long i, double (&fo)[NSP]) {
+#pragma unroll
+      for (int s = 0; s < NSP; s++)
+        fo[s] = !FORCED ? 0.0 : FLDS ? frc[s * 64] : force[NSP * i + s];
     };
     // One loop, one RHS evaluation per pass. A pass is one Newton iteration of the cell's
     // stage; where a setup is due (at y_n, or after max_iters without convergence) the pass
@@ -585,9 +596,12 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     unsigned long long pv = 0;
     // With forcing, r holds the stage's right-hand side plus hg * force, the constant part
     // of z - hg f(z) - r; the forcing is then read at stage changes only.
+    {
+      double fo[NSP];
+      forcing(cell, fo);
 #pragma unroll
-    for (int s = 0; s < NSP; s++)
-      slots[s * 64] = FORCED ? z[s] + hg * forcing(cell, s) : z[s];
+      for (int s = 0; s < NSP; s++) slots[s * 64] = FORCED ? z[s] + hg * fo[s] : z[s];
+    }
     for (;;) {
       // The lane offset and cell index are made opaque on every pass so that the per-lane
       // addresses of the cell's inputs are formed where they are used instead of being held
@@ -608,15 +622,18 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
           // explicit first stage (ESDIRK): its value is y_n and F_0 = f(y_n), this pass's
           // RHS; the first implicit stage's r = y_n + hs a_10 F_0. The pass goes on as that
           // stage's first Newton iteration, with this f at its predictor y_n.
+          double fo[NSP], yn[NSP];
+          forcing(i, fo);
+#pragma unroll
+          for (int s = 0; s < NSP; s++) yn[s] = yst[s * 64];
 #pragma unroll
           for (int s = 0; s < NSP; s++) {
-            const double fo = FORCED ? forcing(i, s) : 0.0;
-            const double F0 = FORCED ? f[s] + fo : f[s];
+            const double F0 = FORCED ? f[s] + fo[s] : f[s];
             Fst[s * fstr] = F0;
             double a = 0.0;
             a += dirk_coef(o, 1, 0) * F0;
-            double rs = yst[s * 64] + hs * a;
-            if (FORCED) rs += hg * fo;
+            double rs = yn[s] + hs * a;
+            if (FORCED) rs += hg * fo[s];
             slots[s * 64] = rs;
           }
           st = 1;
@@ -675,9 +692,10 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
                 halv++;
                 hs = ldexp(h, -halv);
                 hg = hs * o.gamma;
+                double fo[NSP];
+                forcing(i, fo);
 #pragma unroll
-                for (int s = 0; s < NSP; s++)
-                  slots[s * 64] = FORCED ? z[s] + hg * forcing(i, s) : z[s];
+                for (int s = 0; s < NSP; s++) slots[s * 64] = FORCED ? z[s] + hg * fo[s] : z[s];
                 rslot = 0;
                 st = 0;
                 it = 0;
@@ -706,10 +724,19 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
         // (narrow: r_{st-1} and F_{st-1} share slot st - 1; the last stage's r takes slot 0)
         if (!WIDE) rslot = st + 1 < o.nstage ? st * NSP * 64 : 0;
         double *const rnew = slots + rslot;
+        double fo[NSP], yn[NSP];
+        forcing(i, fo);
+        {
+          double ro[NSP];
 #pragma unroll
-        for (int s = 0; s < NSP; s++) {
-          const double F = (z[s] - rold[s * 64]) * ihg;
-          Fst[((st - 1) * NSP + s) * fstr] = FORCED ? F + forcing(i, s) : F;
+          for (int s = 0; s < NSP; s++) ro[s] = rold[s * 64];
+#pragma unroll
+          for (int s = 0; s < NSP; s++) yn[s] = yst[s * 64];
+#pragma unroll
+          for (int s = 0; s < NSP; s++) {
+            const double F = (z[s] - ro[s]) * ihg;
+            Fst[((st - 1) * NSP + s) * fstr] = FORCED ? F + fo[s] : F;
+          }
         }
         double a[NSP];
 #pragma unroll
@@ -728,6 +755,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
             for (int s = 0; s < NSP; s++) u[s] = F0[s * fstr];
 #pragma unroll
             for (int s = 0; s < NSP; s++) v[s] = F1[s * fstr];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < NSP; s++) {
               a[s] += c0 * u[s];
@@ -743,8 +771,8 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
         }
 #pragma unroll
         for (int s = 0; s < NSP; s++) {
-          double rs = yst[s * 64] + hs * a[s];             // the (sub)step start
-          if (FORCED) rs += hg * forcing(i, s);
+          double rs = yn[s] + hs * a[s];                   // the (sub)step start
+          if (FORCED) rs += hg * fo[s];
           rnew[s * 64] = rs;
         }
         it = 0;
@@ -771,10 +799,12 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
       } else {
         setup = true;                                      // substep accepted: the next one
       }
+      double fo[NSP];
+      forcing(i, fo);
 #pragma unroll
       for (int s = 0; s < NSP; s++) {
         yst[s * 64] = z[s];
-        slots[s * 64] = FORCED ? z[s] + hg * forcing(i, s) : z[s];
+        slots[s * 64] = FORCED ? z[s] + hg * fo[s] : z[s];
       }
       rslot = 0;
       start = true;
@@ -1094,7 +1124,7 @@ tord_count(long n, ChemConst cc, ChemPtrsD p, const double *y, const double *for
     double ya[NSP], T = p.Ts[i], dT = p.dTs[i];
 #pragma unroll
     for (int s = 0; s < NSP; s++) ya[s] = y[NSP * i + s] * p.scale[NSP * i + s];
-    chem_temperature(cc, gamma_tabs(gl), ya, T, dT);
+    chem_temperature<true>(cc, gamma_tabs(gl), ya, T, dT);
     tdt[i] = make_double2(T, dT);
     double kr[NRATE], f[NSP];
 #pragma unroll
@@ -1207,7 +1237,8 @@ static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, boo
   // LDS by the number of waves: one or two per CU leave room for more than four do.
   // 167 forced seven-stage steps of 4096 cells: 19.7 ms without, 17.0 (as many full waves),
   // 13.5 with MEM_RATES; one multirate slow step of 32^3 cells 31.0 -> 23.5 ms with
-  // MEM_STAGES; one seven-stage step of 20000 cells 270 -> 192 us.
+  // MEM_STAGES; one seven-stage step of 20000 cells 270 -> 192 us. (Before loads were
+  // issued together and the temperature solve shortened: 11.7, 17.4 ms since.)
   int dev = 0, lim = 0, ncu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
