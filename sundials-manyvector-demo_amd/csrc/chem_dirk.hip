@@ -1609,71 +1609,126 @@ int chem_ls_solve(long n, const double *LU, const unsigned long long *piv, const
 // wave that recomputes ahead of the backward walk. 32^3 cells, 20 steps, K = 5: forward 1.02 ->
 // 0.79 ms, backward 2.43 -> 0.92 ms (1.05 with the nu_k in registers, which spilled).
 // ---------------------------------------------------------------------------------
-__device__ bool cell_step(const ChemConst &cc, const GammaTabs &gt, const CellIn &c, double &Ts,
-                          double &dTs, const DirkDev &o, double h, double (&y)[NSP], double *Fl,
-                          double *Ys, long n, long i) {
+
+// a_{row,col} of an adjoint table, both uniform in the wave (scalar selects; see dirk_coef)
+__device__ inline double adj_coef(const DirkDev &o, int row, int col) {
+  double v = 0.0;
+#pragma unroll
+  for (int r = 0; r < ADJ_MAXSTAGE; r++)
+#pragma unroll
+    for (int q = 0; q <= r; q++)
+      if (r == row && q == col) v = o.A[r * MAXSTAGE + q];
+  return v;
+}
+
+// One step of the lane's cell. Fl: y_n, then the stage derivatives but the last; a stage's
+// right-hand side r lies where its own F will (the last of four stages: where F_0 was, which
+// r has consumed), a step's first correction across the matrix set-up where F_1 will. One loop
+// over all stages and iterations with one RHS evaluation, one matrix and one solve in it, the
+// cells of a wave changing stage together (chem_dirk_batched): unrolled over the stages the
+// two adjoint kernels had 113 and 207 KB of code, and two CUs share 64 KB of instruction cache.
+__device__ inline bool cell_step(const ChemConst &cc, const GammaTabs &gt, const CellIn &c,
+                                 double &Ts, double &dTs, const DirkDev &o, double h,
+                                 double (&y)[NSP], double *Fl, double *Ys, long n, long i) {
 #pragma clang fp contract(on)
-  double z[NSP], f[NSP];
+  double z[NSP], a[NSP][NSP];
+  unsigned long long pv = 0;
 #pragma unroll
   for (int s = 0; s < NSP; s++) {
     z[s] = y[s];
     Fl[s * 64] = y[s];
+    Fl[(NSP + s) * 64] = y[s];                        // r of the first stage
   }
-  double a[NSP][NSP];
-  unsigned long long pv = 0;
-  cell_rhs<true>(cc, gt, c, Ts, dTs, y, o.rhs_scale, f);       // refresh Ts at y_n for J
-  bool ok = true, fresh = true;      // fresh: Ts and dTs are those of z
+  bool ok = true, solved = false, setup = true, start = true, busy = true;
   double crate = 1.0, delp = 0.0;                     // Newton rate estimate, last norm
+  int setups = 0, it = 0;
+#pragma unroll 1
+  for (int st = 0;;) {
+    const double hg = h * adj_coef(o, st, st);
+    double *const rs = Fl + (st + 1 < ADJ_MAXSTAGE ? st + 1 : 1) * NSP * 64;
+    if (busy) {
+      double f[NSP];
+      cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !solved);
+      solved = false;
+      double d[NSP];
 #pragma unroll
-  for (int st = 0; st < ADJ_MAXSTAGE; st++) {
-    if (st < o.nstage && ok) {
-      const double hg = h * o.A[st * MAXSTAGE + st];
-      if (st == 0) {
-        cell_matrix_regs(cc, c, Ts, dTs, y, hg, o.rhs_scale, a);
+      for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * f[s] - rs[s * 64]);
+      bool update = true;
+      if (setup) {
+        if (start) {
+#pragma unroll
+          for (int s = 0; s < NSP; s++) Fl[(2 * NSP + s) * 64] = d[s];
+        }
+        cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a);
         pv = lu_factor_regs<true>(a);
+        setup = false;
+        crate = 1.0;
+        it = 0;
+        if (start) {
+          __asm__ volatile("" ::: "memory");
+#pragma unroll
+          for (int s = 0; s < NSP; s++) {
+            d[s] = Fl[(2 * NSP + s) * 64];
+            z[s] = Fl[s * 64];
+          }
+        } else {
+          solved = true;                              // the next pass evaluates f here again
+          update = false;
+        }
+        start = false;
       }
-      double r[NSP];
-#pragma unroll
-      for (int s = 0; s < NSP; s++) {
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < st; j++) acc += o.A[st * MAXSTAGE + j] * Fl[((j + 1) * NSP + s) * 64];
-        r[s] = Fl[s * 64] + h * acc;
-      }
-      // the stage's Newton iterations; after max_iters or a growing correction, a setup at
-      // the iterate and the iterations start again (up to max_setups times). One loop: the
-      // nested form of the same control flow made this kernel spill ~200 VGPRs.
-      int setups = 0, it = 0;
-      for (;;) {
-        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f, !fresh);
-        fresh = false;
-        double d[NSP];
-#pragma unroll
-        for (int s = 0; s < NSP; s++) d[s] = -(z[s] - hg * f[s] - r[s]);
+      if (update) {
         lu_solve_regs(a, pv, d);
 #pragma unroll
         for (int s = 0; s < NSP; s++) z[s] += d[s];
         const double del = wrms_norm(d, z, o.rtol, o.atol);
         if (it > 0) crate = conv_rate(crate, del, delp);
-        if (conv_ok(crate, del, o.ntol)) break;
         const bool diverging = it > 0 && conv_diverging(del, delp);
         delp = del;
-        if (++it < o.max_iters && !diverging) continue;
-        if (++setups > o.max_setups) { ok = false; break; }
-        cell_rhs<true>(cc, gt, c, Ts, dTs, z, o.rhs_scale, f);   // temperature at the iterate
-        cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a);
-        pv = lu_factor_regs<true>(a);
-        fresh = true;
-        crate = 1.0;
-        it = 0;
+        it++;
+        if (conv_ok(crate, del, o.ntol)) {
+          busy = false;
+        } else if (it >= o.max_iters || diverging) {
+          setup = true;
+          if (++setups > o.max_setups) ok = busy = false;
+        }
       }
+    }
+    if (__builtin_amdgcn_ballot_w64(busy) != 0) continue;   // some cell of the wave iterates
+    // all cells' stages ended. (One that failed, here or at an earlier stage of the step, keeps
+    // its iterate and stops: its later stages store nothing.)
+    if (setups >= 0) {
+      double r[NSP];
+#pragma unroll
+      for (int s = 0; s < NSP; s++) r[s] = rs[s * 64];
+      const double ihg = 1.0 / hg;
       if (st + 1 < ADJ_MAXSTAGE)
 #pragma unroll
-        for (int s = 0; s < NSP; s++) Fl[((st + 1) * NSP + s) * 64] = (z[s] - r[s]) * (1.0 / hg);
+        for (int s = 0; s < NSP; s++) Fl[((st + 1) * NSP + s) * 64] = (z[s] - r[s]) * ihg;
       if (Ys)
 #pragma unroll
         for (int s = 0; s < NSP; s++) Ys[(long)(st * NSP + s) * n + i] = z[s];
     }
+    if (++st >= o.nstage) break;
+    busy = ok;
+    setups = ok ? 0 : -1;
+    it = 0;
+    if (__builtin_amdgcn_ballot_w64(busy) == 0) break;
+    double acc[NSP], yn[NSP];
+#pragma unroll
+    for (int s = 0; s < NSP; s++) acc[s] = 0.0;
+#pragma unroll
+    for (int j = 0; j < ADJ_MAXSTAGE - 1; j++)
+      if (j < st) {
+        const double aj = adj_coef(o, st, j);
+#pragma unroll
+        for (int s = 0; s < NSP; s++) acc[s] += aj * Fl[((j + 1) * NSP + s) * 64];
+      }
+#pragma unroll
+    for (int s = 0; s < NSP; s++) yn[s] = Fl[s * 64];
+    double *const rn = Fl + (st + 1 < ADJ_MAXSTAGE ? st + 1 : 1) * NSP * 64;
+#pragma unroll
+    for (int s = 0; s < NSP; s++) rn[s * 64] = yn[s] + h * acc[s];
   }
 #pragma unroll
   for (int s = 0; s < NSP; s++) y[s] = z[s];
@@ -1798,38 +1853,36 @@ __device__ inline void adj_backward(const ChemConst &cc, const GammaTabs &gt, co
   for (int st = nst - 1; st >= 0; st--) {
     const double Ts = Te[(long)st * n + u];
     const double *Yst = Ys + (long)st * ns * NSP * n;
-    double nu0[NSP];
+    double nu[NSP];                                   // of the stage at hand; nu_0 at the end
+#pragma unroll 1
+    for (int k = ns - 1; k >= 0; k--) {
+      double w[NSP], Y[NSP];
 #pragma unroll
-    for (int k = ADJ_MAXSTAGE - 1; k >= 0; k--) {
-      if (k < ns) {
-        double w[NSP], Y[NSP];
+      for (int s = 0; s < NSP; s++) Y[s] = Yst[(long)(k * NSP + s) * n + u];
+      const double bk = adj_coef(o, ns - 1, k);
 #pragma unroll
-        for (int s = 0; s < NSP; s++) {
-          double acc = dirk_coef(o, ns - 1, k) * lam[s];
-          if (ns - 1 == 0) acc = o.A[k] * lam[s];
+      for (int s = 0; s < NSP; s++) w[s] = bk * lam[s];
 #pragma unroll
-          for (int m = k + 1; m < ADJ_MAXSTAGE; m++)
-            if (m < ns) acc += dirk_coef(o, m, k) * Nl[((m - 1) * NSP + s) * 64];
-          w[s] = acc;
-          Y[s] = Yst[(long)(k * NSP + s) * n + u];
+      for (int m = 1; m < ADJ_MAXSTAGE; m++)
+        if (m > k && m < ns) {
+          const double am = adj_coef(o, m, k);
+#pragma unroll
+          for (int s = 0; s < NSP; s++) w[s] += am * Nl[((m - 1) * NSP + s) * 64];
         }
-        double Mt[NSP][NSP], yb[NSP];
-        stage_adjoint_matrix(cc, gt, c, Ts, Y, o.rhs_scale, h, h * o.A[k * MAXSTAGE + k], w, Mt,
-                             yb);
-        const unsigned long long pv = lu_factor_regs<true>(Mt);
-        lu_solve_regs(Mt, pv, yb);
+      double Mt[NSP][NSP];
+      stage_adjoint_matrix(cc, gt, c, Ts, Y, o.rhs_scale, h, h * adj_coef(o, k, k), w, Mt, nu);
+      const unsigned long long pv = lu_factor_regs<true>(Mt);
+      lu_solve_regs(Mt, pv, nu);
+      if (k > 0)
 #pragma unroll
-        for (int s = 0; s < NSP; s++) {
-          if (k == 0) nu0[s] = yb[s];
-          else Nl[((k - 1) * NSP + s) * 64] = yb[s];
-        }
-      }
+        for (int s = 0; s < NSP; s++) Nl[((k - 1) * NSP + s) * 64] = nu[s];
     }
 #pragma unroll
-    for (int k = 0; k < ADJ_MAXSTAGE; k++)
-      if (k < ns)
+    for (int s = 0; s < NSP; s++) lam[s] += nu[s];
+#pragma unroll 1
+    for (int k = 1; k < ns; k++)
 #pragma unroll
-        for (int s = 0; s < NSP; s++) lam[s] += k == 0 ? nu0[s] : Nl[((k - 1) * NSP + s) * 64];
+      for (int s = 0; s < NSP; s++) lam[s] += Nl[((k - 1) * NSP + s) * 64];
   }
 }
 
