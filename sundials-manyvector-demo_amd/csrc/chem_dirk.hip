@@ -50,7 +50,10 @@ __device__ inline CellIn load_cell(const ChemPtrsD &p, long i) {
 // keeps a RateBin, from the lane's copy of its bin.
 constexpr int RATE_BATCH = 25;        // pairs per wait: each group of tables at once
 struct NoRateBin {
-  static constexpr bool on = false;
+  static constexpr bool on = false, pairs = false;
+};
+struct PairTable : NoRateBin {         // the matrix, too, from the bin-major pairs
+  static constexpr bool pairs = true;
 };
 
 // The pairs of the table bin a lane's temperature lies in, copied to LDS: pair r at
@@ -58,7 +61,7 @@ struct NoRateBin {
 // of T wide) hardly ever changes, and a read back costs 46 conflict-free 16-byte LDS loads
 // instead of as many gathers of up to 64 lines each.
 struct RateBin {
-  static constexpr bool on = true;
+  static constexpr bool on = true, pairs = false;
   double2 *row;
   int bin;
   __device__ void hold(const ChemConst &cc, int b) {
@@ -333,7 +336,9 @@ __device__ constexpr bool CHEM_JNZ[NSP][NSP] = {
 // so that both groups of rates never occupy registers at once. The rates come from the
 // rate-major tables here: with the factors held in registers, the pair table's wider loads
 // cost the batched kernel spills, and it measured faster this way. (Where the lane keeps its
-// bin's pairs in LDS they come from there; the RHS evaluation at this Ts has set it.)
+// bin's pairs in LDS they come from there; the RHS evaluation at this Ts has set it. The adjoint
+// kernels take them from the pair table, loads issued together: 1.37 -> 1.33 ms for 32^3 cells
+// and 20 steps, while the batched kernel loses 1 to 2% that way.)
 template <class Bin>
 __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, double Ts,
                                         double dTs, const double (&y)[NSP], double hg,
@@ -347,10 +352,15 @@ __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, do
   for (int r = 0; r < NRATE; r++) k[r] = dk[r] = 0.0;
   const double hs = hg * srhs;
   double Tdef = 0.0, Tfactor = 0.0;
+  const double2 *pairs = nullptr;
   if constexpr (Bin::on) {
     chem_locate(cc, chem_log(Ts), Tdef);
     Tfactor = fast_rcp(Ts) * cc.idbin;
     chem_rates_at<0, C_BREM, 64>(rb.row, Tdef, Tfactor, k, dk);
+  } else if constexpr (Bin::pairs) {
+    pairs = cc.tabp + (long)chem_locate(cc, chem_log(Ts), Tdef) * NRATE;
+    Tfactor = fast_rcp(Ts) * cc.idbin;
+    chem_rates_batch<0, C_BREM, 1, RATE_BATCH>(pairs, Tdef, Tfactor, k, dk);
   } else chem_rates_range<0, C_BREM>(cc, Ts, k, dk);
   chem_jac_species(ya, k, dk, dTs, M);
 #pragma unroll
@@ -363,6 +373,8 @@ __device__ inline void cell_matrix_regs(const ChemConst &cc, const CellIn &c, do
     }
   }
   if constexpr (Bin::on) chem_rates_at<C_BREM, NRATE, 64>(rb.row, Tdef, Tfactor, k, dk);
+  else if constexpr (Bin::pairs)
+    chem_rates_batch<C_BREM, NRATE, 1, RATE_BATCH>(pairs, Tdef, Tfactor, k, dk);
   else chem_rates_range<C_BREM, NRATE>(cc, Ts, k, dk);
   chem_jac_energy(ya, k, dk, Ts, cc.z, dTs, c.ax, M);
   const double row = hs * c.is(NSP - 1);
@@ -1659,7 +1671,7 @@ __device__ inline bool cell_step(const ChemConst &cc, const GammaTabs &gt, const
 #pragma unroll
           for (int s = 0; s < NSP; s++) Fl[(2 * NSP + s) * 64] = d[s];
         }
-        cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a);
+        cell_matrix_regs(cc, c, Ts, dTs, z, hg, o.rhs_scale, a, PairTable());
         pv = lu_factor_regs<true>(a);
         setup = false;
         crate = 1.0;

@@ -538,6 +538,29 @@ __device__ inline void chem_rates_only_pairs(const ChemConst &c, double T, doubl
   }
 }
 
+// chem_rates_at, its loads issued together the same way.
+template <int R0, int R1, int STRIDE, int BATCH>
+__device__ inline void chem_rates_batch(const double2 *row, double Tdef, double Tfactor,
+                                        double (&k)[NRATE], double (&dk)[NRATE]) {
+#pragma clang fp contract(on)
+  constexpr int R = R0 + BATCH < R1 ? R0 + BATCH : R1;
+  double a[R - R0], b[R - R0];
+#pragma unroll
+  for (int r = R0; r < R; r++) {
+    const double2 v = row[r * STRIDE];
+    a[r - R0] = v.x;
+    b[r - R0] = v.y;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = R0; r < R; r++) {
+    const double w = b[r - R0] - a[r - R0];
+    k[r] = a[r - R0] + Tdef * w;
+    dk[r] = w * Tfactor;
+  }
+  if constexpr (R < R1) chem_rates_batch<R, R1, STRIDE, BATCH>(row, Tdef, Tfactor, k, dk);
+}
+
 struct CellAux {
   double mdensity, inv_mdensity, cie, h2o;
 };
@@ -802,8 +825,10 @@ __device__ inline void chem_vjp_path(const ChemConst &c, const double (&y)[NSP],
 __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NSP], double T,
                                         bool clamped, const CellAux &ax, ChemVjpPre &P) {
 #pragma clang fp contract(on)
-  double k[NRATE], dk[NRATE];
-  chem_rates_pairs<0, NRATE>(c, T, k, dk);
+  double k[NRATE], dk[NRATE], Tdef;
+  const int bn = chem_locate(c, chem_log(T), Tdef);
+  chem_rates_batch<0, NRATE, 1, NRATE / 2>(c.tabp + (long)bn * NRATE, Tdef,
+                                           fast_rcp(T) * c.idbin, k, dk);
 #pragma unroll
   for (int j = 0; j < NREACT; j++) {
     P.k[j] = k[j];
@@ -817,8 +842,6 @@ __device__ inline void chem_vjp_prepare(const ChemConst &c, const double (&y)[NS
 #pragma unroll
   for (int s = 0; s < NSP - 1; s++) P.dgdy[s] = 0.0;
   if (clamped) return;
-  double Tdef;
-  const int bn = chem_locate(c, chem_log(T), Tdef);
   chem_vjp_path(c, y, T, bn, Tdef, fast_rcp(T) * c.idbin, P);
 }
 
