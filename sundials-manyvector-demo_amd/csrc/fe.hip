@@ -647,7 +647,7 @@ fe_xyface_div(Grid g, Fields f, FieldsOut out, double idx, double idy, unsigned 
 }
 
 // ------------------------------------------------------------------------------------
-// one-launch fe() of small grids without tracers
+// one-launch fe() of small grids
 // ------------------------------------------------------------------------------------
 
 // fe() of a grid too small to fill the device is bound by latency: each launch costs its
@@ -674,6 +674,16 @@ struct BoxPoint {
   int lx, ly, lz, cell;
   double sa, sx, sy, sz;
   bool use, core, ox, oy, oz;
+  __device__ bool in_x() const { return lx >= 0 && lx < BX; }
+  __device__ bool in_y() const { return ly >= 0 && ly < BY; }
+  __device__ bool in_z() const { return lz >= 0 && lz < BZ; }
+  // on a line of the box along x, y, z, and its place in the staged field
+  __device__ bool on_x() const { return in_y() && in_z() && !oy && !oz; }
+  __device__ bool on_y() const { return in_x() && in_z() && !ox && !oz; }
+  __device__ bool on_z() const { return in_x() && in_y() && !ox && !oy; }
+  __device__ int at_x() const { return (ly + BY * lz) * BPX + lx + 3; }
+  __device__ int at_y() const { return BOFY + (lx + BX * lz) * BPY + ly + 3; }
+  __device__ int at_z() const { return BOFZ + (lx + BX * ly) * BPY + lz + 3; }
 };
 
 __device__ inline BoxPoint box_point(const Grid &g, int x0, int y0, int z0, int p) {
@@ -716,10 +726,15 @@ __device__ inline BoxPoint box_point(const Grid &g, int x0, int y0, int z0, int 
   return P;
 }
 
-template <int NT>
-__global__ void __launch_bounds__(512, 2)
+// With NC tracers (NT = 0) their faces follow, at most BTP tracers at a time: values of the
+// points loaded before the previous fields' divergence, staged over the dead points, one flux
+// per thread and tracer with the split factors kept from the fluid's face. ST and MODE as in
+// fe_zface_tracers.
+constexpr int BTP = 5;
+template <int NT, int NC = 0, int ST = NC, int MODE = TR_PLAIN>
+__global__ void __launch_bounds__(512, NC > 0 ? 1 : 2)
 fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, double idz,
-       unsigned *flag) {
+       unsigned *flag, FeSlow slow) {
   __shared__ double sh[PT_NF * BFS];
   const int t = threadIdx.x;
   const int nbx = (g.nx + BX - 1) / BX, nby = (g.ny + BY - 1) / BY;
@@ -770,20 +785,15 @@ fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, doub
       if (!(pr > 0.0)) bits |= 4u;
       if (bits) atomicOr(flag, bits);
     }
-    const bool inx = Q.lx >= 0 && Q.lx < BX, iny = Q.ly >= 0 && Q.ly < BY;
-    const bool inz = Q.lz >= 0 && Q.lz < BZ;
     const auto put = [&](int at, double un, double u1, double u2) {
       double *d = sh + at;
       d[PT_R * BFS] = pt[PT_R]; d[PT_U * BFS] = un; d[PT_V * BFS] = u1; d[PT_W * BFS] = u2;
       d[PT_P * BFS] = pt[PT_P]; d[PT_SR * BFS] = pt[PT_SR]; d[PT_C2 * BFS] = pt[PT_C2];
       d[PT_C * BFS] = pt[PT_C];
     };
-    if (iny && inz && !Q.oy && !Q.oz)
-      put((Q.ly + BY * Q.lz) * BPX + Q.lx + 3, pt[PT_U], pt[PT_V], pt[PT_W]);
-    if (inx && inz && !Q.ox && !Q.oz)
-      put(BOFY + (Q.lx + BX * Q.lz) * BPY + Q.ly + 3, pt[PT_V], pt[PT_U], pt[PT_W]);
-    if (inx && iny && !Q.ox && !Q.oy)
-      put(BOFZ + (Q.lx + BX * Q.ly) * BPY + Q.lz + 3, pt[PT_W], pt[PT_V], pt[PT_U]);
+    if (Q.on_x()) put(Q.at_x(), pt[PT_U], pt[PT_V], pt[PT_W]);
+    if (Q.on_y()) put(Q.at_y(), pt[PT_V], pt[PT_U], pt[PT_W]);
+    if (Q.on_z()) put(Q.at_z(), pt[PT_W], pt[PT_V], pt[PT_U]);
   }
   __syncthreads();
   // face t: lines of BX + 1, BY + 1, BZ + 1 faces
@@ -802,10 +812,28 @@ fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, doub
     at = BOFZ + line * BPY + f;
     ok = z0 + f <= g.nz && x0 + line % BX < g.nx && y0 + line / BX < g.ny;
   }
-  double F[5];
-  if (ok)
-    face_flux_lds<PT_U, PT_V, PT_W>(sh + at, BFS, 1, g.gamma, g.igm, face_alpha<PT_U>(sh + at, BFS, 1),
-                                    F);
+  double F[5], hp[NC > 0 ? 5 : 1], hm[NC > 0 ? 5 : 1];
+  if (ok) {
+    const double alpha = face_alpha<PT_U>(sh + at, BFS, 1);
+    face_flux_lds<PT_U, PT_V, PT_W>(sh + at, BFS, 1, g.gamma, g.igm, alpha, F);
+    if constexpr (NC > 0) {
+      double un[6];
+#pragma unroll
+      for (int l = 0; l < 6; l++) un[l] = sh[PT_U * BFS + at + l];
+      tracer_split(un, alpha, hp, hm);
+    }
+  }
+  // the first tracers' values, their latency under the fluid's divergence
+  constexpr int NPASS = NC > 0 ? (NC + BTP - 1) / BTP : 0, TP = NC > 0 ? (NC + NPASS - 1) / NPASS : 1;
+  double tv[NR][TP];
+  const auto load_tracers = [&](int v0) {
+#pragma unroll
+    for (int n = 0; n < NR; n++)
+#pragma unroll
+      for (int v = 0; v < TP; v++)
+        tv[n][v] = P[n].use && v0 + v < NC ? y.chem[(long)ST * P[n].cell + v0 + v] * P[n].sa : 0.0;
+  };
+  if constexpr (NC > 0) load_tracers(0);
   __syncthreads();                    // points dead: their LDS takes the fluxes [comp][face]
   if (ok) {
 #pragma unroll
@@ -822,8 +850,13 @@ fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, doub
     const double *Fy = sh + ay * BNF + BNFX + (lx + BX * lz) * (BY + 1) + ly;
     const double *Fz = sh + az * BNF + BNFX + BNFY + (lx + BX * ly) * (BZ + 1) + lz;
     const double dxy = (Fx[1] - Fx[0]) * idx + (Fy[1] - Fy[0]) * idy;
-    const double rate = 0.0 - (dxy + (Fz[1] - Fz[0]) * idz);
+    double rate = 0.0 - (dxy + (Fz[1] - Fz[0]) * idz);
     const int c = (x0 + lx) + g.nx * ((y0 + ly) + g.ny * (z0 + lz));
+    if (MODE != TR_PLAIN && a == 4) {
+      const long rec = (long)ST * c + NC;
+      out.chem[rec] = MODE == TR_SLOW_SCALED ? rate * slow.eunits / slow.scale[rec] : rate;
+      rate = 0.0;
+    }
     // (selected, not indexed: an index that is not constant would copy the arguments to
     // scratch memory)
     double *o = out.w[0];
@@ -839,7 +872,56 @@ fe_box(Grid g, Fields y, BoxStage s, FieldsOut out, double idx, double idy, doub
       s.y1[a * ncell + c] = v + s.blast * rate;
     }
   }
+  if constexpr (NC > 0) {
+#pragma unroll 1
+    for (int v0 = 0; v0 < NC; v0 += TP) {
+      __syncthreads();                // the previous fluxes are read
+#pragma unroll
+      for (int n = 0; n < NR; n++) {
+        const BoxPoint &Q = P[n];
+        if (!Q.use) continue;
+        const bool ox = Q.on_x(), oy = Q.on_y(), oz = Q.on_z();
+#pragma unroll
+        for (int v = 0; v < TP; v++) {
+          if (ox) sh[v * BFS + Q.at_x()] = tv[n][v];
+          if (oy) sh[v * BFS + Q.at_y()] = tv[n][v];
+          if (oz) sh[v * BFS + Q.at_z()] = tv[n][v];
+        }
+      }
+      __syncthreads();
+      double Ft[TP];
+      if (ok) {
+#pragma unroll
+        for (int v = 0; v < TP; v++) {
+          double cv[6];
+#pragma unroll
+          for (int l = 0; l < 6; l++) cv[l] = sh[v * BFS + at + l];
+          Ft[v] = tracer_face_flux(cv, hp, hm);
+        }
+      }
+      if (v0 + TP < NC) load_tracers(v0 + TP);
+      __syncthreads();                // the values are read
+      if (ok) {
+#pragma unroll
+        for (int v = 0; v < TP; v++) sh[v * BNF + t] = Ft[v];
+      }
+      __syncthreads();
+      for (int n = t; n < TP * BCELLS; n += 512) {
+        const int v = n / BCELLS, q = n % BCELLS;
+        const int lx = q % BX, ly = q / BX % BY, lz = q / (BX * BY);
+        if (v0 + v >= NC || x0 + lx >= g.nx || y0 + ly >= g.ny || z0 + lz >= g.nz) continue;
+        const double *Fx = sh + v * BNF + (ly + BY * lz) * (BX + 1) + lx;
+        const double *Fy = sh + v * BNF + BNFX + (lx + BX * lz) * (BY + 1) + ly;
+        const double *Fz = sh + v * BNF + BNFX + BNFY + (lx + BX * ly) * (BZ + 1) + lz;
+        const double dxy = (Fx[1] - Fx[0]) * idx + (Fy[1] - Fy[0]) * idy;
+        const double rate = 0.0 - (dxy + (Fz[1] - Fz[0]) * idz);
+        const long rec = (long)ST * ((x0 + lx) + g.nx * ((y0 + ly) + g.ny * (z0 + lz))) + v0 + v;
+        out.chem[rec] = MODE == TR_SLOW_SCALED ? rate / slow.scale[rec] : rate;
+      }
+    }
+  }
 }
+static_assert(BTP <= PT_NF, "tracer values over point fields");
 
 __global__ void reset_flag(unsigned *flag) { *flag = 0u; }
 
@@ -851,6 +933,11 @@ static inline unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) 
 
 constexpr int TILE_X = 16, TILE_F = 16;   // fe_zface_tracers' tile
 
+// the number of boxes
+static long fe_boxes(const Grid &g) {
+  return (long)((g.nx + BX - 1) / BX) * ((g.ny + BY - 1) / BY) * ((g.nz + BZ - 1) / BZ);
+}
+
 // NC tracers in records of ST doubles
 template <int NC, int ST = NC, int MODE = TR_PLAIN>
 static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
@@ -859,6 +946,11 @@ static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScrat
   unsigned *const flag = accum ? accum : s.flag;
   if (!accum) hipLaunchKernelGGL(reset_flag, dim3(1), dim3(1), 0, st, s.flag);
   KernelTimer &tm = s.timer;
+  if constexpr (NC > 0) if (!plain && !tm.on && fe_boxes(g) <= FE_BOX_TRACER_MAX) {
+    hipLaunchKernelGGL((fe_box<0, NC, ST, MODE>), dim3((unsigned)fe_boxes(g)), dim3(512), 0, st, g,
+                       f, BoxStage{}, o, 1.0 / g.dx, 1.0 / g.dy, 1.0 / g.dz, flag, slow);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+  }
   if constexpr (MODE == TR_PLAIN) if (plain) {
     tm.begin(PROF_PLAIN_FACES, st);
     hipLaunchKernelGGL(fe_plain_faces<NC>, dim3(nblocks(nxp * nyp * nzp, 256)), dim3(256), 0, st,
@@ -913,7 +1005,7 @@ bool fe_box_fits(const Grid &g) {
 
 int fe_box_launch(const Grid &g, const Fields &y, const BoxStage &bs, const FieldsOut &o,
                   hipStream_t st, unsigned *flag) {
-  const long nb = (long)((g.nx + BX - 1) / BX) * ((g.ny + BY - 1) / BY) * ((g.nz + BZ - 1) / BZ);
+  const long nb = fe_boxes(g);
   const auto kern = bs.nt == 0   ? fe_box<0>
                     : bs.nt == 1 ? fe_box<1>
                     : bs.nt == 2 ? fe_box<2>
@@ -921,7 +1013,7 @@ int fe_box_launch(const Grid &g, const Fields &y, const BoxStage &bs, const Fiel
                     : bs.nt == 4 ? fe_box<4>
                                  : fe_box<5>;
   hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), 0, st, g, y, bs, o, 1.0 / g.dx,
-                     1.0 / g.dy, 1.0 / g.dz, flag);
+                     1.0 / g.dy, 1.0 / g.dz, flag, FeSlow{});
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

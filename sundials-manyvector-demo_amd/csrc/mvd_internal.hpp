@@ -89,6 +89,10 @@ struct BoxStage {
 // kernels, 48^3 46.2 / 48.3, 56^3 54.8 / 55.8, 64^3 62.1 / 59.4 (its boxes recompute a fifth
 // of the faces and load every point five times).
 constexpr long FE_BOX_MAX = 50 * 50 * 50;
+// With tracers, the most boxes: two per CU. fe() of 32^3 cells (256 boxes) with four tracers 39.0
+// us against 49.6 with the three kernels, with ten 42.8 / 56.5 (fslow 47.8 / 61.8); 40^3 (500
+// boxes) with ten 56.8 / 68.5; 48^3 (864) with four 65.4 / 66.7, with ten 81.6 / 80.3.
+constexpr long FE_BOX_TRACER_MAX = 512;
 bool fe_box_fits(const Grid &g);
 int fe_box_launch(const Grid &g, const Fields &y, const BoxStage &bs, const FieldsOut &o,
                   hipStream_t st, unsigned *flag);
