@@ -531,15 +531,16 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
   }
   // The first chunk of each wave is its global wave index; later ones come from the queue
   // (which starts after them), each fetched while the previous chunk is being solved: lane
-  // 0 issues the atomic after the chunk's prologue loads and the wave reads its result at
-  // the end.
+  // 0 issues the atomic at the chunk's start and the wave reads its result at the end. (It
+  // stands in front of the cell's own values: a branch of one lane in their midst made the
+  // compiler save some of them, the cell's index among them, for that lane only.)
   const int nwaves = (int)(gridDim.x * (blockDim.x >> 6));
   int next = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * chunk;
   for (;;) {
     const int base = next;
     if ((long)base >= n) break;
     int q = 0;
-    if (SUBSTEP && lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
+    if (lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
     if (lane < chunk && (long)base + lane < n) {   // the other lanes idle to the chunk's end
     // the lane's cell: queue positions run over the cells in temperature order
     const int cell = order ? order[base + lane] : base + lane;
@@ -597,10 +598,6 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     // on alone and evaluated the RHS again after a setup: 4096 cells, 167 forced
     // seven-stage steps 72.4 -> 19.7 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
     // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included).
-    // the next chunk's queue position, requested once the cell's loads are in flight (lane
-    // 0 is active whenever the chunk is; the substepping variants request it at the chunk's
-    // start, which costs them fewer registers)
-    if (!SUBSTEP && lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
     // (the substepping variants, which hold more state, solve it again: skipping there
     // costs registers that are worth more than the solve)
     bool setup = true, solved = !SUBSTEP && tdt != nullptr;

@@ -53,3 +53,21 @@ def test_batch_equals_parts(mvd, torch_gpu, table, forced, n):
         c = slice(10 * a, 10 * b)
         part = run(mvd, torch, opts, y0[c], yp[c], force[c] if forced else None, h, nsteps)
         assert np.array_equal(part, whole[a:b]), (a, b)
+
+
+@pytest.mark.parametrize("table", ["ark437", "sdirk3"])
+@pytest.mark.parametrize("n", [20000, 8193, 4096, 130])
+def test_forced_steps_without_rejection(mvd, torch_gpu, table, n):
+    """Without step rejection (a kernel variant of its own) the same bits as with it, where no
+    step is rejected."""
+    torch = torch_gpu
+    print(f"[dirk memory, no rejection] {table} n={n}", flush=True)
+    h, nsteps = 50.0, 3
+    y0, _ = problems.chem_cells(n, seed=93)
+    rng = np.random.default_rng(94)
+    yp = 1.0 + 0.02 * rng.uniform(-1, 1, 10 * n)
+    force = rng.standard_normal(10 * n) * 0.02 / (nsteps * h)
+    got = [run(mvd, torch, getattr(mvd, table)(newton_tol=1e-2, max_iters=20, max_halvings=k),
+               y0, yp, force, h, nsteps) for k in (0, 6)]
+    assert np.isfinite(got[0]).all()
+    assert np.array_equal(got[0], got[1])
