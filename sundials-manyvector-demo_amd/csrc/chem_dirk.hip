@@ -597,7 +597,9 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     // the contracted arithmetic (mvd_chem.hpp) and the even chunks, against lanes that ran
     // on alone and evaluated the RHS again after a setup: 4096 cells, 167 forced
     // seven-stage steps 72.4 -> 19.7 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
-    // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included).
+    // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included). With what
+    // followed (DirkMem, loads issued together, the shorter temperature solve, the column-wise
+    // substitution): 10.8, 17.0 and 0.32 ms.
     // (the substepping variants, which hold more state, solve it again: skipping there
     // costs registers that are worth more than the solve)
     bool setup = true, solved = !SUBSTEP && tdt != nullptr;
@@ -1616,7 +1618,8 @@ int chem_ls_solve(long n, const double *LU, const unsigned long long *piv, const
 // taken out or handed to an idle SIMD: gamma tables, scales and stage derivatives in LDS, the last
 // segment kept by the forward run instead of recomputed, and for small batches a second
 // wave that recomputes ahead of the backward walk. 32^3 cells, 20 steps, K = 5: forward 1.02 ->
-// 0.79 ms, backward 2.43 -> 0.92 ms (1.05 with the nu_k in registers, which spilled).
+// 0.79 ms, backward 2.43 -> 0.92 ms (1.05 with the nu_k in registers, which spilled); with one
+// loop over the stages and the table loads issued together 0.57 and 0.68 ms.
 // ---------------------------------------------------------------------------------
 
 // a_{row,col} of an adjoint table, both uniform in the wave (scalar selects; see dirk_coef)
