@@ -68,6 +68,10 @@ int fe_common(mvd_context *ctx, const double *const *w, double *const *wdot, boo
   if (rc) return rc;
   rc = check_ptrs(ctx, (const double *const *)wdot);
   if (rc) return rc;
+  if (!wait) {
+    ctx->fe.async_used = true;
+    ctx->fe.flag_zero = false;
+  }
   rc = mvd::fe_launch(ctx->g, fields_of(ctx, w), fields_out(ctx, wdot), ctx->fe, ctx->stream,
                       plain);
   if (rc == -2) return MVD_UNSUPPORTED;
@@ -78,6 +82,7 @@ int fe_common(mvd_context *ctx, const double *const *w, double *const *wdot, boo
     return MVD_DEVICE_ERROR;
   if (!dev_ok(hipStreamSynchronize(ctx->stream))) return MVD_DEVICE_ERROR;
   ctx->fe.timer.collect();
+  ctx->fe.flag_zero = *ctx->host_flag == 0u && !ctx->fe.async_used;
   return (*ctx->host_flag != 0u) ? MVD_ILLEGAL_STATE : MVD_SUCCESS;
 }
 
@@ -302,6 +307,7 @@ int mvd_fslow(mvd_context *ctx, double t, double *const *w, double *const *wdot)
                              hipMemcpyDeviceToHost, ctx->stream)) ||
       !dev_ok(hipStreamSynchronize(ctx->stream)))
     return MVD_DEVICE_ERROR;
+  ctx->fe.flag_zero = *ctx->host_flag == 0u && !ctx->fe.async_used;
   return (*ctx->host_flag != 0u) ? MVD_ILLEGAL_STATE : MVD_SUCCESS;
 }
 

@@ -52,6 +52,10 @@ struct KernelTimer {
 struct FeScratch {
   double *Fx = nullptr, *Fy = nullptr, *Fz = nullptr;   // face fluxes, [component][face]
   unsigned *flag = nullptr;                             // legal-state bits of the last call
+  // The flag is known to be zero: the last call waited for its kernels and read it so. Never
+  // again once fe() has been queued without waiting (async_used): such a call may sit in a
+  // graph that writes the flag whenever it is replayed.
+  bool flag_zero = false, async_used = false;
   double *red = nullptr;                                // reduction partials
   long red_len = 0;
   KernelTimer timer;
