@@ -96,7 +96,7 @@ __device__ inline void cell_rhs(const ChemConst &cc, const GammaTabs &gt, const 
   double ya[NSP];
 #pragma unroll
   for (int s = 0; s < NSP; s++) ya[s] = y[s] * c.s(s);
-  if (solve_t) chem_temperature<true>(cc, gt, ya, Ts, dTs);
+  if (solve_t) chem_temperature_near(cc, gt, ya, Ts, dTs);
   // species rows from the reaction tables, then the energy row from the cooling tables;
   // the fence keeps the two groups of table loads from being scheduled together
   double k[NRATE];
@@ -1144,7 +1144,7 @@ tord_count(long n, ChemConst cc, ChemPtrsD p, const double *y, const double *for
     double ya[NSP], T = p.Ts[i], dT = p.dTs[i];
 #pragma unroll
     for (int s = 0; s < NSP; s++) ya[s] = y[NSP * i + s] * p.scale[NSP * i + s];
-    chem_temperature<true>(cc, gamma_tabs(gl), ya, T, dT);
+    chem_temperature_near(cc, gamma_tabs(gl), ya, T, dT);
     tdt[i] = make_double2(T, dT);
     double kr[NRATE], f[NSP];
 #pragma unroll

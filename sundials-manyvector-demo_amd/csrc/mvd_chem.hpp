@@ -279,35 +279,57 @@ __device__ inline double temperature_density(const double (&y)[NSP]) {
          4.0026020000000004 * y[7];
 }
 
-// One Newton step of the temperature solve from the input T (kdm = kb / (density * mH)):
-// returns the next iterate and sets dge_dT at T (raja_primordial_network.cpp:943-990).
-__device__ inline double temperature_step(const ChemConst &c, const GammaTabs &gt,
-                                          const double (&y)[NSP], double kdm, double nmono,
-                                          double T, double &dge_dT, double &Tdef) {
-#pragma clang fp contract(on)
-  const int b = chem_locate(c, chem_log(T), Tdef);
-  const double g2a = gt.g2[b], g2b = gt.g2[b + 1], dg2a = gt.dg2[b], dg2b = gt.dg2[b + 1];
-  const double g1a = gt.g1[b], g1b = gt.g1[b + 1], dg1a = gt.dg1[b], dg1b = gt.dg1[b + 1];
+// The gamma tables' values at both nodes of a bin.
+struct GammaBin {
+  double g2a, g2b, dg2a, dg2b, g1a, g1b, dg1a, dg1b;
+};
+
+__device__ inline GammaBin gamma_bin(const GammaTabs &gt, int b) {
+  const GammaBin v{gt.g2[b], gt.g2[b + 1], gt.dg2[b], gt.dg2[b + 1],
+                   gt.g1[b], gt.g1[b + 1], gt.dg1[b], gt.dg1[b + 1]};
   __builtin_amdgcn_sched_barrier(0);                       // all eight loads under one wait
-  const double gH2_2 = g2a + Tdef * (g2b - g2a);
-  const double dgH2_2 = dg2a + Tdef * (dg2b - dg2a);
-  const double gH2_1 = g1a + Tdef * (g1b - g1a);
-  const double dgH2_1 = dg1a + Tdef * (dg1b - dg1a);
+  return v;
+}
+
+// The energy equation at T, Tdef bins above the bin's lower node (kdm = kb / (density * mH)):
+// knum = kb nsum / (density * mH), dge_dT the reference's slope (from the tables of dgamma/dT),
+// slope = d(T knum)/dT of the interpolated energy itself, whose gammas are linear in log T, and
+// curve what with them gives d(dge_dT)/dT = (slope - knum) / T - curve.
+struct EnergyAt {
+  double knum, dge_dT, slope, curve;
+};
+
+__device__ inline EnergyAt energy_at(const ChemConst &c, const GammaBin &v,
+                                     const double (&y)[NSP], double kdm, double nmono, double T,
+                                     double Tdef) {
+#pragma clang fp contract(on)
+  const double d2 = v.g2b - v.g2a, d1 = v.g1b - v.g1a;
+  const double gH2_2 = v.g2a + Tdef * d2;
+  const double dgH2_2 = v.dg2a + Tdef * (v.dg2b - v.dg2a);
+  const double gH2_1 = v.g1a + Tdef * d1;
+  const double dgH2_1 = v.dg1a + Tdef * (v.dg1b - v.dg1a);
   const double g1 = fast_rcp(gH2_1 - 1.0);
   const double g2 = fast_rcp(gH2_2 - 1.0);
   const double a1 = y[0] * g1, a2 = y[1] * g2;
-  const double knum = kdm * (a1 + a2 + nmono);             // kb nsum / dm
-  const double slope = a1 * g1 * dgH2_1 + a2 * g2 * dgH2_2;
-  dge_dT = knum - T * kdm * slope;
-  const double dge = T * knum - y[9];
-  return T - fast_div(dge, dge_dT);
+  const double knum = kdm * (a1 + a2 + nmono);
+  const double b1 = a1 * g1, b2 = a2 * g2, S = kdm * (b1 * dgH2_1 + b2 * dgH2_2);
+  return EnergyAt{knum, knum - T * S, knum - kdm * c.idbin * (b1 * d1 + b2 * d2),
+                  S + kdm * c.idbin * (b1 * ((v.dg1b - v.dg1a) - 2.0 * g1 * d1 * dgH2_1) +
+                                       b2 * ((v.dg2b - v.dg2a) - 2.0 * g2 * d2 * dgH2_2))};
 }
 
+// One Newton step of the temperature solve from the input T: returns the next iterate and sets
+// dge_dT at T (raja_primordial_network.cpp:943-990).
 __device__ inline double temperature_step(const ChemConst &c, const GammaTabs &gt,
                                           const double (&y)[NSP], double kdm, double nmono,
                                           double T, double &dge_dT) {
+#pragma clang fp contract(on)
   double Tdef;
-  return temperature_step(c, gt, y, kdm, nmono, T, dge_dT, Tdef);
+  const int b = chem_locate(c, chem_log(T), Tdef);
+  const EnergyAt e = energy_at(c, gamma_bin(gt, b), y, kdm, nmono, T, Tdef);
+  dge_dT = e.dge_dT;
+  const double dge = T * e.knum - y[9];
+  return T - fast_div(dge, dge_dT);
 }
 
 // kb / (density * mH) and the monatomic species' share of nsum, constant over a solve
@@ -333,15 +355,6 @@ constexpr int TCYCLE = 4;
 // bitwise the values of all ten steps with fewer evaluations. Fixed points and 2-cycles are
 // the common exits of warm-started solves (2-4 steps); 3- and 4-cycles, which rounding
 // makes near some roots, otherwise run the full ten steps and hold up their whole wave.
-//
-// NEAR, for the Newton iterations of the implicit steps: a step shorter than 2^-30 T that stays
-// inside its table bin is the last one. Within a bin the energy is smooth (its curvature,
-// T e''/e', is of order one), so such a step ends at the square of that from the root, 1e-18 T,
-// and further ones only move it within rounding; the slope is that of a point 2^-30 T away,
-// which enters the Newton matrix alone. Across a bin's edge, where the slope jumps, the bitwise
-// rule stands. Warm starts took 3.8 steps per solve of a wave with the bitwise rule alone, and
-// the solve a third of a Newton iteration's time (3500 cycles; now 2050).
-template <bool NEAR = false>
 __device__ inline void chem_temperature(const ChemConst &c, const GammaTabs &gt,
                                         const double (&y)[NSP], double &Ts, double &dTs_ge) {
 #pragma clang fp contract(on)
@@ -353,14 +366,8 @@ __device__ inline void chem_temperature(const ChemConst &c, const GammaTabs &gt,
   for (int q = 0; q < TCYCLE; q++) xh[q] = dh[q] = 0.0;
   for (int it = 0; it < 10; it++) {
     const double T = Ts;
-    double Tdef;
-    Tnew = temperature_step(c, gt, y, kdm, nmono, T, dge_dT, Tdef);
+    Tnew = temperature_step(c, gt, y, kdm, nmono, T, dge_dT);
     Ts = Tnew;
-    if (NEAR) {
-      const double step = Tnew - T, end = Tdef + step * c.idbin * fast_rcp(T);
-      if (fabs(step) <= 0x1p-30 * T && fmin(Tdef, end) > 1e-6 && fmax(Tdef, end) < 1.0 - 1e-6)
-        break;
-    }
 #pragma unroll
     for (int q = TCYCLE - 1; q > 0; q--) {
       xh[q] = xh[q - 1];
@@ -393,6 +400,47 @@ __device__ inline void chem_temperature(const ChemConst &c, const GammaTabs &gt,
   if (Ts < c.tmin) Ts = c.tmin;
   else if (Ts > c.tmax) Ts = c.tmax;
   dTs_ge = fast_rcp(dge_dT);
+}
+
+// The same solve for the Newton iterations of the implicit steps, to the same few ulp of the
+// root in fewer steps. The reference's slope comes from the dgamma tables and is not the
+// derivative of the interpolated energy, so its steps close in on the root only linearly, by a
+// factor of 5e-5 to 1.3e-3 each. Steps shorter than 2^-6 T take the interpolated energy's own
+// slope instead; longer ones are the reference's, so that a start far away goes the same way.
+// Within a bin the energy is smooth (T e''/e' of order one) and Newton's convergence quadratic:
+// a step of at most 2^-30 T ends 1e-18 T from the root and is the last one. Across a bin's edge,
+// where the slope jumps by some 1e-3, steps go on until one is at most 2^-44 T. dTs_ge is the
+// inverse of the reference's slope at the temperature returned (carried from T over the last
+// step by its derivative). Relative errors on 4e5 random cells, largest and rms: T 8.1e-16 and
+// 1.60e-16, dTs_ge 9.0e-16 and 1.62e-16; the ten steps 7.6e-16 and 1.55e-16, 8.2e-16 and
+// 1.62e-16 (the reference's slope with the 2^-30 rule: 1.1e-12 and 2.9e-10 at most). Warm
+// starts 1% away take 2.9 steps, a wave's slowest lane 3.0 (4.0 with the bitwise rule).
+__device__ inline void chem_temperature_near(const ChemConst &c, const GammaTabs &gt,
+                                             const double (&y)[NSP], double &Ts,
+                                             double &dTs_ge) {
+#pragma clang fp contract(on)
+  double kdm, nmono, dge_dT = 0.0, change = 0.0;
+  temperature_consts(y, kdm, nmono);
+  for (int it = 0; it < 10; it++) {
+    const double T = Ts;
+    double Tdef;
+    const GammaBin v = gamma_bin(gt, chem_locate(c, chem_log(T), Tdef));
+    const EnergyAt e = energy_at(c, v, y, kdm, nmono, T, Tdef);
+    dge_dT = e.dge_dT;
+    const double dge = T * e.knum - y[9];
+    Ts = T - fast_div(dge, fabs(dge) <= 0x1p-6 * fabs(T * dge_dT) ? e.slope : dge_dT);
+    const double step = Ts - T, end = Tdef + step * c.idbin * fast_rcp(T);
+    const bool inside = fmin(Tdef, end) > 1e-6 && fmax(Tdef, end) < 1.0 - 1e-6;
+    if (fabs(step) <= (inside ? 0x1p-30 : 0x1p-44) * T) {
+      change = step * fast_rcp(T) * (e.slope - e.knum) - step * e.curve;
+      break;
+    }
+  }
+  if (Ts < c.tmin) Ts = c.tmin;
+  else if (Ts > c.tmax) Ts = c.tmax;
+  // 1 / (dge_dT + change), as fast_rcp with the change in its last sum
+  const double r = __builtin_amdgcn_rcp(dge_dT), e = fma(-dge_dT, r, 1.0);
+  dTs_ge = fma(r, fma(e, e, e) - change * r, r);
 }
 
 // The ten steps without the early exit (the self-check of the exit compares the two)
