@@ -468,6 +468,25 @@ int dirk_fit_block(int block, int nstage, size_t static_lds, size_t limit, bool 
   return fit_block(block, nstage, static_lds, limit, dirk_wide(nstage, esdirk), MEM_SHARED);
 }
 
+// queue += chunk by one lane of the wave; returns the old value to all of them. Called with all
+// lanes. The lane mask is set and restored within the statement, so that there is no branch and
+// no join for the compiler: `if (lane == 0) atomicAdd(...)` in the chunk loop once had the register
+// allocator save live values at the join, ahead of the mask's restoration, for lane 0 only. (64
+// lanes adding 0 to other words instead: one SDIRK3 step of 131072 cells 212 -> 276 us.)
+__device__ inline int queue_take(int *queue, int chunk) {
+  int old;
+  unsigned long long mask;
+  __asm__ volatile("s_mov_b64 %1, exec\n\t"
+                   "s_mov_b64 exec, 1\n\t"
+                   "global_atomic_add %0, %2, %3, %4 sc0\n\t"
+                   "s_waitcnt vmcnt(0)\n\t"
+                   "s_mov_b64 exec, %1"
+                   : "=&v"(old), "=&s"(mask)
+                   : "v"(0), "v"(chunk), "s"(queue)
+                   : "memory");
+  return __builtin_amdgcn_readfirstlane(old);
+}
+
 // FORCED: y' = s_rhs f(y) + force, force constant over the step ([cell][10], the forcing an
 // MRI method hands its fast stepper, multirate_chem_hydro_main.cpp:922-946).
 // SUBSTEP (o.max_halvings > 0): per-cell step rejection. When a cell's Newton budget runs
@@ -530,17 +549,12 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     rb.bin = -1;
   }
   // The first chunk of each wave is its global wave index; later ones come from the queue
-  // (which starts after them), each fetched while the previous chunk is being solved: lane
-  // 0 issues the atomic at the chunk's start and the wave reads its result at the end. (It
-  // stands in front of the cell's own values: a branch of one lane in their midst made the
-  // compiler save some of them, the cell's index among them, for that lane only.)
+  // (which starts after them), asked for when a chunk is done.
   const int nwaves = (int)(gridDim.x * (blockDim.x >> 6));
   int next = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * chunk;
   for (;;) {
     const int base = next;
     if ((long)base >= n) break;
-    int q = 0;
-    if (lane == 0) q = atomicAdd(queue, chunk) + nwaves * chunk;
     if (lane < chunk && (long)base + lane < n) {   // the other lanes idle to the chunk's end
     // the lane's cell: queue positions run over the cells in temperature order
     const int cell = order ? order[base + lane] : base + lane;
@@ -847,7 +861,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     if (nfail) atomicAdd(&bs[STAT_FAILED], nfail);
     atomicAdd(&bs[STAT_HIST + (nit < NHIST - 1 ? nit : NHIST - 1)], 1);
     }
-    next = __builtin_amdgcn_readfirstlane(__shfl(q, 0, 64));
+    next = queue_take(queue, chunk) + nwaves * chunk;
   }
   __syncthreads();
   // block statistics: one row per block; the last block to finish sums the rows into
