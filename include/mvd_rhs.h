@@ -191,8 +191,9 @@ int mvd_erk_evolve(mvd_context *ctx, const mvd_erk_table *tab, double t0, double
  * 1075-1194) over MAGMA's batched getrf/getrs. lsetup factors A = I - gamma*J per cell,
  * J in the mvd_chem_jac layout, with partial pivoting; it returns 0, or the number (> 0,
  * recoverable, as SUNLS_LUFACT_FAIL) of blocks with an exact zero pivot, after which
- * lsolve refuses (MVD_NOT_READY) until a successful lsetup. lsolve solves A x = b for the
- * chemistry subvector ([cell][10]; x may equal b). */
+ * lsolve refuses (MVD_NOT_READY) until a successful lsetup, as it does after an mvd_chem_setup
+ * with another number of cells. lsolve solves A x = b for the chemistry subvector ([cell][10];
+ * x may equal b). */
 int mvd_chem_lsetup(mvd_context *ctx, double gamma, const double *J);
 int mvd_chem_lsolve(mvd_context *ctx, const double *b, double *x);
 /* Setup of the block linear solver from the matrix itself, as SUNLinSolSetup(S, A) receives

@@ -22,11 +22,12 @@ struct mvd_context {
   int dirk_block = 256;   // batched DIRK launch shape (set by mvd_chem_dirk_tune)
   int dirk_waves = 0;     // resident waves of the persistent grid (0: one per SIMD)
   double *vjp_buf = nullptr;   // fe() VJP scratch of the tracers (first use)
-  // block linear solver of the chemistry subvector (allocated by the first lsetup)
+  // block linear solver of the chemistry subvector (allocated by lsetup): room for ls_cells
+  // cells (whole waves), factors of ls_ready cells (0: none)
   double *ls_lu = nullptr;
   unsigned long long *ls_piv = nullptr;
   int *ls_nsing = nullptr;
-  bool ls_ready = false;
+  long ls_cells = 0, ls_ready = 0;
   mvd::ErkState erk;                  // fixed-step ERK evolution (first use)
   double *adj_buf = nullptr;          // chemistry adjoint checkpoints and scratch
   size_t adj_len = 0;
@@ -45,6 +46,42 @@ int check_ptrs(const mvd_context *ctx, const double *const *w) {
     if (!w[v]) return MVD_BAD_ARGUMENT;
   if (ctx->g.nchem > 0 && !w[5]) return MVD_BAD_ARGUMENT;
   return MVD_SUCCESS;
+}
+
+void ls_free(mvd_context *c) {
+  (void)hipFree(c->ls_lu);
+  (void)hipFree(c->ls_piv);
+  (void)hipFree(c->ls_nsing);
+  c->ls_lu = nullptr;
+  c->ls_piv = nullptr;
+  c->ls_nsing = nullptr;
+  c->ls_cells = c->ls_ready = 0;
+}
+
+// Factors I - gamma J, or J itself (formed). The buffers grow with the chemistry: a later
+// mvd_chem_setup may have more cells than the one they were allocated for.
+int ls_setup(mvd_context *c, double gamma, const double *J, bool formed) {
+  const long n = c->chem.n, cells = (n + 63) / 64 * 64;
+  c->ls_ready = 0;
+  if (cells > c->ls_cells) {
+    ls_free(c);
+    if (!dev_ok(hipMalloc(&c->ls_lu, sizeof(double) * 100 * cells)) ||
+        !dev_ok(hipMalloc(&c->ls_piv, sizeof(unsigned long long) * cells)) ||
+        !dev_ok(hipMalloc(&c->ls_nsing, sizeof(int)))) {
+      ls_free(c);
+      return MVD_DEVICE_ERROR;
+    }
+    c->ls_cells = cells;
+  }
+  if (mvd::chem_ls_setup(n, gamma, J, c->ls_lu, c->ls_piv, c->ls_nsing, c->stream, formed))
+    return MVD_DEVICE_ERROR;
+  int nsing = 0;
+  if (!dev_ok(hipMemcpyAsync(&nsing, c->ls_nsing, sizeof(int), hipMemcpyDeviceToHost,
+                             c->stream)) ||
+      !dev_ok(hipStreamSynchronize(c->stream)))
+    return MVD_DEVICE_ERROR;
+  c->ls_ready = nsing == 0 ? n : 0;
+  return nsing;
 }
 
 mvd::Fields fields_of(const mvd_context *ctx, const double *const *w) {
@@ -162,9 +199,7 @@ void mvd_destroy(mvd_context *c) {
   if (c->vjp_buf) (void)hipFree(c->vjp_buf);
   if (c->pack_scratch) (void)hipFree(c->pack_scratch);
   mvd::imex_free(c->imex);
-  if (c->ls_lu) (void)hipFree(c->ls_lu);
-  if (c->ls_piv) (void)hipFree(c->ls_piv);
-  if (c->ls_nsing) (void)hipFree(c->ls_nsing);
+  ls_free(c);
   mvd::erk_free(c->erk);
   if (c->adj_buf) (void)hipFree(c->adj_buf);
   mvd::mri_free(c->mri);
@@ -399,50 +434,18 @@ int mvd_chem_lsetup(mvd_context *ctx, double gamma, const double *J) {
   if (!ctx || !J) return MVD_BAD_ARGUMENT;
   if (!ctx->chem.ready) return MVD_NOT_READY;
   if (!std::isfinite(gamma)) return MVD_BAD_ARGUMENT;
-  const long n = ctx->chem.n;
-  if (!ctx->ls_lu) {
-    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * ((n + 63) / 64 * 64))) ||
-        !dev_ok(hipMalloc(&ctx->ls_piv, sizeof(unsigned long long) * n)) ||
-        !dev_ok(hipMalloc(&ctx->ls_nsing, sizeof(int))))
-      return MVD_DEVICE_ERROR;
-  }
-  ctx->ls_ready = false;
-  if (mvd::chem_ls_setup(n, gamma, J, ctx->ls_lu, ctx->ls_piv, ctx->ls_nsing, ctx->stream))
-    return MVD_DEVICE_ERROR;
-  int nsing = 0;
-  if (!dev_ok(hipMemcpyAsync(&nsing, ctx->ls_nsing, sizeof(int), hipMemcpyDeviceToHost,
-                             ctx->stream)) ||
-      !dev_ok(hipStreamSynchronize(ctx->stream)))
-    return MVD_DEVICE_ERROR;
-  ctx->ls_ready = nsing == 0;
-  return nsing;
+  return ls_setup(ctx, gamma, J, false);
 }
 
 int mvd_chem_lsetup_matrix(mvd_context *ctx, const double *A) {
   if (!ctx || !A) return MVD_BAD_ARGUMENT;
   if (!ctx->chem.ready) return MVD_NOT_READY;
-  const long n = ctx->chem.n;
-  if (!ctx->ls_lu) {
-    if (!dev_ok(hipMalloc(&ctx->ls_lu, sizeof(double) * 100 * ((n + 63) / 64 * 64))) ||
-        !dev_ok(hipMalloc(&ctx->ls_piv, sizeof(unsigned long long) * n)) ||
-        !dev_ok(hipMalloc(&ctx->ls_nsing, sizeof(int))))
-      return MVD_DEVICE_ERROR;
-  }
-  ctx->ls_ready = false;
-  if (mvd::chem_ls_setup(n, 0.0, A, ctx->ls_lu, ctx->ls_piv, ctx->ls_nsing, ctx->stream, true))
-    return MVD_DEVICE_ERROR;
-  int nsing = 0;
-  if (!dev_ok(hipMemcpyAsync(&nsing, ctx->ls_nsing, sizeof(int), hipMemcpyDeviceToHost,
-                             ctx->stream)) ||
-      !dev_ok(hipStreamSynchronize(ctx->stream)))
-    return MVD_DEVICE_ERROR;
-  ctx->ls_ready = nsing == 0;
-  return nsing;
+  return ls_setup(ctx, 0.0, A, true);
 }
 
 int mvd_chem_lsolve(mvd_context *ctx, const double *b, double *x) {
   if (!ctx || !b || !x) return MVD_BAD_ARGUMENT;
-  if (!ctx->ls_ready) return MVD_NOT_READY;
+  if (!ctx->ls_ready || ctx->ls_ready != ctx->chem.n) return MVD_NOT_READY;
   if (mvd::chem_ls_solve(ctx->chem.n, ctx->ls_lu, ctx->ls_piv, b, x, ctx->stream) ||
       !dev_ok(hipStreamSynchronize(ctx->stream)))
     return MVD_DEVICE_ERROR;
