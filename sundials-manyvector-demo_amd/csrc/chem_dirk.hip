@@ -517,7 +517,9 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
   // its cells (dirk_wave_words): the constants read at every RHS evaluation, loaded from HBM
   // once per cell, and the stage derivatives and step start read at stage changes.
   __shared__ int bs[NSTAT];
-  extern __shared__ double lds[];
+  // (16-byte accesses: the rate pairs of MEM_RATES, whose rows lie at multiples of 64 doubles)
+  extern __shared__ __attribute__((aligned(16))) double lds[];
+  static_assert(4 * TLEN % 64 == 0 && sizeof(double2) == 16, "rate pairs at 16-byte addresses");
   if (threadIdx.x < NSTAT) bs[threadIdx.x] = 0;
   // the wide tables' matrix, for a stage index held per lane
   __shared__ double tabA[WIDE ? MAXSTAGE * MAXSTAGE : 1];
