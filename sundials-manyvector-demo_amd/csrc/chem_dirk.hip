@@ -1263,8 +1263,9 @@ struct BatchedPlan {
   size_t bytes() const { return b_rows + b_ord + b_cnt + b_key + b_tdt + b_fst; }
 };
 
+// max_rows: the most blocks (statistics rows) the caller has room for (0: any number).
 static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, bool forced,
-                        int nsteps, BatchedPlan &p) {
+                        int nsteps, BatchedPlan &p, long max_rows = 0) {
   if (n <= 0 || n > (1L << 30)) return -1;
   if (block != 64 && block != 128 && block != 256) return -1;
   if (o.nstage < 1 || o.nstage > MAXSTAGE) return -1;
@@ -1313,6 +1314,9 @@ static int batched_plan(long n, const DirkDev &o, int grid_waves, int block, boo
   if (p.chunk < 32) p.chunk = 32;
   if (p.mem != MEM_SHARED && full == spread && full < want)
     p.chunk = nsteps == 1 && n <= 32 * 64 ? 32 : 64;
+  // full waves where spreading the cells would take more blocks than there are rows for
+  if (max_rows && std::min<long>(want, (n + p.chunk - 1) / p.chunk) > max_rows * p.wpb)
+    p.chunk = 64;
   const long chunks = (n + p.chunk - 1) / p.chunk;
   const long waves = want < chunks ? want : chunks;
   p.grid = (waves + p.wpb - 1) / p.wpb;
@@ -1422,7 +1426,7 @@ int dirk_batched_launch_noalloc(ChemState &s, const DirkDev &o, double h, double
   if (s.n > NOALLOC_MAX_CELLS) return MVD_BAD_ARGUMENT;
   if (dirk_wide(o.nstage, o.esdirk != 0)) return MVD_UNSUPPORTED;   // no room for its stage buffer
   BatchedPlan p;
-  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, 1, p)) return -1;
+  if (batched_plan(s.n, o, grid_waves, block, force != nullptr, 1, p, NOALLOC_MAX_ROWS)) return -1;
   if (p.nrow > NOALLOC_MAX_ROWS || p.bytes() > NOALLOC_WORK) return MVD_BAD_ARGUMENT;
   unsigned char *base = dirk_noalloc_scratch();
   if (!base) return -1;
