@@ -79,8 +79,11 @@ int erk_evolve(const Grid &g, FeScratch &fe, ErkState &e, const ErkTable &tab, d
   const long len = (5L + g.nchem) * ncell;
   const unsigned nb = (unsigned)((len + 255) / 256);
   if (!e.Y[0]) {
-    if (hipMalloc(&e.Y[0], sizeof(double) * len * (3 + ERK_MAXSTAGE)) != hipSuccess) return -1;
-    if (hipMalloc(&e.flag, sizeof(unsigned)) != hipSuccess) return -1;
+    if (hipMalloc(&e.Y[0], sizeof(double) * len * (3 + ERK_MAXSTAGE)) != hipSuccess ||
+        hipMalloc(&e.flag, sizeof(unsigned)) != hipSuccess) {
+      erk_free(e);                          // (all or nothing: the next call tries again)
+      return -1;
+    }
     e.Y[1] = e.Y[0] + len;
     e.Z = e.Y[1] + len;
     e.K = e.Z + len;

@@ -64,8 +64,11 @@ int imex_evolve(const Grid &g, FeScratch &fe, ChemState &ch, double eunit_inv, I
   if (!m.Y || m.S != S || m.len != len) {
     imex_free(m);
     // Yn | Z | R | Fe_0..Fe_{S-1} | Fi_0..Fi_{S-1} (chemistry only)
-    if (hipMalloc(&m.Y, sizeof(double) * (len * (3 + S) + nc * S)) != hipSuccess) return -1;
-    if (hipMalloc(&m.flag, 2 * sizeof(unsigned)) != hipSuccess) return -1;
+    if (hipMalloc(&m.Y, sizeof(double) * (len * (3 + S) + nc * S)) != hipSuccess ||
+        hipMalloc(&m.flag, 2 * sizeof(unsigned)) != hipSuccess) {
+      imex_free(m);                         // (all or nothing: the next call tries again)
+      return -1;
+    }
     m.nfail = (int *)(m.flag + 1);
     m.S = S;
     m.len = len;

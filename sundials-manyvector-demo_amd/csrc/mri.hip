@@ -135,12 +135,15 @@ int mri_evolve(const Grid &g, FeScratch &fe, ChemState &ch, double eunit_inv, Mr
   const long len = (5L + g.nchem) * n;
   if (!m.Y) {
     // Y | F_0 F_1 F_2 | R
-    if (hipMalloc(&m.Y, sizeof(double) * len * 5) != hipSuccess) return -1;
+    if (hipMalloc(&m.Y, sizeof(double) * len * 5) != hipSuccess ||
+        hipMalloc(&m.flag, 2 * sizeof(unsigned)) != hipSuccess ||
+        hipStreamCreateWithFlags(&m.cap, hipStreamNonBlocking) != hipSuccess) {
+      mri_free(m);                        // (all or nothing: the next call tries again)
+      return -1;
+    }
     m.F = m.Y + len;
     m.R = m.F + 3 * len;
-    if (hipMalloc(&m.flag, 2 * sizeof(unsigned)) != hipSuccess) return -1;
     m.nfail = (int *)(m.flag + 1);
-    if (hipStreamCreateWithFlags(&m.cap, hipStreamNonBlocking) != hipSuccess) return -1;
   }
   for (int q = 0; q < 5; q++)
     if (hipMemcpyAsync(m.Y + q * n, w[q], sizeof(double) * n, hipMemcpyDeviceToDevice, st) !=
