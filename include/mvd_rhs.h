@@ -113,7 +113,9 @@ int mvd_postprocess_step(mvd_context *ctx, double t, double *const *w);
  * and enables; mvd_profile_read returns the number of slots and fills per-slot total
  * milliseconds and launch counts. Slots: 0, 1 unused (kept so that the numbering stays),
  * 2 the z-face kernels (fluid, then tracers when nchem > 0), 3 fe_plain_faces,
- * 4 fe_plain_div, 5 fe_xyface_div (the x- and y-faces for every nchem). */
+ * 4 fe_plain_div, 5 fe_xyface_div (the x- and y-faces for every nchem), 6 fe_box (all of fe()
+ * on small grids). The kernels timed are those that run without it; with on = 2 fe() takes the
+ * kernels of slots 2 and 5 on small grids too (results equal to rounding). */
 int mvd_profile(mvd_context *ctx, int on);
 int mvd_profile_read(mvd_context *ctx, double *ms, long *count, int nslot);
 

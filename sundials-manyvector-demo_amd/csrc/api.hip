@@ -290,6 +290,7 @@ int mvd_profile(mvd_context *ctx, int on) {
     for (int i = 0; i < 2 * mvd::PROF_NSLOT; i++) (void)hipEventDestroy(t.ev[i]);
   }
   t.on = on != 0;
+  t.faces = on == 2;
   for (int s = 0; s < mvd::PROF_NSLOT; s++) { t.ms[s] = 0.0; t.count[s] = 0; t.pending[s] = false; }
   return MVD_SUCCESS;
 }

@@ -953,9 +953,11 @@ static int launch_fe(const Grid &g, const Fields &f, const FieldsOut &o, FeScrat
   unsigned *const flag = accum ? accum : s.flag;
   if (!accum) clear_flag(s, st);
   KernelTimer &tm = s.timer;
-  if constexpr (NC > 0) if (!plain && !tm.on && fe_boxes(g) <= FE_BOX_TRACER_MAX) {
+  if constexpr (NC > 0) if (!plain && !(tm.on && tm.faces) && fe_boxes(g) <= FE_BOX_TRACER_MAX) {
+    tm.begin(PROF_FE_BOX, st);
     hipLaunchKernelGGL((fe_box<0, NC, ST, MODE>), dim3((unsigned)fe_boxes(g)), dim3(512), 0, st, g,
                        f, BoxStage{}, o, 1.0 / g.dx, 1.0 / g.dy, 1.0 / g.dz, flag, slow);
+    tm.end(PROF_FE_BOX, st);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   if constexpr (MODE == TR_PLAIN) if (plain) {
@@ -1027,9 +1029,12 @@ int fe_box_launch(const Grid &g, const Fields &y, const BoxStage &bs, const Fiel
 int fe_launch(const Grid &g, const Fields &f, const FieldsOut &o, FeScratch &s,
               hipStream_t st, bool plain, unsigned *accum) {
   if (fe_too_large(g)) return -2;
-  if (!plain && fe_box_fits(g) && !s.timer.on) {
+  if (!plain && fe_box_fits(g) && !(s.timer.on && s.timer.faces)) {
     if (!accum) clear_flag(s, st);
-    return fe_box_launch(g, f, BoxStage{}, o, st, accum ? accum : s.flag);
+    s.timer.begin(PROF_FE_BOX, st);
+    const int rc = fe_box_launch(g, f, BoxStage{}, o, st, accum ? accum : s.flag);
+    s.timer.end(PROF_FE_BOX, st);
+    return rc;
   }
   switch (g.nchem) {
     case 0: return launch_fe<0>(g, f, o, s, st, plain, accum);

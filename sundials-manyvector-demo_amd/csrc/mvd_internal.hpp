@@ -18,10 +18,11 @@ struct FieldsOut {
 // Kernel timing slots (HIP events recorded on the launch stream around each kernel).
 // (slots 0 and 1 are unused; the numbering is part of mvd_profile_read's interface)
 enum { PROF_UNUSED0 = 0, PROF_UNUSED1, PROF_ZFACE_DIV, PROF_PLAIN_FACES, PROF_PLAIN_DIV,
-       PROF_XYFACE_DIV, PROF_NSLOT };
+       PROF_XYFACE_DIV, PROF_FE_BOX, PROF_NSLOT };
 
 struct KernelTimer {
   bool on = false;
+  bool faces = false;        // while on: fe() by its face kernels on every grid (no fe_box)
   hipEvent_t ev[2 * PROF_NSLOT] = {};
   bool pending[PROF_NSLOT] = {};
   double ms[PROF_NSLOT] = {};

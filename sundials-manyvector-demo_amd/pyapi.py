@@ -448,7 +448,7 @@ class Context:
 
     # slots 0 and 1 are unused; slot 2 times the z-face kernels (fluid, then tracers)
     PROFILE_SLOTS = ("unused0", "unused1", "fe_zface_div", "fe_plain_faces", "fe_plain_div",
-                     "fe_xyface_div")
+                     "fe_xyface_div", "fe_box")
 
     def profile(self, on=True):
         _check("mvd_profile", lib().mvd_profile(self.h, 1 if on else 0))
