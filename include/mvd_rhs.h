@@ -55,7 +55,9 @@ int mvd_set_stream(mvd_context *ctx, void *stream);
 
 /* fEuler (utilities.cpp:17-253; ARKRhsFn signature euler3D.hpp:1480) with zero external
  * forcing: wdot = -div F(w). Returns MVD_ILLEGAL_STATE when any cell has rho, et or p <= 0
- * (mvd_last_state_flags gives the 1/2/4 bits). */
+ * (mvd_last_state_flags gives the 1/2/4 bits). The units must keep the squared sound speed above
+ * 3e-17 and the split fluxes (density times wave speed times velocity) below 1e19: beyond, the
+ * products of the WENO weights leave the range of a double (mvd_fe_plain has no such limits). */
 int mvd_fe(mvd_context *ctx, double t, const double *const *w, double *const *wdot);
 /* The same result from the plain one-thread-per-cell kernels with the reference's operation
  * order and no FMA contraction (the comparator; bitwise reproducible on the CPU). */

@@ -32,7 +32,7 @@ namespace {
 //   dQ = sum o_k dq_k - 2 sum (o_k / e_k) (q_k - Q) de_k,
 //   de_1 = 2 t1 dt1 + (39/32) c dc and so on.
 // One reciprocal (of the common denominator times e_1 e_2 e_3: seven factors, finite for
-// |beta| < 1e43); 77 operations. Returns Q.
+// |beta| < 1e43 and normal for eps > 1e-43); 77 operations. Returns Q.
 __device__ inline double weno5_adj(double f0, double f1, double f2, double f3, double f4,
                                    double epsb, double y, double (&x)[5]) {
   const double a = f1 - f0, b = f2 - f1, c = f3 - f2, d = f4 - f3;
@@ -374,7 +374,13 @@ __device__ inline void face_adjoint(const double *P, const int (&off)[6], double
     y4 = hci * (Sb + Tb);
     y3 = 0.5 * B0;
   }
-  const double eps04 = (16.0 * WENO_EPSB) * (cs * cs), eps13 = 4.0 * WENO_EPSB;
+  // The acoustic values are reconstructed times the power of two next to 1 / cs: the seven factors
+  // of size eps04 in weno5_adj's denominator stay of order 1e-5 each however small cs is (with
+  // eps in units of cs^2 their product underflows below cs = 3e-20). W0, W4 and sfx carry
+  // that factor until the end.
+  const int ecs = __builtin_amdgcn_frexp_exp(cs);
+  const double css = ldexp(cs, -ecs);
+  const double eps04 = (16.0 * WENO_EPSB) * (css * css), eps13 = 4.0 * WENO_EPSB;
   double W0 = 0.0, W1 = 0.0, W2 = 0.0, W3 = 0.0, W4 = 0.0;
   double sfx = 0.0, skx = 0.0, ub = 0.0, vb = 0.0, wb = 0.0;
   double X[5] = {y0, y1, y2, y3, y4};
@@ -393,7 +399,7 @@ __device__ inline void face_adjoint(const double *P, const int (&off)[6], double
       x[l] = q[Q_R * FS] * (un + al);
       D[l] = gmh * fma(du, du, fma(dv, dv, dw * dw));
       K[l] = fma(p, fma(gamma, un, tt), x[l] * D[l]);
-      f[l] = K[l] - fma(x[l], du, p);
+      f[l] = ldexp(K[l] - fma(x[l], du, p), -ecs);
     }
     {
       const double Q0 = weno5_adj(f[0], f[1], f[2], f[3], f[4], eps04, y0, Ab);
@@ -406,7 +412,7 @@ __device__ inline void face_adjoint(const double *P, const int (&off)[6], double
 #pragma unroll
     for (int l = 0; l < 5; l++) {
       const double *q = pt(l, o);
-      f[l] = K[l] + fma(x[l], q[Q_U * FS] - u, q[Q_P * FS]);
+      f[l] = ldexp(K[l] + fma(x[l], q[Q_U * FS] - u, q[Q_P * FS]), -ecs);
     }
     {
       double x4[5];
@@ -485,8 +491,9 @@ __device__ inline void face_adjoint(const double *P, const int (&off)[6], double
   // the Roe state: from the back-projection, then to the two points
   double csb;
   {
-    const double S = hci * (W4 + W0), T = hci * (W4 - W0), F0 = fma(0.5, W3, S);
-    csb = fma(ci, fma(ci, skx, -sfx), fma(igm * Fb[4], S, T * tb));
+    const double h04 = ldexp(hci, ecs), S = h04 * (W4 + W0), T = h04 * (W4 - W0);
+    const double F0 = fma(0.5, W3, S);
+    csb = fma(ci, fma(ci, skx, -ldexp(sfx, ecs)), fma(igm * Fb[4], S, T * tb));
     ub += fma(Fb[1], F0, Fb[4] * fma(u, F0, cs * T));
     vb += fma(Fb[2], F0, Fb[4] * fma(v, F0, 0.5 * W1));
     wb += fma(Fb[3], F0, Fb[4] * fma(w, F0, 0.5 * W2));

@@ -271,7 +271,8 @@ __device__ inline void weno5_sd(double f0, double f1, double f2, double f3, doub
 
 // The corrections of the f+ and f- reconstructions together, with a single reciprocal:
 //   q = S+ / den+ + S- / den-,   f+ + f- = f2+ + f2- + (2/3) q
-// (den+ den- is a product of eight (eps + beta) factors: finite for |beta| < 1e38).
+// (den+ den- is a product of eight (eps + beta) factors: finite for |beta| < 1e38, and normal for
+// eps > 1e-38, which holds the acoustic components, with their 12e-6 cs^2, to cs > 3e-17).
 // fp: f+ at points 0..4; fm: f- at points 5..1 (reversed).
 __device__ inline double weno5_q(const double (&fp)[5], const double (&fm)[5], double epsb) {
   double Sp, dp, Sm, dm;
