@@ -465,23 +465,8 @@ __device__ inline void chem_temperature(const ChemConst &c, const double (&y)[NS
   chem_temperature(c, gamma_tabs(c), y, Ts, dTs_ge);
 }
 
-// linear-in-log(T) interpolation of every rate table and its T derivative
-// (raja_primordial_network.cpp:1046-1245)
-__device__ inline void chem_rates(const ChemConst &c, double T, double (&k)[NRATE],
-                                  double (&dk)[NRATE]) {
-#pragma clang fp contract(on)
-  double Tdef;
-  const int b = chem_locate(c, chem_log(T), Tdef);
-  const double Tfactor = fast_rcp(T) * c.idbin;
-#pragma unroll
-  for (int r = 0; r < NRATE; r++) {
-    const double a0 = c.tab[r * TLEN + b], a1 = c.tab[r * TLEN + b + 1];
-    k[r] = a0 + Tdef * (a1 - a0);
-    dk[r] = (a1 - a0) * Tfactor;
-  }
-}
-
-// Rates and derivatives of tables [r0, r1) only.
+// Linear-in-log(T) interpolation of the rate tables [R0, R1) and their T derivatives
+// (raja_primordial_network.cpp:1046-1245).
 template <int R0, int R1>
 __device__ inline void chem_rates_range(const ChemConst &c, double T, double (&k)[NRATE],
                                         double (&dk)[NRATE]) {
@@ -828,11 +813,10 @@ __device__ constexpr signed char CHEM_STO[NSP - 1][NREACT] = {
 // of its expression (chem_energy_grad). `clamped`: T sits on a clamp bound, so it
 // does not depend on y.
 //
-// In two parts: chem_vjp_prepare forms what does not depend on vp (reaction rates and
-// their T-derivatives, the gas-energy row's tangents, the temperature path's dg/dT and
-// dg/dy), chem_vjp_apply contracts one cotangent with it; chem_vjp_row gives the row
-// vp = v e_r with the same arithmetic restricted to its nonzero terms (the exact Jacobian
-// one row at a time, for many cotangents at one state).
+// chem_vjp_kernel contracts one cotangent (chem_vjp_species, chem_energy_grad, chem_vjp_path).
+// For the exact Jacobian one row at a time, chem_vjp_prepare forms what the rows share (reaction
+// rates and their T-derivatives, the gas-energy row's tangents, the temperature path's dg/dT and
+// dg/dy) and chem_vjp_row gives the row of vp = v e_r from its nonzero terms.
 struct ChemVjpPre {
   double k[NREACT], dk[NREACT];   // reaction rates and T-derivatives (reaction order)
   double e9[NSP];                 // d f_9 / d y_s (H2_1, H_1, H_2, He_1..3, de); [9]: d/dT
@@ -926,23 +910,7 @@ __device__ inline void chem_vjp_species(const double (&k)[N], const double (&dk)
   }
 }
 
-__device__ inline void chem_vjp_apply(const ChemVjpPre &P, const double (&y)[NSP],
-                                      const double (&vp)[NSP], double (&yab)[NSP]) {
-#pragma clang fp contract(on)
-#pragma unroll
-  for (int s = 0; s < NSP; s++) yab[s] = 0.0;
-  double Tb = 0.0;
-  chem_vjp_species(P.k, P.dk, y, vp, yab, Tb);
-  // gas-energy row
-  constexpr int dirs[7] = {0, 2, 3, 5, 6, 7, 8};
-#pragma unroll
-  for (int q = 0; q < 7; q++) yab[dirs[q]] += vp[9] * P.e9[dirs[q]];
-  Tb += vp[9] * P.e9[NSP - 1];
-  chem_vjp_temperature(P, Tb, yab);
-}
-
-// chem_vjp_apply for vp = v e_r (row r of the Jacobian times v): the terms of the other
-// rows, all zero, are left out.
+// Row r of the Jacobian times v.
 __device__ inline void chem_vjp_row(const ChemVjpPre &P, const double (&y)[NSP], int r,
                                     double v, double (&row)[NSP]) {
 #pragma clang fp contract(on)
