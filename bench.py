@@ -302,7 +302,7 @@ def bench_fe_tracers(api, problems, torch, n, seed, reps):
 
 def bench_sod(api, problems, torch, cpu=True):
     """Config-1 Sod shock tube: 128x3x3 cells, Neumann, 2000 fixed steps of 1e-4 to t=0.2 with
-    Bogacki-Shampine 3 (mvd_erk_evolve, one captured step replayed); the oracle's ERK on one
+    Bogacki-Shampine 3 (mvd_erk_evolve, one launch per stage); the oracle's ERK on one
     host core for the same run, and the largest field-relative difference between the two."""
     sys.path.insert(0, os.path.join(ROOT, "tests"))
     import orc
@@ -310,7 +310,7 @@ def bench_sod(api, problems, torch, cpu=True):
     w0 = [np.ascontiguousarray(a, dtype=np.float64).reshape(-1) for a in problems.sod(nx)[:5]]
     ctx = api.Context(api.make_params(nx, 3, 3, 0, (1,) * 6))
     wd = [torch.from_numpy(a.copy()).to("cuda") for a in w0] + [None]
-    ctx.erk_evolve(wd, h, 10)                     # capture the step graph
+    ctx.erk_evolve(wd, h, 10)                     # (allocates its buffers)
     for q in range(5):
         wd[q].copy_(torch.from_numpy(w0[q]))
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

@@ -215,11 +215,12 @@ int mvd_chem_vjp(mvd_context *ctx, double t, const double *y, const double *v, d
                  double *ydot);
 /* Self-check of the device temperature solve (no counterpart in the reference; for tests
  * and diagnostics): the ten Newton steps of cvklu_calculate_temperature
- * (raja_primordial_network.cpp:908-1011) end early at the first bitwise repeat of the
- * iteration (a cycle of period <= 4, whose remaining steps are known). Runs the early form
- * and the full ten steps from the warm starts Ts0 ([cell]) for every cell of y (scaled,
- * [cell][10]) and stores the number of cells whose (T, dTs_ge) differ bitwise; the
- * per-cell chemistry state is not changed. */
+ * (raja_primordial_network.cpp:908-1011) end early, in the RHS and VJP calls and the
+ * adjoint's Jacobians (the implicit steps solve for the same root to a few ulp), at the
+ * first bitwise repeat of the iteration (a cycle of period <= 4, whose remaining steps are
+ * known). Runs the early form and the full ten steps from the warm starts Ts0 ([cell]) for
+ * every cell of y (scaled, [cell][10]) and stores the number of cells whose (T, dTs_ge) differ
+ * bitwise; the per-cell chemistry state is not changed. */
 int mvd_chem_temperature_check(mvd_context *ctx, const double *y, const double *Ts0,
                                long *mismatches);
 /* device pointers of per-cell chemistry state: 0 scale, 1 inv_scale, 2 Ts, 3 dTs_ge,
@@ -409,9 +410,12 @@ int mvd_chem_dirk_set_shape(mvd_context *ctx, int block, int waves);
  * three stages and 64 with four; for tables of more than four stages (and
  * explicit-first-stage tables, which this call does not see) 54, the stage derivatives
  * going to a device buffer of 80 * (nstage - 1) bytes per thread of the persistent grid
- * instead. Halves the block until it fits; 0 when not even one wave fits. (A launch of at
- * most two waves per CU keeps more in LDS, with blocks of as many waves: the forcing, the
- * stage derivatives and, at one wave per CU, the rate pairs of each cell's table bin.) */
+ * instead. Halves the block until it fits; 0 when not even one wave fits. This is the layout
+ * of launches of many waves only. Where the cells' 64-cell waves number at most one per CU, a
+ * wave also keeps the forcing, the rate pairs of each cell's table bin and, for the long
+ * tables, the stage derivatives in LDS; long tables keep forcing and stage derivatives there
+ * up to two waves per CU (in blocks of two waves: a requested block of 64 keeps to the
+ * layout above). Such launches may run with smaller blocks than this call says. */
 int mvd_chem_dirk_fit_block(int block, int nstage, long static_lds, long lds_limit);
 int mvd_chem_dirk_get_shape(mvd_context *ctx, int *block, int *waves);
 

@@ -615,7 +615,7 @@ chem_dirk_batched(long n, ChemConst cc, ChemPtrsD p, DirkDev o, double h, double
     // seven-stage steps 72.4 -> 19.7 ms; one multirate slow step of 32^3 cells 77.3 -> 31.6
     // ms; one SDIRK3 step of 64^3 cells 0.471 -> 0.382 ms (ordering pass included). With what
     // followed (DirkMem, loads issued together, the shorter temperature solve, the column-wise
-    // substitution): 10.8, 17.0 and 0.32 ms.
+    // substitution): 10.8, 16.9 and 0.33 ms.
     // (the substepping variants, which hold more state, solve it again: skipping there
     // costs registers that are worth more than the solve)
     bool setup = true, solved = !SUBSTEP && tdt != nullptr;

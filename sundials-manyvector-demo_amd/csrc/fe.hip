@@ -313,7 +313,7 @@ fe_zface_tracers(Grid g, Fields f, FieldsOut out, double idz, FeSlow slow) {
 // first loads are waited for, no point is loaded or converted twice within a segment, and
 // the last five rows and the last face's flux are carried over. A kernel that loaded 37
 // rows for 32 faces and then computed them issued 65% of the time; at 256^3 the z faces went
-// from 0.72 to 0.55 ms with this form (0.74 at four waves per SIMD, where it spills).
+// from 0.78 to 0.56 ms with this form (0.74 at four waves per SIMD, where it spills).
 constexpr int ZX = 16, ZC = 16, ZROWS = ZC + 5;
 __global__ void __launch_bounds__(256, 3)
 fe_zface_div_xy(Grid g, Fields f, FieldsOut out, double idz, int nseg, int len) {
@@ -414,9 +414,9 @@ fe_zface_div_xy(Grid g, Fields f, FieldsOut out, double idz, int nseg, int len) 
 // point fields were, one tracer per field; u, v and c stay, for the faces' split factors;
 // each thread forms its x- and y-face's tracer fluxes from LDS. The kernel is bound by its
 // FP64 instructions: 8 point fields and the y fluxes (40 KB) let four blocks share a CU, so
-// that four waves per SIMD hide the LDS and dependency latency (128 registers, 84% of the
-// issue rate). At 256^3: 0.92 ms, 1.26 before (three waves per SIMD, ten point fields, 786
-// FP64 instructions per face where there are now 557).
+// that four waves per SIMD hide the LDS and dependency latency (128 registers, vector
+// instructions issued in 81% of the cycles). At 256^3: 0.94 ms, 1.26 before (three waves per
+// SIMD, ten point fields, 786 FP64 instructions per face with its share of the staging; now 638).
 constexpr int XY_TX = 16, XY_TY = 15;
 constexpr int XY_PX = XY_TX + 6, XY_PY = XY_TY + 6;      // point window 22 x 21
 constexpr int XY_NP = XY_PX * XY_PY;
